@@ -342,10 +342,8 @@ std::unique_ptr<PbMatrix> pb_build_host(const cpp::MatrixCSR &c) {
   // entry e of the used range is colidx[e], e = rowptr[i] - rowptr[0] + k (MatrixCSR.cpp:135)
   if (static_cast<long>(ci.size()) < nnz) bad("CSR rowptr points past colidx");
   auto pb = std::unique_ptr<PbMatrix>(new PbMatrix());
-  pb->n = n;
-  pb->nbins = (n + kPbRows - 1) / kPbRows;
-  pb->nsb = (n + kPbCols - 1) / kPbCols;
-  const int nb = pb->nbins, ns = pb->nsb;
+  pb->set_widths(n);
+  const int nb = pb->nbins, rows = pb->rows;
   // pass 1: counts per bin (far; local groups) and per column (far).  The
   // local groups of a bin are formed in row order: an entry opens a new
   // group when the current one is full or its row is kPbLocalPad or more
@@ -354,12 +352,12 @@ std::unique_ptr<PbMatrix> pb_build_host(const cpp::MatrixCSR &c) {
       loccnt(static_cast<std::size_t>(nb) + 1, 0);
   int gfill = kPbLocalGroup, gbase = 0;  // the current bin's open group
   for (int r = 0; r < n; r++) {
-    const int b = r >> kPbShift;
-    if ((r & (kPbRows - 1)) == 0) gfill = kPbLocalGroup;  // a new bin
+    const int b = r / rows;
+    if (r % rows == 0) gfill = kPbLocalGroup;  // a new bin
     for (long e = rp[static_cast<std::size_t>(r)] - r0; e < rp[static_cast<std::size_t>(r) + 1] - r0; e++) {
       const int col = ci[static_cast<std::size_t>(e)] - c.get_f_col();
       if (col < 0 || col >= n) bad("CSR column index outside the matrix");
-      if ((col >> kPbShift) == b) {
+      if (col / rows == b) {
         if (gfill == kPbLocalGroup || r - gbase >= kPbLocalPad) {
           loccnt[static_cast<std::size_t>(b) + 1] += kPbLocalGroup;
           gfill = 0;
@@ -392,25 +390,25 @@ std::unique_ptr<PbMatrix> pb_build_host(const cpp::MatrixCSR &c) {
   int lslot = 0;   // next slot in the open group (kPbLocalGroup: none open)
   gfill = kPbLocalGroup;
   for (int r = 0; r < n; r++) {
-    const int b = r >> kPbShift;
-    if ((r & (kPbRows - 1)) == 0) {
+    const int b = r / rows;
+    if (r % rows == 0) {
       gfill = kPbLocalGroup;
       lnext = loccnt[static_cast<std::size_t>(b)];
     }
     for (long e = rp[static_cast<std::size_t>(r)] - r0; e < rp[static_cast<std::size_t>(r) + 1] - r0; e++) {
       const int col = ci[static_cast<std::size_t>(e)] - c.get_f_col();
-      if ((col >> kPbShift) == b) {
+      if (col / rows == b) {
         if (gfill == kPbLocalGroup || r - gbase >= kPbLocalPad) {
           lslot = static_cast<int>(lnext);
           lnext += kPbLocalGroup;
           gfill = 0;
           gbase = r;
-          lbase[static_cast<std::size_t>(lslot / kPbLocalGroup)] = static_cast<unsigned short>(r & (kPbRows - 1));
+          lbase[static_cast<std::size_t>(lslot / kPbLocalGroup)] = static_cast<unsigned short>(r % rows);
         }
         const std::size_t k = static_cast<std::size_t>(lslot + gfill);
         gfill++;
         loc_src_h[k] = static_cast<int>(e);
-        lkey[k] = static_cast<unsigned short>((col & (kPbRows - 1)) | ((r - gbase) << kPbShift));
+        lkey[k] = static_cast<unsigned short>((col % rows) | ((r - gbase) << kPbShift));
       } else {
         const int k = ccur[static_cast<std::size_t>(col)]++;
         csc_src[static_cast<std::size_t>(k)] = static_cast<int>(e);
@@ -423,19 +421,17 @@ std::unique_ptr<PbMatrix> pb_build_host(const cpp::MatrixCSR &c) {
   std::vector<unsigned short> frow(nf);
   for (std::size_t k = 0; k < nf; k++) {
     const int r = csc_row[k];
-    const int sl = bcur[static_cast<std::size_t>(r >> kPbShift)]++;
+    const int sl = bcur[static_cast<std::size_t>(r / rows)]++;
     slot_csc[k] = sl;
-    frow[static_cast<std::size_t>(sl)] = static_cast<unsigned short>(r & (kPbRows - 1));
+    frow[static_cast<std::size_t>(sl)] = static_cast<unsigned short>(r % rows);
   }
   // scatter order over superblocks of `cols` columns: superblocks in
   // order, within a superblock by (bin, column).  Per superblock, the runs
   // of entries bound for one bin, in bin order: entry o of a run lands in
   // slot o + delta, with delta the run's first slot minus its first entry.
   constexpr int kNoDelta = std::numeric_limits<int>::min();
-  auto scatter_side = [&](int cols, int &nsb_out, std::vector<int> &far_src, DevBuf &sp_d, DevBuf &fkey_d,
+  auto scatter_side = [&](int cols, int ns2, std::vector<int> &far_src, DevBuf &sp_d, DevBuf &fkey_d,
                           DevBuf &rp_d, DevBuf &rdelta_d, DevBuf &cbase_d, DevBuf &cp_d) {
-    const int ns2 = (n + cols - 1) / cols;
-    nsb_out = ns2;
     std::vector<int> spc(static_cast<std::size_t>(ns2) + 1, 0);
     for (int s2 = 0; s2 < ns2; s2++)
       spc[static_cast<std::size_t>(s2) + 1] =
@@ -448,7 +444,7 @@ std::unique_ptr<PbMatrix> pb_build_host(const cpp::MatrixCSR &c) {
     for (int s2 = 0; s2 < ns2; s2++) {
       const int k0 = spc[static_cast<std::size_t>(s2)], k1 = spc[static_cast<std::size_t>(s2) + 1];
       std::fill(cnt.begin(), cnt.end(), 0);
-      for (int k = k0; k < k1; k++) cnt[static_cast<std::size_t>(csc_row[static_cast<std::size_t>(k)] >> kPbShift) + 1]++;
+      for (int k = k0; k < k1; k++) cnt[static_cast<std::size_t>(csc_row[static_cast<std::size_t>(k)] / rows) + 1]++;
       // run index of each non-empty bin, and its slot delta (the run's
       // entries are consecutive in CSC order within the bin's slots)
       std::fill(run_of.begin(), run_of.end(), -1);
@@ -461,12 +457,12 @@ std::unique_ptr<PbMatrix> pb_build_host(const cpp::MatrixCSR &c) {
       rdelta.resize(rbase + static_cast<std::size_t>(nr), kNoDelta);
       erun.assign(static_cast<std::size_t>(k1 - k0), -1);
       for (int k = k0; k < k1; k++) {  // column order, so each bin's run stays in column order
-        const int b = csc_row[static_cast<std::size_t>(k)] >> kPbShift;
+        const int b = csc_row[static_cast<std::size_t>(k)] / rows;
         const int o = k0 + cnt[static_cast<std::size_t>(b)]++;
         const int r = run_of[static_cast<std::size_t>(b)];
         far_src[static_cast<std::size_t>(o)] = csc_src[static_cast<std::size_t>(k)];
-        const int col = (ci[static_cast<std::size_t>(csc_src[static_cast<std::size_t>(k)])] - c.get_f_col()) &
-                        (cols - 1);
+        const int col = (ci[static_cast<std::size_t>(csc_src[static_cast<std::size_t>(k)])] - c.get_f_col()) %
+                        cols;
         const bool starts = o - k0 == first[static_cast<std::size_t>(b)];
         fkey[static_cast<std::size_t>(o)] = static_cast<unsigned short>(col | (starts ? kPbRunStart : 0u));
         erun[static_cast<std::size_t>(o - k0)] = r;
@@ -502,11 +498,10 @@ std::unique_ptr<PbMatrix> pb_build_host(const cpp::MatrixCSR &c) {
     cbase_d.upload(cbase.data(), cbase.size() * sizeof(int));
     cp_d.upload(chp.data(), chp.size() * sizeof(int));
   };
-  int ns_check = 0;
-  scatter_side(kPbCols, ns_check, far_src_h, pb->sp, pb->fkey, pb->rp, pb->rdelta, pb->cbase, pb->cp);
-  if (ns_check != ns) bad("propagation-blocked layout: superblock count");
-  scatter_side(kPbColsWide, pb->nsb_w, far_src_w_h, pb->sp_w, pb->fkey_w, pb->rp_w, pb->rdelta_w, pb->cbase_w,
-               pb->cp_w);
+  scatter_side(pb->cols, pb->nsb, far_src_h, pb->sp, pb->fkey, pb->rp, pb->rdelta, pb->cbase, pb->cp);
+  if (pb->cols_w != pb->cols)
+    scatter_side(pb->cols_w, pb->nsb_w, far_src_w_h, pb->sp_w, pb->fkey_w, pb->rp_w, pb->rdelta_w, pb->cbase_w,
+                 pb->cp_w);
   pb->frow.upload(frow.data(), frow.size() * sizeof(unsigned short));
   pb->bp.upload(bincnt.data(), bincnt.size() * sizeof(int));
   pb->lp.upload(loccnt.data(), loccnt.size() * sizeof(int));
@@ -521,9 +516,10 @@ std::unique_ptr<PbMatrix> pb_build_host(const cpp::MatrixCSR &c) {
 }
 
 std::string pb_layout_compare(const PbMatrix &a, const PbMatrix &b) {
-  if (a.n != b.n || a.nbins != b.nbins || a.nsb != b.nsb || a.nsb_w != b.nsb_w || a.n_far != b.n_far ||
-      a.n_loc != b.n_loc)
+  if (a.n != b.n || a.nbins != b.nbins || a.nsb != b.nsb || a.nsb_w != b.nsb_w || a.rows != b.rows ||
+      a.cols != b.cols || a.cols_w != b.cols_w || a.n_far != b.n_far || a.n_loc != b.n_loc)
     return "sizes";
+  const bool wide = a.cols_w != a.cols;  // (else there is no separate wide order)
   auto dl = [](const DevBuf &d, std::size_t bytes) {
     std::vector<unsigned char> v(bytes);
     if (bytes) TBSLA_HIP_CHECK(hipMemcpy(v.data(), d.get(), bytes, hipMemcpyDeviceToHost));
@@ -542,22 +538,23 @@ std::string pb_layout_compare(const PbMatrix &a, const PbMatrix &b) {
     std::size_t bytes;
   };
   const std::size_t ra = last(a.rp, a.nsb), rb = last(b.rp, b.nsb), ca = last(a.cp, a.nsb), cb = last(b.cp, b.nsb);
-  const std::size_t raw = last(a.rp_w, a.nsb_w), rbw = last(b.rp_w, b.nsb_w);
-  const std::size_t caw = last(a.cp_w, a.nsb_w), cbw = last(b.cp_w, b.nsb_w);
+  const std::size_t raw = wide ? last(a.rp_w, a.nsb_w) : 0, rbw = wide ? last(b.rp_w, b.nsb_w) : 0;
+  const std::size_t caw = wide ? last(a.cp_w, a.nsb_w) : 0, cbw = wide ? last(b.cp_w, b.nsb_w) : 0;
   if (ra != rb || ca != cb || raw != rbw || caw != cbw) return "run or chunk counts";
-  const std::size_t ns1 = static_cast<std::size_t>(a.nsb) + 1, nw1 = static_cast<std::size_t>(a.nsb_w) + 1;
+  const std::size_t ns1 = static_cast<std::size_t>(a.nsb) + 1, nw1 = wide ? static_cast<std::size_t>(a.nsb_w) + 1 : 0;
+  const std::size_t nfw = wide ? nf : 0;
   const std::size_t nb1 = static_cast<std::size_t>(a.nbins) + 1;
   const Item items[] = {
       {"sp", a.sp, b.sp, ns1 * i4},           {"fkey", a.fkey, b.fkey, nf * u2},
       {"rp", a.rp, b.rp, ns1 * i4},           {"rdelta", a.rdelta, b.rdelta, ra * i4},
       {"cbase", a.cbase, b.cbase, ca * i4},   {"cp", a.cp, b.cp, ns1 * i4},
-      {"sp_w", a.sp_w, b.sp_w, nw1 * i4},     {"fkey_w", a.fkey_w, b.fkey_w, nf * u2},
+      {"sp_w", a.sp_w, b.sp_w, nw1 * i4},     {"fkey_w", a.fkey_w, b.fkey_w, nfw * u2},
       {"rp_w", a.rp_w, b.rp_w, nw1 * i4},     {"rdelta_w", a.rdelta_w, b.rdelta_w, raw * i4},
       {"cbase_w", a.cbase_w, b.cbase_w, caw * i4}, {"cp_w", a.cp_w, b.cp_w, nw1 * i4},
       {"frow", a.frow, b.frow, nf * u2},      {"bp", a.bp, b.bp, nb1 * i4},
       {"lp", a.lp, b.lp, nb1 * i4},           {"lkey", a.lkey, b.lkey, nl * u2},
       {"lbase", a.lbase, b.lbase, nl / kPbLocalGroup * u2},
-      {"far_src", a.far_src, b.far_src, nf * i4}, {"far_src_w", a.far_src_w, b.far_src_w, nf * i4},
+      {"far_src", a.far_src, b.far_src, nf * i4}, {"far_src_w", a.far_src_w, b.far_src_w, nfw * i4},
       {"loc_src", a.loc_src, b.loc_src, nl * i4}};
   for (const Item &it : items)
     if (dl(it.x, it.bytes) != dl(it.y, it.bytes)) return it.name;

@@ -25,6 +25,7 @@
 #include <tbsla/cpp/Matrix.hpp>
 #include <tbsla/cpp/MatrixCSR.hpp>
 
+#include <algorithm>
 #include <memory>
 #include <string>
 #include <mutex>
@@ -71,9 +72,9 @@ struct DeviceMatrix {
 };
 
 // Propagation-blocked layout of a square CSR matrix for PageRank.  Rows are
-// grouped in bins of kPbRows; an entry whose column lies in its row's bin is
-// "local", every other entry is "far".  Columns are grouped in superblocks of
-// kPbCols.
+// grouped in bins of `rows` (at most kPbRows); an entry whose column lies in
+// its row's bin is "local", every other entry is "far".  Columns are grouped
+// in superblocks of `cols` (at most kPbCols).
 //   far    stored twice over: in scatter order -- by (column superblock,
 //          row bin, column) -- with the column offset in the superblock, the
 //          value and the slot of its product (sp: superblock boundaries), and
@@ -95,8 +96,8 @@ constexpr int kPbColShift = 13;
 constexpr int kPbLocalGroup = 4;
 constexpr int kPbLocalPad = 7;  // the row field of a padding key (3 bits above the column)
 constexpr int kPbCols = 1 << kPbColShift;
-// the wide scatter order: superblocks of kPbColsWide columns, for the FP32
-// delta products of mixed runs (a 4-byte x slice of that width fills the
+// the wide scatter order: superblocks of at most kPbColsWide columns, for the
+// FP32 delta products of mixed runs (a 4-byte x slice of that width fills the
 // same 64 KB of LDS as an 8-byte slice of kPbCols)
 constexpr int kPbColShiftWide = 14;
 constexpr int kPbColsWide = 1 << kPbColShiftWide;
@@ -107,9 +108,38 @@ constexpr int kPbChunk = 64;
 static_assert(kPbShift + 3 <= 16, "local keys hold the column and a 3-bit row offset in 16 bits");
 static_assert(kPbCols <= 0x2000, "scatter keys hold the column in 13 bits");
 static_assert(kPbColsWide <= kPbRunStart, "wide scatter keys hold the column in 15 bits");
+// A gather (scatter) launch has one workgroup per bin (superblock), of which
+// the 256 CUs hold 512 (256) at a time.  The width is the smallest that
+// gives whole rounds of them: ceil(n / (slots * rounds)) with the fewest
+// rounds that keep it at or under the cap, in multiples of 64 so that a
+// bin's rows start on a cache line.  With the width fixed at the cap, graphs
+// under 2^21 nodes left most CUs idle and others ended in a nearly empty
+// round (16 entries a row, FP64 iteration: 2^16 nodes 52.1 -> 18.1 us, 2^18
+// 55.9 -> 26.6, 2^20 71.2 -> 52.7, 2^22 246 -> 238).  Under kPbMinWidth a
+// workgroup is shorter than its own start-up.
+constexpr int kPbGatherSlots = 512;
+constexpr int kPbScatterSlots = 256;
+constexpr int kPbMinWidth = 256;
+inline int pb_width(int n, int slots, int cap) {
+  const long per_round = static_cast<long>(slots) * cap;
+  const long blocks = std::max(1L, (n + per_round - 1) / per_round) * slots;
+  const long w = ((n + blocks - 1) / blocks + 63) / 64 * 64;
+  return static_cast<int>(std::min<long>(cap, std::max<long>(kPbMinWidth, w)));
+}
 
 struct PbMatrix {
   int n = 0, nbins = 0, nsb = 0;
+  int rows = 0, cols = 0, cols_w = 0;  // rows per bin, columns per superblock (narrow and wide order)
+  // sizes all of these from n
+  void set_widths(int n_) {
+    n = n_;
+    rows = pb_width(n, kPbGatherSlots, kPbRows);
+    cols = pb_width(n, kPbScatterSlots, kPbCols);
+    cols_w = pb_width(n, kPbScatterSlots, kPbColsWide);
+    nbins = (n + rows - 1) / rows;
+    nsb = (n + cols - 1) / cols;
+    nsb_w = (n + cols_w - 1) / cols_w;
+  }
   long n_far = 0, n_loc = 0;  // n_loc counts the padding entries too
   // far entries in scatter order: fkey (16 bits) = column within the
   // superblock, | kPbRunStart on the first entry of a run. A run is the far
@@ -122,9 +152,10 @@ struct PbMatrix {
   // values by Dtype F64, F32, BF16 (built on demand); the far values in the
   // scatter order that reads them: F64 and F32 narrow, BF16 wide
   DevBuf fval[3], lval[3];
-  // The far entries in the wide scatter order (superblocks of kPbColsWide
+  // The far entries in the wide scatter order (superblocks of cols_w
   // columns, the same product slots), read by the delta products of BF16 and
-  // value-free mixed runs.
+  // value-free mixed runs.  Where cols_w == cols the narrow arrays serve
+  // both and these stay empty.
   int nsb_w = 0;
   DevBuf sp_w, fkey_w, rp_w, rdelta_w, cbase_w, cp_w;
   DevBuf prod;              // 8-byte product slots, n_far + kPbChunk (spare slots that

@@ -568,6 +568,7 @@ struct PbScatterArgs {
   const int *cbase;           // run of the first entry of each 64-entry chunk
   const int *cp;              // chunks of superblock s: [cp[s], cp[s+1])
   int nsb, n;
+  int cols;                   // columns per superblock
   long nfar;                  // product slots; kPbChunk spare slots follow them
 };
 
@@ -591,7 +592,7 @@ struct AnchorMove {
 // The far products of one superblock (picked from blockIdx): its slice of x
 // staged in xs (LDS), then every far product v * x[c] written to its slot.
 // With MOVE the slice is the anchor move's result instead of x.  COLS: the
-// superblock width of the layout `a` (kPbCols or kPbColsWide).
+// widest superblock of the layout `a` (kPbCols or kPbColsWide).
 template <typename VT, typename XT, typename AT, bool MOVE, int COLS>
 __device__ inline void pb_scatter_sb(const PbScatterArgs &a, const VT *__restrict__ val, const XT *__restrict__ x,
                                      AT *__restrict__ prod, XT *xs, const AnchorMove &am, double *red,
@@ -608,8 +609,8 @@ __device__ inline void pb_scatter_sb(const PbScatterArgs &a, const VT *__restric
   const int k0 = a.sp[sb], k1 = a.sp[sb + 1];
   const int *__restrict__ delta = a.rdelta + a.rp[sb];  // slot - entry of each run of this superblock
   const int *__restrict__ cbase = a.cbase + a.cp[sb];   // run of the first entry of each chunk
-  const long c0 = static_cast<long>(sb) * COLS;
-  const int nc = static_cast<int>(min(static_cast<long>(COLS), static_cast<long>(a.n) - c0));
+  const long c0 = static_cast<long>(sb) * a.cols;
+  const int nc = static_cast<int>(min(static_cast<long>(a.cols), static_cast<long>(a.n) - c0));
   {
     constexpr int S = COLS / kPbScatterThreads;  // x values per thread, all loads issued first
     XT t[S];
@@ -700,7 +701,7 @@ __device__ inline void pb_scatter_sb(const PbScatterArgs &a, const VT *__restric
       const int d = __shfl(g.dl[u], below + static_cast<int>((s1 >> lane) & 1ull), 64);
       // lanes past the end write a spare slot, so the store is unconditional
       const long o = e < nent ? static_cast<long>(k0 + e + d) : a.nfar + lane;
-      prod[o] = g.v[u] * static_cast<AT>(xs[g.key[u] & static_cast<unsigned>(COLS - 1)]);
+      prod[o] = g.v[u] * static_cast<AT>(xs[g.key[u] & (kPbRunStart - 1)]);
     }
   };
   // iteration it: the loads of stage it + 1 (its chunk runs were loaded in
@@ -755,10 +756,10 @@ constexpr bool pb_anchor_wide() {
 
 // Mixed runs, one launch per iteration: in an iteration that moves the
 // anchor, the anchor move and the FP64 anchor product's far products (values
-// VA, FP64, layout a of superblock width kPbColsWide for value-free anchors,
-// else kPbCols); otherwise the delta product's (values VD, delta XD, sums AD)
-// over layout ad of superblock width DCOLS (kPbColsWide: the 4-byte x slice
-// fills the LDS of a narrow FP64 slice).
+// VA, FP64, layout a: the wide order for value-free anchors, else the
+// narrow one); otherwise the delta product's (values VD, delta XD, sums AD)
+// over layout ad of superblocks up to DCOLS wide (kPbColsWide: the 4-byte x
+// slice fills the LDS of a narrow FP64 slice).
 template <typename VA, typename VD, typename XD, typename AD, int DCOLS>
 __global__ __launch_bounds__(kPbScatterThreads) void pb_scatter_mx(PbScatterArgs a, PbScatterArgs ad,
                                                                    const VA *__restrict__ vala,
@@ -783,7 +784,7 @@ __global__ __launch_bounds__(kPbScatterThreads) void pb_scatter_mx(PbScatterArgs
 struct PbView {
   const int *bp, *lp;
   const unsigned short *frow, *lkey, *lbase;
-  int n;
+  int n, rows;  // rows per bin
 };
 
 // Two products of type T in one vector load.
@@ -799,7 +800,7 @@ struct PbPair<double> {
 };
 
 // The row sums of one bin (blockIdx) into the FP64 LDS accumulator ybin
-// (kPbRows entries): the bin's far products and its local products, x read
+// (v.rows <= kPbRows entries): the bin's far products and its local products, x read
 // from the bin's own slice (XCS: x[j] scaled by xcs[j], the value-free anchor
 // product's input colscale .* xhat; else by xsc).  Ends with a barrier.
 template <typename VT, typename XT, typename AT, bool XCS = false>
@@ -808,8 +809,8 @@ __device__ inline void pb_accumulate(const PbView &v, const VT *__restrict__ lva
                                      const double *__restrict__ xcs = nullptr) {
 #pragma clang fp contract(off)
   const int bin = blockIdx.x, tid = threadIdx.x;
-  const int base = bin << kPbShift;
-  for (int i = tid; i < kPbRows; i += 1024) ybin[i] = 0.0;
+  const int base = bin * v.rows;
+  for (int i = tid; i < v.rows; i += 1024) ybin[i] = 0.0;
   __syncthreads();
   const int f1 = v.bp[bin + 1], l1 = v.lp[bin + 1];
   // far products in pairs: one 4-byte load of two rows and one 8- or
@@ -940,8 +941,8 @@ __global__ __launch_bounds__(1024) void pb_gather(PbView v, const VT *__restrict
   __shared__ double red[16];
   pb_accumulate<VT, XT, AT>(v, lval, x, prod, ybin, static_cast<XT>(st->raw ? st->xscale : 1.0));
   const int bin = blockIdx.x, tid = threadIdx.x;
-  const int base = bin << kPbShift;
-  const int rows = min(kPbRows, v.n - base);
+  const int base = bin * v.rows;
+  const int rows = min(v.rows, v.n - base);
   double lmax = -INFINITY;
   const double beta = st->beta, tele = st->tele;
   for (int i = tid; i < rows; i += 1024) {
@@ -980,8 +981,8 @@ __global__ __launch_bounds__(1024) void pb_gather_sn(PbView v, const VT *__restr
   __shared__ double red[48];
   pb_accumulate<VT, XT, AT>(v, lval, x, prod, ybin);
   const int bin = blockIdx.x, tid = threadIdx.x;
-  const int base = bin << kPbShift;
-  const int rows = min(kPbRows, v.n - base);
+  const int base = bin * v.rows;
+  const int rows = min(v.rows, v.n - base);
   const double beta = st->beta, tele = st->tele, inv = st->inv_sum;
   double err = 0.0;
   CSum cs{0, 0};
@@ -1040,8 +1041,8 @@ __global__ __launch_bounds__(1024) void pb_gather_mx(PbView v, const VA *__restr
   else
     pb_accumulate<VD, XD, AD>(v, lvald, xd, static_cast<const AD *>(prod), ybin);
   const int bin = blockIdx.x, tid = threadIdx.x;
-  const int base = bin << kPbShift;
-  const int rows = min(kPbRows, v.n - base);
+  const int base = bin * v.rows;
+  const int rows = min(v.rows, v.n - base);
   const double beta = st->beta, c = st->inv_sum;
   // the anchor iteration's teleport term and scale (kept by the finalize
   // pass of that iteration for the phase)
@@ -1081,13 +1082,13 @@ __global__ __launch_bounds__(1024) void pb_gather_mx(PbView v, const VA *__restr
 
 PbView pb_view(const PbMatrix &pb) {
   return PbView{pb.bp.as<int>(), pb.lp.as<int>(), pb.frow.as<unsigned short>(), pb.lkey.as<unsigned short>(),
-                pb.lbase.as<unsigned short>(), pb.n};
+                pb.lbase.as<unsigned short>(), pb.n, pb.rows};
 }
 
 PbScatterArgs pb_args(const PbMatrix &pb) {
   return PbScatterArgs{pb.sp.as<int>(),    pb.fkey.as<unsigned short>(), pb.rp.as<int>(), pb.rdelta.as<int>(),
                        pb.cbase.as<int>(), pb.cp.as<int>(),              pb.nsb,          pb.n,
-                       pb.n_far};
+                       pb.cols,            pb.n_far};
 }
 
 // The scatter order of the delta products with values VD (the far values of
@@ -1098,9 +1099,10 @@ constexpr bool pb_delta_wide() {
 }
 
 PbScatterArgs pb_args_wide(const PbMatrix &pb) {
+  if (pb.cols_w == pb.cols) return pb_args(pb);
   return PbScatterArgs{pb.sp_w.as<int>(),    pb.fkey_w.as<unsigned short>(), pb.rp_w.as<int>(), pb.rdelta_w.as<int>(),
                        pb.cbase_w.as<int>(), pb.cp_w.as<int>(),              pb.nsb_w,          pb.n,
-                       pb.n_far};
+                       pb.cols_w,            pb.n_far};
 }
 
 dim3 pb_scatter_grid(const PbMatrix &pb) { return dim3((pb.nsb + 7) / 8 * 8); }

@@ -50,14 +50,15 @@ __global__ __launch_bounds__(kT) void pbb_rows(const int *__restrict__ rowptr, i
 // far flag of every entry (its column outside its row's bin); err[0] for a
 // column outside [0, n)
 __global__ __launch_bounds__(kT) void pbb_far(const int *__restrict__ colidx, const int *__restrict__ row_of, long nnz,
-                                              int f_col, int n, int *__restrict__ far, int *__restrict__ err) {
+                                              int f_col, int n, int rows, int *__restrict__ far,
+                                              int *__restrict__ err) {
   for (long e = blockIdx.x * static_cast<long>(kT) + threadIdx.x; e < nnz; e += static_cast<long>(gridDim.x) * kT) {
     const int c = colidx[e] - f_col;
     if (c < 0 || c >= n) {
       err[0] = 1;
       far[e] = 0;
     } else {
-      far[e] = (c >> kPbShift) != (row_of[e] >> kPbShift) ? 1 : 0;
+      far[e] = c / rows != row_of[e] / rows ? 1 : 0;
     }
   }
 }
@@ -66,7 +67,7 @@ __global__ __launch_bounds__(kT) void pbb_far(const int *__restrict__ colidx, co
 // scan of the far flags); the local ones: row, column in the bin, entry
 __global__ __launch_bounds__(kT) void pbb_compact(const int *__restrict__ far, const int *__restrict__ fpos,
                                                   const int *__restrict__ colidx, const int *__restrict__ row_of,
-                                                  long nnz, int f_col, unsigned long long *__restrict__ fkey,
+                                                  long nnz, int f_col, int rows, unsigned long long *__restrict__ fkey,
                                                   int *__restrict__ fval, int *__restrict__ lrow,
                                                   int *__restrict__ lcol, int *__restrict__ le) {
   for (long e = blockIdx.x * static_cast<long>(kT) + threadIdx.x; e < nnz; e += static_cast<long>(gridDim.x) * kT) {
@@ -78,7 +79,7 @@ __global__ __launch_bounds__(kT) void pbb_compact(const int *__restrict__ far, c
     } else {
       const int li = static_cast<int>(e) - fpos[e];
       lrow[li] = row_of[e];
-      lcol[li] = c & (kPbRows - 1);
+      lcol[li] = c % rows;
       le[li] = static_cast<int>(e);
     }
   }
@@ -86,9 +87,10 @@ __global__ __launch_bounds__(kT) void pbb_compact(const int *__restrict__ far, c
 
 // key = bin of the entry's row, val = its CSC position
 __global__ __launch_bounds__(kT) void pbb_bin_keys(const int *__restrict__ csc_e, const int *__restrict__ row_of,
-                                                   long nf, unsigned long long *__restrict__ key, int *__restrict__ val) {
+                                                   long nf, int rows, unsigned long long *__restrict__ key,
+                                                   int *__restrict__ val) {
   for (long k = blockIdx.x * static_cast<long>(kT) + threadIdx.x; k < nf; k += static_cast<long>(gridDim.x) * kT) {
-    key[k] = static_cast<unsigned long long>(row_of[csc_e[k]] >> kPbShift);
+    key[k] = static_cast<unsigned long long>(row_of[csc_e[k]] / rows);
     val[k] = static_cast<int>(k);
   }
 }
@@ -114,23 +116,24 @@ __global__ __launch_bounds__(kT) void pbb_bounds(const unsigned long long *__res
 
 // slot s holds CSC position slot_list[s]: its inverse and the row in the bin
 __global__ __launch_bounds__(kT) void pbb_slots(const int *__restrict__ slot_list, const int *__restrict__ csc_e,
-                                                const int *__restrict__ row_of, long nf, int *__restrict__ slot_of,
+                                                const int *__restrict__ row_of, long nf, int rows,
+                                                int *__restrict__ slot_of,
                                                 unsigned short *__restrict__ frow) {
   for (long s = blockIdx.x * static_cast<long>(kT) + threadIdx.x; s < nf; s += static_cast<long>(gridDim.x) * kT) {
     const int k = slot_list[s];
     slot_of[k] = static_cast<int>(s);
-    frow[s] = static_cast<unsigned short>(row_of[csc_e[k]] & (kPbRows - 1));
+    frow[s] = static_cast<unsigned short>(row_of[csc_e[k]] % rows);
   }
 }
 
 // key = superblock << binbits | bin, val = CSC position
 __global__ __launch_bounds__(kT) void pbb_sc_keys(const unsigned long long *__restrict__ csc_col,
                                                   const int *__restrict__ csc_e, const int *__restrict__ row_of, long nf,
-                                                  int colshift, int binbits, unsigned long long *__restrict__ key,
+                                                  int cols, int rows, int binbits, unsigned long long *__restrict__ key,
                                                   int *__restrict__ val) {
   for (long k = blockIdx.x * static_cast<long>(kT) + threadIdx.x; k < nf; k += static_cast<long>(gridDim.x) * kT) {
-    const int sb = static_cast<int>(csc_col[k] >> colshift);
-    const int b = row_of[csc_e[k]] >> kPbShift;
+    const int sb = static_cast<int>(csc_col[k]) / cols;
+    const int b = row_of[csc_e[k]] / rows;
     key[k] = (static_cast<unsigned long long>(sb) << binbits) | static_cast<unsigned long long>(b);
     val[k] = static_cast<int>(k);
   }
@@ -148,7 +151,7 @@ __global__ __launch_bounds__(kT) void pbb_sc_entries(const unsigned long long *_
   for (long o = blockIdx.x * static_cast<long>(kT) + threadIdx.x; o < nf; o += static_cast<long>(gridDim.x) * kT) {
     const int k = sc[o];
     const bool st = o == 0 || key[o] != key[o - 1];
-    fkey[o] = static_cast<unsigned short>(static_cast<unsigned>(csc_col[k] & static_cast<unsigned long long>(cols - 1)) |
+    fkey[o] = static_cast<unsigned short>((static_cast<unsigned>(csc_col[k]) % static_cast<unsigned>(cols)) |
                                           (st ? kPbRunStart : 0u));
     far_src[o] = csc_e[k];
     start[o] = st ? 1 : 0;
@@ -192,10 +195,10 @@ __global__ __launch_bounds__(kT) void pbb_cbase(const unsigned long long *__rest
 
 // local entries [lbeg[b], lbeg[b + 1]) of bin b (in row order)
 __global__ __launch_bounds__(kT) void pbb_local_begin(const int *__restrict__ rowptr, int rp0,
-                                                      const int *__restrict__ fpos, long nnz, int n, int nb,
-                                                      int nloc, int *__restrict__ lbeg) {
+                                                      const int *__restrict__ fpos, long nnz, int n, int rows,
+                                                      int nb, int nloc, int *__restrict__ lbeg) {
   for (long b = blockIdx.x * static_cast<long>(kT) + threadIdx.x; b <= nb; b += static_cast<long>(gridDim.x) * kT) {
-    const long r = b << kPbShift;
+    const long r = b * rows;
     int v = nloc;
     if (r < n) {
       const long e = rowptr[r] - rp0;
@@ -248,17 +251,17 @@ __global__ __launch_bounds__(kT) void pbb_local_walk(const int *__restrict__ lbe
 // the group's first entry (padding slots keep their fill)
 __global__ __launch_bounds__(kT) void pbb_local_place(const int *__restrict__ rel, const int *__restrict__ lrow,
                                                       const int *__restrict__ lcol, const int *__restrict__ le,
-                                                      const int *__restrict__ lp, long nloc,
+                                                      const int *__restrict__ lp, long nloc, int rows,
                                                       unsigned short *__restrict__ lkey, unsigned short *__restrict__ lbase,
                                                       int *__restrict__ loc_src) {
   for (long li = blockIdx.x * static_cast<long>(kT) + threadIdx.x; li < nloc; li += static_cast<long>(gridDim.x) * kT) {
     const int r = lrow[li], q = rel[li];
     const int pos = q % kPbLocalGroup;
     const int base = lrow[li - pos];  // the group's first entry
-    const int k = lp[r >> kPbShift] + q;
+    const int k = lp[r / rows] + q;
     loc_src[k] = le[li];
     lkey[k] = static_cast<unsigned short>(lcol[li] | ((r - base) << kPbShift));
-    if (pos == 0) lbase[k / kPbLocalGroup] = static_cast<unsigned short>(base & (kPbRows - 1));
+    if (pos == 0) lbase[k / kPbLocalGroup] = static_cast<unsigned short>(base % rows);
   }
 }
 
@@ -315,14 +318,10 @@ std::vector<T> download(const DevBuf &b, std::size_t n) {
 
 // One scatter order (superblocks of `cols` columns) of the CSC-ordered far
 // entries: sp, fkey, rp, rdelta, cbase, cp and far_src.
-void scatter_order(int cols, int n, int nb, long nf, const DevBuf &csc_col, const DevBuf &csc_e, const DevBuf &row_of,
-                   const DevBuf &slot_of, int &nsb, DevBuf &sp_d, DevBuf &fkey_d, DevBuf &rp_d, DevBuf &rdelta_d,
+void scatter_order(int cols, int rows, int nb, long nf, const DevBuf &csc_col, const DevBuf &csc_e, const DevBuf &row_of,
+                   const DevBuf &slot_of, int ns, DevBuf &sp_d, DevBuf &fkey_d, DevBuf &rp_d, DevBuf &rdelta_d,
                    DevBuf &cbase_d, DevBuf &cp_d, DevBuf &far_src_d, DevBuf &err) {
   const hipStream_t s = nullptr;
-  int colshift = 0;
-  while ((1 << colshift) < cols) colshift++;
-  const int ns = (n + cols - 1) / cols;
-  nsb = ns;
   const int binbits = bits_for(nb - 1), sbbits = bits_for(ns - 1);
   DevBuf key, val, k2, v2, spb;
   spb.alloc(sizeof(int) * (static_cast<std::size_t>(ns) + 1));
@@ -335,7 +334,7 @@ void scatter_order(int cols, int n, int nb, long nf, const DevBuf &csc_col, cons
     k2.alloc(sizeof(unsigned long long) * static_cast<std::size_t>(nf));
     v2.alloc(sizeof(int) * static_cast<std::size_t>(nf));
     hipLaunchKernelGGL(pbb_sc_keys, dim3(blocks_for(nf)), dim3(kT), 0, s, csc_col.as<unsigned long long>(),
-                       csc_e.as<int>(), row_of.as<int>(), nf, colshift, binbits, key.as<unsigned long long>(),
+                       csc_e.as<int>(), row_of.as<int>(), nf, cols, rows, binbits, key.as<unsigned long long>(),
                        val.as<int>());
     radix_sort_pairs(key.as<unsigned long long>(), val.as<int>(), k2.as<unsigned long long>(), v2.as<int>(), nf,
                      binbits + sbbits, s);
@@ -398,10 +397,8 @@ std::unique_ptr<PbMatrix> pb_build_gpu(const DeviceMatrix &d, int n) {
   const long nnz = d.noop ? 0 : d.entries;  // no values: no entries (MatrixCSR.cpp:130-131)
   if (nnz >= (1L << 31)) bad("propagation-blocked layout limited to 2^31 entries");
   auto pb = std::unique_ptr<PbMatrix>(new PbMatrix());
-  pb->n = n;
-  pb->nbins = (n + kPbRows - 1) / kPbRows;
-  pb->nsb = (n + kPbCols - 1) / kPbCols;
-  const int nb = pb->nbins;
+  pb->set_widths(n);
+  const int nb = pb->nbins, rows = pb->rows;
   DevBuf err, row_of, far, fpos;
   err.alloc(4 * sizeof(int));
   const std::size_t e1 = static_cast<std::size_t>(std::max(1L, nnz));
@@ -412,7 +409,7 @@ std::unique_ptr<PbMatrix> pb_build_gpu(const DeviceMatrix &d, int n) {
   if (nnz > 0) {
     hipLaunchKernelGGL(pbb_rows, dim3(blocks_for(n)), dim3(kT), 0, s, d.rowptr.as<int>(), d.rp0, n, row_of.as<int>());
     hipLaunchKernelGGL(pbb_far, dim3(blocks_for(nnz)), dim3(kT), 0, s, d.colidx.as<int>(), row_of.as<int>(), nnz,
-                       d.f_col, n, far.as<int>(), err.as<int>());
+                       d.f_col, n, rows, far.as<int>(), err.as<int>());
     TBSLA_HIP_CHECK(hipMemcpyAsync(fpos.get(), far.get(), sizeof(int) * static_cast<std::size_t>(nnz),
                                    hipMemcpyDeviceToDevice, s));
     exclusive_scan(fpos.as<int>(), nnz, s);
@@ -430,7 +427,7 @@ std::unique_ptr<PbMatrix> pb_build_gpu(const DeviceMatrix &d, int n) {
   le.alloc(sizeof(int) * static_cast<std::size_t>(std::max(1L, nloc)));
   if (nnz > 0)
     hipLaunchKernelGGL(pbb_compact, dim3(blocks_for(nnz)), dim3(kT), 0, s, far.as<int>(), fpos.as<int>(),
-                       d.colidx.as<int>(), row_of.as<int>(), nnz, d.f_col, csc_col.as<unsigned long long>(),
+                       d.colidx.as<int>(), row_of.as<int>(), nnz, d.f_col, rows, csc_col.as<unsigned long long>(),
                        csc_e.as<int>(), lrow.as<int>(), lcol.as<int>(), le.as<int>());
   if (nf > 0) {
     k2.alloc(sizeof(unsigned long long) * static_cast<std::size_t>(nf));
@@ -446,14 +443,14 @@ std::unique_ptr<PbMatrix> pb_build_gpu(const DeviceMatrix &d, int n) {
   if (nf > 0) {
     bkey.alloc(sizeof(unsigned long long) * static_cast<std::size_t>(nf));
     slot_list.alloc(sizeof(int) * static_cast<std::size_t>(nf));
-    hipLaunchKernelGGL(pbb_bin_keys, dim3(blocks_for(nf)), dim3(kT), 0, s, csc_e.as<int>(), row_of.as<int>(), nf,
+    hipLaunchKernelGGL(pbb_bin_keys, dim3(blocks_for(nf)), dim3(kT), 0, s, csc_e.as<int>(), row_of.as<int>(), nf, rows,
                        bkey.as<unsigned long long>(), slot_list.as<int>());
     radix_sort_pairs(bkey.as<unsigned long long>(), slot_list.as<int>(), k2.as<unsigned long long>(), v2.as<int>(), nf,
                      bits_for(nb - 1), s);
     hipLaunchKernelGGL(pbb_bounds, dim3(blocks_for(nb + 1L)), dim3(kT), 0, s, bkey.as<unsigned long long>(), nf, nb, 0,
                        bpb.as<int>());
     hipLaunchKernelGGL(pbb_slots, dim3(blocks_for(nf)), dim3(kT), 0, s, slot_list.as<int>(), csc_e.as<int>(),
-                       row_of.as<int>(), nf, slot_of.as<int>(), pb->frow.as<unsigned short>());
+                       row_of.as<int>(), nf, rows, slot_of.as<int>(), pb->frow.as<unsigned short>());
   }
   if (nf > 0) {
     pb->bp = std::move(bpb);
@@ -465,13 +462,12 @@ std::unique_ptr<PbMatrix> pb_build_gpu(const DeviceMatrix &d, int n) {
   v2.release();
   bkey.release();
   slot_list.release();
-  // the two scatter orders
-  int ns_check = 0;
-  scatter_order(kPbCols, n, nb, nf, csc_col, csc_e, row_of, slot_of, ns_check, pb->sp, pb->fkey, pb->rp, pb->rdelta,
+  // the two scatter orders (one where both have the same width)
+  scatter_order(pb->cols, rows, nb, nf, csc_col, csc_e, row_of, slot_of, pb->nsb, pb->sp, pb->fkey, pb->rp, pb->rdelta,
                 pb->cbase, pb->cp, pb->far_src, err);
-  if (ns_check != pb->nsb) bad("propagation-blocked layout: superblock count");
-  scatter_order(kPbColsWide, n, nb, nf, csc_col, csc_e, row_of, slot_of, pb->nsb_w, pb->sp_w, pb->fkey_w, pb->rp_w,
-                pb->rdelta_w, pb->cbase_w, pb->cp_w, pb->far_src_w, err);
+  if (pb->cols_w != pb->cols)
+    scatter_order(pb->cols_w, rows, nb, nf, csc_col, csc_e, row_of, slot_of, pb->nsb_w, pb->sp_w, pb->fkey_w, pb->rp_w,
+                  pb->rdelta_w, pb->cbase_w, pb->cp_w, pb->far_src_w, err);
   if (read_int(err.as<int>() + 1)) bad("propagation-blocked layout: run slots are not consecutive");
   // local groups
   DevBuf lbeg, ngroups, rel;
@@ -480,7 +476,7 @@ std::unique_ptr<PbMatrix> pb_build_gpu(const DeviceMatrix &d, int n) {
   rel.alloc(sizeof(int) * static_cast<std::size_t>(std::max(1L, nloc)));
   if (nloc > 0) {
     hipLaunchKernelGGL(pbb_local_begin, dim3(blocks_for(nb + 1)), dim3(kT), 0, s, d.rowptr.as<int>(), d.rp0,
-                       fpos.as<int>(), nnz, n, nb, static_cast<int>(nloc), lbeg.as<int>());
+                       fpos.as<int>(), nnz, n, rows, nb, static_cast<int>(nloc), lbeg.as<int>());
     hipLaunchKernelGGL(pbb_local_walk, dim3((nb + kT / 64 - 1) / (kT / 64)), dim3(kT), 0, s, lbeg.as<int>(),
                        lrow.as<int>(), nb, rel.as<int>(), ngroups.as<int>());
   }
@@ -503,7 +499,7 @@ std::unique_ptr<PbMatrix> pb_build_gpu(const DeviceMatrix &d, int n) {
                        static_cast<unsigned short>(kPbLocalPad << kPbShift));
     hipLaunchKernelGGL(pbb_fill_i32, dim3(blocks_for(nl)), dim3(kT), 0, s, pb->loc_src.as<int>(), nl, -1);
     hipLaunchKernelGGL(pbb_local_place, dim3(blocks_for(nloc)), dim3(kT), 0, s, rel.as<int>(), lrow.as<int>(),
-                       lcol.as<int>(), le.as<int>(), pb->lp.as<int>(), nloc, pb->lkey.as<unsigned short>(),
+                       lcol.as<int>(), le.as<int>(), pb->lp.as<int>(), nloc, rows, pb->lkey.as<unsigned short>(),
                        pb->lbase.as<unsigned short>(), pb->loc_src.as<int>());
   }
   pb->prod.alloc(sizeof(double) * (static_cast<std::size_t>(nf) + kPbChunk));  // + spare slots
@@ -518,7 +514,7 @@ void pb_build_values(PbMatrix &pb, const DeviceMatrix &d, Dtype vdt) {
   const long nf = pb.n_far, nl = pb.n_loc;
   // far values in the scatter order that reads them: F64 (anchor and FP64
   // products) and F32 (delta products) narrow, BF16 (delta products) wide
-  const DevBuf &fsrc = vdt == Dtype::BF16 ? pb.far_src_w : pb.far_src;
+  const DevBuf &fsrc = vdt == Dtype::BF16 && pb.cols_w != pb.cols ? pb.far_src_w : pb.far_src;
   const std::size_t esz = vdt == Dtype::F64 ? 8 : (vdt == Dtype::F32 ? 4 : 2);
   pb.fval[slot].alloc(esz * static_cast<std::size_t>(std::max(1L, nf)));
   pb.lval[slot].alloc(esz * static_cast<std::size_t>(std::max(1L, nl)));
