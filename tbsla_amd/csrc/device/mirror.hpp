@@ -171,9 +171,12 @@ struct DeviceCache {
   std::unique_ptr<DeviceMatrix> transposed;
   std::unique_ptr<PbMatrix> pb;
   DevBuf x_stage, y_stage;
-  // count-stochastic CSR: the value of each column (fl(1/count)) in FP64 and
-  // FP32, 0 for a column with no entries (built by the PageRank engine)
-  DevBuf colscale64, colscale32;
+  // the value of each column of a CSR matrix whose stored entries agree
+  // within every column (fl(1/count) after fill_cqmat_stochastic), in FP64,
+  // in FP32, and rounded to BF16 (held in FP32); 0 for a column with no
+  // entries (found and built by the PageRank engine)
+  enum ColValues { kUnknown, kPerColumn, kDiffer } col_values = kUnknown;
+  DevBuf colscale64, colscale32, colscale_bf16;
 };
 
 // Build (or fetch) the mirror of `m` with values of type vdt.

@@ -506,8 +506,65 @@ __global__ __launch_bounds__(256) void scale_into_f32(const double *__restrict__
     z[i] = static_cast<float>(s[i] * v);
 }
 
+// bad[0] = 1 unless every stored value of column j has the bits of cs[j]
+// (colscale_kernel's: one of the column's stored values).
+__global__ __launch_bounds__(256) void colscale_check(const int *__restrict__ colidx, const double *__restrict__ vals,
+                                                      long nnz, int f_col, const double *__restrict__ cs,
+                                                      int *__restrict__ bad) {
+  if (*bad) return;  // (another block found one: nothing left to decide)
+  for (long k = blockIdx.x * 256L + threadIdx.x; k < nnz; k += static_cast<long>(gridDim.x) * 256)
+    if (__double_as_longlong(vals[k]) != __double_as_longlong(cs[static_cast<long>(colidx[k]) - f_col])) *bad = 1;
+}
+__global__ __launch_bounds__(256) void to_bf16_f32(const double *__restrict__ a, float *__restrict__ b, long n) {
+  for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += static_cast<long>(gridDim.x) * 256)
+    b[i] = dev::Val<dev::bf16>::cvt(dev::bf16_of(a[i]));
+}
+
 unsigned grid_for(long n, long cap = kNormBlocks) {
   return static_cast<unsigned>(std::max<long>(1, std::min<long>(cap, (n + 255) / 256)));
+}
+
+// Whether the stored entries of every column of an n-column CSR matrix hold
+// one value (true of fill_cqmat_stochastic's by construction, found from the
+// values otherwise).  If so the column values (0 for a column with no
+// entries) are in the matrix's device cache in FP64, FP32 and as BF16 rounds
+// them.  Decided once per matrix; x_need <= n has been checked.
+bool column_values(const cpp::Matrix &m, const DeviceMatrix &d64, long n, hipStream_t s) {
+  DeviceCache &cache = m.device_cache();
+  std::lock_guard<std::mutex> g(cache.mu);
+  if (cache.col_values != DeviceCache::kUnknown) return cache.col_values == DeviceCache::kPerColumn;
+  DevBuf c64, c32, cbf, bad;
+  c64.alloc(sizeof(double) * static_cast<std::size_t>(n));
+  const unsigned ge = grid_for(d64.entries, 16L * kNormBlocks), gn = grid_for(n);
+  hipLaunchKernelGGL(fill_f64, dim3(gn), dim3(256), 0, s, c64.as<double>(), n, 0.0);
+  int differs = 0;
+  if (d64.entries > 0) {
+    hipLaunchKernelGGL(colscale_kernel, dim3(ge), dim3(256), 0, s, d64.colidx.as<int>(), d64.vals.as<double>(),
+                       d64.entries, d64.f_col, n, c64.as<double>());
+    if (!m.count_stochastic()) {
+      bad.alloc(sizeof(double));
+      hipLaunchKernelGGL(fill_f64, dim3(1), dim3(256), 0, s, bad.as<double>(), 1L, 0.0);
+      hipLaunchKernelGGL(colscale_check, dim3(ge), dim3(256), 0, s, d64.colidx.as<int>(), d64.vals.as<double>(),
+                         d64.entries, d64.f_col, c64.as<double>(), bad.as<int>());
+      TBSLA_HIP_CHECK(hipMemcpyAsync(&differs, bad.get(), sizeof(int), hipMemcpyDeviceToHost, s));
+      TBSLA_HIP_CHECK(hipStreamSynchronize(s));
+    }
+  }
+  if (!differs) {
+    c32.alloc(sizeof(float) * static_cast<std::size_t>(n));
+    cbf.alloc(sizeof(float) * static_cast<std::size_t>(n));
+    hipLaunchKernelGGL(to_f32, dim3(gn), dim3(256), 0, s, c64.as<double>(), c32.as<float>(), n);
+    hipLaunchKernelGGL(to_bf16_f32, dim3(gn), dim3(256), 0, s, c64.as<double>(), cbf.as<float>(), n);
+  }
+  TBSLA_HIP_CHECK(hipGetLastError());
+  TBSLA_HIP_CHECK(hipStreamSynchronize(s));
+  if (!differs) {
+    cache.colscale64 = std::move(c64);
+    cache.colscale32 = std::move(c32);
+    cache.colscale_bf16 = std::move(cbf);
+  }
+  cache.col_values = differs ? DeviceCache::kDiffer : DeviceCache::kPerColumn;
+  return !differs;
 }
 
 // ---------------------------------------------------------------------------
@@ -592,11 +649,12 @@ struct AnchorMove {
 // The far products of one superblock (picked from blockIdx): its slice of x
 // staged in xs (LDS), then every far product v * x[c] written to its slot.
 // With MOVE the slice is the anchor move's result instead of x.  COLS: the
-// widest superblock of the layout `a` (kPbCols or kPbColsWide).
-template <typename VT, typename XT, typename AT, bool MOVE, int COLS>
+// widest superblock of the layout `a` (kPbCols or kPbColsWide).  xcs (value-
+// free FP64 products): the column values; the slice is xcs .* x.
+template <typename VT, typename XT, typename AT, bool MOVE, int COLS, bool XCS = false>
 __device__ inline void pb_scatter_sb(const PbScatterArgs &a, const VT *__restrict__ val, const XT *__restrict__ x,
                                      AT *__restrict__ prod, XT *xs, const AnchorMove &am, double *red,
-                                     XT xsc = XT(1)) {
+                                     XT xsc = XT(1), const XT *__restrict__ xcs = nullptr) {
 #pragma clang fp contract(off)
   // superblocks of one XCD (blockIdx % 8) are contiguous, so the runs that
   // share a cache line at a run boundary are written through the same L2
@@ -632,6 +690,7 @@ __device__ inline void pb_scatter_sb(const PbScatterArgs &a, const VT *__restric
         }
       } else {
         t[u] = i < nc ? static_cast<XT>(x[c0 + i] * xsc) : XT(0);
+        if (XCS && i < nc) t[u] *= xcs[c0 + i];
       }
     }
 #pragma unroll
@@ -730,22 +789,24 @@ __device__ inline void pb_scatter_sb(const PbScatterArgs &a, const VT *__restric
   if (it < nit) store(it, s0);
 }
 
-// FP64 runs: the far products of x.
-template <typename VT, typename XT, typename AT, int COLS>
-__global__ __launch_bounds__(kPbScatterThreads) void pb_scatter(PbScatterArgs a, const VT *__restrict__ val,
-                                                                const XT *__restrict__ x, AT *__restrict__ prod,
-                                                                const PrState *st) {
-  if (st->done) return;
-  __shared__ XT xs[COLS];
-  // (raw reference-rule runs: x is the unnormalised b, the iterate x * xscale)
-  pb_scatter_sb<VT, XT, AT, false, COLS>(a, val, x, prod, xs, AnchorMove{}, nullptr,
-                                         static_cast<XT>(st->raw ? st->xscale : 1.0));
-}
-
 template <typename VT>
 constexpr bool pb_value_free() {
   return std::is_same<VT, dev::Pattern>::value;
 }
+
+// FP64 runs: the far products of x (value-free: of cs .* x).
+template <typename VT, int COLS>
+__global__ __launch_bounds__(kPbScatterThreads) void pb_scatter(PbScatterArgs a, const VT *__restrict__ val,
+                                                                const double *__restrict__ cs,
+                                                                const double *__restrict__ x,
+                                                                double *__restrict__ prod, const PrState *st) {
+  if (st->done) return;
+  __shared__ double xs[COLS];
+  // (raw reference-rule runs: x is the unnormalised b, the iterate x * xscale)
+  pb_scatter_sb<VT, double, double, false, COLS, pb_value_free<VT>()>(a, val, x, prod, xs, AnchorMove{}, nullptr,
+                                                                      st->raw ? st->xscale : 1.0, cs);
+}
+
 // The value-free FP64 anchor product takes the wide scatter order (a 128 KB
 // x slice, runs of about 32 products), as the value-free FP64 runs do; with
 // FP64 values the narrow order was faster.
@@ -801,8 +862,8 @@ struct PbPair<double> {
 
 // The row sums of one bin (blockIdx) into the FP64 LDS accumulator ybin
 // (v.rows <= kPbRows entries): the bin's far products and its local products, x read
-// from the bin's own slice (XCS: x[j] scaled by xcs[j], the value-free anchor
-// product's input colscale .* xhat; else by xsc).  Ends with a barrier.
+// from the bin's own slice, scaled by xsc (XCS: and by xcs[j], the column
+// values of a value-free FP64 product).  Ends with a barrier.
 template <typename VT, typename XT, typename AT, bool XCS = false>
 __device__ inline void pb_accumulate(const PbView &v, const VT *__restrict__ lval, const XT *__restrict__ x,
                                      const AT *__restrict__ prod, double *ybin, XT xsc = XT(1),
@@ -907,7 +968,7 @@ __device__ inline void pb_accumulate(const PbView &v, const VT *__restrict__ lva
 #pragma unroll
       for (int u = 0; u < 4; u++) {
         const int j = base + c[g][u];
-        xv[g][u] = static_cast<AT>(XCS ? xcs[j] * x[j] : x[j] * xsc);
+        xv[g][u] = static_cast<AT>(XCS ? xcs[j] * (x[j] * xsc) : x[j] * xsc);
       }
 #pragma unroll
     for (int g = 0; g < LU; g++) {
@@ -931,15 +992,16 @@ __device__ inline void pb_accumulate(const PbView &v, const VT *__restrict__ lva
 
 // FP64 runs under the reference rule: b = beta*(A x) + t into out, block
 // max into the slots (normalised by a separate pass).
-template <typename VT, typename XT, typename AT, int TM>
-__global__ __launch_bounds__(1024) void pb_gather(PbView v, const VT *__restrict__ lval, const XT *__restrict__ x,
-                                                  const AT *__restrict__ prod, Teleport tp, double *__restrict__ out,
-                                                  PrState *st, unsigned long long *slots) {
+template <typename VT, int TM>
+__global__ __launch_bounds__(1024) void pb_gather(PbView v, const VT *__restrict__ lval, const double *__restrict__ cs,
+                                                  const double *__restrict__ x, const double *__restrict__ prod,
+                                                  Teleport tp, double *__restrict__ out, PrState *st,
+                                                  unsigned long long *slots) {
 #pragma clang fp contract(off)
   if (st->done) return;
-  __shared__ double ybin[kPbRows];  // FP64 sums (products may be FP32)
+  __shared__ double ybin[kPbRows];
   __shared__ double red[16];
-  pb_accumulate<VT, XT, AT>(v, lval, x, prod, ybin, static_cast<XT>(st->raw ? st->xscale : 1.0));
+  pb_accumulate<VT, double, double, pb_value_free<VT>()>(v, lval, x, prod, ybin, st->raw ? st->xscale : 1.0, cs);
   const int bin = blockIdx.x, tid = threadIdx.x;
   const int base = bin * v.rows;
   const int rows = min(v.rows, v.n - base);
@@ -966,20 +1028,19 @@ __global__ __launch_bounds__(1024) void pb_gather(PbView v, const VT *__restrict
 // pass: x' = (beta*(A x) + t) * inv_sum, where inv_sum = 1 / sum(x) (the
 // sum-normalised iterate does not depend on the scale, so the scale of the
 // last iterate serves), with sum|x' - x| and the compensated sum of x' as
-// per-bin partials.  PAT: also z' = colscale .* x' for the next value-free
-// product (x is then the product's input z, xprev the iterate).
-template <typename VT, typename XT, typename AT, int TM, bool PAT>
-__global__ __launch_bounds__(1024) void pb_gather_sn(PbView v, const VT *__restrict__ lval, const XT *__restrict__ x,
-                                                     const AT *__restrict__ prod, Teleport tp,
-                                                     const double *__restrict__ xprev, double *__restrict__ xout,
-                                                     double *__restrict__ zout, const double *__restrict__ colscale,
-                                                     const PrState *st, double *__restrict__ perr,
-                                                     double *__restrict__ ps, double *__restrict__ pc) {
+// per-bin partials.
+template <typename VT, int TM>
+__global__ __launch_bounds__(1024) void pb_gather_sn(PbView v, const VT *__restrict__ lval,
+                                                     const double *__restrict__ colscale,
+                                                     const double *__restrict__ x, const double *__restrict__ prod,
+                                                     Teleport tp, double *__restrict__ xout, const PrState *st,
+                                                     double *__restrict__ perr, double *__restrict__ ps,
+                                                     double *__restrict__ pc) {
 #pragma clang fp contract(off)
   if (st->done) return;
   __shared__ double ybin[kPbRows];
   __shared__ double red[48];
-  pb_accumulate<VT, XT, AT>(v, lval, x, prod, ybin);
+  pb_accumulate<VT, double, double, pb_value_free<VT>()>(v, lval, x, prod, ybin, 1.0, colscale);
   const int bin = blockIdx.x, tid = threadIdx.x;
   const int base = bin * v.rows;
   const int rows = min(v.rows, v.n - base);
@@ -990,8 +1051,7 @@ __global__ __launch_bounds__(1024) void pb_gather_sn(PbView v, const VT *__restr
     const int r = base + i;
     const double xn = add_teleport<TM>(beta * ybin[i], tele, tp, r) * inv;
     xout[r] = xn;
-    if (PAT) zout[r] = colscale[r] * xn;
-    err += fabs(xn - xprev[r]);
+    err += fabs(xn - x[r]);
     csum_add(cs, xn);
   }
   double e;
@@ -1117,42 +1177,18 @@ dim3 pb_scatter_grid_wide(const PbMatrix &pb) { return dim3((pb.nsb_w + 7) / 8 *
 // and FP32, the wide order measured slower).
 constexpr unsigned kPbScatterLdsPad = 24 * 1024;
 
-// The far products of one FP64-sum iteration (values VT, x of type XT):
-// value-free ones over the wide order, the others over the narrow one.
-template <typename VT, typename XT, typename AT>
-void launch_pb_scatter(const PbMatrix &pb, const VT *fval, const XT *x, AT *prod, const PrState *st, hipStream_t s) {
+// The far products of one FP64 iteration (values VT): value-free ones (cs:
+// the column values) over the wide order, the others over the narrow one.
+template <typename VT>
+void launch_pb_scatter(const PbMatrix &pb, const VT *fval, const double *cs, const double *x, double *prod,
+                       const PrState *st, hipStream_t s) {
   if (pb.n_far == 0) return;
-  if constexpr (std::is_same<VT, dev::Pattern>::value && sizeof(XT) == 8)
-    hipLaunchKernelGGL((pb_scatter<VT, XT, AT, kPbColsWide>), pb_scatter_grid_wide(pb), dim3(kPbScatterThreads), 0, s,
-                       pb_args_wide(pb), fval, x, prod, st);
+  if constexpr (pb_value_free<VT>())
+    hipLaunchKernelGGL((pb_scatter<VT, kPbColsWide>), pb_scatter_grid_wide(pb), dim3(kPbScatterThreads), 0, s,
+                       pb_args_wide(pb), fval, cs, x, prod, st);
   else
-    hipLaunchKernelGGL((pb_scatter<VT, XT, AT, kPbCols>), pb_scatter_grid(pb), dim3(kPbScatterThreads),
-                       kPbScatterLdsPad, s, pb_args(pb), fval, x, prod, st);
-}
-
-// One propagation-blocked product with the reference-rule update (FP64
-// runs): values of type VT from `pb` (dev::Pattern: value-free), x of type
-// XT, sums of type AT.
-template <typename VT, typename XT, typename AT, int TM>
-void launch_pb(const PbMatrix &pb, int vslot, const XT *x, const Teleport &tp, double *out, PrState *st,
-               unsigned long long *slots, hipStream_t s) {
-  const VT *fval = vslot >= 0 ? pb.fval[vslot].as<VT>() : nullptr;
-  const VT *lval = vslot >= 0 ? pb.lval[vslot].as<VT>() : nullptr;
-  AT *prod = pb.prod.as<AT>();
-  launch_pb_scatter<VT, XT, AT>(pb, fval, x, prod, st, s);
-  hipLaunchKernelGGL((pb_gather<VT, XT, AT, TM>), dim3(pb.nbins), dim3(1024), 0, s, pb_view(pb), lval, x, prod, tp,
-                     out, st, slots);
-}
-
-template <typename VT, typename XT, typename AT>
-void launch_pb_update(int tmode, const PbMatrix &pb, int vslot, const XT *x, const Teleport &tp, double *out,
-                      PrState *st, unsigned long long *slots, hipStream_t s) {
-  if (tmode == 1)
-    launch_pb<VT, XT, AT, 1>(pb, vslot, x, tp, out, st, slots, s);
-  else if (tmode == 2)
-    launch_pb<VT, XT, AT, 2>(pb, vslot, x, tp, out, st, slots, s);
-  else
-    launch_pb<VT, XT, AT, 0>(pb, vslot, x, tp, out, st, slots, s);
+    hipLaunchKernelGGL((pb_scatter<VT, kPbCols>), pb_scatter_grid(pb), dim3(kPbScatterThreads), kPbScatterLdsPad, s,
+                       pb_args(pb), fval, cs, x, prod, st);
 }
 
 // The per-bin partials of a sum-normalised iteration.
@@ -1160,31 +1196,41 @@ struct SnPartials {
   double *perr, *ps, *pc;
 };
 
-// One sum-normalised FP64 iteration (PAT: value-free over z): scatter and
-// gather; the finalize pass follows.
-template <typename VT, int TM, bool PAT>
-void launch_pb_sn_tm(const PbMatrix &pb, int vslot, const double *xin, const double *z, const Teleport &tp,
-                     double *xout, double *zout, const double *colscale, PrState *st, const SnPartials &sp,
-                     hipStream_t s) {
-  const VT *fval = vslot >= 0 ? pb.fval[vslot].as<VT>() : nullptr;
-  const VT *lval = vslot >= 0 ? pb.lval[vslot].as<VT>() : nullptr;
-  const double *x = PAT ? z : xin;
+// One FP64 iteration on the blocked products (values VT; dev::Pattern: value-
+// free, cs the column values): scatter and gather.  sp == nullptr: the
+// reference-rule update, block maxima into the slots; else the sum-normalised
+// one with its partials.  The finalize passes follow.
+template <typename VT, int TM>
+void launch_pb_tm(const PbMatrix &pb, const double *cs, const double *x, const Teleport &tp, double *out, PrState *st,
+                  unsigned long long *slots, const SnPartials *sp, hipStream_t s) {
+  constexpr int slot = static_cast<int>(Dtype::F64);
+  const VT *fval = pb_value_free<VT>() ? nullptr : pb.fval[slot].as<VT>();
+  const VT *lval = pb_value_free<VT>() ? nullptr : pb.lval[slot].as<VT>();
   double *prod = pb.prod.as<double>();
-  launch_pb_scatter<VT, double, double>(pb, fval, x, prod, st, s);
-  hipLaunchKernelGGL((pb_gather_sn<VT, double, double, TM, PAT>), dim3(pb.nbins), dim3(1024), 0, s, pb_view(pb), lval,
-                     x, prod, tp, xin, xout, zout, colscale, st, sp.perr, sp.ps, sp.pc);
+  launch_pb_scatter<VT>(pb, fval, cs, x, prod, st, s);
+  if (sp)
+    hipLaunchKernelGGL((pb_gather_sn<VT, TM>), dim3(pb.nbins), dim3(1024), 0, s, pb_view(pb), lval, cs, x, prod, tp,
+                       out, st, sp->perr, sp->ps, sp->pc);
+  else
+    hipLaunchKernelGGL((pb_gather<VT, TM>), dim3(pb.nbins), dim3(1024), 0, s, pb_view(pb), lval, cs, x, prod, tp, out,
+                       st, slots);
 }
 
-template <typename VT, bool PAT>
-void launch_pb_sn(int tmode, const PbMatrix &pb, int vslot, const double *xin, const double *z, const Teleport &tp,
-                  double *xout, double *zout, const double *colscale, PrState *st, const SnPartials &sp,
-                  hipStream_t s) {
-  if (tmode == 1)
-    launch_pb_sn_tm<VT, 1, PAT>(pb, vslot, xin, z, tp, xout, zout, colscale, st, sp, s);
-  else if (tmode == 2)
-    launch_pb_sn_tm<VT, 2, PAT>(pb, vslot, xin, z, tp, xout, zout, colscale, st, sp, s);
+void launch_pb(int tmode, const PbMatrix &pb, const double *cs, const double *x, const Teleport &tp, double *out,
+               PrState *st, unsigned long long *slots, const SnPartials *sp, hipStream_t s) {
+  const auto go = [&](auto tag) {
+    using VT = decltype(tag);
+    if (tmode == 1)
+      launch_pb_tm<VT, 1>(pb, cs, x, tp, out, st, slots, sp, s);
+    else if (tmode == 2)
+      launch_pb_tm<VT, 2>(pb, cs, x, tp, out, st, slots, sp, s);
+    else
+      launch_pb_tm<VT, 0>(pb, cs, x, tp, out, st, slots, sp, s);
+  };
+  if (cs)
+    go(dev::Pattern());
   else
-    launch_pb_sn_tm<VT, 0, PAT>(pb, vslot, xin, z, tp, xout, zout, colscale, st, sp, s);
+    go(double());
 }
 
 // Buffers of a mixed sum-normalised iteration.
@@ -1208,9 +1254,9 @@ void launch_pb_mx_tm(const PbMatrix &pb, int va, int vd, const MxBufs &b, const 
   const VD *fd = vd >= 0 ? pb.fval[vd].as<VD>() : nullptr;
   const VD *ld = vd >= 0 ? pb.lval[vd].as<VD>() : nullptr;
   const XD *xd = static_cast<const XD *>(b.xd);
-  // the delta products of BF16 and value-free runs take the wide scatter
-  // order, FP32-valued ones the narrow one (measured: value-free FP32 delta
-  // scatter 154 -> 140 us wide, BF16 196 -> 192, FP32 191 -> 196)
+  // the delta products of BF16-valued and value-free runs take the wide
+  // scatter order, FP32-valued ones the narrow one (measured: value-free FP32
+  // delta scatter 154 -> 140 us wide, BF16 196 -> 192, FP32 191 -> 196)
   constexpr bool wide = pb_delta_wide<VD>();
   // (a wide anchor's 128 KB slice leaves room for one block per CU without
   // the LDS pad)
@@ -1314,7 +1360,7 @@ struct Workspace {
 
 struct Scratch {
   WsBuf st, slots, perr, ps, pc, total, member, nodes, hsum, hcomp;
-  WsBuf X0, X1, Z, Z1, yhat, xhat, xhat32, D0, D1, ZD0, ZD1, W;
+  WsBuf X0, X1, Z, yhat, xhat, xhat32, D0, D1, ZD0, ZD1, W;
 };
 
 // zd = fl32(colscale32 * d) of a constant FP32 delta d
@@ -1425,6 +1471,7 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
   PageRankReport rep;
   if (n == 0) return rep;
   const bool pat32 = p.precision == PrPrecision::PATTERN_F32;
+  const bool pattern = p.precision == PrPrecision::PATTERN;
   const bool mixed = p.precision == PrPrecision::F32 || p.precision == PrPrecision::BF16 || pat32;
   const bool csr = m.format() == cpp::FORMAT_CSR;
   if ((mixed || p.precision == PrPrecision::PATTERN) && !csr)
@@ -1437,6 +1484,9 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
     throw std::invalid_argument("tbsla: explicit edge values need a CSR matrix and FP64 precision");
 
   const DeviceMatrix &d64 = mirror(m, Dtype::F64);
+  if (csr && !d64.noop && d64.rows != n)
+    throw std::invalid_argument("tbsla: CSR rowptr does not cover every row");
+  if (d64.x_need > n) throw std::invalid_argument("tbsla: column index beyond n_col");
   const bool fused = csr && !d64.noop && d64.rows == n;
   // propagation-blocked products: explicit choice, or by default on graphs
   // of 2^16 nodes and more, whatever the stopping rule (their row sums are
@@ -1444,21 +1494,23 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
   // products, whose sums are the reference's)
   const bool use_pb = fused && !p.values && (p.gather == 2 || (p.gather == 0 && n >= (1L << 16)));
   const PbMatrix *pbm = nullptr;
+  // Blocked products of a matrix whose stored entries agree within every
+  // column (a link graph: 1/out-degree) read no values: the input is scaled
+  // by the column's value once, which gives the same rounded products.  (On
+  // fill_cqmat_stochastic(2^24,2^24,8,0.5,7): FP64 iteration 696 -> 536 us,
+  // FP32 437 -> 385, BF16 436 -> 428.)
+  bool vfree = false;
   if (use_pb) {
-    const bool mixed_pat = mixed && m.count_stochastic();
-    pbm = &pb_mirror(m, (p.precision == PrPrecision::PATTERN || mixed_pat) ? Dtype::PATTERN : Dtype::F64);
-    if (p.precision == PrPrecision::F32) pbm = &pb_mirror(m, Dtype::F32);
-    if (p.precision == PrPrecision::BF16) pbm = &pb_mirror(m, Dtype::BF16);
+    vfree = column_values(m, d64, n, s);
+    pbm = &pb_mirror(m, vfree ? Dtype::PATTERN : Dtype::F64);
+    if (!vfree && p.precision == PrPrecision::F32) pbm = &pb_mirror(m, Dtype::F32);
+    if (!vfree && p.precision == PrPrecision::BF16) pbm = &pb_mirror(m, Dtype::BF16);
   }
   // the tile products of a mixed run read the values in the low precision
   // (the blocked ones read them from the blocked layout)
   const DeviceMatrix *dlo = nullptr;
   if (!use_pb && p.precision == PrPrecision::F32) dlo = &mirror(m, Dtype::F32);
   if (!use_pb && p.precision == PrPrecision::BF16) dlo = &mirror(m, Dtype::BF16);
-  if (csr && !d64.noop && d64.rows != n)
-    throw std::invalid_argument("tbsla: CSR rowptr does not cover every row");
-  if (d64.x_need > n) throw std::invalid_argument("tbsla: column index beyond n_col");
-
   Scratch w;
   Workspace ws{arena, cap, 0};
   const unsigned gN = grid_for(n);
@@ -1501,32 +1553,17 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
     ws.upload(w.member, mem.data(), mem.size(), s);
     tp.member = w.member.as<unsigned char>();
   }
-  const bool pattern = p.precision == PrPrecision::PATTERN;
-  // 1/count per column (the value every entry of column j holds after
-  // fill_cqmat_stochastic), computed from the FP64 mirror on the GPU once
-  // per matrix and kept in its device cache
+  // the column values of a value-free run (1/count per column after
+  // fill_cqmat_stochastic), and those of its deltas in FP32 (as rounded for
+  // the run's precision)
   const double *colscale64 = nullptr;
   const float *colscale32 = nullptr;
-  if (pattern || pat32 || (mixed && m.count_stochastic())) {
+  if (vfree || pattern || pat32 || (mixed && m.count_stochastic())) {
     if (arena) throw std::invalid_argument("tbsla: the allocation-free entry point runs FP64 only");
-    DeviceCache &cache = m.device_cache();
-    std::lock_guard<std::mutex> g(cache.mu);
-    if (!cache.colscale64.get()) {
-      DevBuf c64, c32;
-      c64.alloc(sizeof(double) * static_cast<std::size_t>(n));
-      c32.alloc(sizeof(float) * static_cast<std::size_t>(n));
-      hipLaunchKernelGGL(fill_f64, dim3(gN), dim3(256), 0, s, c64.as<double>(), n, 0.0);
-      if (d64.entries > 0)
-        hipLaunchKernelGGL(colscale_kernel, dim3(grid_for(d64.entries)), dim3(256), 0, s, d64.colidx.as<int>(),
-                           d64.vals.as<double>(), d64.entries, d64.f_col, n, c64.as<double>());
-      hipLaunchKernelGGL(to_f32, dim3(gN), dim3(256), 0, s, c64.as<double>(), c32.as<float>(), n);
-      TBSLA_HIP_CHECK(hipGetLastError());
-      TBSLA_HIP_CHECK(hipStreamSynchronize(s));
-      cache.colscale64 = std::move(c64);
-      cache.colscale32 = std::move(c32);
-    }
+    (void)column_values(m, d64, n, s);
+    const DeviceCache &cache = m.device_cache();
     colscale64 = cache.colscale64.as<double>();
-    colscale32 = cache.colscale32.as<float>();
+    colscale32 = p.precision == PrPrecision::BF16 ? cache.colscale_bf16.as<float>() : cache.colscale32.as<float>();
   }
   PrState h{};
   h.beta = p.beta;
@@ -1556,7 +1593,7 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
   // update's b unnormalised and carry its scale (1/max) to the readers of
   // the iterate, so the normalise pass writes nothing (a pass over the
   // iterate less per iteration)
-  h.raw = (fused && pbm && !sn && !mixed && !pattern) ? 1 : 0;
+  h.raw = (fused && pbm && !sn && !mixed) ? 1 : 0;
   h.xscale = 1.0;
   // mixed runs start from the anchor xhat = 0 (so yhat = A xhat = 0 with no
   // product) and delta = b0: the first phase carries the whole iterate in the
@@ -1606,8 +1643,10 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
       hipLaunchKernelGGL(fill_f64, dim3(gN), dim3(256), 0, s, w.yhat.as<double>(), n, 0.0);
     }
   }
+  // value-free deltas: the product's input zd = colscale32 .* delta
+  const bool zdelta = pat32 || (pb_mixed && vfree);
   float *ZD[2] = {nullptr, nullptr};
-  if (pat32) {
+  if (zdelta) {
     ws.alloc(w.ZD0, sizeof(float) * n);
     ws.alloc(w.ZD1, sizeof(float) * n);
     ZD[0] = w.ZD0.as<float>();
@@ -1619,18 +1658,10 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
       hipLaunchKernelGGL(scale_into_f32, dim3(gN), dim3(256), 0, s, colscale64, b0, ZD[0], n);
     hipLaunchKernelGGL(fill_f32, dim3(gN), dim3(256), 0, s, ZD[1], n, 0.0f);
   }
-  // (propagation-blocked mixed runs form z = colscale .* xhat where they
-  // read it)
-  if (pattern || (mixed && m.count_stochastic() && !pb_mixed)) {
+  // (propagation-blocked runs form z = colscale .* x where they read it)
+  if (!pbm && (pattern || (mixed && m.count_stochastic()))) {
     ws.alloc(w.Z, sizeof(double) * n);
     hipLaunchKernelGGL(scale_into, dim3(gN), dim3(256), 0, s, colscale64, X[0], w.Z.as<double>(), n);
-  }
-  // value-free FP64 sum-normalised runs write the next z beside the next
-  // iterate, so z alternates between two buffers like the iterate
-  double *ZP[2] = {w.Z.as<double>(), nullptr};
-  if (sn && pattern) {
-    ws.alloc(w.Z1, sizeof(double) * n);
-    ZP[1] = w.Z1.as<double>();
   }
   TBSLA_HIP_CHECK(hipGetLastError());
   // the set-up copies read pageable host memory (state, node set, 1/count)
@@ -1665,33 +1696,26 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
         const SnPartials sp{w.perr.as<double>(), w.ps.as<double>(), w.pc.as<double>()};
         if (mixed) {
           MxBufs b;
-          b.am = AnchorMove{w.xhat.as<double>(), w.xhat32.as<float>(), D[it & 1], mixed_pattern ? colscale : nullptr,
-                            w.hsum.as<double>(), w.hcomp.as<double>(), 0};
-          b.xd = pat32 ? static_cast<const void *>(ZD[it & 1]) : static_cast<const void *>(D[it & 1]);
+          b.am = AnchorMove{w.xhat.as<double>(), w.xhat32.as<float>(), D[it & 1], colscale, w.hsum.as<double>(),
+                            w.hcomp.as<double>(), 0};
+          b.xd = vfree ? static_cast<const void *>(ZD[it & 1]) : static_cast<const void *>(D[it & 1]);
           b.w = w.W.as<float>();
           b.dold = D[it & 1];
           b.dnew = D[(it + 1) & 1];
-          b.zdnew = pat32 ? ZD[(it + 1) & 1] : nullptr;
+          b.zdnew = vfree ? ZD[(it + 1) & 1] : nullptr;
           b.colscale32 = colscale32;
-          if (pat32)
+          if (vfree)
             launch_pb_mx<dev::Pattern, dev::Pattern, float, true>(tmode, *pbm, -1, -1, b, tp, st, sp, s);
-          else if (mixed_pattern && p.precision == PrPrecision::F32)
-            launch_pb_mx<dev::Pattern, float, float, false>(tmode, *pbm, -1, 1, b, tp, st, sp, s);
-          else if (mixed_pattern)
-            launch_pb_mx<dev::Pattern, dev::bf16, float, false>(tmode, *pbm, -1, 2, b, tp, st, sp, s);
           else if (p.precision == PrPrecision::F32)
             launch_pb_mx<double, float, float, false>(tmode, *pbm, 0, 1, b, tp, st, sp, s);
           else
             launch_pb_mx<double, dev::bf16, float, false>(tmode, *pbm, 0, 2, b, tp, st, sp, s);
-        } else if (pattern) {
-          launch_pb_sn<dev::Pattern, true>(tmode, *pbm, -1, xin, ZP[it & 1], tp, xout, ZP[(it + 1) & 1], colscale, st,
-                                           sp, s);
         } else {
-          launch_pb_sn<double, false>(tmode, *pbm, 0, xin, nullptr, tp, xout, nullptr, nullptr, st, sp, s);
+          launch_pb(tmode, *pbm, colscale, xin, tp, xout, st, nullptr, &sp, s);
         }
         // (the anchor move's sum partials: one per superblock of the anchor
         // product's scatter order)
-        const int nsb_anchor = (pat32 || mixed_pattern) ? pbm->nsb_w : pbm->nsb;
+        const int nsb_anchor = vfree ? pbm->nsb_w : pbm->nsb;
         hipLaunchKernelGGL(pr_finalize_sn, dim3(1), dim3(kTileThreads), 0, s, sp.perr, sp.ps, sp.pc, pbm->nbins,
                            mixed ? w.hsum.as<double>() : nullptr, mixed ? w.hcomp.as<double>() : nullptr, nsb_anchor,
                            st);
@@ -1726,30 +1750,26 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
                                nullptr, nullptr, nullptr, nullptr, n, st, w.perr.as<double>(), w.ps.as<double>(),
                                w.pc.as<double>());
           fin_norm(gM);
+        } else if (pbm) {
+          launch_pb(tmode, *pbm, colscale, xin, tp, xout, st, slots, nullptr, s);
+          fin_max();
+          hipLaunchKernelGGL(pr_normalize<4>, dim3(gN), dim3(kTileThreads), 0, s, xout, xin, nullptr, nullptr, nullptr,
+                             nullptr, nullptr, nullptr, nullptr, n, st, w.perr.as<double>(), w.ps.as<double>(),
+                             w.pc.as<double>());
+          fin_norm(gN);
         } else if (pattern) {
-          if (pbm)
-            launch_pb_update<dev::Pattern, double, double>(tmode, *pbm, -1, Z, tp, xout, st, slots, s);
-          else
-            launch_update<dev::Pattern, double, false>(tmode, d64, nullptr, Z, nullptr, tp, xout, st, slots, s);
+          launch_update<dev::Pattern, double, false>(tmode, d64, nullptr, Z, nullptr, tp, xout, st, slots, s);
           fin_max();
           hipLaunchKernelGGL(pr_normalize<2>, dim3(gN), dim3(kTileThreads), 0, s, xout, xin, nullptr, nullptr,
                              nullptr, Z, colscale, nullptr, nullptr, n, st, w.perr.as<double>(), w.ps.as<double>(),
                              w.pc.as<double>());
           fin_norm(gN);
         } else {
-          if (pbm)
-            launch_pb_update<double, double, double>(tmode, *pbm, 0, xin, tp, xout, st, slots, s);
-          else
-            launch_update<double, double, false>(tmode, d64, p.values, xin, nullptr, tp, xout, st, slots, s);
+          launch_update<double, double, false>(tmode, d64, p.values, xin, nullptr, tp, xout, st, slots, s);
           fin_max();
-          if (pbm)
-            hipLaunchKernelGGL(pr_normalize<4>, dim3(gN), dim3(kTileThreads), 0, s, xout, xin, nullptr, nullptr,
-                               nullptr, nullptr, nullptr, nullptr, nullptr, n, st, w.perr.as<double>(),
-                               w.ps.as<double>(), w.pc.as<double>());
-          else
-            hipLaunchKernelGGL(pr_normalize<0>, dim3(gN), dim3(kTileThreads), 0, s, xout, xin, nullptr, nullptr,
-                               nullptr, nullptr, nullptr, nullptr, nullptr, n, st, w.perr.as<double>(),
-                               w.ps.as<double>(), w.pc.as<double>());
+          hipLaunchKernelGGL(pr_normalize<0>, dim3(gN), dim3(kTileThreads), 0, s, xout, xin, nullptr, nullptr,
+                             nullptr, nullptr, nullptr, nullptr, nullptr, n, st, w.perr.as<double>(),
+                             w.ps.as<double>(), w.pc.as<double>());
           fin_norm(gN);
         }
       } else {

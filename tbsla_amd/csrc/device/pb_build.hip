@@ -24,6 +24,7 @@
 
 #include "mirror.hpp"
 #include "sort.hpp"
+#include "tile_csr.hpp"
 
 namespace tbsla {
 namespace hip {
@@ -273,13 +274,6 @@ __global__ __launch_bounds__(kT) void pbb_fill_i32(int *__restrict__ a, long n, 
 }
 
 // value of entry src[k] (0 for padding, src < 0) in the stored type
-__device__ inline unsigned short bf16_of(double d) {  // round to nearest even via FP32, as the host build
-  const float f = static_cast<float>(d);
-  unsigned u = __float_as_uint(f);
-  if ((u & 0x7f800000u) == 0x7f800000u) return static_cast<unsigned short>(u >> 16);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return static_cast<unsigned short>(u >> 16);
-}
 template <typename T>
 __device__ inline T conv(double d);
 template <>
@@ -292,7 +286,7 @@ __device__ inline float conv<float>(double d) {
 }
 template <>
 __device__ inline unsigned short conv<unsigned short>(double d) {
-  return bf16_of(d);
+  return dev::bf16_of(d);
 }
 template <typename T>
 __global__ __launch_bounds__(kT) void pbb_values(const double *__restrict__ vals, const int *__restrict__ src, long m,

@@ -25,6 +25,15 @@ struct bf16 {
   unsigned short bits;
 };
 
+// round to nearest even via FP32, as the CSR mirror's values
+__device__ inline unsigned short bf16_of(double d) {
+  const float f = static_cast<float>(d);
+  unsigned u = __float_as_uint(f);
+  if ((u & 0x7f800000u) == 0x7f800000u) return static_cast<unsigned short>(u >> 16);
+  u += 0x7fffu + ((u >> 16) & 1u);
+  return static_cast<unsigned short>(u >> 16);
+}
+
 typedef double v2d __attribute__((ext_vector_type(2)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef int v4i __attribute__((ext_vector_type(4)));
