@@ -64,16 +64,16 @@ struct SumRow {
   double acc;
   __device__ void operator()(int, double s) { acc += s; }
 };
-template <bool LONG>
+template <int TN, bool LONG>
 __global__ __launch_bounds__(kTileThreads) void adj_spmv_sum(dev::CsrView<double> m, const double *__restrict__ x,
                                                              double *__restrict__ part, int part_off) {
-  __shared__ dev::CsrTileLds<double> lds;
+  __shared__ dev::CsrTileLds<double, TN> lds;
   __shared__ double red[1][kTileThreads];
   SumRow epi{0.0};
-  if (LONG)
-    dev::csr_long_row<double, double>(m, x, lds, epi);
+  if constexpr (LONG)
+    dev::csr_long_row<double, double, TN>(m, x, lds, epi);
   else
-    dev::csr_tile_rows<double, double>(m, x, lds, epi);
+    dev::csr_tile_rows<double, double, TN>(m, x, lds, epi);
   double v[1] = {epi.acc};
   block_sums<1>(v, red);
   if (threadIdx.x == 0) part[part_off + blockIdx.x] = v[0];
@@ -145,7 +145,7 @@ struct AdjRow {
   }
 };
 
-template <typename VT, typename UT, bool LONG>
+template <typename VT, typename UT, int TN, bool LONG>
 __global__ __launch_bounds__(kTileThreads) void adj_update(dev::CsrView<VT> mT, const UT *__restrict__ u,
                                                            const double *__restrict__ w,
                                                            const double *__restrict__ lam,
@@ -154,15 +154,15 @@ __global__ __launch_bounds__(kTileThreads) void adj_update(dev::CsrView<VT> mT, 
                                                            double *__restrict__ part, int part_off) {
   if (st->done) return;
   using AT = typename dev::Val<VT>::A;
-  __shared__ dev::CsrTileLds<AT> lds;
+  __shared__ dev::CsrTileLds<AT, TN> lds;
   __shared__ double red[4][kTileThreads];
   const double beta = st->beta;
   const double vu = (st->c - st->a * st->sv) / st->s;
   AdjRow<AT> epi{w, lam, p, v, lam_new, beta, (1.0 - beta) * vu, st->inv_n, {0, 0, 0, 0}};
-  if (LONG)
-    dev::csr_long_row<VT, UT>(mT, u, lds, epi);
+  if constexpr (LONG)
+    dev::csr_long_row<VT, UT, TN>(mT, u, lds, epi);
   else
-    dev::csr_tile_rows<VT, UT>(mT, u, lds, epi);
+    dev::csr_tile_rows<VT, UT, TN>(mT, u, lds, epi);
   block_sums<4>(epi.q, red);
   if (threadIdx.x == 0)
     for (int k = 0; k < 4; k++) part[4 * (part_off + blockIdx.x) + k] = epi.q[k];
@@ -279,10 +279,12 @@ void run_adjoint(const DeviceMatrix &d64, const DeviceMatrix &dT, const AdjointP
   dev::CsrView<double> a = dev::csr_view<double>(d64);
   a.vals = src;
   if (d64.ntiles > 0)
-    hipLaunchKernelGGL(adj_spmv_sum<false>, dim3(d64.ntiles), dim3(kTileThreads), 0, s, a, pr, part_ap.as<double>(),
-                       0);
+    with_tile_size(d64, [&](auto tn) {
+      hipLaunchKernelGGL((adj_spmv_sum<decltype(tn)::value, false>), dim3(d64.ntiles), dim3(kTileThreads), 0, s, a, pr,
+                         part_ap.as<double>(), 0);
+    });
   if (d64.nlong > 0)
-    hipLaunchKernelGGL(adj_spmv_sum<true>, dim3(d64.nlong), dim3(kTileThreads), 0, s, a, pr, part_ap.as<double>(),
+    hipLaunchKernelGGL((adj_spmv_sum<kTileThreads, true>), dim3(d64.nlong), dim3(kTileThreads), 0, s, a, pr, part_ap.as<double>(),
                        d64.ntiles);
   hipLaunchKernelGGL(adj_sums, dim3(gN), dim3(kTileThreads), 0, s, pr, p.teleport, w, h.inv_n, n,
                      part4.as<double>());
@@ -306,10 +308,12 @@ void run_adjoint(const DeviceMatrix &d64, const DeviceMatrix &dT, const AdjointP
       double *lin = L[it & 1], *lout = L[(it + 1) & 1];
       hipLaunchKernelGGL((adj_prep<UT>), dim3(gN), dim3(256), 0, s, lin, U.as<UT>(), n, dst);
       if (dT.ntiles > 0)
-        hipLaunchKernelGGL((adj_update<VT, UT, false>), dim3(dT.ntiles), dim3(kTileThreads), 0, s, mt, U.as<UT>(), w,
-                           lin, lout, pr, p.teleport, dst, part.as<double>(), 0);
+        with_tile_size(dT, [&](auto tn) {
+          hipLaunchKernelGGL((adj_update<VT, UT, decltype(tn)::value, false>), dim3(dT.ntiles), dim3(kTileThreads), 0,
+                             s, mt, U.as<UT>(), w, lin, lout, pr, p.teleport, dst, part.as<double>(), 0);
+        });
       if (dT.nlong > 0)
-        hipLaunchKernelGGL((adj_update<VT, UT, true>), dim3(dT.nlong), dim3(kTileThreads), 0, s, mt, U.as<UT>(), w,
+        hipLaunchKernelGGL((adj_update<VT, UT, kTileThreads, true>), dim3(dT.nlong), dim3(kTileThreads), 0, s, mt, U.as<UT>(), w,
                            lin, lout, pr, p.teleport, dst, part.as<double>(), dT.ntiles);
       hipLaunchKernelGGL(adj_finalize, dim3(1), dim3(kTileThreads), 0, s, part.as<double>(), nparts, dst);
     }

@@ -77,6 +77,21 @@ MinMax minmax_offset(const int *a, std::size_t n, long off) {
   return out;
 }
 
+// Entries per tile.  A CU holds six workgroups with 3072-entry tiles (LDS) and
+// eight with smaller ones, so up to two rounds of them (9.4 M entries) 2048
+// fills the last round better (500,009 rows of 16: 30.8 -> 26.7 us; 300,007
+// of 12: 14.0 -> 13.1; 1,000,003 of 16, past the line: 51.8 against 53.9).  Up
+// to a tile of 1024 per workgroup slot's half, PageRank's updates are latency
+// alone and take the smallest (a row per thread, and the step decision merged
+// in).  A row that runs past its tile is finished by one thread from memory:
+// with rows over 256 entries the large tiles stay.
+int tile_size(long nnz, const int *rowptr, int rows) {
+  int longest = 0;
+  for (int i = 0; i < rows; i++) longest = std::max(longest, rowptr[i + 1] - rowptr[i]);
+  if (longest > 256 || nnz > 2L * 1536 * kCsrTileNnz) return kCsrTileNnz;
+  return nnz <= (1L << 20) ? 1024 : 2048;
+}
+
 [[noreturn]] void bad(const char *what) { throw std::invalid_argument(std::string("tbsla: ") + what); }
 
 void build_csr(DeviceMatrix &d, const cpp::MatrixCSR &m, Dtype vdt) {
@@ -105,7 +120,8 @@ void build_csr(DeviceMatrix &d, const cpp::MatrixCSR &m, Dtype vdt) {
   // entry j of row i is values[rowptr[i] - rowptr[0] + k] (MatrixCSR.cpp:135)
   d.colidx.upload(ci.data(), static_cast<std::size_t>(used) * sizeof(int));
   upload_values(d.vals, vals.data(), static_cast<std::size_t>(used), vdt);
-  std::vector<int> t = csr_entry_tiles(rp.data(), d.rows, kCsrTileNnz);
+  d.tile_nnz = tile_size(used, rp.data(), d.rows);
+  std::vector<int> t = csr_entry_tiles(rp.data(), d.rows, d.tile_nnz);
   d.ntiles = static_cast<int>(t.size()) - 1;
   d.tiles.upload(t.data(), t.size() * sizeof(int));
   std::vector<int> lr;
@@ -215,7 +231,8 @@ void build_coo_like(DeviceMatrix &d, const M &m, Dtype vdt, bool scoo) {
   d.segrow.upload(segrow.data(), segrow.size() * sizeof(int));
   d.colidx.upload(pcol, n * sizeof(int));
   upload_values(d.vals, pval, n, vdt);
-  std::vector<int> t = csr_entry_tiles(segptr.data(), d.nseg, kCsrTileNnz);
+  d.tile_nnz = tile_size(static_cast<long>(n), segptr.data(), d.nseg);
+  std::vector<int> t = csr_entry_tiles(segptr.data(), d.nseg, d.tile_nnz);
   d.ntiles = static_cast<int>(t.size()) - 1;
   d.tiles.upload(t.data(), t.size() * sizeof(int));
   std::vector<int> lr;
@@ -317,7 +334,8 @@ const DeviceMatrix &transpose_mirror(const cpp::Matrix &m) {
   d->rowptr.upload(ptr.data(), ptr.size() * sizeof(int));
   d->colidx.upload(ridx.data(), ridx.size() * sizeof(int));
   d->perm.upload(perm.data(), perm.size() * sizeof(int));
-  std::vector<int> t = csr_entry_tiles(ptr.data(), cols, kCsrTileNnz);
+  d->tile_nnz = tile_size(used, ptr.data(), cols);
+  std::vector<int> t = csr_entry_tiles(ptr.data(), cols, d->tile_nnz);
   d->ntiles = static_cast<int>(t.size()) - 1;
   d->tiles.upload(t.data(), t.size() * sizeof(int));
   std::vector<int> lr;

@@ -29,6 +29,7 @@
 #include <memory>
 #include <string>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "common.hpp"
@@ -54,6 +55,7 @@ struct DeviceMatrix {
   // CSR
   DevBuf rowptr, colidx, vals, tiles, long_rows;
   int ntiles = 0, nlong = 0, rp0 = 0;
+  int tile_nnz = kCsrTileNnz;  // entries per tile of the table in `tiles`
   // ELL (sliced column-major)
   int K = 0;
   DevBuf ecols, evals;
@@ -178,6 +180,17 @@ struct DeviceCache {
   enum ColValues { kUnknown, kPerColumn, kDiffer } col_values = kUnknown;
   DevBuf colscale64, colscale32, colscale_bf16;
 };
+
+// f(integral_constant<int, tile size>) for the tile size of d's table.
+template <typename F>
+inline void with_tile_size(const DeviceMatrix &d, F &&f) {
+  if (d.tile_nnz == 1024)
+    f(std::integral_constant<int, 1024>());
+  else if (d.tile_nnz == 2048)
+    f(std::integral_constant<int, 2048>());
+  else
+    f(std::integral_constant<int, kCsrTileNnz>());
+}
 
 // Build (or fetch) the mirror of `m` with values of type vdt.
 const DeviceMatrix &mirror(const cpp::Matrix &m, Dtype vdt);

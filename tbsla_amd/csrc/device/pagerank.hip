@@ -1,15 +1,19 @@
 // PageRank iteration kernels and their host driver (see pagerank.hpp).
 //
-// One iteration of the CSR engine is four launches (five with long rows):
-//   pr_update_csr     entry-tile SpMV of the current iterate fused with
-//                     b = beta*(A b_t) + tele and the block max of b, merged
-//                     into 64 atomic-max slots.
-//   pr_finalize_max   one wavefront: max over the slots into the state.
-//   pr_normalize      b /= max, the L1 residual against b_t and the
-//                     compensated sum of b, as per-block partials.
-//   pr_finalize_norm  one block: merges the partials and updates the state:
-//                     iteration count, convergence, the next teleport term,
-//                     and (mixed precision) whether to move the anchor.
+// One iteration of the CSR engine is two launches (three with long rows):
+//   pr_update_csr     first the step decision of the iteration before (every
+//                     block merges that normalise pass's partials, at most
+//                     256, and takes the same decision; block 0 stores it),
+//                     then the entry-tile SpMV of the current iterate fused
+//                     with b = beta*(A b_t) + tele and the block max of b,
+//                     merged into 64 atomic-max slots.
+//   pr_normalize      the max over the slots (every block), then b /= max, the
+//                     L1 residual against b_t and the compensated sum of b,
+//                     as per-block partials.
+// The step decision updates the state: iteration count, convergence, the next
+// teleport term, and (mixed precision) whether to move the anchor.  A launch
+// of its own (pr_finalize_norm) takes it at the end of a launch batch, before
+// the host reads the state.
 // Partial results cross workgroups only at kernel boundaries, so no kernel
 // needs a device-wide fence.
 // Every kernel returns at once when the state says the run has converged, so
@@ -52,12 +56,19 @@ struct PrState {
   // reference-rule runs with propagation-blocked products keep the update's
   // unnormalised b (raw = 1): the iterate is b * xscale, xscale = 1 / max of
   // the update that wrote it (1 for the start and in every other run)
-  double xscale;
+  // xnext: that scale as the normalise pass leaves it for the next products,
+  // before the step decision moves it to xscale
+  double xscale, xnext;
   int it, max_it, done, rule;
   int need_anchor, anchors, anchor_it, mixed, raw;
 };
 
 constexpr int kNormBlocks = 1024;
+// blocks of a normalise pass (1024 threads each): as many partials as the
+// first wavefront of the next kernel merges in one step of four loads a lane
+// (mixed runs, six streams instead of three: twice as many)
+constexpr int kPassBlocks = 256;
+constexpr int kMergeTileNnz = 1024;
 
 // Neumaier-compensated running sum and its exact-error merge (TwoSum).
 struct CSum {
@@ -94,19 +105,20 @@ __device__ inline double wave_sum(double v) {
 __device__ inline void block1024_err_csum(double err, CSum cs, double *red, double &err_out, CSum &cs_out) {
   err = wave_sum(err);
   cs = wave_csum(cs);
-  const int w = threadIdx.x >> 6;
-  if ((threadIdx.x & 63) == 0) {
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  if (lane == 0) {
     red[w] = err;
     red[16 + w] = cs.s;
     red[32 + w] = cs.c;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    err_out = 0;
-    cs_out = CSum{0, 0};
-    for (int i = 0; i < 16; i++) {
-      err_out += red[i];
-      cs_out = csum_merge(cs_out, CSum{red[16 + i], red[32 + i]});
+  if (w == 0) {  // the 16 wavefronts' sums on 16 lanes (each 16-lane group the same)
+    err_out = red[lane & 15];
+    cs_out = CSum{red[16 + (lane & 15)], red[32 + (lane & 15)]};
+#pragma unroll
+    for (int off = 8; off > 0; off >>= 1) {
+      err_out += __shfl_xor(err_out, off, 64);
+      cs_out = csum_merge(cs_out, CSum{__shfl_xor(cs_out.s, off, 64), __shfl_xor(cs_out.c, off, 64)});
     }
   }
 }
@@ -144,17 +156,26 @@ __device__ inline double add_teleport(double bi, double tele, const Teleport &tp
   return bi + tele * tp.v[i];
 }
 
+// What an update needs of the state, in LDS (written by the first wavefront
+// before the products, read after the barrier that ends them).
+struct StepIn {
+  double beta, tele;
+  int go;  // 0: the run had converged, nothing is written
+};
+
 // Per-row update epilogue: b = beta*(yhat + s) + teleport (MIXED) or beta*s + teleport.
 template <typename AT, bool MIXED, int TM>
 struct UpdateRow {
   double *b;
   const double *yhat;
   Teleport tp;
-  double beta, tele, lmax;
+  const StepIn *in;
+  double lmax;
   __device__ void operator()(int row, AT s) {
 #pragma clang fp contract(off)
+    if (!in->go) return;
     const double v = MIXED ? yhat[row] + static_cast<double>(s) : static_cast<double>(s);
-    const double bi = add_teleport<TM>(beta * v, tele, tp, row);
+    const double bi = add_teleport<TM>(in->beta * v, in->tele, tp, row);
     b[row] = bi;
     lmax = fmax(lmax, bi);
   }
@@ -178,60 +199,31 @@ __device__ inline void slot_max(unsigned long long *slots, double v, double *red
   if (threadIdx.x == 0) atomicMax(slots + (blockIdx.x % kMaxSlots), ord_encode(bm));
 }
 
-// Fused update over the CSR tiles (LONG = false) or the long rows (LONG =
-// true): b = beta * (A x) + tele, block max into the slots.  VT = dev::Pattern
-// is the value-free product over z = colscale .* b_t.
-template <typename VT, typename XT, bool MIXED, int TM, bool LONG>
-__global__ __launch_bounds__(kTileThreads) void pr_update_csr(dev::CsrView<VT> m, const XT *__restrict__ x,
-                                                              const double *__restrict__ yhat, Teleport tp,
-                                                              double *__restrict__ b, PrState *st,
-                                                              unsigned long long *slots) {
-  if (st->done) return;
-  using AT = typename dev::Val<VT>::A;
-  __shared__ dev::CsrTileLds<AT> lds;
-  __shared__ double red[kTileThreads];
-  UpdateRow<AT, MIXED, TM> epi{b, yhat, tp, st->beta, st->tele, -INFINITY};
-  if (LONG)
-    dev::csr_long_row<VT, XT>(m, x, lds, epi);
-  else
-    dev::csr_tile_rows<VT, XT>(m, x, lds, epi);
-  slot_max(slots, epi.lmax, red);
+__device__ inline double step_bound(double err, double S, double sum_prev) {
+  return err / S + fabs(sum_prev / S - 1.0);
+}
+__device__ inline bool step_converged(const PrState &st, double err, double bound) {
+  return st.rule == 0 ? (err < st.eps) : (bound <= st.bound_target);
 }
 
-// Update for any format after a plain product y = A b_t (generic engine).
-template <int TM>
-__global__ __launch_bounds__(kTileThreads) void pr_update_vec(double *__restrict__ b, long n, Teleport tp,
-                                                              PrState *st, unsigned long long *slots) {
-#pragma clang fp contract(off)
-  if (st->done) return;
-  __shared__ double red[kTileThreads];
-  const double beta = st->beta, tele = st->tele;
-  double lmax = -INFINITY;
-  for (long i = blockIdx.x * static_cast<long>(kTileThreads) + threadIdx.x; i < n;
-       i += static_cast<long>(gridDim.x) * kTileThreads) {
-    const double bi = add_teleport<TM>(beta * b[i], tele, tp, i);
-    b[i] = bi;
-    lmax = fmax(lmax, bi);
-  }
-  slot_max(slots, lmax, red);
-}
-
-// Decision logic of the last block of pr_normalize (one thread).
+// The step decision from an iteration's residual and sum (one thread).
+// MIXED = false leaves out what only mixed runs do.
+template <bool MIXED = true>
 __device__ inline void finalize_step(PrState *st, double err, double S) {
   // (mixed runs) this iteration moved the anchor: its step is the FP64
   // anchor product's, so its bound is free of the low-precision error
-  const bool moved = st->mixed && st->need_anchor;
+  const bool moved = MIXED && st->mixed && st->need_anchor;
   st->it += 1;
   st->err_prev = st->err;
   st->err = err;
   st->sum_prev = st->sum;
   st->sum = S;
-  const double bound = err / S + fabs(st->sum_prev / S - 1.0);
+  const double bound = step_bound(err, S, st->sum_prev);
   st->bound_prev = st->bound;
   st->bound = bound;
-  bool converged = st->rule == 0 ? (err < st->eps) : (bound <= st->bound_target);
+  bool converged = step_converged(*st, err, bound);
   int anchor = 0;
-  if (st->mixed) {
+  if (MIXED && st->mixed) {
     // A low-precision phase converges to a point off the FP64 fixed point by
     // up to about floor_eps * (bound at its anchor) / (1 - rho)^2, rho the
     // phase's mean contraction per iteration.  When that may exceed the
@@ -261,6 +253,136 @@ __device__ inline void finalize_step(PrState *st, double err, double S) {
   st->need_anchor = anchor;
   st->done = (converged || st->it >= st->max_it) ? 1 : 0;
   st->tele = S * st->tele_scale;
+  st->xscale = st->xnext;
+}
+
+// The partials of a normalise pass; n = 0: the state is up to date.
+struct Partials {
+  const double *perr, *ps, *pc;
+  int n;
+};
+
+// The first wavefront of every block of an update: merges the partials of
+// the iteration before (at most kPassBlocks, four a lane) and takes its step
+// decision, the same in every block; block 0 stores the new state to `out`
+// (a buffer of its own: other blocks still read `in`).  issue() loads,
+// finish() decides; both are the Pre work of a tile, so the loads wait beside
+// the tile's.
+struct StepMerge {
+  static constexpr int U = kPassBlocks / 64;
+  const PrState *in;
+  PrState *out;
+  Partials pp;
+  StepIn *sh;
+  double pe[U], pv[U], pw[U];
+
+  __device__ void issue() {
+    if (threadIdx.x >= 64) return;
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int i = max(0, min(static_cast<int>(threadIdx.x) + 64 * u, pp.n - 1));
+      pe[u] = pp.perr[i];
+      pv[u] = pp.ps[i];
+      pw[u] = pp.pc[i];
+    }
+  }
+  __device__ void finish() {
+    if (threadIdx.x >= 64) return;
+    double e = 0, S = 0;
+    if (pp.n > 0) {
+      CSum t{0, 0};
+#pragma unroll
+      for (int u = 0; u < U; u++)
+        if (static_cast<int>(threadIdx.x) + 64 * u < pp.n) {
+          e += pe[u];
+          t = csum_merge(t, CSum{pv[u], pw[u]});
+        }
+      e = wave_sum(e);
+      t = wave_csum(t);
+      S = t.s + t.c;
+    }
+    if (threadIdx.x != 0) return;
+    if (blockIdx.x == 0) {
+      *out = *in;
+      if (pp.n > 0) finalize_step<false>(out, e, S);
+    }
+    // what finalize_step leaves in tele and done
+    StepIn v{in->beta, in->tele, !in->done};
+    if (pp.n > 0) {
+      v.tele = S * in->tele_scale;
+      v.go = !(step_converged(*in, e, step_bound(e, S, in->sum)) || in->it + 1 >= in->max_it);
+    }
+    *sh = v;
+  }
+};
+// The state is up to date and only read.
+struct StepRead {
+  const PrState *in;
+  StepIn *sh;
+  __device__ void issue() {}
+  __device__ void finish() {
+    if (threadIdx.x == 0) *sh = StepIn{in->beta, in->tele, !in->done};
+  }
+};
+
+// Fused update over the CSR tiles (LONG = false) or the long rows (LONG =
+// true): b = beta * (A x) + tele, block max into the slots.  VT = dev::Pattern
+// is the value-free product over z = colscale .* b_t.
+// MERGE: the step decision of the iteration before is taken here (StepMerge).
+template <typename VT, typename XT, bool MIXED, int TM, int TN, bool MERGE, bool LONG>
+__global__ __launch_bounds__(kTileThreads) void pr_update_csr(dev::CsrView<VT> m, const XT *__restrict__ x,
+                                                              const double *__restrict__ yhat, Teleport tp,
+                                                              double *__restrict__ b, const PrState *st,
+                                                              PrState *st_out, Partials pp,
+                                                              unsigned long long *slots) {
+  if (st->done) {
+    if (MERGE && blockIdx.x == 0 && threadIdx.x == 0) *st_out = *st;
+    return;
+  }
+  using AT = typename dev::Val<VT>::A;
+  __shared__ dev::CsrTileLds<AT, TN> lds;
+  __shared__ double red[kTileThreads];
+  __shared__ StepIn in;
+  UpdateRow<AT, MIXED, TM> epi{b, yhat, tp, &in, -INFINITY};
+  if constexpr (LONG) {
+    StepRead{st, &in}.finish();
+    __syncthreads();
+    dev::csr_long_row<VT, XT, TN>(m, x, lds, epi);
+  } else if constexpr (MERGE) {
+    StepMerge pre{st, st_out, pp, &in};
+    dev::csr_tile_rows<VT, XT, TN>(m, x, lds, epi, pre);
+  } else {
+    dev::csr_tile_rows<VT, XT, TN>(m, x, lds, epi, StepRead{st, &in});
+  }
+  if (in.go) slot_max(slots, epi.lmax, red);
+}
+
+// Update for any format after a plain product y = A b_t (generic engine).
+template <int TM>
+__global__ __launch_bounds__(kTileThreads) void pr_update_vec(double *__restrict__ b, long n, Teleport tp,
+                                                              const PrState *st, PrState *st_out, Partials pp,
+                                                              unsigned long long *slots) {
+#pragma clang fp contract(off)
+  if (st->done) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *st_out = *st;
+    return;
+  }
+  __shared__ double red[kTileThreads];
+  __shared__ StepIn in;
+  StepMerge pre{st, st_out, pp, &in};
+  pre.issue();
+  pre.finish();
+  __syncthreads();
+  if (!in.go) return;
+  const double beta = in.beta, tele = in.tele;
+  double lmax = -INFINITY;
+  for (long i = blockIdx.x * static_cast<long>(kTileThreads) + threadIdx.x; i < n;
+       i += static_cast<long>(gridDim.x) * kTileThreads) {
+    const double bi = add_teleport<TM>(beta * b[i], tele, tp, i);
+    b[i] = bi;
+    lmax = fmax(lmax, bi);
+  }
+  slot_max(slots, lmax, red);
 }
 
 // MODE 0: FP64, b normalised in place, previous iterate `prev`.
@@ -270,105 +392,119 @@ __device__ inline void finalize_step(PrState *st, double err, double S) {
 // MODE 2: FP64 + z = colscale .* b for the next value-free product.
 // MODE 3: MODE 1 + zd = colscale .* (b - xhat) in FP32 (colscale32) for the
 //         next value-free FP32 product.
+//
+// Every block takes the maximum of the update's slots (64 loads by its first
+// wavefront); block 0 leaves it in the state and clears slots_next, the slots
+// of the next update (the two sets alternate).
 template <int MODE>
-__global__ __launch_bounds__(kTileThreads) void pr_normalize(double *__restrict__ b, const double *__restrict__ prev,
-                                                             const double *__restrict__ xhat,
-                                                             const float *__restrict__ dold, float *__restrict__ dnew,
-                                                             double *__restrict__ z,
-                                                             const double *__restrict__ colscale,
-                                                             float *__restrict__ zd,
-                                                             const float *__restrict__ colscale32, long n, PrState *st,
-                                                             double *__restrict__ perr, double *__restrict__ ps,
-                                                             double *__restrict__ pc) {
+__global__ __launch_bounds__(1024) void pr_normalize(double *__restrict__ b, const double *__restrict__ prev,
+                                                     const double *__restrict__ xhat, const float *__restrict__ dold,
+                                                     float *__restrict__ dnew, double *__restrict__ z,
+                                                     const double *__restrict__ colscale, float *__restrict__ zd,
+                                                     const float *__restrict__ colscale32, long n, PrState *st,
+                                                     const unsigned long long *slots, unsigned long long *slots_next,
+                                                     double *__restrict__ perr, double *__restrict__ ps,
+                                                     double *__restrict__ pc) {
 #pragma clang fp contract(off)
   if (st->done) return;
-  __shared__ double red_s[kTileThreads], red_c[kTileThreads];
-  const double m = st->maxv;
-  const double inv_m = 1.0 / m, pscale = st->xscale;  // (MODE 4)
-  const bool moved = st->need_anchor != 0;
+  __shared__ double red[48];
+  __shared__ double smax;
+  const long stride = static_cast<long>(gridDim.x) * 1024;
+  const long i_first = blockIdx.x * 1024L + threadIdx.x;
+  // four elements of the thread's sequence per step, loads first; the first
+  // step's are in flight beside the slots
+  double bv[4], pv[4];
+  const auto load4 = [&](long i0) {
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const long i = min(i0 + u * stride, n - 1);
+      bv[u] = b[i];
+      pv[u] = prev[i];
+    }
+  };
+  if (MODE == 4 || MODE == 0) load4(i_first);
+  if (threadIdx.x < 64) {
+    unsigned long long u = __hip_atomic_load(slots + threadIdx.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+      const unsigned long long o = __shfl_xor(u, off, 64);
+      u = o > u ? o : u;
+    }
+    if (threadIdx.x == 0) smax = ord_decode(u);
+  }
+  if (blockIdx.x == 0 && threadIdx.x >= 64 && threadIdx.x < 64 + kMaxSlots)
+    __hip_atomic_store(slots_next + (threadIdx.x - 64), 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const double pscale = st->xscale;  // (MODE 4)
+  const bool moved = st->need_anchor != 0, raw = st->raw != 0;
+  __syncthreads();
+  const double m = smax, inv_m = 1.0 / m;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    st->maxv = m;
+    st->xnext = raw ? inv_m : 1.0;  // the scale of the b just written
+  }
   double err = 0;
   CSum cs{0, 0};
-  if (MODE == 4) {
-    // four elements of the thread's sequence per step, loads first (the
-    // same order of additions as one element per step)
-    const long stride = static_cast<long>(gridDim.x) * kTileThreads;
-    for (long i0 = blockIdx.x * static_cast<long>(kTileThreads) + threadIdx.x; i0 < n; i0 += 4 * stride) {
-      double bv[4], pv[4];
-#pragma unroll
-      for (int u = 0; u < 4; u++) {
-        const long i = min(i0 + u * stride, n - 1);
-        bv[u] = b[i];
-        pv[u] = prev[i];
-      }
+  if (MODE == 4 || MODE == 0) {
+    for (long i0 = i_first; i0 < n; i0 += 4 * stride) {
+      if (i0 != i_first) load4(i0);
 #pragma unroll
       for (int u = 0; u < 4; u++)
         if (i0 + u * stride < n) {
-          const double bi = bv[u] * inv_m;
-          err += fabs(bi - pv[u] * pscale);
+          const double bi = MODE == 4 ? bv[u] * inv_m : bv[u] / m;
+          err += fabs(bi - (MODE == 4 ? pv[u] * pscale : pv[u]));
           csum_add(cs, bi);
+          if (MODE == 0) b[i0 + u * stride] = bi;
         }
     }
-  }
-  for (long i = blockIdx.x * static_cast<long>(kTileThreads) + threadIdx.x; MODE != 4 && i < n;
-       i += static_cast<long>(gridDim.x) * kTileThreads) {
-    const double bi = b[i] / m;
-    const bool mixed = MODE == 1 || MODE == 3;
-    // an iteration that moved the anchor starts from xhat itself (its delta
-    // was folded into xhat and is not read)
-    const double pi = mixed ? (moved ? xhat[i] : xhat[i] + static_cast<double>(dold[i])) : prev[i];
-    err += fabs(bi - pi);
-    csum_add(cs, bi);
-    if (mixed) {
-      const double dd = bi - xhat[i];
-      dnew[i] = static_cast<float>(dd);
-      if (MODE == 3) zd[i] = static_cast<float>(static_cast<double>(colscale32[i]) * dd);
-    } else {
-      b[i] = bi;
-      if (MODE == 2) z[i] = colscale[i] * bi;
+  } else {
+    for (long i = blockIdx.x * 1024L + threadIdx.x; i < n; i += stride) {
+      const double bi = b[i] / m;
+      const bool mixed = MODE == 1 || MODE == 3;
+      // an iteration that moved the anchor starts from xhat itself (its delta
+      // was folded into xhat and is not read)
+      const double pi = mixed ? (moved ? xhat[i] : xhat[i] + static_cast<double>(dold[i])) : prev[i];
+      err += fabs(bi - pi);
+      csum_add(cs, bi);
+      if (mixed) {
+        const double dd = bi - xhat[i];
+        dnew[i] = static_cast<float>(dd);
+        if (MODE == 3) zd[i] = static_cast<float>(static_cast<double>(colscale32[i]) * dd);
+      } else {
+        b[i] = bi;
+        z[i] = colscale[i] * bi;
+      }
     }
   }
-  const double berr = dev::block_tree_sum<double>(err, red_s);
-  const CSum bs = block_csum(cs, red_s, red_c);
+  double e;
+  CSum t;
+  block1024_err_csum(err, cs, red, e, t);
   if (threadIdx.x == 0) {
-    perr[blockIdx.x] = berr;
-    ps[blockIdx.x] = bs.s;
-    pc[blockIdx.x] = bs.c;
+    perr[blockIdx.x] = e;
+    ps[blockIdx.x] = t.s;
+    pc[blockIdx.x] = t.c;
   }
-}
-
-// One wavefront: the maximum over the slots, which are cleared for the next
-// update.  Slots are read and cleared with device-scope atomics.
-__global__ __launch_bounds__(64) void pr_finalize_max(unsigned long long *slots, PrState *st) {
-  if (st->done) return;
-  unsigned long long u = __hip_atomic_load(slots + threadIdx.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  __hip_atomic_store(slots + threadIdx.x, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    const unsigned long long o = __shfl_xor(u, off, 64);
-    u = o > u ? o : u;
-  }
-  if (threadIdx.x == 0) st->maxv = ord_decode(u);
 }
 
 // Sum of the per-block partials (err, compensated sum) over nb blocks by one
-// kTileThreads block, in the fixed order thread t: t, t + kTileThreads, ...
+// block of T threads, in the fixed order thread t: t, t + T, ...
 // The loads of 8 partials per thread are issued together (a loop that loads
 // one partial per step waits for each load in turn).
+template <int T = kTileThreads>
 __device__ inline void sum_partials(const double *__restrict__ perr, const double *__restrict__ ps,
                                     const double *__restrict__ pc, int nb, double &e, CSum &t) {
   constexpr int U = 8;
-  for (int i0 = threadIdx.x; i0 < nb; i0 += U * kTileThreads) {
+  for (int i0 = threadIdx.x; i0 < nb; i0 += U * T) {
     double pe[U], pv[U], pw[U];
 #pragma unroll
     for (int u = 0; u < U; u++) {
-      const int i = min(i0 + u * kTileThreads, nb - 1);
+      const int i = min(i0 + u * T, nb - 1);
       pe[u] = perr ? perr[i] : 0.0;
       pv[u] = ps[i];
       pw[u] = pc[i];
     }
 #pragma unroll
     for (int u = 0; u < U; u++)
-      if (i0 + u * kTileThreads < nb) {
+      if (i0 + u * T < nb) {
         e += pe[u];
         t = csum_merge(t, CSum{pv[u], pw[u]});
       }
@@ -387,10 +523,7 @@ __global__ __launch_bounds__(kTileThreads) void pr_finalize_norm(const double *_
   sum_partials(perr, ps, pc, nb, e, t);
   e = dev::block_tree_sum<double>(e, red_s);
   t = block_csum(t, red_s, red_c);
-  if (threadIdx.x == 0) {
-    finalize_step(st, e, t.s + t.c);
-    if (st->raw) st->xscale = 1.0 / st->maxv;  // the scale of the b just written
-  }
+  if (threadIdx.x == 0) finalize_step(st, e, t.s + t.c);
 }
 
 // Mixed precision with tile products: move the anchor to the current iterate
@@ -423,53 +556,47 @@ struct StoreRowD {
 
 // Mixed precision: the FP64 anchor product yhat = A64 xhat (VT = double) or
 // its value-free form over z = colscale .* xhat (VT = dev::Pattern).
-template <typename VT, bool LONG>
+template <typename VT, int TN, bool LONG>
 __global__ __launch_bounds__(kTileThreads) void pr_anchor_spmv(dev::CsrView<VT> m, const double *__restrict__ x,
                                                                double *__restrict__ yhat, const PrState *st) {
   if (st->done || !st->need_anchor) return;
-  __shared__ dev::CsrTileLds<double> lds;
+  __shared__ dev::CsrTileLds<double, TN> lds;
   StoreRowD<double> epi{yhat};
-  if (LONG)
-    dev::csr_long_row<VT, double>(m, x, lds, epi);
+  if constexpr (LONG)
+    dev::csr_long_row<VT, double, TN>(m, x, lds, epi);
   else
-    dev::csr_tile_rows<VT, double>(m, x, lds, epi);
+    dev::csr_tile_rows<VT, double, TN>(m, x, lds, epi);
 }
 
-// v = a (+ d) ; out = v / sum(v) with a compensated sum (two passes).
-// (the element is (a + d) * xscale: xscale is 1 except in raw runs)
-__global__ __launch_bounds__(kTileThreads) void pr_sum_kernel(const double *__restrict__ a,
-                                                              const float *__restrict__ d, long n,
-                                                              const PrState *st, double *__restrict__ ps,
-                                                              double *__restrict__ pc) {
+// Mixed runs on the tile products: the state's sum becomes the compensated
+// sum of the anchor plus the FP32 delta (one block; once per run).
+__global__ __launch_bounds__(1024) void pr_sum_rounded(const double *__restrict__ a, const float *__restrict__ d,
+                                                       long n, PrState *st) {
 #pragma clang fp contract(off)
-  __shared__ double red_s[kTileThreads], red_c[kTileThreads];
-  const double sc = st->xscale;
-  CSum cs{0, 0};
-  for (long i = blockIdx.x * static_cast<long>(kTileThreads) + threadIdx.x; i < n;
-       i += static_cast<long>(gridDim.x) * kTileThreads)
-    csum_add(cs, (d ? a[i] + static_cast<double>(d[i]) : a[i]) * sc);
-  const CSum bs = block_csum(cs, red_s, red_c);
-  if (threadIdx.x == 0) {
-    ps[blockIdx.x] = bs.s;
-    pc[blockIdx.x] = bs.c;
+  __shared__ double red[48];
+  CSum cs{0, 0}, t;
+  for (long i0 = threadIdx.x; i0 < n; i0 += 8 * 1024) {
+    double v[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+      const long i = min(i0 + u * 1024, n - 1);
+      v[u] = a[i] + static_cast<double>(d[i]);
+    }
+#pragma unroll
+    for (int u = 0; u < 8; u++)
+      if (i0 + u * 1024 < n) csum_add(cs, v[u]);
   }
+  double unused;
+  block1024_err_csum(0.0, cs, red, unused, t);
+  if (threadIdx.x == 0) st->sum = t.s + t.c;
 }
 
-__global__ __launch_bounds__(kTileThreads) void pr_sum_finalize(const double *__restrict__ ps,
-                                                                const double *__restrict__ pc, int nb,
-                                                                double *__restrict__ total) {
-  __shared__ double red_s[kTileThreads], red_c[kTileThreads];
-  CSum t{0, 0};
-  for (int i = threadIdx.x; i < nb; i += kTileThreads) t = csum_merge(t, CSum{ps[i], pc[i]});
-  t = block_csum(t, red_s, red_c);
-  if (threadIdx.x == 0) *total = t.s + t.c;
-}
-
+// out = v / sum(v), v = (a (+ d)) * xscale (xscale is 1 except in raw runs):
+// the state holds the compensated sum of the last iterate.
 __global__ __launch_bounds__(256) void pr_scale_kernel(const double *__restrict__ a, const float *__restrict__ d,
-                                                       long n, const PrState *st, const double *__restrict__ total,
-                                                       double *__restrict__ out) {
+                                                       long n, const PrState *st, double *__restrict__ out) {
 #pragma clang fp contract(off)
-  const double S = *total, sc = st->xscale;
+  const double S = st->sum, sc = st->xscale;
   for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += static_cast<long>(gridDim.x) * 256)
     out[i] = ((d ? a[i] + static_cast<double>(d[i]) : a[i]) * sc) / S;
 }
@@ -492,18 +619,44 @@ __global__ __launch_bounds__(256) void to_f32(const double *__restrict__ a, floa
 __global__ __launch_bounds__(256) void fill_f64(double *y, long n, double v) {
   for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += static_cast<long>(gridDim.x) * 256) y[i] = v;
 }
-__global__ __launch_bounds__(256) void fill_f32(float *y, long n, float v) {
-  for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += static_cast<long>(gridDim.x) * 256) y[i] = v;
-}
-__global__ __launch_bounds__(256) void scale_into(const double *__restrict__ s, const double *__restrict__ x,
-                                                  double *__restrict__ z, long n) {
-  for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += static_cast<long>(gridDim.x) * 256) z[i] = s[i] * x[i];
+// Everything a run starts from: the state, the max slots (both sets) and the
+// start vectors that are not nullptr.
+struct PrInit {
+  PrState h;
+  PrState *st;
+  unsigned long long *slots;
+  long n;
+  double *x;          // = x0
+  double x0;
+  double *xhat, *yhat, *z;  // = 0, 0, z_scale .* x0
+  const double *z_scale;
+  float *d, *w, *xhat32;    // = fl32(x0), 0, 0
+  float *zd;                // = fl32(zd_scale32 .* fl32(x0)), or fl32(zd_scale64 * x0)
+  const float *zd_scale32;
+  const double *zd_scale64;
+};
+__global__ __launch_bounds__(256) void pr_init(PrInit a) {
+  if (blockIdx.x == 0) {
+    if (threadIdx.x == 0) *a.st = a.h;
+    if (threadIdx.x < 2 * kMaxSlots) a.slots[threadIdx.x] = 0;
+  }
+  const float f0 = static_cast<float>(a.x0);
+  for (long i = blockIdx.x * 256L + threadIdx.x; i < a.n; i += static_cast<long>(gridDim.x) * 256) {
+    if (a.x) a.x[i] = a.x0;
+    if (a.xhat) a.xhat[i] = 0.0;
+    if (a.yhat) a.yhat[i] = 0.0;
+    if (a.z) a.z[i] = a.z_scale[i] * a.x0;
+    if (a.d) a.d[i] = f0;
+    if (a.w) a.w[i] = 0.0f;
+    if (a.xhat32) a.xhat32[i] = 0.0f;
+    if (a.zd)
+      a.zd[i] = a.zd_scale32 ? static_cast<float>(static_cast<double>(a.zd_scale32[i]) * static_cast<double>(f0))
+                             : static_cast<float>(a.zd_scale64[i] * a.x0);
+  }
 }
 
-__global__ __launch_bounds__(256) void scale_into_f32(const double *__restrict__ s, double v, float *__restrict__ z,
-                                                      long n) {
-  for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += static_cast<long>(gridDim.x) * 256)
-    z[i] = static_cast<float>(s[i] * v);
+unsigned grid_for(long n, long cap = kNormBlocks) {
+  return static_cast<unsigned>(std::max<long>(1, std::min<long>(cap, (n + 255) / 256)));
 }
 
 // bad[0] = 1 unless every stored value of column j has the bits of cs[j]
@@ -518,10 +671,6 @@ __global__ __launch_bounds__(256) void colscale_check(const int *__restrict__ co
 __global__ __launch_bounds__(256) void to_bf16_f32(const double *__restrict__ a, float *__restrict__ b, long n) {
   for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += static_cast<long>(gridDim.x) * 256)
     b[i] = dev::Val<dev::bf16>::cvt(dev::bf16_of(a[i]));
-}
-
-unsigned grid_for(long n, long cap = kNormBlocks) {
-  return static_cast<unsigned>(std::max<long>(1, std::min<long>(cap, (n + 255) / 256)));
 }
 
 // Whether the stored entries of every column of an n-column CSR matrix hold
@@ -794,17 +943,35 @@ constexpr bool pb_value_free() {
   return std::is_same<VT, dev::Pattern>::value;
 }
 
-// FP64 runs: the far products of x (value-free: of cs .* x).
+// FP64 runs: the far products of x (value-free: of cs .* x).  The last block
+// takes the step decision of the iteration before from its partials instead
+// (pp.n > 0): the products need only the iterate and, in raw runs, its scale
+// xnext, so the decision costs no launch of its own.  The other blocks may
+// read `done` before or after it is set; a scatter past convergence writes
+// products that nothing reads.
 template <typename VT, int COLS>
 __global__ __launch_bounds__(kPbScatterThreads) void pb_scatter(PbScatterArgs a, const VT *__restrict__ val,
                                                                 const double *__restrict__ cs,
                                                                 const double *__restrict__ x,
-                                                                double *__restrict__ prod, const PrState *st) {
+                                                                double *__restrict__ prod, PrState *st, Partials pp) {
   if (st->done) return;
   __shared__ double xs[COLS];
-  // (raw reference-rule runs: x is the unnormalised b, the iterate x * xscale)
+  if (blockIdx.x == gridDim.x - 1) {
+    if (pp.n > 0) {
+      double e = 0, eb = 0;
+      CSum t{0, 0}, tb{0, 0};
+      sum_partials<kPbScatterThreads>(pp.perr, pp.ps, pp.pc, pp.n, e, t);
+      block1024_err_csum(e, t, xs, eb, tb);
+      if (threadIdx.x == 0) {
+        finalize_step<false>(st, eb, tb.s + tb.c);
+        st->inv_sum = 1.0 / (tb.s + tb.c);
+      }
+    }
+    return;
+  }
+  // (raw reference-rule runs: x is the unnormalised b, the iterate x * xnext)
   pb_scatter_sb<VT, double, double, false, COLS, pb_value_free<VT>()>(a, val, x, prod, xs, AnchorMove{}, nullptr,
-                                                                      st->raw ? st->xscale : 1.0, cs);
+                                                                      st->xnext, cs);
 }
 
 // The value-free FP64 anchor product takes the wide scatter order (a 128 KB
@@ -1001,7 +1168,7 @@ __global__ __launch_bounds__(1024) void pb_gather(PbView v, const VT *__restrict
   if (st->done) return;
   __shared__ double ybin[kPbRows];
   __shared__ double red[16];
-  pb_accumulate<VT, double, double, pb_value_free<VT>()>(v, lval, x, prod, ybin, st->raw ? st->xscale : 1.0, cs);
+  pb_accumulate<VT, double, double, pb_value_free<VT>()>(v, lval, x, prod, ybin, st->xnext, cs);
   const int bin = blockIdx.x, tid = threadIdx.x;
   const int base = bin * v.rows;
   const int rows = min(v.rows, v.n - base);
@@ -1181,14 +1348,13 @@ constexpr unsigned kPbScatterLdsPad = 24 * 1024;
 // the column values) over the wide order, the others over the narrow one.
 template <typename VT>
 void launch_pb_scatter(const PbMatrix &pb, const VT *fval, const double *cs, const double *x, double *prod,
-                       const PrState *st, hipStream_t s) {
-  if (pb.n_far == 0) return;
+                       PrState *st, const Partials &pp, hipStream_t s) {
   if constexpr (pb_value_free<VT>())
-    hipLaunchKernelGGL((pb_scatter<VT, kPbColsWide>), pb_scatter_grid_wide(pb), dim3(kPbScatterThreads), 0, s,
-                       pb_args_wide(pb), fval, cs, x, prod, st);
+    hipLaunchKernelGGL((pb_scatter<VT, kPbColsWide>), dim3(pb_scatter_grid_wide(pb).x + 1), dim3(kPbScatterThreads),
+                       0, s, pb_args_wide(pb), fval, cs, x, prod, st, pp);
   else
-    hipLaunchKernelGGL((pb_scatter<VT, kPbCols>), pb_scatter_grid(pb), dim3(kPbScatterThreads), kPbScatterLdsPad, s,
-                       pb_args(pb), fval, cs, x, prod, st);
+    hipLaunchKernelGGL((pb_scatter<VT, kPbCols>), dim3(pb_scatter_grid(pb).x + 1), dim3(kPbScatterThreads),
+                       kPbScatterLdsPad, s, pb_args(pb), fval, cs, x, prod, st, pp);
 }
 
 // The per-bin partials of a sum-normalised iteration.
@@ -1199,15 +1365,16 @@ struct SnPartials {
 // One FP64 iteration on the blocked products (values VT; dev::Pattern: value-
 // free, cs the column values): scatter and gather.  sp == nullptr: the
 // reference-rule update, block maxima into the slots; else the sum-normalised
-// one with its partials.  The finalize passes follow.
+// one with its partials.  pp: the partials of the iteration before, whose step
+// decision the scatter takes (pp.n = 0: taken already).
 template <typename VT, int TM>
 void launch_pb_tm(const PbMatrix &pb, const double *cs, const double *x, const Teleport &tp, double *out, PrState *st,
-                  unsigned long long *slots, const SnPartials *sp, hipStream_t s) {
+                  unsigned long long *slots, const SnPartials *sp, const Partials &pp, hipStream_t s) {
   constexpr int slot = static_cast<int>(Dtype::F64);
   const VT *fval = pb_value_free<VT>() ? nullptr : pb.fval[slot].as<VT>();
   const VT *lval = pb_value_free<VT>() ? nullptr : pb.lval[slot].as<VT>();
   double *prod = pb.prod.as<double>();
-  launch_pb_scatter<VT>(pb, fval, cs, x, prod, st, s);
+  launch_pb_scatter<VT>(pb, fval, cs, x, prod, st, pp, s);
   if (sp)
     hipLaunchKernelGGL((pb_gather_sn<VT, TM>), dim3(pb.nbins), dim3(1024), 0, s, pb_view(pb), lval, cs, x, prod, tp,
                        out, st, sp->perr, sp->ps, sp->pc);
@@ -1217,15 +1384,15 @@ void launch_pb_tm(const PbMatrix &pb, const double *cs, const double *x, const T
 }
 
 void launch_pb(int tmode, const PbMatrix &pb, const double *cs, const double *x, const Teleport &tp, double *out,
-               PrState *st, unsigned long long *slots, const SnPartials *sp, hipStream_t s) {
+               PrState *st, unsigned long long *slots, const SnPartials *sp, const Partials &pp, hipStream_t s) {
   const auto go = [&](auto tag) {
     using VT = decltype(tag);
     if (tmode == 1)
-      launch_pb_tm<VT, 1>(pb, cs, x, tp, out, st, slots, sp, s);
+      launch_pb_tm<VT, 1>(pb, cs, x, tp, out, st, slots, sp, pp, s);
     else if (tmode == 2)
-      launch_pb_tm<VT, 2>(pb, cs, x, tp, out, st, slots, sp, s);
+      launch_pb_tm<VT, 2>(pb, cs, x, tp, out, st, slots, sp, pp, s);
     else
-      launch_pb_tm<VT, 0>(pb, cs, x, tp, out, st, slots, sp, s);
+      launch_pb_tm<VT, 0>(pb, cs, x, tp, out, st, slots, sp, pp, s);
   };
   if (cs)
     go(dev::Pattern());
@@ -1280,43 +1447,58 @@ void launch_pb_mx(int tmode, const PbMatrix &pb, int va, int vd, const MxBufs &b
     launch_pb_mx_tm<VA, VD, XD, 0, PAT32>(pb, va, vd, b, tp, st, sp, s);
 }
 
+// The state an update reads, where its block 0 leaves the state after the
+// step decision it takes (nullptr: none to take), and the partials for it.
+struct StepArgs {
+  const PrState *in;
+  PrState *out;
+  Partials pp;
+};
+
 template <typename VT, typename XT, bool MIXED, int TM>
 void launch_update(const DeviceMatrix &d, const VT *vals, const XT *x, const double *yhat, const Teleport &tp,
-                   double *b, PrState *st, unsigned long long *slots, hipStream_t s) {
+                   double *b, const StepArgs &a, unsigned long long *slots, hipStream_t s) {
   dev::CsrView<VT> m = dev::csr_view<VT>(d);
   if (vals) m.vals = vals;
-  if (d.ntiles > 0)
-    hipLaunchKernelGGL((pr_update_csr<VT, XT, MIXED, TM, false>), dim3(d.ntiles), dim3(kTileThreads), 0, s, m, x,
-                       yhat, tp, b, st, slots);
+  // (nnz / tile size + 1 tiles, so at least one block stores the state)
+  if constexpr (!MIXED) {
+    if (a.out)
+      hipLaunchKernelGGL((pr_update_csr<VT, XT, MIXED, TM, kMergeTileNnz, true, false>), dim3(d.ntiles),
+                         dim3(kTileThreads), 0, s, m, x, yhat, tp, b, a.in, a.out, a.pp, slots);
+  }
+  if (!a.out)
+    with_tile_size(d, [&](auto tn) {
+      hipLaunchKernelGGL((pr_update_csr<VT, XT, MIXED, TM, decltype(tn)::value, false, false>), dim3(d.ntiles),
+                         dim3(kTileThreads), 0, s, m, x, yhat, tp, b, a.in, a.out, a.pp, slots);
+    });
   if (d.nlong > 0)
-    hipLaunchKernelGGL((pr_update_csr<VT, XT, MIXED, TM, true>), dim3(d.nlong), dim3(kTileThreads), 0, s, m, x, yhat,
-                       tp, b, st, slots);
+    hipLaunchKernelGGL((pr_update_csr<VT, XT, MIXED, TM, kTileThreads, false, true>), dim3(d.nlong),
+                       dim3(kTileThreads), 0, s, m, x, yhat, tp, b, a.out ? a.out : a.in,
+                       static_cast<PrState *>(nullptr), Partials{}, slots);
 }
 
 // Values override `vals` (nullptr: the mirror's own values).
 template <typename VT, typename XT, bool MIXED>
 void launch_update(int tmode, const DeviceMatrix &d, const VT *vals, const XT *x, const double *yhat,
-                   const Teleport &tp, double *b, PrState *st, unsigned long long *slots, hipStream_t s) {
+                   const Teleport &tp, double *b, const StepArgs &a, unsigned long long *slots, hipStream_t s) {
   if (tmode == 1)
-    launch_update<VT, XT, MIXED, 1>(d, vals, x, yhat, tp, b, st, slots, s);
+    launch_update<VT, XT, MIXED, 1>(d, vals, x, yhat, tp, b, a, slots, s);
   else if (tmode == 2)
-    launch_update<VT, XT, MIXED, 2>(d, vals, x, yhat, tp, b, st, slots, s);
+    launch_update<VT, XT, MIXED, 2>(d, vals, x, yhat, tp, b, a, slots, s);
   else
-    launch_update<VT, XT, MIXED, 0>(d, vals, x, yhat, tp, b, st, slots, s);
+    launch_update<VT, XT, MIXED, 0>(d, vals, x, yhat, tp, b, a, slots, s);
 }
 
 template <typename VT>
 void launch_anchor(const DeviceMatrix &d, const double *x, double *yhat, const PrState *st, hipStream_t s) {
   const dev::CsrView<VT> m = dev::csr_view<VT>(d);
   if (d.ntiles > 0)
-    hipLaunchKernelGGL((pr_anchor_spmv<VT, false>), dim3(d.ntiles), dim3(kTileThreads), 0, s, m, x, yhat, st);
+    with_tile_size(d, [&](auto tn) {
+      hipLaunchKernelGGL((pr_anchor_spmv<VT, decltype(tn)::value, false>), dim3(d.ntiles), dim3(kTileThreads), 0, s, m,
+                         x, yhat, st);
+    });
   if (d.nlong > 0)
-    hipLaunchKernelGGL((pr_anchor_spmv<VT, true>), dim3(d.nlong), dim3(kTileThreads), 0, s, m, x, yhat, st);
-}
-
-__global__ void zero_u64(unsigned long long *p, int n) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = 0;
+    hipLaunchKernelGGL((pr_anchor_spmv<VT, kTileThreads, true>), dim3(d.nlong), dim3(kTileThreads), 0, s, m, x, yhat, st);
 }
 
 // One device buffer of a run: owned (allocated for the run) or a slice of
@@ -1359,16 +1541,9 @@ struct Workspace {
 };
 
 struct Scratch {
-  WsBuf st, slots, perr, ps, pc, total, member, nodes, hsum, hcomp;
+  WsBuf st, slots, perr, ps, pc, member, nodes, hsum, hcomp;
   WsBuf X0, X1, Z, yhat, xhat, xhat32, D0, D1, ZD0, ZD1, W;
 };
-
-// zd = fl32(colscale32 * d) of a constant FP32 delta d
-__global__ __launch_bounds__(256) void scale_into_f32_32(const float *__restrict__ s, float d, float *__restrict__ z,
-                                                         long n) {
-  for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += static_cast<long>(gridDim.x) * 256)
-    z[i] = static_cast<float>(static_cast<double>(s[i]) * static_cast<double>(d));
-}
 
 // One block: the step decision of a sum-normalised propagation-blocked
 // iteration from the gather's per-bin partials (nb) and, after a mixed run's
@@ -1514,43 +1689,40 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
   Scratch w;
   Workspace ws{arena, cap, 0};
   const unsigned gN = grid_for(n);
-  // the mixed normalise pass (six streams) measured faster with twice the
-  // blocks (four and eight times: slower); the FP64 one (three streams) slower
-  const unsigned gM = mixed ? grid_for(n, 2L * kNormBlocks) : gN;
+  // blocks of the normalise pass.  The mixed one (six streams) measured
+  // faster with twice the blocks (four and eight times: slower); the FP64 one
+  // (three streams) slower
+  const unsigned gM = static_cast<unsigned>(std::min<long>(mixed ? 2 * kPassBlocks : kPassBlocks, (n + 1023) / 1024));
   // sum-normalised rule with propagation-blocked products: the update, the
-  // normalisation and the residual in the gather pass, one finalize pass
+  // normalisation and the residual in the gather pass
   const bool sn = pbm && p.rule == PrRule::SUMNORM;
-  const unsigned nparts = std::max(std::max(gN, gM), sn ? static_cast<unsigned>(pbm->nbins) : 0u);
-  ws.alloc(w.st, sizeof(PrState));
-  ws.alloc(w.slots, sizeof(unsigned long long) * kMaxSlots);
+  const unsigned nparts = std::max(gM, sn ? static_cast<unsigned>(pbm->nbins) : 0u);
+  ws.alloc(w.st, 2 * sizeof(PrState));
+  ws.alloc(w.slots, 2 * sizeof(unsigned long long) * kMaxSlots);
   ws.alloc(w.perr, sizeof(double) * nparts);
   ws.alloc(w.ps, sizeof(double) * nparts);
   ws.alloc(w.pc, sizeof(double) * nparts);
-  ws.alloc(w.total, sizeof(double));
-  ws.alloc(w.X0, sizeof(double) * n);
-  ws.alloc(w.X1, sizeof(double) * n);
+  // (mixed runs on propagation-blocked products keep the iterate as the
+  // anchor plus the delta and never use X)
+  const bool pb_mixed = mixed && sn;
+  if (!pb_mixed) {
+    ws.alloc(w.X0, sizeof(double) * n);
+    ws.alloc(w.X1, sizeof(double) * n);
+  }
   // teleport mode: 0 uniform, 1 node set (Matrix.cpp:63-114), 2 distribution vector
   const int tmode = p.teleport ? 2 : (p.personalized ? 1 : 0);
   Teleport tp{nullptr, p.teleport};
   const double b0 = p.personalized && !p.teleport ? 0.25 : 1.0;
-  std::vector<unsigned char> mem;
-  if (tmode == 1 && arena) {
-    // no host staging vector: the node list goes to the scratch buffer and
-    // a kernel sets the flags
+  if (tmode == 1) {
     ws.alloc(w.member, static_cast<std::size_t>(n));
     hipLaunchKernelGGL(fill_u8, dim3(grid_for(n)), dim3(256), 0, s, w.member.as<unsigned char>(), n,
                        static_cast<unsigned char>(0));
     if (p.n_nodes > 0) {
+      // (p.nodes stays valid until the run has ended)
       ws.upload(w.nodes, p.nodes, sizeof(int) * static_cast<std::size_t>(p.n_nodes), s);
       hipLaunchKernelGGL(set_members, dim3(grid_for(p.n_nodes)), dim3(256), 0, s, w.member.as<unsigned char>(), n,
                          w.nodes.as<int>(), p.n_nodes);
     }
-    tp.member = w.member.as<unsigned char>();
-  } else if (tmode == 1) {
-    mem.assign(static_cast<std::size_t>(n), 0);
-    for (int k = 0; k < p.n_nodes; k++)
-      if (p.nodes[k] >= 0 && p.nodes[k] < n) mem[static_cast<std::size_t>(p.nodes[k])] = 1;
-    ws.upload(w.member, mem.data(), mem.size(), s);
     tp.member = w.member.as<unsigned char>();
   }
   // the column values of a value-free run (1/count per column after
@@ -1595,6 +1767,7 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
   // iterate less per iteration)
   h.raw = (fused && pbm && !sn && !mixed) ? 1 : 0;
   h.xscale = 1.0;
+  h.xnext = 1.0;
   // mixed runs start from the anchor xhat = 0 (so yhat = A xhat = 0 with no
   // product) and delta = b0: the first phase carries the whole iterate in the
   // low precision, and the first anchor move comes when it has converged to
@@ -1607,40 +1780,38 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
   // more iteration; FP32 3e-6 and 1e-6 -> 1 move, 1e-5 and above -> 2)
   h.anchor_tau = p.anchor_tau > 0 ? p.anchor_tau : (p.precision == PrPrecision::BF16 ? 1e-2 : 3e-6);
   h.done = p.max_iteration <= 0 ? 1 : 0;
-  TBSLA_HIP_CHECK(hipMemcpyAsync(w.st.get(), &h, sizeof(h), hipMemcpyHostToDevice, s));
-  PrState *st = w.st.as<PrState>();
+  // one launch writes the state, the slots and every start vector (the other
+  // buffers are written before they are read)
+  PrInit in{};
+  in.h = h;
+  in.st = w.st.as<PrState>();
+  in.slots = w.slots.as<unsigned long long>();
+  in.n = n;
+  in.x = w.X0.as<double>();
+  in.x0 = x0;
+  PrState *const st = w.st.as<PrState>();
   double *X[2] = {w.X0.as<double>(), w.X1.as<double>()};
-  // (mixed runs on propagation-blocked products keep the iterate as the
-  // anchor plus the delta and never read X)
-  const bool pb_mixed = mixed && sn;
-  if (!pb_mixed) {
-    hipLaunchKernelGGL(fill_f64, dim3(gN), dim3(256), 0, s, X[0], n, x0);
-    hipLaunchKernelGGL(fill_f64, dim3(gN), dim3(256), 0, s, X[1], n, 0.0);
-  }
-  unsigned long long *slots = w.slots.as<unsigned long long>();
-  hipLaunchKernelGGL(zero_u64, dim3(1), dim3(kMaxSlots), 0, s, slots, kMaxSlots);
+  unsigned long long *const slots = w.slots.as<unsigned long long>();
   float *D[2] = {nullptr, nullptr};
   if (mixed) {
     ws.alloc(w.xhat, sizeof(double) * n);
     ws.alloc(w.D0, sizeof(float) * n);
     ws.alloc(w.D1, sizeof(float) * n);
-    D[0] = w.D0.as<float>();
+    D[0] = in.d = w.D0.as<float>();
     D[1] = w.D1.as<float>();
-    hipLaunchKernelGGL(fill_f64, dim3(gN), dim3(256), 0, s, w.xhat.as<double>(), n, 0.0);
-    hipLaunchKernelGGL(fill_f32, dim3(gN), dim3(256), 0, s, D[0], n, static_cast<float>(x0));
-    hipLaunchKernelGGL(fill_f32, dim3(gN), dim3(256), 0, s, D[1], n, 0.0f);
+    in.xhat = w.xhat.as<double>();
     if (sn) {
       // the anchor's FP32 one-step change (0 before the first anchor, whose
       // anchor is 0) and the scatter's per-superblock sums of a moved anchor
       ws.alloc(w.W, sizeof(float) * n);
-      hipLaunchKernelGGL(fill_f32, dim3(gN), dim3(256), 0, s, w.W.as<float>(), n, 0.0f);
       ws.alloc(w.xhat32, sizeof(float) * n);
-      hipLaunchKernelGGL(fill_f32, dim3(gN), dim3(256), 0, s, w.xhat32.as<float>(), n, 0.0f);
+      in.w = w.W.as<float>();
+      in.xhat32 = w.xhat32.as<float>();
       ws.alloc(w.hsum, sizeof(double) * std::max(1, pbm->nsb));
       ws.alloc(w.hcomp, sizeof(double) * std::max(1, pbm->nsb));
     } else {
       ws.alloc(w.yhat, sizeof(double) * n);
-      hipLaunchKernelGGL(fill_f64, dim3(gN), dim3(256), 0, s, w.yhat.as<double>(), n, 0.0);
+      in.yhat = w.yhat.as<double>();
     }
   }
   // value-free deltas: the product's input zd = colscale32 .* delta
@@ -1649,27 +1820,26 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
   if (zdelta) {
     ws.alloc(w.ZD0, sizeof(float) * n);
     ws.alloc(w.ZD1, sizeof(float) * n);
-    ZD[0] = w.ZD0.as<float>();
+    ZD[0] = in.zd = w.ZD0.as<float>();
     ZD[1] = w.ZD1.as<float>();
     if (sn)
-      hipLaunchKernelGGL(scale_into_f32_32, dim3(gN), dim3(256), 0, s, colscale32,
-                         static_cast<float>(x0), ZD[0], n);
+      in.zd_scale32 = colscale32;
     else
-      hipLaunchKernelGGL(scale_into_f32, dim3(gN), dim3(256), 0, s, colscale64, b0, ZD[0], n);
-    hipLaunchKernelGGL(fill_f32, dim3(gN), dim3(256), 0, s, ZD[1], n, 0.0f);
+      in.zd_scale64 = colscale64;
   }
   // (propagation-blocked runs form z = colscale .* x where they read it)
   if (!pbm && (pattern || (mixed && m.count_stochastic()))) {
     ws.alloc(w.Z, sizeof(double) * n);
-    hipLaunchKernelGGL(scale_into, dim3(gN), dim3(256), 0, s, colscale64, X[0], w.Z.as<double>(), n);
+    in.z = w.Z.as<double>();
+    in.z_scale = colscale64;
   }
+  hipLaunchKernelGGL(pr_init, dim3(gN), dim3(256), 0, s, in);
   TBSLA_HIP_CHECK(hipGetLastError());
-  // the set-up copies read pageable host memory (state, node set, 1/count)
-  TBSLA_HIP_CHECK(hipStreamSynchronize(s));
 
   // device time of the loop: HIP events, or (allocation-free runs, which
   // create no events) the host clock between two stream synchronisations
   hipEvent_t e0 = nullptr, e1 = nullptr;
+  if (arena) TBSLA_HIP_CHECK(hipStreamSynchronize(s));
   const auto h0 = std::chrono::steady_clock::now();
   if (!arena) {
     TBSLA_HIP_CHECK(hipEventCreate(&e0));
@@ -1681,19 +1851,39 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
   PrState hs{};
   int launched = 0;
   const bool mixed_pattern = mixed && m.count_stochastic();
-  auto fin_max = [&]() { hipLaunchKernelGGL(pr_finalize_max, dim3(1), dim3(kMaxSlots), 0, s, slots, st); };
-  auto fin_norm = [&](unsigned nb) {
-    hipLaunchKernelGGL(pr_finalize_norm, dim3(1), dim3(kTileThreads), 0, s, w.perr.as<double>(), w.ps.as<double>(),
-                       w.pc.as<double>(), static_cast<int>(nb), st);
-  };
+  // runs whose updates take the step decision of the iteration before: the
+  // tile products and the generic engine in one precision (their state
+  // alternates between two buffers).  On larger matrices than those with
+  // kMergeTileNnz-entry tiles the decision repeated in every block costs more
+  // than a launch of its own.
+  const bool merged = !pbm && !mixed && (!fused || d64.tile_nnz == kMergeTileNnz);
+  const auto state = [&](int it) { return merged ? st + (it & 1) : st; };
+  const SnPartials sp{w.perr.as<double>(), w.ps.as<double>(), w.pc.as<double>()};
+  const Partials parts{sp.perr, sp.ps, sp.pc, static_cast<int>(sn ? static_cast<unsigned>(pbm->nbins) : gM)};
+  const Partials none{sp.perr, sp.ps, sp.pc, 0};
   double *Z = w.Z.as<double>();
   const double *colscale = colscale64;
+  const auto normalize = [&](auto mode, double *xout, const double *xin, const float *dcur, float *dnext, float *zdnext,
+                             double *z, int it) {
+    hipLaunchKernelGGL(pr_normalize<decltype(mode)::value>, dim3(gM), dim3(1024), 0, s, xout, xin,
+                       w.xhat.as<double>(), dcur, dnext, z, colscale, zdnext, colscale32, n, state(it + 1),
+                       slots + (it & 1) * kMaxSlots, slots + ((it + 1) & 1) * kMaxSlots, sp.perr, sp.ps, sp.pc);
+  };
+  const auto decide = [&](PrState *to) {
+    hipLaunchKernelGGL(pr_finalize_norm, dim3(1), dim3(kTileThreads), 0, s, sp.perr, sp.ps, sp.pc,
+                       static_cast<int>(gM), to);
+  };
+  using std::integral_constant;
   auto launch_batch = [&](int batch) {
     for (int k = 0; k < batch; k++) {
       const int it = launched + k;
       double *xin = X[it & 1], *xout = X[(it + 1) & 1];
+      // the step decision of the iteration before is taken by this one, the
+      // last of the batch's by a launch of its own
+      const Partials &pp = k > 0 ? parts : none;
+      unsigned long long *const slot = slots + (it & 1) * kMaxSlots;
+      const StepArgs step = merged ? StepArgs{state(it), state(it + 1), pp} : StepArgs{st, nullptr, none};
       if (sn) {
-        const SnPartials sp{w.perr.as<double>(), w.ps.as<double>(), w.pc.as<double>()};
         if (mixed) {
           MxBufs b;
           b.am = AnchorMove{w.xhat.as<double>(), w.xhat32.as<float>(), D[it & 1], colscale, w.hsum.as<double>(),
@@ -1711,14 +1901,15 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
           else
             launch_pb_mx<double, dev::bf16, float, false>(tmode, *pbm, 0, 2, b, tp, st, sp, s);
         } else {
-          launch_pb(tmode, *pbm, colscale, xin, tp, xout, st, nullptr, &sp, s);
+          launch_pb(tmode, *pbm, colscale, xin, tp, xout, st, nullptr, &sp, pp, s);
         }
         // (the anchor move's sum partials: one per superblock of the anchor
         // product's scatter order)
         const int nsb_anchor = vfree ? pbm->nsb_w : pbm->nsb;
-        hipLaunchKernelGGL(pr_finalize_sn, dim3(1), dim3(kTileThreads), 0, s, sp.perr, sp.ps, sp.pc, pbm->nbins,
-                           mixed ? w.hsum.as<double>() : nullptr, mixed ? w.hcomp.as<double>() : nullptr, nsb_anchor,
-                           st);
+        if (mixed || k == batch - 1)
+          hipLaunchKernelGGL(pr_finalize_sn, dim3(1), dim3(kTileThreads), 0, s, sp.perr, sp.ps, sp.pc, pbm->nbins,
+                             mixed ? w.hsum.as<double>() : nullptr, mixed ? w.hcomp.as<double>() : nullptr,
+                             nsb_anchor, st);
       } else if (fused) {
         if (mixed) {
           float *dcur = D[it & 1], *dnext = D[(it + 1) & 1];
@@ -1734,59 +1925,46 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
             else
               launch_anchor<double>(d64, xhat, yhat, st, s);
             if (pat32)
-              launch_update<dev::Pattern, float, true>(tmode, d64, nullptr, zdcur, yhat, tp, xout, st, slots, s);
+              launch_update<dev::Pattern, float, true>(tmode, d64, nullptr, zdcur, yhat, tp, xout, step, slot, s);
             else if (p.precision == PrPrecision::F32)
-              launch_update<float, float, true>(tmode, *dlo, nullptr, dcur, yhat, tp, xout, st, slots, s);
+              launch_update<float, float, true>(tmode, *dlo, nullptr, dcur, yhat, tp, xout, step, slot, s);
             else
-              launch_update<dev::bf16, float, true>(tmode, *dlo, nullptr, dcur, yhat, tp, xout, st, slots, s);
+              launch_update<dev::bf16, float, true>(tmode, *dlo, nullptr, dcur, yhat, tp, xout, step, slot, s);
           }
-          fin_max();
           if (pat32)
-            hipLaunchKernelGGL(pr_normalize<3>, dim3(gM), dim3(kTileThreads), 0, s, xout, nullptr, xhat, dcur, dnext,
-                               nullptr, nullptr, zdnext, colscale32, n, st, w.perr.as<double>(),
-                               w.ps.as<double>(), w.pc.as<double>());
+            normalize(integral_constant<int, 3>(), xout, nullptr, dcur, dnext, zdnext, nullptr, it);
           else
-            hipLaunchKernelGGL(pr_normalize<1>, dim3(gM), dim3(kTileThreads), 0, s, xout, nullptr, xhat, dcur, dnext,
-                               nullptr, nullptr, nullptr, nullptr, n, st, w.perr.as<double>(), w.ps.as<double>(),
-                               w.pc.as<double>());
-          fin_norm(gM);
+            normalize(integral_constant<int, 1>(), xout, nullptr, dcur, dnext, nullptr, nullptr, it);
+          decide(st);
         } else if (pbm) {
-          launch_pb(tmode, *pbm, colscale, xin, tp, xout, st, slots, nullptr, s);
-          fin_max();
-          hipLaunchKernelGGL(pr_normalize<4>, dim3(gN), dim3(kTileThreads), 0, s, xout, xin, nullptr, nullptr, nullptr,
-                             nullptr, nullptr, nullptr, nullptr, n, st, w.perr.as<double>(), w.ps.as<double>(),
-                             w.pc.as<double>());
-          fin_norm(gN);
-        } else if (pattern) {
-          launch_update<dev::Pattern, double, false>(tmode, d64, nullptr, Z, nullptr, tp, xout, st, slots, s);
-          fin_max();
-          hipLaunchKernelGGL(pr_normalize<2>, dim3(gN), dim3(kTileThreads), 0, s, xout, xin, nullptr, nullptr,
-                             nullptr, Z, colscale, nullptr, nullptr, n, st, w.perr.as<double>(), w.ps.as<double>(),
-                             w.pc.as<double>());
-          fin_norm(gN);
+          launch_pb(tmode, *pbm, colscale, xin, tp, xout, st, slot, nullptr, pp, s);
+          normalize(integral_constant<int, 4>(), xout, xin, nullptr, nullptr, nullptr, nullptr, it);
+          if (k == batch - 1) decide(st);
         } else {
-          launch_update<double, double, false>(tmode, d64, p.values, xin, nullptr, tp, xout, st, slots, s);
-          fin_max();
-          hipLaunchKernelGGL(pr_normalize<0>, dim3(gN), dim3(kTileThreads), 0, s, xout, xin, nullptr, nullptr,
-                             nullptr, nullptr, nullptr, nullptr, nullptr, n, st, w.perr.as<double>(),
-                             w.ps.as<double>(), w.pc.as<double>());
-          fin_norm(gN);
+          if (pattern) {
+            launch_update<dev::Pattern, double, false>(tmode, d64, nullptr, Z, nullptr, tp, xout, step, slot, s);
+            normalize(integral_constant<int, 2>(), xout, xin, nullptr, nullptr, nullptr, Z, it);
+          } else {
+            launch_update<double, double, false>(tmode, d64, p.values, xin, nullptr, tp, xout, step, slot, s);
+            normalize(integral_constant<int, 0>(), xout, xin, nullptr, nullptr, nullptr, nullptr, it);
+          }
+          if (!merged || k == batch - 1) decide(state(it + 1));
         }
       } else {
         // any format: y = 0 (accumulating formats), y += A b_t, update, normalise
         hipLaunchKernelGGL(fill_f64, dim3(gN), dim3(256), 0, s, xout, n, 0.0);
         if (!d64.noop) launch_spmv(d64, xin, Dtype::F64, xout, Dtype::F64, 0, s);
         if (tmode == 1)
-          hipLaunchKernelGGL(pr_update_vec<1>, dim3(gN), dim3(kTileThreads), 0, s, xout, n, tp, st, slots);
+          hipLaunchKernelGGL(pr_update_vec<1>, dim3(gN), dim3(kTileThreads), 0, s, xout, n, tp, step.in, step.out, pp,
+                             slot);
         else if (tmode == 2)
-          hipLaunchKernelGGL(pr_update_vec<2>, dim3(gN), dim3(kTileThreads), 0, s, xout, n, tp, st, slots);
+          hipLaunchKernelGGL(pr_update_vec<2>, dim3(gN), dim3(kTileThreads), 0, s, xout, n, tp, step.in, step.out, pp,
+                             slot);
         else
-          hipLaunchKernelGGL(pr_update_vec<0>, dim3(gN), dim3(kTileThreads), 0, s, xout, n, tp, st, slots);
-        fin_max();
-        hipLaunchKernelGGL(pr_normalize<0>, dim3(gN), dim3(kTileThreads), 0, s, xout, xin, nullptr, nullptr,
-                           nullptr, nullptr, nullptr, nullptr, nullptr, n, st, w.perr.as<double>(),
-                           w.ps.as<double>(), w.pc.as<double>());
-        fin_norm(gN);
+          hipLaunchKernelGGL(pr_update_vec<0>, dim3(gN), dim3(kTileThreads), 0, s, xout, n, tp, step.in, step.out, pp,
+                             slot);
+        normalize(integral_constant<int, 0>(), xout, xin, nullptr, nullptr, nullptr, nullptr, it);
+        if (k == batch - 1) decide(state(it + 1));
       }
     }
     TBSLA_HIP_CHECK(hipGetLastError());
@@ -1809,7 +1987,7 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
     // allocation-free runs: the state is read after every batch
     while (launched < p.max_iteration) {
       launch_batch(std::min(next, p.max_iteration - launched));
-      TBSLA_HIP_CHECK(hipMemcpyAsync(&hs, st, sizeof(hs), hipMemcpyDeviceToHost, s));
+      TBSLA_HIP_CHECK(hipMemcpyAsync(&hs, state(launched), sizeof(hs), hipMemcpyDeviceToHost, s));
       TBSLA_HIP_CHECK(hipStreamSynchronize(s));
       if (hs.done) break;
       next = next_batch(hs, check);
@@ -1826,7 +2004,7 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
     auto enqueue = [&](int batch) {
       launch_batch(batch);
       const int sl = (head + npend) & 1;
-      TBSLA_HIP_CHECK(hipMemcpyAsync(hbuf + sl, st, sizeof(PrState), hipMemcpyDeviceToHost, s));
+      TBSLA_HIP_CHECK(hipMemcpyAsync(hbuf + sl, state(launched), sizeof(PrState), hipMemcpyDeviceToHost, s));
       TBSLA_HIP_CHECK(hipEventRecord(cev[sl], s));
       npend++;
     };
@@ -1854,11 +2032,9 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
   // final sum normalisation (Matrix.cpp:52-59), compensated
   const double *a = mixed ? w.xhat.as<double>() : X[it & 1];
   const float *dd = mixed ? D[it & 1] : nullptr;
-  hipLaunchKernelGGL(pr_sum_kernel, dim3(gN), dim3(kTileThreads), 0, s, a, dd, n, st, w.ps.as<double>(),
-                     w.pc.as<double>());
-  hipLaunchKernelGGL(pr_sum_finalize, dim3(1), dim3(kTileThreads), 0, s, w.ps.as<double>(), w.pc.as<double>(),
-                     static_cast<int>(gN), w.total.as<double>());
-  hipLaunchKernelGGL(pr_scale_kernel, dim3(gN), dim3(256), 0, s, a, dd, n, st, w.total.as<double>(), out_dev);
+  if (mixed && !sn)  // the state's sum is that of the FP64 update; the result's elements are rounded
+    hipLaunchKernelGGL(pr_sum_rounded, dim3(1), dim3(1024), 0, s, a, dd, n, st);
+  hipLaunchKernelGGL(pr_scale_kernel, dim3(gN), dim3(256), 0, s, a, dd, n, state(launched), out_dev);
   TBSLA_HIP_CHECK(hipGetLastError());
   TBSLA_HIP_CHECK(hipStreamSynchronize(s));
   float ms = 0;
@@ -1914,10 +2090,9 @@ std::size_t slice(std::size_t bytes) { return (std::max<std::size_t>(bytes, 1) +
 }  // namespace
 
 std::size_t page_rank_noalloc_bytes(long n, int n_nodes) {
-  const std::size_t gN = grid_for(n);
-  std::size_t b = slice(sizeof(PrState)) + slice(sizeof(unsigned long long) * kMaxSlots) +
-                  3 * slice(sizeof(double) * gN) + slice(sizeof(double)) +
-                  2 * slice(sizeof(double) * static_cast<std::size_t>(n));
+  const std::size_t gM = static_cast<std::size_t>(std::min<long>(kPassBlocks, (n + 1023) / 1024));
+  std::size_t b = slice(2 * sizeof(PrState)) + slice(2 * sizeof(unsigned long long) * kMaxSlots) +
+                  3 * slice(sizeof(double) * gM) + 2 * slice(sizeof(double) * static_cast<std::size_t>(n));
   if (n_nodes > 0) b += slice(static_cast<std::size_t>(n)) + slice(sizeof(int) * static_cast<std::size_t>(n_nodes));
   return b;
 }

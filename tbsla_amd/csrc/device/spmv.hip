@@ -42,20 +42,20 @@ struct StoreRow {
   }
 };
 
-template <typename VT, typename XT, typename YT>
+template <typename VT, typename XT, typename YT, int TN>
 __global__ __launch_bounds__(kTileThreads) void csr_tile_kernel(dev::CsrView<VT> m, const XT *__restrict__ x,
                                                                 YT *__restrict__ y) {
-  __shared__ dev::CsrTileLds<typename Val<VT>::A> lds;
+  __shared__ dev::CsrTileLds<typename Val<VT>::A, TN> lds;
   StoreRow<YT> epi{y};
-  dev::csr_tile_rows<VT, XT>(m, x, lds, epi);
+  dev::csr_tile_rows<VT, XT, TN>(m, x, lds, epi);
 }
 
 template <typename VT, typename XT, typename YT>
 __global__ __launch_bounds__(kTileThreads) void csr_long_kernel(dev::CsrView<VT> m, const XT *__restrict__ x,
                                                                 YT *__restrict__ y) {
-  __shared__ dev::CsrTileLds<typename Val<VT>::A> lds;
+  __shared__ dev::CsrTileLds<typename Val<VT>::A, kTileThreads> lds;
   StoreRow<YT> epi{y};
-  dev::csr_long_row<VT, XT>(m, x, lds, epi);
+  dev::csr_long_row<VT, XT, kTileThreads>(m, x, lds, epi);
 }
 
 // ELL: one row per thread, one workgroup per slice of kEllSlice rows, whose
@@ -145,16 +145,16 @@ struct AccRow {
   }
 };
 
-template <typename VT, typename XT, typename YT, bool LONG>
+template <typename VT, typename XT, typename YT, int TN, bool LONG>
 __global__ __launch_bounds__(kTileThreads) void coo_tile_kernel(dev::CsrView<VT> m, const XT *__restrict__ x,
                                                                 YT *__restrict__ y, const int *__restrict__ segrow,
                                                                 long y_off) {
-  __shared__ dev::CsrTileLds<typename Val<VT>::A> lds;
+  __shared__ dev::CsrTileLds<typename Val<VT>::A, TN> lds;
   AccRow<YT> epi{y, segrow, y_off};
-  if (LONG)
-    dev::csr_long_row<VT, XT>(m, x, lds, epi);
+  if constexpr (LONG)
+    dev::csr_long_row<VT, XT, TN>(m, x, lds, epi);
   else
-    dev::csr_tile_rows<VT, XT>(m, x, lds, epi);
+    dev::csr_tile_rows<VT, XT, TN>(m, x, lds, epi);
 }
 
 // kDenseRows consecutive rows per wavefront, so each x load serves all of
@@ -235,7 +235,10 @@ void run_typed(const DeviceMatrix &d, const XT *x, YT *y, int vect_incr, hipStre
     case cpp::FORMAT_CSR: {
       const dev::CsrView<VT> m = dev::csr_view<VT>(d);
       if (d.ntiles > 0)
-        hipLaunchKernelGGL((csr_tile_kernel<VT, XT, YT>), dim3(d.ntiles), dim3(kTileThreads), 0, s, m, x, y);
+        with_tile_size(d, [&](auto tn) {
+          hipLaunchKernelGGL((csr_tile_kernel<VT, XT, YT, decltype(tn)::value>), dim3(d.ntiles), dim3(kTileThreads), 0,
+                             s, m, x, y);
+        });
       if (d.nlong > 0)
         hipLaunchKernelGGL((csr_long_kernel<VT, XT, YT>), dim3(d.nlong), dim3(kTileThreads), 0, s, m, x, y);
       break;
@@ -252,10 +255,12 @@ void run_typed(const DeviceMatrix &d, const XT *x, YT *y, int vect_incr, hipStre
       const dev::CsrView<VT> m = dev::csr_view<VT>(d);
       const long y_off = vect_incr - (d.format == cpp::FORMAT_SCOO ? d.f_row : 0);
       if (d.ntiles > 0)
-        hipLaunchKernelGGL((coo_tile_kernel<VT, XT, YT, false>), dim3(d.ntiles), dim3(kTileThreads), 0, s, m, x, y,
-                           d.segrow.as<int>(), y_off);
+        with_tile_size(d, [&](auto tn) {
+          hipLaunchKernelGGL((coo_tile_kernel<VT, XT, YT, decltype(tn)::value, false>), dim3(d.ntiles),
+                             dim3(kTileThreads), 0, s, m, x, y, d.segrow.as<int>(), y_off);
+        });
       if (d.nlong > 0)
-        hipLaunchKernelGGL((coo_tile_kernel<VT, XT, YT, true>), dim3(d.nlong), dim3(kTileThreads), 0, s, m, x, y,
+        hipLaunchKernelGGL((coo_tile_kernel<VT, XT, YT, kTileThreads, true>), dim3(d.nlong), dim3(kTileThreads), 0, s, m, x, y,
                            d.segrow.as<int>(), y_off);
       break;
     }

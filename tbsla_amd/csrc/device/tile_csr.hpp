@@ -138,7 +138,7 @@ constexpr int kSumRun = 16;
 
 // TN: entries per tile (kCsrTileNnz unless a caller builds its own tile
 // table with another size); rows longer than TN / 2 go to csr_long_row.
-template <typename AT, int TN = kCsrTileNnz>
+template <typename AT, int TN>
 struct CsrTileLds {
   AT prod[TN + kSumRun];
 };
@@ -246,12 +246,20 @@ struct TileEntries {
   }
 };
 
+// Work of the caller's own that a tile does beside its loads: issue() (loads)
+// after the tile's index and value loads, finish() after its products, before
+// the barrier that precedes the row sums.
+struct NoPre {
+  __device__ void issue() {}
+  __device__ void finish() {}
+};
+
 // The bounds of the thread's first owned row, then the index/value loads,
 // gathers and products into prod.  (Issuing the row table first measured
 // faster than deferring it behind the tile loads.)
-template <bool FULL, typename VT, typename XT, int TN>
+template <bool FULL, typename VT, typename XT, int TN, typename Pre>
 __device__ inline void csr_tile_stage(const CsrView<VT> &m, const XT *__restrict__ x, typename Val<VT>::A *prod,
-                                      long e0, int ne, int rlo, int rhi, int &a, int &b) {
+                                      long e0, int ne, int rlo, int rhi, int &a, int &b, Pre &pre) {
   // loaded with no branch so they stay in flight under the tile loads
   // (indices clamped to rhi <= rows: in bounds, and exact for every thread
   // that owns a row)
@@ -259,17 +267,20 @@ __device__ inline void csr_tile_stage(const CsrView<VT> &m, const XT *__restrict
   b = m.rowptr[min(rlo + static_cast<int>(threadIdx.x) + 1, rhi)] - m.rp0;
   TileEntries<FULL, VT, XT, TN> t;
   t.load(m, e0, ne);
+  pre.issue();
   typename Val<VT>::A p[TileEntries<FULL, VT, XT, TN>::G][4];
   t.products(m, x, e0, ne, p);
+  pre.finish();
   TileEntries<FULL, VT, XT, TN>::store(p, prod, ne);
 }
 
 // Rows of entry tile `tile`; epi(row, sum) once per owned row by the thread
 // that sums it, rows longer than LT left to csr_long_row.  The caller
 // synchronises the block before reusing `lds`.
-template <typename VT, typename XT, typename Epi, int TN = kCsrTileNnz, int LT = TN / 2>
+template <typename VT, typename XT, typename Epi, int TN, int LT, typename Pre = NoPre>
 __device__ inline void csr_tile_rows_at(const CsrView<VT> &m, const XT *__restrict__ x,
-                                        CsrTileLds<typename Val<VT>::A, TN> &lds, Epi &epi, int tile) {
+                                        CsrTileLds<typename Val<VT>::A, TN> &lds, Epi &epi, int tile,
+                                        Pre &&pre = Pre()) {
 #pragma clang fp contract(off)
   using AT = typename Val<VT>::A;
   const int tid = threadIdx.x;
@@ -278,9 +289,9 @@ __device__ inline void csr_tile_rows_at(const CsrView<VT> &m, const XT *__restri
   const int rlo = m.tile_row[tile], rhi = m.tile_row[tile + 1];
   int a, b;
   if (ne == TN)
-    csr_tile_stage<true, VT, XT, TN>(m, x, lds.prod, e0, ne, rlo, rhi, a, b);
+    csr_tile_stage<true, VT, XT, TN>(m, x, lds.prod, e0, ne, rlo, rhi, a, b, pre);
   else
-    csr_tile_stage<false, VT, XT, TN>(m, x, lds.prod, e0, ne, rlo, rhi, a, b);
+    csr_tile_stage<false, VT, XT, TN>(m, x, lds.prod, e0, ne, rlo, rhi, a, b, pre);
   __syncthreads();
   const long e1 = e0 + ne;
   for (int r = rlo + tid; r < rhi; r += kTileThreads) {
@@ -315,16 +326,16 @@ __device__ inline void csr_tile_rows_at(const CsrView<VT> &m, const XT *__restri
 }
 
 // Rows of entry tile blockIdx.x.
-template <typename VT, typename XT, typename Epi>
+template <typename VT, typename XT, int TN, typename Epi, typename Pre = NoPre>
 __device__ inline void csr_tile_rows(const CsrView<VT> &m, const XT *__restrict__ x,
-                                     CsrTileLds<typename Val<VT>::A> &lds, Epi &epi) {
-  csr_tile_rows_at<VT, XT, Epi>(m, x, lds, epi, blockIdx.x);
+                                     CsrTileLds<typename Val<VT>::A, TN> &lds, Epi &epi, Pre &&pre = Pre()) {
+  csr_tile_rows_at<VT, XT, Epi, TN, kCsrLongRow>(m, x, lds, epi, blockIdx.x, pre);
 }
 
 // One long row (m.long_rows[idx]) per workgroup: chunk products (LC
 // entries per chunk), a fixed-order tree per chunk, chunk totals added in
 // order.  epi by thread 0.
-template <typename VT, typename XT, typename Epi, int TN = kCsrTileNnz, int LC = TN>
+template <typename VT, typename XT, typename Epi, int TN, int LC>
 __device__ inline void csr_long_row_at(const CsrView<VT> &m, const XT *__restrict__ x,
                                        CsrTileLds<typename Val<VT>::A, TN> &lds, Epi &epi, int idx) {
   using AT = typename Val<VT>::A;
@@ -340,10 +351,10 @@ __device__ inline void csr_long_row_at(const CsrView<VT> &m, const XT *__restric
   if (threadIdx.x == 0) epi(r, epi_init<AT>(epi, r, 0) + total);
 }
 
-template <typename VT, typename XT, typename Epi>
+template <typename VT, typename XT, int TN, typename Epi>
 __device__ inline void csr_long_row(const CsrView<VT> &m, const XT *__restrict__ x,
-                                    CsrTileLds<typename Val<VT>::A> &lds, Epi &epi) {
-  csr_long_row_at<VT, XT, Epi>(m, x, lds, epi, blockIdx.x);
+                                    CsrTileLds<typename Val<VT>::A, TN> &lds, Epi &epi) {
+  csr_long_row_at<VT, XT, Epi, TN, kCsrTileNnz>(m, x, lds, epi, blockIdx.x);
 }
 
 }  // namespace dev
