@@ -243,35 +243,35 @@ unsigned grid_for(long n) {
 
 template <typename VT, typename UT>
 void run_adjoint(const DeviceMatrix &d64, const DeviceMatrix &dT, const AdjointParams &p, const double *pr,
-                 const double *w, double *grad_values, double *grad_teleport, hipStream_t s, AdjointReport &rep) {
+                 const double *w, double *grad_values, double *grad_teleport, RunSpaces &spaces, hipStream_t s,
+                 AdjointReport &rep) {
   const long n = dT.rows;
   const long nnz = dT.entries;
   const unsigned gN = grid_for(n);
   const double *src = p.values ? p.values : d64.vals.as<double>();
-  DevBuf valsT, L0, L1, U, st, part, part_ap, part4;
-  valsT.alloc(sizeof(VT) * static_cast<std::size_t>(std::max(1L, nnz)));
-  L0.alloc(sizeof(double) * n);
-  L1.alloc(sizeof(double) * n);
-  U.alloc(sizeof(UT) * n);
-  st.alloc(sizeof(AdjState));
+  WsBuf valsT, L0, L1, U, st, part, part_ap, part4;
+  RunLayout ws;
+  ws.alloc(valsT, sizeof(VT) * static_cast<std::size_t>(std::max(1L, nnz)));
+  ws.alloc(L0, sizeof(double) * n);
+  ws.alloc(L1, sizeof(double) * n);
+  ws.alloc(U, sizeof(UT) * n);
+  ws.alloc(st, sizeof(AdjState));
   const int nparts = dT.ntiles + dT.nlong;
-  part.alloc(sizeof(double) * 4 * static_cast<std::size_t>(std::max(1, nparts)));
+  ws.alloc(part, sizeof(double) * 4 * static_cast<std::size_t>(std::max(1, nparts)));
   const int n_ap = d64.ntiles + d64.nlong;
-  part_ap.alloc(sizeof(double) * static_cast<std::size_t>(std::max(1, n_ap)));
-  part4.alloc(sizeof(double) * 4 * gN);
+  ws.alloc(part_ap, sizeof(double) * static_cast<std::size_t>(std::max(1, n_ap)));
+  ws.alloc(part4, sizeof(double) * 4 * gN);
+  std::unique_ptr<RunSpace> space = spaces.take(ws.bytes());
+  ws.place(space->mem.get());
 
   AdjState h{};
   h.beta = p.beta;
   h.eps = p.epsilon;
   h.inv_n = 1.0 / static_cast<double>(n);
   h.max_it = p.max_iteration;
-  TBSLA_HIP_CHECK(hipMemcpyAsync(st.get(), &h, sizeof(h), hipMemcpyHostToDevice, s));
+  TBSLA_HIP_CHECK(hipMemcpyAsync(st.p, &h, sizeof(h), hipMemcpyHostToDevice, s));
   AdjState *dst = st.as<AdjState>();
-
-  hipEvent_t e0, e1;
-  TBSLA_HIP_CHECK(hipEventCreate(&e0));
-  TBSLA_HIP_CHECK(hipEventCreate(&e1));
-  TBSLA_HIP_CHECK(hipEventRecord(e0, s));
+  TBSLA_HIP_CHECK(hipEventRecord(space->timing[0], s));
   if (nnz > 0)
     hipLaunchKernelGGL((adj_gather<VT>), dim3(grid_for(nnz)), dim3(256), 0, s, dT.perm.as<int>(), src,
                        valsT.as<VT>(), nnz);
@@ -290,7 +290,7 @@ void run_adjoint(const DeviceMatrix &d64, const DeviceMatrix &dT, const AdjointP
                      part4.as<double>());
   hipLaunchKernelGGL(adj_init, dim3(1), dim3(kTileThreads), 0, s, part_ap.as<double>(), n_ap, part4.as<double>(),
                      static_cast<int>(gN), dst);
-  TBSLA_HIP_CHECK(hipMemcpyAsync(L0.get(), w, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
+  TBSLA_HIP_CHECK(hipMemcpyAsync(L0.p, w, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
   TBSLA_HIP_CHECK(hipGetLastError());
   // the state copy above reads host memory
   TBSLA_HIP_CHECK(hipStreamSynchronize(s));
@@ -334,12 +334,11 @@ void run_adjoint(const DeviceMatrix &d64, const DeviceMatrix &dT, const AdjointP
     hipLaunchKernelGGL(adj_grad_values, dim3((d64.rows + 255) / 256), dim3(256), 0, s, d64.rowptr.as<int>(),
                        d64.colidx.as<int>(), d64.rows, d64.rp0, d64.f_col, lam, pr, grad_values, dst);
   TBSLA_HIP_CHECK(hipGetLastError());
-  TBSLA_HIP_CHECK(hipEventRecord(e1, s));
-  TBSLA_HIP_CHECK(hipEventSynchronize(e1));
+  TBSLA_HIP_CHECK(hipEventRecord(space->timing[1], s));
+  TBSLA_HIP_CHECK(hipEventSynchronize(space->timing[1]));
   float ms = 0;
-  TBSLA_HIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
-  (void)hipEventDestroy(e0);
-  (void)hipEventDestroy(e1);
+  TBSLA_HIP_CHECK(hipEventElapsedTime(&ms, space->timing[0], space->timing[1]));
+  spaces.give(std::move(space));
   rep.iterations = hs.it;
   rep.last_change = hs.norm > 0 ? hs.diff / hs.norm : 0.0;
   rep.s = hs.s;
@@ -362,9 +361,9 @@ AdjointReport page_rank_adjoint(const cpp::Matrix &m, const AdjointParams &p, co
   if (d64.x_need > n) throw std::invalid_argument("tbsla: column index beyond n_col");
   const DeviceMatrix &dT = transpose_mirror(m);
   if (p.precision == Dtype::F32)
-    run_adjoint<float, float>(d64, dT, p, pr, w, grad_values, grad_teleport, s, rep);
+    run_adjoint<float, float>(d64, dT, p, pr, w, grad_values, grad_teleport, m.device_cache().spaces, s, rep);
   else if (p.precision == Dtype::F64)
-    run_adjoint<double, double>(d64, dT, p, pr, w, grad_values, grad_teleport, s, rep);
+    run_adjoint<double, double>(d64, dT, p, pr, w, grad_values, grad_teleport, m.device_cache().spaces, s, rep);
   else
     throw std::invalid_argument("tbsla: the PageRank adjoint runs in F32 or F64");
   return rep;

@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstddef>
 #include <cstdint>
 #include <stdexcept>
@@ -67,10 +68,15 @@ class DevBuf {
 
   void alloc(std::size_t bytes) {
     if (bytes <= bytes_ && p_) return;
+    reserve(bytes);
+    TBSLA_HIP_CHECK(hipMemset(p_, 0, bytes_ + 256));
+  }
+  // alloc without clearing the memory
+  void reserve(std::size_t bytes) {
+    if (bytes <= bytes_ && p_) return;
     release();
     std::size_t padded = ((bytes ? bytes : 1) + 255 + 256) & ~std::size_t(255);
     TBSLA_HIP_CHECK(hipMalloc(&p_, padded));
-    TBSLA_HIP_CHECK(hipMemset(p_, 0, padded));
     bytes_ = padded - 256;
   }
   void upload(const void *src, std::size_t bytes, hipStream_t s = nullptr) {

@@ -33,6 +33,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "runspace.hpp"
 
 namespace tbsla {
 namespace hip {
@@ -173,6 +174,7 @@ struct DeviceCache {
   std::unique_ptr<DeviceMatrix> transposed;
   std::unique_ptr<PbMatrix> pb;
   DevBuf x_stage, y_stage;
+  RunSpaces spaces;  // memory of PageRank and adjoint runs, kept between them
   // the value of each column of a CSR matrix whose stored entries agree
   // within every column (fl(1/count) after fill_cqmat_stochastic), in FP64,
   // in FP32, and rounded to BF16 (held in FP32); 0 for a column with no

@@ -1501,48 +1501,9 @@ void launch_anchor(const DeviceMatrix &d, const double *x, double *yhat, const P
     hipLaunchKernelGGL((pr_anchor_spmv<VT, kTileThreads, true>), dim3(d.nlong), dim3(kTileThreads), 0, s, m, x, yhat, st);
 }
 
-// One device buffer of a run: owned (allocated for the run) or a slice of
-// the fixed scratch buffer of the allocation-free entry point.  Unlike
-// DevBuf, a slice is not cleared: every buffer below is written before it
-// is read.
-struct WsBuf {
-  DevBuf own;
-  void *p = nullptr;
-  template <class T>
-  T *as() const {
-    return static_cast<T *>(p);
-  }
-  void *get() const { return p; }
-};
-
-// Where a run's buffers come from: hipMalloc (arena == nullptr) or
-// consecutive 256-byte-aligned slices of `arena` (cap bytes), which is
-// never allocated or freed here.
-struct Workspace {
-  unsigned char *arena = nullptr;
-  std::size_t cap = 0, used = 0;
-  void alloc(WsBuf &b, std::size_t bytes) {
-    if (!arena) {
-      b.own.alloc(bytes);
-      b.p = b.own.get();
-      return;
-    }
-    const std::size_t need = (std::max<std::size_t>(bytes, 1) + 255) & ~std::size_t(255);
-    if (need > cap - used)
-      throw std::invalid_argument("tbsla: the allocation-free PageRank needs more than its " +
-                                  std::to_string(cap >> 20) + " MiB scratch buffer");
-    b.p = arena + used;
-    used += need;
-  }
-  void upload(WsBuf &b, const void *src, std::size_t bytes, hipStream_t s) {
-    alloc(b, bytes);
-    if (bytes) TBSLA_HIP_CHECK(hipMemcpyAsync(b.p, src, bytes, hipMemcpyHostToDevice, s));
-  }
-};
-
 struct Scratch {
   WsBuf st, slots, perr, ps, pc, member, nodes, hsum, hcomp;
-  WsBuf X0, X1, Z, yhat, xhat, xhat32, D0, D1, ZD0, ZD1, W;
+  WsBuf X0, X1, Z, yhat, xhat, xhat32, D0, D1, ZD0, ZD1, W, out;
 };
 
 // One block: the step decision of a sum-normalised propagation-blocked
@@ -1633,11 +1594,12 @@ int iterations_left(const PrState &h, int check) {
 
 namespace {
 
-// The engine.  arena != nullptr: every buffer of the run is a slice of the
+// The engine.  The result goes to out_dev, or (out_dev == nullptr) to a buffer
+// of the run, and from there to out_host if given.  arena != nullptr: every buffer of the run is a slice of the
 // arena (cap bytes) and nothing is allocated (the caller has checked that
 // the mirror exists and that no lazily built layout is needed).
-PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, double *out_dev, hipStream_t s,
-                             unsigned char *arena, std::size_t cap) {
+PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, double *out_dev, double *out_host,
+                             hipStream_t s, unsigned char *arena, std::size_t cap) {
   const long n = m.get_n_col();
   // (COO keeps NR/NC in ln_row/ln_col, MatrixCOO.cpp:344-345, so the block
   // layout is read from NR/NC)
@@ -1687,7 +1649,7 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
   if (!use_pb && p.precision == PrPrecision::F32) dlo = &mirror(m, Dtype::F32);
   if (!use_pb && p.precision == PrPrecision::BF16) dlo = &mirror(m, Dtype::BF16);
   Scratch w;
-  Workspace ws{arena, cap, 0};
+  RunLayout ws;
   const unsigned gN = grid_for(n);
   // blocks of the normalise pass.  The mixed one (six streams) measured
   // faster with twice the blocks (four and eight times: slower); the FP64 one
@@ -1715,11 +1677,51 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
   const double b0 = p.personalized && !p.teleport ? 0.25 : 1.0;
   if (tmode == 1) {
     ws.alloc(w.member, static_cast<std::size_t>(n));
+    ws.alloc(w.nodes, sizeof(int) * static_cast<std::size_t>(std::max(0, p.n_nodes)));
+  }
+  if (mixed) {
+    ws.alloc(w.xhat, sizeof(double) * n);
+    ws.alloc(w.D0, sizeof(float) * n);
+    ws.alloc(w.D1, sizeof(float) * n);
+    if (sn) {
+      // the anchor's FP32 one-step change and FP32 copy, and the scatter's
+      // per-superblock sums of a moved anchor
+      ws.alloc(w.W, sizeof(float) * n);
+      ws.alloc(w.xhat32, sizeof(float) * n);
+      ws.alloc(w.hsum, sizeof(double) * std::max(1, pbm->nsb));
+      ws.alloc(w.hcomp, sizeof(double) * std::max(1, pbm->nsb));
+    } else {
+      ws.alloc(w.yhat, sizeof(double) * n);
+    }
+  }
+  // value-free deltas: the product's input zd = colscale32 .* delta
+  const bool zdelta = pat32 || (pb_mixed && vfree);
+  if (zdelta) {
+    ws.alloc(w.ZD0, sizeof(float) * n);
+    ws.alloc(w.ZD1, sizeof(float) * n);
+  }
+  // (propagation-blocked runs form z = colscale .* x where they read it)
+  const bool stored_z = !pbm && (pattern || (mixed && m.count_stochastic()));
+  if (stored_z) ws.alloc(w.Z, sizeof(double) * n);
+  if (!out_dev) ws.alloc(w.out, sizeof(double) * n);
+  std::unique_ptr<RunSpace> space;
+  if (arena) {
+    if (ws.bytes() > cap)
+      throw std::invalid_argument("tbsla: the allocation-free PageRank needs more than its " +
+                                  std::to_string(cap >> 20) + " MiB scratch buffer");
+    ws.place(arena);
+  } else {
+    space = m.device_cache().spaces.take(ws.bytes());
+    ws.place(space->mem.get());
+  }
+  if (!out_dev) out_dev = w.out.as<double>();
+  if (tmode == 1) {
     hipLaunchKernelGGL(fill_u8, dim3(grid_for(n)), dim3(256), 0, s, w.member.as<unsigned char>(), n,
                        static_cast<unsigned char>(0));
     if (p.n_nodes > 0) {
       // (p.nodes stays valid until the run has ended)
-      ws.upload(w.nodes, p.nodes, sizeof(int) * static_cast<std::size_t>(p.n_nodes), s);
+      TBSLA_HIP_CHECK(hipMemcpyAsync(w.nodes.p, p.nodes, sizeof(int) * static_cast<std::size_t>(p.n_nodes),
+                                     hipMemcpyHostToDevice, s));
       hipLaunchKernelGGL(set_members, dim3(grid_for(p.n_nodes)), dim3(256), 0, s, w.member.as<unsigned char>(), n,
                          w.nodes.as<int>(), p.n_nodes);
     }
@@ -1794,42 +1796,26 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
   unsigned long long *const slots = w.slots.as<unsigned long long>();
   float *D[2] = {nullptr, nullptr};
   if (mixed) {
-    ws.alloc(w.xhat, sizeof(double) * n);
-    ws.alloc(w.D0, sizeof(float) * n);
-    ws.alloc(w.D1, sizeof(float) * n);
     D[0] = in.d = w.D0.as<float>();
     D[1] = w.D1.as<float>();
     in.xhat = w.xhat.as<double>();
     if (sn) {
-      // the anchor's FP32 one-step change (0 before the first anchor, whose
-      // anchor is 0) and the scatter's per-superblock sums of a moved anchor
-      ws.alloc(w.W, sizeof(float) * n);
-      ws.alloc(w.xhat32, sizeof(float) * n);
+      // (w is 0 before the first anchor, whose anchor is 0)
       in.w = w.W.as<float>();
       in.xhat32 = w.xhat32.as<float>();
-      ws.alloc(w.hsum, sizeof(double) * std::max(1, pbm->nsb));
-      ws.alloc(w.hcomp, sizeof(double) * std::max(1, pbm->nsb));
     } else {
-      ws.alloc(w.yhat, sizeof(double) * n);
       in.yhat = w.yhat.as<double>();
     }
   }
-  // value-free deltas: the product's input zd = colscale32 .* delta
-  const bool zdelta = pat32 || (pb_mixed && vfree);
-  float *ZD[2] = {nullptr, nullptr};
+  float *ZD[2] = {w.ZD0.as<float>(), w.ZD1.as<float>()};
   if (zdelta) {
-    ws.alloc(w.ZD0, sizeof(float) * n);
-    ws.alloc(w.ZD1, sizeof(float) * n);
-    ZD[0] = in.zd = w.ZD0.as<float>();
-    ZD[1] = w.ZD1.as<float>();
+    in.zd = ZD[0];
     if (sn)
       in.zd_scale32 = colscale32;
     else
       in.zd_scale64 = colscale64;
   }
-  // (propagation-blocked runs form z = colscale .* x where they read it)
-  if (!pbm && (pattern || (mixed && m.count_stochastic()))) {
-    ws.alloc(w.Z, sizeof(double) * n);
+  if (stored_z) {
     in.z = w.Z.as<double>();
     in.z_scale = colscale64;
   }
@@ -1838,14 +1824,9 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
 
   // device time of the loop: HIP events, or (allocation-free runs, which
   // create no events) the host clock between two stream synchronisations
-  hipEvent_t e0 = nullptr, e1 = nullptr;
   if (arena) TBSLA_HIP_CHECK(hipStreamSynchronize(s));
   const auto h0 = std::chrono::steady_clock::now();
-  if (!arena) {
-    TBSLA_HIP_CHECK(hipEventCreate(&e0));
-    TBSLA_HIP_CHECK(hipEventCreate(&e1));
-    TBSLA_HIP_CHECK(hipEventRecord(e0, s));
-  }
+  if (space) TBSLA_HIP_CHECK(hipEventRecord(space->timing[0], s));
   const int check = fused ? std::max(1, p.check_every) : 1;
   int next = check;  // iterations in the next launch batch
   PrState hs{};
@@ -1970,19 +1951,6 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
     TBSLA_HIP_CHECK(hipGetLastError());
     launched += batch;
   };
-  // pinned state copies of the two batches in flight and their events
-  // (released on every exit; the stream has drained by then or the run failed)
-  struct ReadBack {
-    PrState *hbuf = nullptr;
-    hipEvent_t cev[2] = {nullptr, nullptr};
-    ~ReadBack() {
-      if (hbuf) (void)hipHostFree(hbuf);
-      for (hipEvent_t e : cev)
-        if (e) (void)hipEventDestroy(e);
-    }
-  } rb;
-  PrState *&hbuf = rb.hbuf;
-  hipEvent_t *cev = rb.cev;
   if (arena) {
     // allocation-free runs: the state is read after every batch
     while (launched < p.max_iteration) {
@@ -1998,8 +1966,9 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
     // state, the next batch is already queued when the state read before
     // predicts more iterations than are in flight, so the GPU does not idle
     // at the reads (kernels launched past convergence return at once).
-    TBSLA_HIP_CHECK(hipHostMalloc(reinterpret_cast<void **>(&hbuf), 2 * sizeof(PrState), hipHostMallocDefault));
-    for (int k = 0; k < 2; k++) TBSLA_HIP_CHECK(hipEventCreateWithFlags(&cev[k], hipEventDisableTiming));
+    static_assert(2 * sizeof(PrState) <= kReadBackBytes, "two states fit the read-back buffer");
+    PrState *const hbuf = static_cast<PrState *>(space->pinned);
+    hipEvent_t *const cev = space->ready;
     int head = 0, npend = 0;  // slot of the oldest batch in flight, batches in flight
     auto enqueue = [&](int batch) {
       launch_batch(batch);
@@ -2026,7 +1995,7 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
       if (npend == 0 && launched < p.max_iteration) enqueue(std::min(next_batch(hs, check), p.max_iteration - launched));
     }
   }
-  if (!arena) TBSLA_HIP_CHECK(hipEventRecord(e1, s));
+  if (space) TBSLA_HIP_CHECK(hipEventRecord(space->timing[1], s));
   const double host_seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - h0).count();
   const int it = hs.it;
   // final sum normalisation (Matrix.cpp:52-59), compensated
@@ -2036,12 +2005,14 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
     hipLaunchKernelGGL(pr_sum_rounded, dim3(1), dim3(1024), 0, s, a, dd, n, st);
   hipLaunchKernelGGL(pr_scale_kernel, dim3(gN), dim3(256), 0, s, a, dd, n, state(launched), out_dev);
   TBSLA_HIP_CHECK(hipGetLastError());
+  if (out_host)
+    TBSLA_HIP_CHECK(hipMemcpyAsync(out_host, out_dev, sizeof(double) * static_cast<std::size_t>(n),
+                                   hipMemcpyDeviceToHost, s));
   TBSLA_HIP_CHECK(hipStreamSynchronize(s));
   float ms = 0;
-  if (!arena) {
-    TBSLA_HIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
+  if (space) {
+    TBSLA_HIP_CHECK(hipEventElapsedTime(&ms, space->timing[0], space->timing[1]));
+    m.device_cache().spaces.give(std::move(space));
   }
   rep.iterations = it;
   rep.anchors = hs.anchors;
@@ -2054,7 +2025,7 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
 }  // namespace
 
 PageRankReport page_rank_device(const cpp::Matrix &m, const PageRankParams &p, double *out_dev, hipStream_t s) {
-  return run_page_rank(m, p, out_dev, s, nullptr, 0);
+  return run_page_rank(m, p, out_dev, nullptr, s, nullptr, 0);
 }
 
 // ---- allocation-free PageRank ----------------------------------------------
@@ -2116,16 +2087,11 @@ PageRankReport page_rank_device_noalloc(const cpp::Matrix &m, const PageRankPara
                                 "tbsla_hip_prepare(m, TBSLA_F64) first");
   PageRankParams q = p;
   q.gather = 1;
-  return run_page_rank(m, q, out_dev, s, scratch_of_current_device(), kNoAllocScratchBytes);
+  return run_page_rank(m, q, out_dev, nullptr, s, scratch_of_current_device(), kNoAllocScratchBytes);
 }
 
 PageRankReport page_rank(const cpp::Matrix &m, const PageRankParams &p, double *out) {
-  const long n = m.get_n_col();
-  DevBuf o;
-  o.alloc(sizeof(double) * static_cast<std::size_t>(std::max(1L, n)));
-  PageRankReport r = page_rank_device(m, p, o.as<double>(), nullptr);
-  if (n > 0) TBSLA_HIP_CHECK(hipMemcpy(out, o.get(), sizeof(double) * static_cast<std::size_t>(n), hipMemcpyDeviceToHost));
-  return r;
+  return run_page_rank(m, p, nullptr, out, nullptr, nullptr, 0);
 }
 
 }  // namespace hip
