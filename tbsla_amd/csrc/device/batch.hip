@@ -39,7 +39,9 @@ constexpr int kChunkRows = 2048;     // rows per pass item, single-RHS graphs
 constexpr int kBatchTiles[3] = {1024, 2048, 3072};
 constexpr int kBatchLongRow = 512;
 constexpr int kBatchLongChunk = 1024;
-constexpr int kSpmmChunkRows = 1024;  // rows per pass item, SpMM groups
+// rows per pass item of an SpMM group: 64 to 1024, so that a group has about
+// 2048 items (each leaves a partial per RHS to merge)
+int spmm_chunk_rows(int rows) { return std::max(64, std::min(1024, (rows / 2048 + 63) / 64 * 64)); }
 constexpr int kMaxGroups = 64;
 constexpr int kQueues = 8;           // one per XCD
 
@@ -47,7 +49,7 @@ int tile_index(int tile_nnz) { return tile_nnz == 1024 ? 0 : (tile_nnz == 3072 ?
 int rpw_index(int spmm_rows) { return spmm_rows == 32 ? 0 : (spmm_rows == 128 ? 2 : 1); }
 
 struct RhsState {
-  double tele_scale, tele, maxv, err, sum, sum_prev, bound, total;
+  double tele_scale, tele, err, sum, sum_prev, bound;
   int it, done, pad0, pad1;
 };
 
@@ -86,7 +88,8 @@ struct BatchDev {
   XT *xa0, *xa1, *xb0, *xb1;  // iterate buffers by parity
   const SpmmGroup<VT> *g;     // n_groups descriptors (device memory)
   RhsState *rs;
-  unsigned long long *slots;
+  int n_rhs_total;
+  unsigned long long *slots;  // kSlots per RHS, two sets (by parity)
   const int *q_items;
   const int *q_off;           // kQueues + 1 queue boundaries in q_items
   int xcd_map;
@@ -361,6 +364,12 @@ void batch_step(BatchDev<VT, XT> d, int par) {
   using AT = typename dev::Val<VT>::A;
   __shared__ dev::CsrTileLds<AT, TN> lds;
   __shared__ double red[kTileThreads];
+  {  // nothing left to do once every set is done (a replay may run on past it)
+    int active = 0;
+    for (int r = threadIdx.x; r < d.n_rhs_total; r += kTileThreads) active |= !d.rs[r].done;
+    if (!__syncthreads_or(active)) return;
+  }
+  d.slots += static_cast<long>(par) * kSlots * d.n_rhs_total;
   const XT *xa_in = par ? d.xa1 : d.xa0, *xb_in = par ? d.xb1 : d.xb0;
   XT *xa_out = par ? d.xa0 : d.xa1, *xb_out = par ? d.xb0 : d.xb1;
   int q, local, stride;
@@ -409,58 +418,65 @@ void batch_step(BatchDev<VT, XT> d, int par) {
   }
 }
 
-// One wavefront per RHS: max over its slots (cleared for the next step).
-__global__ __launch_bounds__(64) void batch_finalize_max(RhsState *rs, unsigned long long *slots) {
-  const int r = blockIdx.x, l = threadIdx.x;
-  if (rs[r].done) return;
-  unsigned long long u = 0;
-  if (l < kSlots) {
-    u = __hip_atomic_load(slots + r * kSlots + l, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(slots + r * kSlots + l, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    const unsigned long long o = __shfl_xor(u, off, 64);
-    u = o > u ? o : u;
-  }
-  if (l == 0) rs[r].maxv = ord_decode(u);
-}
-
-// MODE 0: normalise the step's output (b /= max, residual, compensated sum).
-// MODE 1: compensated sum of each RHS's final iterate.
-// MODE 2: out = final iterate / total.
-template <typename VT, typename XT, int MODE>
-__global__ __launch_bounds__(kTileThreads) void batch_pass(BatchDev<VT, XT> d, const PassItem *__restrict__ items,
-                                                           PassPart *__restrict__ part,
-                                                           const long *__restrict__ out_off,
-                                                           double *__restrict__ out, int par) {
+// Normalise pass: b /= max, residual against the previous iterate and
+// compensated sum, one partial per item (SpMM: per item and RHS).  The
+// maximum of each RHS is taken from its slots by every block; the block of
+// the RHS's first item clears the other set, the next step's.
+//
+// Bound by its three streams of the iterates (read, read, write).  SpMM
+// items: 16 lanes per row, an RHS quad each (16-byte accesses in FP32), U
+// rows per lane loaded before any is used.  With one RHS per lane and one row
+// at a time the pass over 2^20 rows x 64 FP32 sets and 48 single graphs took
+// 296 us; 173 us now, 4.7 TB/s.
+template <typename VT, typename XT>
+__global__ __launch_bounds__(kTileThreads) void batch_normalize(BatchDev<VT, XT> d, const PassItem *__restrict__ items,
+                                                                PassPart *__restrict__ part, int par) {
 #pragma clang fp contract(off)
   __shared__ double red_e[kTileThreads], red_s[kTileThreads], red_c[kTileThreads];
+  __shared__ double smax[kLanes];
   const PassItem it = items[blockIdx.x];
+  const long set = static_cast<long>(kSlots) * d.n_rhs_total;
+  const unsigned long long *slots = d.slots + par * set;
+  unsigned long long *next = d.slots + (1 - par) * set;
   if (it.kind == 0) {
     const int g = it.id;
     const RhsState &st = d.rs[g];
-    if (MODE == 0 && st.done) return;
-    XT *cur = MODE == 0 ? (par ? d.xa0 : d.xa1) : ((st.it & 1) ? d.xa1 : d.xa0);
+    if (st.done) return;
+    XT *cur = par ? d.xa0 : d.xa1;
     const XT *prev = par ? d.xa1 : d.xa0;
-    const double m = st.maxv, S = st.total;
+    constexpr int U = kChunkRows / kTileThreads;  // the item's rows of a thread
+    XT cv[U], pv[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int i = min(it.r0 + static_cast<int>(threadIdx.x) + u * kTileThreads, it.r1 - 1);
+      cv[u] = cur[i];
+      pv[u] = prev[i];
+    }
+    if (threadIdx.x < 64) {
+      unsigned long long s = threadIdx.x < kSlots ? slots[g * kSlots + threadIdx.x] : 0ull;
+#pragma unroll
+      for (int off = kSlots / 2; off > 0; off >>= 1) {
+        const unsigned long long o = __shfl_xor(s, off, 64);
+        s = o > s ? o : s;
+      }
+      if (threadIdx.x == 0) smax[0] = ord_decode(s);
+      if (it.r0 == d.row_base[g] && threadIdx.x < kSlots) next[g * kSlots + threadIdx.x] = 0;
+    }
+    __syncthreads();
+    const double m = smax[0];
     double err = 0;
     CSum cs{0, 0};
-    const long o = out_off[g] - d.row_base[g];
-    for (int i = it.r0 + threadIdx.x; i < it.r1; i += kTileThreads) {
-      if (MODE == 0) {
-        const XT bs = static_cast<XT>(static_cast<double>(cur[i]) / m);
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int i = it.r0 + static_cast<int>(threadIdx.x) + u * kTileThreads;
+      if (i < it.r1) {
+        const XT bs = static_cast<XT>(static_cast<double>(cv[u]) / m);
         const double bi = static_cast<double>(bs);
-        err += fabs(bi - static_cast<double>(prev[i]));
+        err += fabs(bi - static_cast<double>(pv[u]));
         csum_add(cs, bi);
         cur[i] = bs;
-      } else if (MODE == 1) {
-        csum_add(cs, static_cast<double>(cur[i]));
-      } else {
-        out[o + i] = static_cast<double>(cur[i]) / S;
       }
     }
-    if (MODE == 2) return;
     err = dev::block_tree_sum<double>(err, red_e);
     // compensated merge across the block, fixed order
     red_s[threadIdx.x] = cs.s;
@@ -478,67 +494,176 @@ __global__ __launch_bounds__(kTileThreads) void batch_pass(BatchDev<VT, XT> d, c
     if (threadIdx.x == 0) part[it.part] = PassPart{err, red_s[0], red_c[0]};
     return;
   }
-  // SpMM group: wave w takes rows r0 + w, r0 + w + 4, ...; lane = RHS
+  // SpMM group: rows r0 + 4 * wave + sub, 16 apart; lane quad q = RHS 4q .. 4q + 3
   const SpmmGroup<VT> &G = d.g[it.id];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int rhs = G.rhs_base + lane;
-  const bool valid = lane < G.n_rhs;
-  const RhsState *st = valid ? &d.rs[rhs] : nullptr;
-  const bool active = valid && (MODE != 0 || !st->done);
-  double err = 0;
-  CSum cs{0, 0};
-  if (active) {
-    XT *cur = (MODE == 0 ? (par ? d.xb0 : d.xb1) : ((st->it & 1) ? d.xb1 : d.xb0)) + G.xoff;
-    const XT *prev = (par ? d.xb1 : d.xb0) + G.xoff;
-    const double m = st->maxv, S = st->total;
-    for (int i = it.r0 + wave; i < it.r1; i += 4) {
-      const long k = static_cast<long>(i) * kLanes + lane;
-      if (MODE == 0) {
-        const XT bs = static_cast<XT>(static_cast<double>(cur[k]) / m);
-        const double bi = static_cast<double>(bs);
-        err += fabs(bi - static_cast<double>(prev[k]));
-        csum_add(cs, bi);
-        cur[k] = bs;
-      } else if (MODE == 1) {
-        csum_add(cs, static_cast<double>(cur[k]));
-      } else {
-        out[out_off[rhs] + i] = static_cast<double>(cur[k]) / S;
+  const int sub = lane >> 4, q = lane & 15;
+  const int n_rhs = G.n_rhs, rhs0 = G.rhs_base;
+  {
+    constexpr int P = kTileThreads / kLanes;  // threads per RHS
+    const int j = threadIdx.x / P, k0 = (threadIdx.x % P) * (kSlots / P);
+    unsigned long long s = 0;
+    if (j < n_rhs)
+#pragma unroll
+      for (int k = 0; k < kSlots / P; k++) {
+        const unsigned long long o = slots[(rhs0 + j) * kSlots + k0 + k];
+        s = o > s ? o : s;
+        if (it.r0 == 0) next[(rhs0 + j) * kSlots + k0 + k] = 0;
       }
+#pragma unroll
+    for (int off = P / 2; off > 0; off >>= 1) {
+      const unsigned long long o = __shfl_xor(s, off, 64);
+      s = o > s ? o : s;
+    }
+    if (threadIdx.x % P == 0) smax[j] = ord_decode(s);
+  }
+  __syncthreads();
+  bool act[4];
+  double m[4], err[4] = {0, 0, 0, 0};
+  CSum cs[4] = {};
+  bool any = false, all = true;
+#pragma unroll
+  for (int t = 0; t < 4; t++) {
+    act[t] = 4 * q + t < n_rhs && !d.rs[rhs0 + 4 * q + t].done;
+    m[t] = smax[4 * q + t];
+    any = any || act[t];
+    all = all && act[t];
+  }
+  XT *cur = (par ? d.xb0 : d.xb1) + G.xoff + 4 * q;
+  const XT *prev = (par ? d.xb1 : d.xb0) + G.xoff + 4 * q;
+  constexpr int U = sizeof(XT) == 4 ? 4 : 2;
+  if (any)
+    for (int i0 = it.r0 + wave * 4 + sub; i0 < it.r1; i0 += 16 * U) {
+      XT cv[U][4], pv[U][4];
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const long k = static_cast<long>(min(i0 + 16 * u, it.r1 - 1)) * kLanes;
+        Quad<XT>::load(cur + k, cv[u]);
+        Quad<XT>::load(prev + k, pv[u]);
+      }
+#pragma unroll
+      for (int u = 0; u < U; u++)
+        if (i0 + 16 * u < it.r1) {
+#pragma unroll
+          for (int t = 0; t < 4; t++) {
+            const XT bs = static_cast<XT>(static_cast<double>(cv[u][t]) / m[t]);
+            const double bi = static_cast<double>(bs);
+            err[t] += fabs(bi - static_cast<double>(pv[u][t]));
+            csum_add(cs[t], bi);
+            cv[u][t] = bs;
+          }
+          XT *p = cur + static_cast<long>(i0 + 16 * u) * kLanes;
+          if (all) {
+            Quad<XT>::store(p, cv[u]);
+          } else {
+#pragma unroll
+            for (int t = 0; t < 4; t++)
+              if (act[t]) p[t] = cv[u][t];
+          }
+        }
+    }
+  // the four rows of a wavefront, then the four wavefronts, in a fixed order
+#pragma unroll
+  for (int t = 0; t < 4; t++) {
+#pragma unroll
+    for (int off = 16; off <= 32; off <<= 1) {
+      err[t] += __shfl_xor(err[t], off, 64);
+      cs[t] = csum_merge(cs[t], CSum{__shfl_xor(cs[t].s, off, 64), __shfl_xor(cs[t].c, off, 64)});
+    }
+    if (sub == 0) {
+      red_e[wave * 64 + 4 * q + t] = err[t];
+      red_s[wave * 64 + 4 * q + t] = cs[t].s;
+      red_c[wave * 64 + 4 * q + t] = cs[t].c;
     }
   }
-  if (MODE == 2) return;
-  red_e[threadIdx.x] = err;
-  red_s[threadIdx.x] = cs.s;
-  red_c[threadIdx.x] = cs.c;
   __syncthreads();
-  if (wave == 0) {
+  if (wave == 0 && lane < n_rhs && !d.rs[rhs0 + lane].done) {
     double e = red_e[lane];
     CSum t{red_s[lane], red_c[lane]};
     for (int w = 1; w < 4; w++) {
       e += red_e[w * 64 + lane];
       t = csum_merge(t, CSum{red_s[w * 64 + lane], red_c[w * 64 + lane]});
     }
-    if (active) part[it.part + lane] = PassPart{e, t.s, t.c};
+    part[it.part + lane] = PassPart{e, t.s, t.c};
   }
 }
 
-// One wavefront per RHS: merge its partials in a fixed order.  FINAL = 0:
-// the step decision (reference residual or sum-normalised bound) and the
-// next teleport term; FINAL = 1: the total of the final iterate.
-template <int FINAL>
+// out = final iterate / its sum (FP64), each RHS's vector contiguous.  An
+// SpMM group's iterate is row-major (n x 64): tiles of 64 rows are turned
+// through LDS, so each store is 64 consecutive rows of one RHS.  Stored
+// straight from the row-major order, 8 bytes to each of 64 vectors per
+// wavefront, 2^20 rows x 64 sets took 2058 us; 312 us so.
+template <typename VT, typename XT>
+__global__ __launch_bounds__(kTileThreads) void batch_output(BatchDev<VT, XT> d, const PassItem *__restrict__ items,
+                                                             const long *__restrict__ out_off,
+                                                             double *__restrict__ out) {
+  __shared__ XT tile[kLanes][kLanes + 1];
+  const PassItem it = items[blockIdx.x];
+  if (it.kind == 0) {
+    const int g = it.id;
+    const RhsState &st = d.rs[g];
+    const XT *cur = (st.it & 1) ? d.xa1 : d.xa0;
+    const double S = st.sum;
+    const long o = out_off[g] - d.row_base[g];
+    for (int i = it.r0 + threadIdx.x; i < it.r1; i += kTileThreads) out[o + i] = static_cast<double>(cur[i]) / S;
+    return;
+  }
+  const SpmmGroup<VT> &G = d.g[it.id];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int sub = lane >> 4, q = lane & 15;
+  const int n_rhs = G.n_rhs, rhs0 = G.rhs_base;
+  // which buffer holds each RHS's final iterate (its own parity)
+  bool odd[4], any0 = false, any1 = false;
+#pragma unroll
+  for (int t = 0; t < 4; t++) {
+    odd[t] = 4 * q + t < n_rhs && (d.rs[rhs0 + 4 * q + t].it & 1);
+    any0 = any0 || (4 * q + t < n_rhs && !odd[t]);
+    any1 = any1 || odd[t];
+  }
+  const XT *x0 = d.xb0 + G.xoff + 4 * q, *x1 = d.xb1 + G.xoff + 4 * q;
+  for (int r0 = it.r0; r0 < it.r1; r0 += kLanes) {
+    XT v0[4][4] = {}, v1[4][4] = {};
+#pragma unroll
+    for (int u = 0; u < 4; u++) {  // rows r0 + 16 * wave + 4 * u + sub
+      const long k = static_cast<long>(min(r0 + 16 * wave + 4 * u + sub, it.r1 - 1)) * kLanes;
+      if (any0) Quad<XT>::load(x0 + k, v0[u]);
+      if (any1) Quad<XT>::load(x1 + k, v1[u]);
+    }
+    __syncthreads();  // (the tile's readers of the round before)
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+#pragma unroll
+      for (int t = 0; t < 4; t++) tile[4 * q + t][16 * wave + 4 * u + sub] = odd[t] ? v1[u][t] : v0[u][t];
+    __syncthreads();
+    const int i = r0 + lane;
+    for (int j = wave; j < n_rhs; j += 4)
+      if (i < it.r1) out[out_off[rhs0 + j] + i] = static_cast<double>(tile[j][lane]) / d.rs[rhs0 + j].sum;
+  }
+}
+
+// One wavefront per RHS: merge its partials in a fixed order, then the step
+// decision (reference residual or sum-normalised bound) and the next teleport
+// term.
 __global__ __launch_bounds__(64) void batch_finalize_norm(RhsState *rs, const RhsInfo *__restrict__ info,
                                                           const PassPart *__restrict__ part, double eps,
                                                           double bound_target, int rule, int max_it) {
   const int r = blockIdx.x, l = threadIdx.x;
   RhsState &st = rs[r];
-  if (!FINAL && st.done) return;
+  if (st.done) return;
   const RhsInfo in = info[r];
   double e = 0;
   CSum t{0, 0};
-  for (int k = l; k < in.count; k += 64) {
-    const PassPart p = part[in.base + static_cast<long>(k) * in.stride];
-    e += p.e;
-    t = csum_merge(t, CSum{p.s, p.c});
+  constexpr int U = 4;  // partials of a lane loaded before they are merged, in order
+  for (int k0 = l; k0 < in.count; k0 += 64 * U) {
+    PassPart p[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) p[u] = part[in.base + static_cast<long>(min(k0 + 64 * u, in.count - 1)) * in.stride];
+#pragma unroll
+    for (int u = 0; u < U; u++)
+      if (k0 + 64 * u < in.count) {
+        e += p[u].e;
+        t = csum_merge(t, CSum{p[u].s, p[u].c});
+      }
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
@@ -549,10 +674,6 @@ __global__ __launch_bounds__(64) void batch_finalize_norm(RhsState *rs, const Rh
   }
   if (l != 0) return;
   const double S = t.s + t.c;
-  if (FINAL) {
-    st.total = S;
-    return;
-  }
   st.it += 1;
   st.err = e;
   st.sum_prev = st.sum;
@@ -987,8 +1108,9 @@ void PageRankBatch::Impl::build() {
       const int rows = sgraphs[static_cast<std::size_t>(gr.sgraph)]->rows;
       const long first = np;
       int cnt = 0;
-      for (int r0 = 0; r0 < rows; r0 += kSpmmChunkRows) {
-        it.push_back(PassItem{1, static_cast<int>(s), r0, std::min(rows, r0 + kSpmmChunkRows), np});
+      const int chunk = spmm_chunk_rows(rows);
+      for (int r0 = 0; r0 < rows; r0 += chunk) {
+        it.push_back(PassItem{1, static_cast<int>(s), r0, std::min(rows, r0 + chunk), np});
         np += kLanes;
         cnt++;
       }
@@ -1002,7 +1124,7 @@ void PageRankBatch::Impl::build() {
   parts.alloc(sizeof(PassPart) * static_cast<std::size_t>(std::max(1L, np)));
   out_off.upload(dev_out.data(), dev_out.size() * sizeof(long));
   rs.alloc(sizeof(RhsState) * static_cast<std::size_t>(std::max(1, n_rhs_total)));
-  slots.alloc(sizeof(unsigned long long) * kSlots * static_cast<std::size_t>(std::max(1, n_rhs_total)));
+  slots.alloc(sizeof(unsigned long long) * 2 * kSlots * static_cast<std::size_t>(std::max(1, n_rhs_total)));
 
   // ---- work items and queues of every (tile size, SpMM rows) layout
   {
@@ -1051,6 +1173,7 @@ BatchDev<VT, XT> PageRankBatch::Impl::dev_view(const BatchConfig &c, double beta
   d.xb1 = xb[1].as<XT>();
   d.g = w.group_desc.as<SpmmGroup<VT>>();
   d.rs = rs.as<RhsState>();
+  d.n_rhs_total = n_rhs_total;
   d.slots = slots.as<unsigned long long>();
   d.q_items = w.q_items[xcd_map].as<int>();
   d.q_off = w.q_off_dev[xcd_map].as<int>();
@@ -1096,11 +1219,10 @@ void PageRankBatch::Impl::enqueue_iteration(const BatchDev<VT, XT> &d, int par, 
 template <typename VT, typename XT>
 void PageRankBatch::Impl::enqueue_rest(const BatchDev<VT, XT> &d, int par, const BatchParams &p,
                                        hipStream_t s) const {
-  hipLaunchKernelGGL(batch_finalize_max, dim3(n_rhs_total), dim3(64), 0, s, d.rs, d.slots);
   if (n_items)
-    hipLaunchKernelGGL((batch_pass<VT, XT, 0>), dim3(n_items), dim3(kTileThreads), 0, s, d, items.as<PassItem>(),
-                       parts.as<PassPart>(), out_off.as<long>(), static_cast<double *>(nullptr), par);
-  hipLaunchKernelGGL(batch_finalize_norm<0>, dim3(n_rhs_total), dim3(64), 0, s, d.rs, info.as<RhsInfo>(),
+    hipLaunchKernelGGL((batch_normalize<VT, XT>), dim3(n_items), dim3(kTileThreads), 0, s, d, items.as<PassItem>(),
+                       parts.as<PassPart>(), par);
+  hipLaunchKernelGGL(batch_finalize_norm, dim3(n_rhs_total), dim3(64), 0, s, d.rs, info.as<RhsInfo>(),
                      parts.as<PassPart>(), p.epsilon, p.epsilon * (1.0 - p.beta) / p.beta, static_cast<int>(p.rule),
                      p.max_iteration);
 }
@@ -1124,7 +1246,7 @@ void PageRankBatch::Impl::init_state(const BatchParams &p, hipStream_t s) {
     if (a_rows) hipLaunchKernelGGL(batch_fill<float>, dim3(fill_grid(a_rows)), dim3(256), 0, s, xa[0].as<float>(), static_cast<long>(a_rows), 0.25f);
     if (xb_len) hipLaunchKernelGGL(batch_fill<float>, dim3(fill_grid(xb_len)), dim3(256), 0, s, xb[0].as<float>(), xb_len, 0.25f);
   }
-  const long ns = static_cast<long>(kSlots) * n_rhs_total;
+  const long ns = 2L * kSlots * n_rhs_total;
   hipLaunchKernelGGL(batch_fill<unsigned long long>, dim3(fill_grid(ns)), dim3(256), 0, s, slots.as<unsigned long long>(), ns, 0ull);
   TBSLA_HIP_CHECK(hipGetLastError());
   TBSLA_HIP_CHECK(hipStreamSynchronize(s));  // the state copy reads host memory
@@ -1242,15 +1364,11 @@ BatchReport PageRankBatch::Impl::run_typed(const BatchParams &p, double *out, hi
     if (all) break;
   }
   TBSLA_HIP_CHECK(hipEventRecord(e1, s));
-  // final sum normalisation of every RHS (Matrix.cpp:105-111), compensated
-  if (n_items) {
-    hipLaunchKernelGGL((batch_pass<VT, XT, 1>), dim3(n_items), dim3(kTileThreads), 0, s, d, items.as<PassItem>(),
-                       parts.as<PassPart>(), out_off.as<long>(), out, 0);
-    hipLaunchKernelGGL(batch_finalize_norm<1>, dim3(n_rhs_total), dim3(64), 0, s, d.rs, info.as<RhsInfo>(),
-                       parts.as<PassPart>(), 0.0, 0.0, 0, 0);
-    hipLaunchKernelGGL((batch_pass<VT, XT, 2>), dim3(n_items), dim3(kTileThreads), 0, s, d, items.as<PassItem>(),
-                       parts.as<PassPart>(), out_off.as<long>(), out, 0);
-  }
+  // final sum normalisation of every RHS (Matrix.cpp:105-111), by the
+  // compensated sum of its last normalise pass
+  if (n_items)
+    hipLaunchKernelGGL((batch_output<VT, XT>), dim3(n_items), dim3(kTileThreads), 0, s, d, items.as<PassItem>(),
+                       out_off.as<long>(), out);
   TBSLA_HIP_CHECK(hipGetLastError());
   TBSLA_HIP_CHECK(hipStreamSynchronize(s));
   float ms = 0;

@@ -14,15 +14,15 @@
 //                      row-major n x 64 so a gathered row of X is 64
 //                      consecutive values (one coalesced load per wavefront).
 //
-// One iteration is four launches, captured in a hipGraph and replayed:
+// One iteration is three launches, captured in a hipGraph and replayed:
 //   batch_step          persistent work-queue kernel over every tile of the
 //                       block-diagonal matrix and every 64-row block of the
 //                       multi-RHS graphs (SpMM: lane = RHS), fused with
 //                       b = beta*(A b_t) + t and per-RHS maxima (atomic max
 //                       slots); per-XCD queues keep a graph's tiles on one
 //                       XCD so its iterate stays in that XCD's L2
-//   batch_finalize_max  per-RHS maximum
-//   batch_pass<0>       b /= max, residual and compensated sum partials
+//   batch_normalize     per-RHS maximum from the slots, b /= max, residual and
+//                       compensated sum partials
 //   batch_finalize_norm per-RHS decision, teleport term for the next step
 // The launch shape (workgroups per CU, queue mapping, gathers in flight)
 // is chosen by an autotuner that times candidate shapes on the first
