@@ -111,21 +111,23 @@ constexpr int kPbChunk = 64;
 static_assert(kPbShift + 3 <= 16, "local keys hold the column and a 3-bit row offset in 16 bits");
 static_assert(kPbCols <= 0x2000, "scatter keys hold the column in 13 bits");
 static_assert(kPbColsWide <= kPbRunStart, "wide scatter keys hold the column in 15 bits");
-// A gather (scatter) launch has one workgroup per bin (superblock), of which
-// the 256 CUs hold 512 (256) at a time.  The width is the smallest that
-// gives whole rounds of them: ceil(n / (slots * rounds)) with the fewest
-// rounds that keep it at or under the cap, in multiples of 64 so that a
-// bin's rows start on a cache line.  With the width fixed at the cap, graphs
-// under 2^21 nodes left most CUs idle and others ended in a nearly empty
-// round (16 entries a row, FP64 iteration: 2^16 nodes 52.1 -> 18.1 us, 2^18
-// 55.9 -> 26.6, 2^20 71.2 -> 52.7, 2^22 246 -> 238).  Under kPbMinWidth a
-// workgroup is shorter than its own start-up.
-constexpr int kPbGatherSlots = 512;
-constexpr int kPbScatterSlots = 256;
+// A gather (scatter) launch has one workgroup per bin (superblock).  The
+// width is the smallest that gives whole rounds of one workgroup per CU:
+// ceil(n / (256 * rounds)) with the fewest rounds that keep it at or under
+// the cap, in multiples of 64 so that a bin's rows start on a cache line.
+// With the width fixed at the cap, graphs under 2^21 nodes left most CUs idle
+// and others ended in a nearly empty round (16 entries a row, FP64
+// iteration: 2^16 nodes 52.1 -> 18.1 us, 2^18 55.9 -> 26.6, 2^20 71.2 -> 52.7,
+// 2^22 246 -> 238).  Two gather workgroups fit a CU, but rounds of 512 were
+// slower (66,000 nodes of 8: 13.1 against 14.6 us, 300,007 of 16 21.0 against
+// 22.5, 5,000,011 of 8 151.9 against 155.8), and so were two rounds of
+// scatter workgroups on small graphs (a round costs 4 us).  Under kPbMinWidth
+// a workgroup is shorter than its own start-up.
+constexpr int kPbSlots = 256;
 constexpr int kPbMinWidth = 256;
-inline int pb_width(int n, int slots, int cap) {
-  const long per_round = static_cast<long>(slots) * cap;
-  const long blocks = std::max(1L, (n + per_round - 1) / per_round) * slots;
+inline int pb_width(int n, int cap) {
+  const long per_round = static_cast<long>(kPbSlots) * cap;
+  const long blocks = std::max(1L, (n + per_round - 1) / per_round) * kPbSlots;
   const long w = ((n + blocks - 1) / blocks + 63) / 64 * 64;
   return static_cast<int>(std::min<long>(cap, std::max<long>(kPbMinWidth, w)));
 }
@@ -136,9 +138,9 @@ struct PbMatrix {
   // sizes all of these from n
   void set_widths(int n_) {
     n = n_;
-    rows = pb_width(n, kPbGatherSlots, kPbRows);
-    cols = pb_width(n, kPbScatterSlots, kPbCols);
-    cols_w = pb_width(n, kPbScatterSlots, kPbColsWide);
+    rows = pb_width(n, kPbRows);
+    cols = pb_width(n, kPbCols);
+    cols_w = pb_width(n, kPbColsWide);
     nbins = (n + rows - 1) / rows;
     nsb = (n + cols - 1) / cols;
     nsb_w = (n + cols_w - 1) / cols_w;
