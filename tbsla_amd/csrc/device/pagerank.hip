@@ -92,15 +92,64 @@ __device__ inline CSum csum_merge(CSum a, CSum b) {
 // Fixed-order butterfly reductions over one wavefront (every lane gets the
 // result) and over the 16 wavefronts of a 1024-thread workgroup (thread 0
 // gets the result; red holds 48 doubles).
+// The partner of each step holds the other group's value: lanes 1 and 2 away
+// (quad permutes), then the mirrored lane of 8 and of 16 (every lane of a
+// group holds the group's value), which are VALU moves; the 16-lane rows are
+// exchanged through LDS shuffles.  (Six LDS shuffles in a chain take three
+// times as long.)
+template <int CTRL>
+__device__ inline double dpp_f64(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_mov_dpp(static_cast<int>(b), CTRL, 0xF, 0xF, false);
+  const int hi = __builtin_amdgcn_mov_dpp(static_cast<int>(b >> 32), CTRL, 0xF, 0xF, false);
+  return __longlong_as_double((static_cast<long long>(hi) << 32) | static_cast<unsigned>(lo));
+}
+constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppHalfMirror = 0x141, kDppMirror = 0x140;
+// f(partner) over the steps of a 16-lane row
+template <typename T, typename Get, typename Op>
+__device__ inline T row_reduce(T v, Get get, Op op) {
+  v = op(v, get(std::integral_constant<int, kDppXor1>(), v));
+  v = op(v, get(std::integral_constant<int, kDppXor2>(), v));
+  v = op(v, get(std::integral_constant<int, kDppHalfMirror>(), v));
+  v = op(v, get(std::integral_constant<int, kDppMirror>(), v));
+  return v;
+}
+struct GetF64 {
+  template <typename C>
+  __device__ double operator()(C, double v) const {
+    return dpp_f64<C::value>(v);
+  }
+};
+struct GetCSum {
+  template <typename C>
+  __device__ CSum operator()(C, CSum v) const {
+    return CSum{dpp_f64<C::value>(v.s), dpp_f64<C::value>(v.c)};
+  }
+};
+struct AddF64 {
+  __device__ double operator()(double a, double b) const { return a + b; }
+};
+struct MaxF64 {
+  __device__ double operator()(double a, double b) const { return fmax(a, b); }
+};
+struct MergeCSum {
+  __device__ CSum operator()(CSum a, CSum b) const { return csum_merge(a, b); }
+};
 __device__ inline CSum wave_csum(CSum v) {
+  v = row_reduce(v, GetCSum(), MergeCSum());
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = csum_merge(v, CSum{__shfl_xor(v.s, off, 64), __shfl_xor(v.c, off, 64)});
+  for (int off = 16; off <= 32; off <<= 1) v = csum_merge(v, CSum{__shfl_xor(v.s, off, 64), __shfl_xor(v.c, off, 64)});
   return v;
 }
 __device__ inline double wave_sum(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
+  v = row_reduce(v, GetF64(), AddF64());
+  v += __shfl_xor(v, 16, 64);
+  return v + __shfl_xor(v, 32, 64);
+}
+__device__ inline double wave_max(double v) {
+  v = row_reduce(v, GetF64(), MaxF64());
+  v = fmax(v, __shfl_xor(v, 16, 64));
+  return fmax(v, __shfl_xor(v, 32, 64));
 }
 __device__ inline void block1024_err_csum(double err, CSum cs, double *red, double &err_out, CSum &cs_out) {
   err = wave_sum(err);
@@ -115,11 +164,8 @@ __device__ inline void block1024_err_csum(double err, CSum cs, double *red, doub
   if (w == 0) {  // the 16 wavefronts' sums on 16 lanes (each 16-lane group the same)
     err_out = red[lane & 15];
     cs_out = CSum{red[16 + (lane & 15)], red[32 + (lane & 15)]};
-#pragma unroll
-    for (int off = 8; off > 0; off >>= 1) {
-      err_out += __shfl_xor(err_out, off, 64);
-      cs_out = csum_merge(cs_out, CSum{__shfl_xor(cs_out.s, off, 64), __shfl_xor(cs_out.c, off, 64)});
-    }
+    err_out = row_reduce(err_out, GetF64(), AddF64());
+    cs_out = row_reduce(cs_out, GetCSum(), MergeCSum());
   }
 }
 
@@ -545,6 +591,152 @@ __global__ __launch_bounds__(256) void pr_anchor_move(double *__restrict__ xhat,
   }
 }
 
+// A small graph's whole run in one workgroup and one launch (at most
+// `iterations` of them, so that every launch ends): the iterate, the update
+// and the row bounds stay in LDS, and the entries are read from L2, row by
+// row, C per thread at a time.  The arithmetic is that of pr_update_csr and
+// pr_normalize (row sums left to right, b = beta*s + tele, b / max).  VF: the
+// entries of a column agree, so only the indices are read and the products
+// are those of the column values (cs), formed once per column in LDS.
+//
+// Bound by the latency of a row's loads and by the cache lines one CU reads
+// (a lane reads its own row); the two launches of an iteration took 11.5 us
+// whatever the size.  Value-free, 8 entries a row, us an iteration: 100 nodes
+// 11.6 -> 2.5, 1,000 12.2 -> 3.2, 2,500 12.1 -> 4.1, 5,003 12.5 -> 6.1; 4,000
+// of 16 12.4 -> 8.1.  With stored values (three times the bytes, and most of
+// each line another lane's) 2,500 of 8 took 6.2 and 5,003 9.5, 3,000 of 16
+// 16.3: the lines kOneBlockEntries* draw.
+constexpr int kOneBlockRows = 5632;  // 28 bytes a row: 154 KB of LDS
+constexpr long kOneBlockEntries = 65536;       // value-free
+constexpr long kOneBlockEntriesVal = 24576;    // with stored values
+constexpr int kOneBlockLenBits = 11;
+static_assert(kCsrLongRow < (1 << kOneBlockLenBits) && kOneBlockEntries < (1L << (31 - kOneBlockLenBits)),
+              "a row's first entry and length fit one int");
+
+typedef int v4i_u __attribute__((ext_vector_type(4), aligned(4)));
+typedef double v2d_u __attribute__((ext_vector_type(2), aligned(8)));
+
+// C entries from entry e (past the row's end they are the next row's, or the
+// mirror's zeroed padding: loaded, never added).
+template <bool VF, int C>
+struct RowChunk {
+  v4i_u c[C / 4];
+  v2d_u v[VF ? 1 : C / 2];
+  __device__ void load(const dev::CsrView<double> &m, int e) {
+#pragma unroll
+    for (int k = 0; k < C / 4; k++) c[k] = reinterpret_cast<const v4i_u *>(m.colidx + e)[k];
+    if (!VF)
+#pragma unroll
+      for (int k = 0; k < C / 2; k++) v[k] = reinterpret_cast<const v2d_u *>(m.vals + e)[k];
+  }
+  // s plus the first `len` products, in entry order
+  __device__ double add(double s, int len, const double *xs) const {
+#pragma clang fp contract(off)
+    double p[C];
+#pragma unroll
+    for (int k = 0; k < C / 4; k++) {
+      p[4 * k] = xs[c[k].x];
+      p[4 * k + 1] = xs[c[k].y];
+      p[4 * k + 2] = xs[c[k].z];
+      p[4 * k + 3] = xs[c[k].w];
+      if (!VF) {
+        p[4 * k] = v[2 * k].x * p[4 * k];
+        p[4 * k + 1] = v[2 * k].y * p[4 * k + 1];
+        p[4 * k + 2] = v[2 * k + 1].x * p[4 * k + 2];
+        p[4 * k + 3] = v[2 * k + 1].y * p[4 * k + 3];
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < C; k++) s = k < len ? s + p[k] : s;
+    return s;
+  }
+};
+
+template <int TM, bool VF, int C>
+__global__ __launch_bounds__(1024) void pr_one_block(dev::CsrView<double> m, const double *__restrict__ colval, int n,
+                                                     Teleport tp, double *__restrict__ x, double *__restrict__ out,
+                                                     PrState *st, int iterations) {
+#pragma clang fp contract(off)
+  __shared__ double xs[kOneBlockRows], ys[kOneBlockRows], zbuf[VF ? kOneBlockRows : 1];
+  __shared__ int bounds[kOneBlockRows];  // first entry << kOneBlockLenBits | length
+  __shared__ double red[48];
+  __shared__ PrState sh;
+  double *const zs = VF ? zbuf : xs;  // the products' input
+  constexpr int T = 1024, kLen = (1 << kOneBlockLenBits) - 1;
+  const int tid = threadIdx.x;
+  if (tid == 0) sh = *st;
+  for (int r = tid; r < n; r += T) {
+    const int a = m.rowptr[r] - m.rp0, b = m.rowptr[r + 1] - m.rp0;
+    bounds[r] = a << kOneBlockLenBits | (b - a);
+    const double v = x[r];
+    xs[r] = v;
+    if (VF) zs[r] = colval[r] * v;
+  }
+  __syncthreads();
+  for (int it = 0; it < iterations && !sh.done; it++) {
+    const double beta = sh.beta, tele = sh.tele;
+    double lmax = -INFINITY;
+    // the first chunk of the thread's next row is loaded while this one is summed
+    RowChunk<VF, C> ck;
+    int bd = tid < n ? bounds[tid] : 0;
+    ck.load(m, bd >> kOneBlockLenBits);
+#pragma unroll 1
+    for (int r = tid; r < n; r += T) {
+      const int bn = r + T < n ? bounds[r + T] : 0;
+      RowChunk<VF, C> nx;
+      nx.load(m, bn >> kOneBlockLenBits);
+      const int a = bd >> kOneBlockLenBits, len = bd & kLen;
+      double s = ck.add(0.0, len, zs);
+      for (int k = C; k < len; k += C) {
+        RowChunk<VF, C> c;
+        c.load(m, a + k);
+        s = c.add(s, len - k, zs);
+      }
+      const double b = add_teleport<TM>(beta * s, tele, tp, r);
+      ys[r] = b;
+      lmax = fmax(lmax, b);
+      ck = nx;
+      bd = bn;
+    }
+    lmax = wave_max(lmax);
+    if ((tid & 63) == 0) red[tid >> 6] = lmax;
+    __syncthreads();  // (every read of the old iterate by a row sum is done too)
+    const double mx = row_reduce(red[tid & 15], GetF64(), MaxF64());
+    double err = 0, e;
+    CSum cs{0, 0}, t;
+    for (int r = tid; r < n; r += T) {
+      const double b = ys[r] / mx;
+      err += fabs(b - xs[r]);
+      csum_add(cs, b);
+      xs[r] = b;
+      if (VF) zs[r] = colval[r] * b;
+    }
+    __syncthreads();  // (red is written again)
+    block1024_err_csum(err, cs, red, e, t);
+    if (tid == 0) {
+      sh.maxv = mx;
+      finalize_step<false>(&sh, e, t.s + t.c);
+    }
+    __syncthreads();
+  }
+  const double S = sh.sum;
+  for (int r = tid; r < n; r += T) {
+    x[r] = xs[r];
+    if (sh.done) out[r] = xs[r] / S;
+  }
+  if (tid == 0) *st = sh;
+}
+
+template <int TM>
+void launch_one_block(const DeviceMatrix &d, const double *colval, int n, const Teleport &tp, double *x, double *out,
+                      PrState *st, int iterations, hipStream_t s) {
+  const dev::CsrView<double> m = dev::csr_view<double>(d);
+  const auto kernel = !colval ? pr_one_block<TM, false, 8>
+                      : d.entries > 10L * n ? pr_one_block<TM, true, 16>
+                                            : pr_one_block<TM, true, 8>;
+  hipLaunchKernelGGL(kernel, dim3(1), dim3(1024), 0, s, m, colval, n, tp, x, out, st, iterations);
+}
+
 template <typename YT>
 struct StoreRowD {
   YT *y;
@@ -673,47 +865,52 @@ __global__ __launch_bounds__(256) void to_bf16_f32(const double *__restrict__ a,
     b[i] = dev::Val<dev::bf16>::cvt(dev::bf16_of(a[i]));
 }
 
-// Whether the stored entries of every column of an n-column CSR matrix hold
-// one value (true of fill_cqmat_stochastic's by construction, found from the
-// values otherwise).  If so the column values (0 for a column with no
-// entries) are in the matrix's device cache in FP64, FP32 and as BF16 rounds
-// them.  Decided once per matrix; x_need <= n has been checked.
+// The column values of an n-column CSR matrix into cs (0 for a column with no
+// entries).  Returns whether the stored entries of every column hold one
+// value: true of fill_cqmat_stochastic's by construction, found from the
+// values otherwise (with `flag`, 8 bytes).  x_need <= n has been checked.
+bool find_column_values(const cpp::Matrix &m, const DeviceMatrix &d64, long n, double *cs, double *flag,
+                        hipStream_t s) {
+  const unsigned ge = grid_for(d64.entries, 16L * kNormBlocks);
+  hipLaunchKernelGGL(fill_f64, dim3(grid_for(n)), dim3(256), 0, s, cs, n, 0.0);
+  if (d64.entries == 0) return true;
+  hipLaunchKernelGGL(colscale_kernel, dim3(ge), dim3(256), 0, s, d64.colidx.as<int>(), d64.vals.as<double>(),
+                     d64.entries, d64.f_col, n, cs);
+  if (m.count_stochastic()) return true;
+  int differs = 0;
+  hipLaunchKernelGGL(fill_f64, dim3(1), dim3(256), 0, s, flag, 1L, 0.0);
+  hipLaunchKernelGGL(colscale_check, dim3(ge), dim3(256), 0, s, d64.colidx.as<int>(), d64.vals.as<double>(),
+                     d64.entries, d64.f_col, cs, reinterpret_cast<int *>(flag));
+  TBSLA_HIP_CHECK(hipMemcpyAsync(&differs, flag, sizeof(int), hipMemcpyDeviceToHost, s));
+  TBSLA_HIP_CHECK(hipStreamSynchronize(s));
+  return !differs;
+}
+
+// find_column_values, decided once per matrix: if true, the column values are
+// in the matrix's device cache in FP64, FP32 and as BF16 rounds them.
 bool column_values(const cpp::Matrix &m, const DeviceMatrix &d64, long n, hipStream_t s) {
   DeviceCache &cache = m.device_cache();
   std::lock_guard<std::mutex> g(cache.mu);
   if (cache.col_values != DeviceCache::kUnknown) return cache.col_values == DeviceCache::kPerColumn;
-  DevBuf c64, c32, cbf, bad;
-  c64.alloc(sizeof(double) * static_cast<std::size_t>(n));
-  const unsigned ge = grid_for(d64.entries, 16L * kNormBlocks), gn = grid_for(n);
-  hipLaunchKernelGGL(fill_f64, dim3(gn), dim3(256), 0, s, c64.as<double>(), n, 0.0);
-  int differs = 0;
-  if (d64.entries > 0) {
-    hipLaunchKernelGGL(colscale_kernel, dim3(ge), dim3(256), 0, s, d64.colidx.as<int>(), d64.vals.as<double>(),
-                       d64.entries, d64.f_col, n, c64.as<double>());
-    if (!m.count_stochastic()) {
-      bad.alloc(sizeof(double));
-      hipLaunchKernelGGL(fill_f64, dim3(1), dim3(256), 0, s, bad.as<double>(), 1L, 0.0);
-      hipLaunchKernelGGL(colscale_check, dim3(ge), dim3(256), 0, s, d64.colidx.as<int>(), d64.vals.as<double>(),
-                         d64.entries, d64.f_col, c64.as<double>(), bad.as<int>());
-      TBSLA_HIP_CHECK(hipMemcpyAsync(&differs, bad.get(), sizeof(int), hipMemcpyDeviceToHost, s));
-      TBSLA_HIP_CHECK(hipStreamSynchronize(s));
-    }
-  }
-  if (!differs) {
-    c32.alloc(sizeof(float) * static_cast<std::size_t>(n));
-    cbf.alloc(sizeof(float) * static_cast<std::size_t>(n));
-    hipLaunchKernelGGL(to_f32, dim3(gn), dim3(256), 0, s, c64.as<double>(), c32.as<float>(), n);
-    hipLaunchKernelGGL(to_bf16_f32, dim3(gn), dim3(256), 0, s, c64.as<double>(), cbf.as<float>(), n);
+  DevBuf c64, c32, cbf, flag;
+  c64.reserve(sizeof(double) * static_cast<std::size_t>(n));
+  flag.reserve(sizeof(double));
+  const bool same = find_column_values(m, d64, n, c64.as<double>(), flag.as<double>(), s);
+  if (same) {
+    c32.reserve(sizeof(float) * static_cast<std::size_t>(n));
+    cbf.reserve(sizeof(float) * static_cast<std::size_t>(n));
+    hipLaunchKernelGGL(to_f32, dim3(grid_for(n)), dim3(256), 0, s, c64.as<double>(), c32.as<float>(), n);
+    hipLaunchKernelGGL(to_bf16_f32, dim3(grid_for(n)), dim3(256), 0, s, c64.as<double>(), cbf.as<float>(), n);
   }
   TBSLA_HIP_CHECK(hipGetLastError());
   TBSLA_HIP_CHECK(hipStreamSynchronize(s));
-  if (!differs) {
+  if (same) {
     cache.colscale64 = std::move(c64);
     cache.colscale32 = std::move(c32);
     cache.colscale_bf16 = std::move(cbf);
   }
-  cache.col_values = differs ? DeviceCache::kDiffer : DeviceCache::kPerColumn;
-  return !differs;
+  cache.col_values = same ? DeviceCache::kPerColumn : DeviceCache::kDiffer;
+  return same;
 }
 
 // ---------------------------------------------------------------------------
@@ -1503,7 +1700,7 @@ void launch_anchor(const DeviceMatrix &d, const double *x, double *yhat, const P
 
 struct Scratch {
   WsBuf st, slots, perr, ps, pc, member, nodes, hsum, hcomp;
-  WsBuf X0, X1, Z, yhat, xhat, xhat32, D0, D1, ZD0, ZD1, W, out;
+  WsBuf X0, X1, Z, yhat, xhat, xhat32, D0, D1, ZD0, ZD1, W, out, cs, flag;
 };
 
 // One block: the step decision of a sum-normalised propagation-blocked
@@ -1631,12 +1828,19 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
   // products, whose sums are the reference's)
   const bool use_pb = fused && !p.values && (p.gather == 2 || (p.gather == 0 && n >= (1L << 16)));
   const PbMatrix *pbm = nullptr;
+  // small graphs with no long row: the whole run in one workgroup.  (The
+  // stored values' padding is read, so explicit ones take the tiles; f_col is
+  // 0 in a matrix of one block.)
+  const bool small = fused && !use_pb && !mixed && !p.values && n <= kOneBlockRows && d64.nlong == 0 &&
+                     d64.f_col == 0 && p.max_iteration > 0;
   // Blocked products of a matrix whose stored entries agree within every
   // column (a link graph: 1/out-degree) read no values: the input is scaled
   // by the column's value once, which gives the same rounded products.  (On
   // fill_cqmat_stochastic(2^24,2^24,8,0.5,7): FP64 iteration 696 -> 536 us,
   // FP32 437 -> 385, BF16 436 -> 428.)
   bool vfree = false;
+  const bool try_vfree = small && d64.entries <= kOneBlockEntries;
+  if (try_vfree && !arena) vfree = column_values(m, d64, n, s);
   if (use_pb) {
     vfree = column_values(m, d64, n, s);
     pbm = &pb_mirror(m, vfree ? Dtype::PATTERN : Dtype::F64);
@@ -1704,6 +1908,11 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
   const bool stored_z = !pbm && (pattern || (mixed && m.count_stochastic()));
   if (stored_z) ws.alloc(w.Z, sizeof(double) * n);
   if (!out_dev) ws.alloc(w.out, sizeof(double) * n);
+  // (allocation-free runs find the column values again in each run)
+  if (try_vfree && arena) {
+    ws.alloc(w.cs, sizeof(double) * n);
+    ws.alloc(w.flag, sizeof(double));
+  }
   std::unique_ptr<RunSpace> space;
   if (arena) {
     if (ws.bytes() > cap)
@@ -1732,13 +1941,16 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
   // the run's precision)
   const double *colscale64 = nullptr;
   const float *colscale32 = nullptr;
-  if (vfree || pattern || pat32 || (mixed && m.count_stochastic())) {
-    if (arena) throw std::invalid_argument("tbsla: the allocation-free entry point runs FP64 only");
+  if (arena) {
+    if (try_vfree) vfree = find_column_values(m, d64, n, w.cs.as<double>(), w.flag.as<double>(), s);
+    if (vfree) colscale64 = w.cs.as<double>();
+  } else if (vfree || pattern || pat32 || (mixed && m.count_stochastic())) {
     (void)column_values(m, d64, n, s);
     const DeviceCache &cache = m.device_cache();
     colscale64 = cache.colscale64.as<double>();
     colscale32 = p.precision == PrPrecision::BF16 ? cache.colscale_bf16.as<float>() : cache.colscale32.as<float>();
   }
+  const bool one_block = small && d64.entries <= (vfree ? kOneBlockEntries : kOneBlockEntriesVal);
   PrState h{};
   h.beta = p.beta;
   h.eps = p.epsilon;
@@ -1827,7 +2039,7 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
   if (arena) TBSLA_HIP_CHECK(hipStreamSynchronize(s));
   const auto h0 = std::chrono::steady_clock::now();
   if (space) TBSLA_HIP_CHECK(hipEventRecord(space->timing[0], s));
-  const int check = fused ? std::max(1, p.check_every) : 1;
+  const int check = one_block ? 256 : (fused ? std::max(1, p.check_every) : 1);
   int next = check;  // iterations in the next launch batch
   PrState hs{};
   int launched = 0;
@@ -1837,7 +2049,7 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
   // alternates between two buffers).  On larger matrices than those with
   // kMergeTileNnz-entry tiles the decision repeated in every block costs more
   // than a launch of its own.
-  const bool merged = !pbm && !mixed && (!fused || d64.tile_nnz == kMergeTileNnz);
+  const bool merged = !pbm && !mixed && !one_block && (!fused || d64.tile_nnz == kMergeTileNnz);
   const auto state = [&](int it) { return merged ? st + (it & 1) : st; };
   const SnPartials sp{w.perr.as<double>(), w.ps.as<double>(), w.pc.as<double>()};
   const Partials parts{sp.perr, sp.ps, sp.pc, static_cast<int>(sn ? static_cast<unsigned>(pbm->nbins) : gM)};
@@ -1856,7 +2068,15 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
   };
   using std::integral_constant;
   auto launch_batch = [&](int batch) {
-    for (int k = 0; k < batch; k++) {
+    if (one_block) {
+      if (tmode == 1)
+        launch_one_block<1>(d64, colscale64, static_cast<int>(n), tp, X[0], out_dev, st, batch, s);
+      else if (tmode == 2)
+        launch_one_block<2>(d64, colscale64, static_cast<int>(n), tp, X[0], out_dev, st, batch, s);
+      else
+        launch_one_block<0>(d64, colscale64, static_cast<int>(n), tp, X[0], out_dev, st, batch, s);
+    }
+    for (int k = 0; k < batch && !one_block; k++) {
       const int it = launched + k;
       double *xin = X[it & 1], *xout = X[(it + 1) & 1];
       // the step decision of the iteration before is taken by this one, the
@@ -1980,7 +2200,7 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
     bool have = false;  // hs holds a state read back
     if (launched < p.max_iteration) enqueue(std::min(check, p.max_iteration - launched));
     while (npend > 0) {
-      if (npend == 1 && launched < p.max_iteration) {
+      if (npend == 1 && launched < p.max_iteration && !one_block) {
         int nb = check;
         if (have) nb = std::min(check, iterations_left(hs, check) - (launched - hs.it));
         nb = std::min(nb, p.max_iteration - launched);
@@ -2003,7 +2223,8 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
   const float *dd = mixed ? D[it & 1] : nullptr;
   if (mixed && !sn)  // the state's sum is that of the FP64 update; the result's elements are rounded
     hipLaunchKernelGGL(pr_sum_rounded, dim3(1), dim3(1024), 0, s, a, dd, n, st);
-  hipLaunchKernelGGL(pr_scale_kernel, dim3(gN), dim3(256), 0, s, a, dd, n, state(launched), out_dev);
+  if (!one_block)  // (which wrote the result)
+    hipLaunchKernelGGL(pr_scale_kernel, dim3(gN), dim3(256), 0, s, a, dd, n, state(launched), out_dev);
   TBSLA_HIP_CHECK(hipGetLastError());
   if (out_host)
     TBSLA_HIP_CHECK(hipMemcpyAsync(out_host, out_dev, sizeof(double) * static_cast<std::size_t>(n),
@@ -2064,6 +2285,7 @@ std::size_t page_rank_noalloc_bytes(long n, int n_nodes) {
   const std::size_t gM = static_cast<std::size_t>(std::min<long>(kPassBlocks, (n + 1023) / 1024));
   std::size_t b = slice(2 * sizeof(PrState)) + slice(2 * sizeof(unsigned long long) * kMaxSlots) +
                   3 * slice(sizeof(double) * gM) + 2 * slice(sizeof(double) * static_cast<std::size_t>(n));
+  if (n <= kOneBlockRows) b += slice(sizeof(double) * static_cast<std::size_t>(n)) + slice(sizeof(double));
   if (n_nodes > 0) b += slice(static_cast<std::size_t>(n)) + slice(sizeof(int) * static_cast<std::size_t>(n_nodes));
   return b;
 }
