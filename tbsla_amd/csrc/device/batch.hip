@@ -401,7 +401,7 @@ void batch_step(BatchDev<VT, XT> d, int par) {
       TileEpi<XT> epi{xa_out, d.row_graph, d.rs, d.a_member, d.slots, d.beta, gA, gB, w % kSlots,
                       -INFINITY, -INFINITY};
       if (tile)
-        dev::csr_tile_rows_at<VT, XT, TileEpi<XT>, TN, kBatchLongRow>(d.a, xa_in, lds, epi, w);
+        dev::csr_tile_rows_at<VT, XT, TileEpi<XT>, TN, kBatchLongRow, dev::kPlain>(d.a, xa_in, lds, epi, w);
       else
         dev::csr_long_row_at<VT, XT, TileEpi<XT>, TN, kBatchLongChunk>(d.a, xa_in, lds, epi, w - d.a_ntiles);
       const double bA = dev::block_tree_max<double>(epi.mA, red);

@@ -1,5 +1,7 @@
 #include "mirror.hpp"
 
+#include "kernels.hpp"
+
 #include <tbsla/cpp/MatrixCOO.hpp>
 #include <tbsla/cpp/MatrixCSR.hpp>
 #include <tbsla/cpp/MatrixDENSE.hpp>
@@ -119,6 +121,7 @@ void build_csr(DeviceMatrix &d, const cpp::MatrixCSR &m, Dtype vdt) {
   d.rowptr.upload(rp.data(), rp.size() * sizeof(int));
   // entry j of row i is values[rowptr[i] - rowptr[0] + k] (MatrixCSR.cpp:135)
   d.colidx.upload(ci.data(), static_cast<std::size_t>(used) * sizeof(int));
+  pack_columns(d);
   upload_values(d.vals, vals.data(), static_cast<std::size_t>(used), vdt);
   d.tile_nnz = tile_size(used, rp.data(), d.rows);
   std::vector<int> t = csr_entry_tiles(rp.data(), d.rows, d.tile_nnz);
@@ -230,6 +233,7 @@ void build_coo_like(DeviceMatrix &d, const M &m, Dtype vdt, bool scoo) {
   d.rowptr.upload(segptr.data(), segptr.size() * sizeof(int));
   d.segrow.upload(segrow.data(), segrow.size() * sizeof(int));
   d.colidx.upload(pcol, n * sizeof(int));
+  pack_columns(d);
   upload_values(d.vals, pval, n, vdt);
   d.tile_nnz = tile_size(static_cast<long>(n), segptr.data(), d.nseg);
   std::vector<int> t = csr_entry_tiles(segptr.data(), d.nseg, d.tile_nnz);
@@ -333,6 +337,7 @@ const DeviceMatrix &transpose_mirror(const cpp::Matrix &m) {
   d->x_need = rows;
   d->rowptr.upload(ptr.data(), ptr.size() * sizeof(int));
   d->colidx.upload(ridx.data(), ridx.size() * sizeof(int));
+  pack_columns(*d);
   d->perm.upload(perm.data(), perm.size() * sizeof(int));
   d->tile_nnz = tile_size(used, ptr.data(), cols);
   std::vector<int> t = csr_entry_tiles(ptr.data(), cols, d->tile_nnz);

@@ -6,7 +6,8 @@
 //                   that starts in the tile is then summed by one thread in
 //                   entry order.  With FP64 this reproduces the reference loop
 //                   MatrixCSR.cpp:133-139 bit for bit (product rounded, then a
-//                   left-to-right sum starting from 0).
+//                   left-to-right sum starting from 0).  Columns are read
+//                   packed in three bytes where they fit (pack_columns).
 // csr_long_kernel   rows longer than 1536 entries, one workgroup each.
 // ell_kernel        one row per thread over the sliced column-major slots (one
 //                   contiguous block per workgroup), eight slots per step;
@@ -20,6 +21,8 @@
 // dense_kernel      four rows per wavefront sharing each x load, butterfly reduction
 //                   (MatrixDENSE.cpp:67-72, different summation order).
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "kernels.hpp"
 #include "tile_csr.hpp"
@@ -42,12 +45,12 @@ struct StoreRow {
   }
 };
 
-template <typename VT, typename XT, typename YT, int TN>
+template <typename VT, typename XT, typename YT, int TN, bool PACK>
 __global__ __launch_bounds__(kTileThreads) void csr_tile_kernel(dev::CsrView<VT> m, const XT *__restrict__ x,
                                                                 YT *__restrict__ y) {
   __shared__ dev::CsrTileLds<typename Val<VT>::A, TN> lds;
   StoreRow<YT> epi{y};
-  dev::csr_tile_rows<VT, XT, TN>(m, x, lds, epi);
+  dev::csr_tile_rows<VT, XT, TN, PACK ? dev::kPacked : dev::kPlain>(m, x, lds, epi);
 }
 
 template <typename VT, typename XT, typename YT>
@@ -145,7 +148,7 @@ struct AccRow {
   }
 };
 
-template <typename VT, typename XT, typename YT, int TN, bool LONG>
+template <typename VT, typename XT, typename YT, int TN, bool PACK, bool LONG>
 __global__ __launch_bounds__(kTileThreads) void coo_tile_kernel(dev::CsrView<VT> m, const XT *__restrict__ x,
                                                                 YT *__restrict__ y, const int *__restrict__ segrow,
                                                                 long y_off) {
@@ -154,7 +157,7 @@ __global__ __launch_bounds__(kTileThreads) void coo_tile_kernel(dev::CsrView<VT>
   if constexpr (LONG)
     dev::csr_long_row<VT, XT, TN>(m, x, lds, epi);
   else
-    dev::csr_tile_rows<VT, XT, TN>(m, x, lds, epi);
+    dev::csr_tile_rows<VT, XT, TN, PACK ? dev::kPacked : dev::kPlain>(m, x, lds, epi);
 }
 
 // kDenseRows consecutive rows per wavefront, so each x load serves all of
@@ -227,6 +230,19 @@ __global__ void fill_kernel(T *y, long n, T v) {
   for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += static_cast<long>(gridDim.x) * 256) y[i] = v;
 }
 
+// three words of packed columns for entries 4g .. 4g + 3 (0 past the end)
+__global__ __launch_bounds__(256) void pack24_kernel(const int *__restrict__ colidx, long nnz, int f_col,
+                                                     unsigned *__restrict__ out) {
+  const long groups = (nnz + 3) / 4;
+  for (long g = blockIdx.x * 256L + threadIdx.x; g < groups; g += static_cast<long>(gridDim.x) * 256) {
+    unsigned c[4];
+    for (int q = 0; q < 4; q++) c[q] = 4 * g + q < nnz ? static_cast<unsigned>(colidx[4 * g + q] - f_col) : 0u;
+    out[3 * g] = c[0] | c[1] << 24;
+    out[3 * g + 1] = c[1] >> 8 | c[2] << 16;
+    out[3 * g + 2] = c[2] >> 16 | c[3] << 8;
+  }
+}
+
 inline unsigned blocks_for(long n, int per_block) { return static_cast<unsigned>((n + per_block - 1) / per_block); }
 
 template <typename VT, typename XT, typename YT>
@@ -236,8 +252,9 @@ void run_typed(const DeviceMatrix &d, const XT *x, YT *y, int vect_incr, hipStre
       const dev::CsrView<VT> m = dev::csr_view<VT>(d);
       if (d.ntiles > 0)
         with_tile_size(d, [&](auto tn) {
-          hipLaunchKernelGGL((csr_tile_kernel<VT, XT, YT, decltype(tn)::value>), dim3(d.ntiles), dim3(kTileThreads), 0,
-                             s, m, x, y);
+          constexpr int TN = decltype(tn)::value;
+          const auto kernel = m.col24 ? csr_tile_kernel<VT, XT, YT, TN, true> : csr_tile_kernel<VT, XT, YT, TN, false>;
+          hipLaunchKernelGGL(kernel, dim3(d.ntiles), dim3(kTileThreads), 0, s, m, x, y);
         });
       if (d.nlong > 0)
         hipLaunchKernelGGL((csr_long_kernel<VT, XT, YT>), dim3(d.nlong), dim3(kTileThreads), 0, s, m, x, y);
@@ -256,11 +273,13 @@ void run_typed(const DeviceMatrix &d, const XT *x, YT *y, int vect_incr, hipStre
       const long y_off = vect_incr - (d.format == cpp::FORMAT_SCOO ? d.f_row : 0);
       if (d.ntiles > 0)
         with_tile_size(d, [&](auto tn) {
-          hipLaunchKernelGGL((coo_tile_kernel<VT, XT, YT, decltype(tn)::value, false>), dim3(d.ntiles),
-                             dim3(kTileThreads), 0, s, m, x, y, d.segrow.as<int>(), y_off);
+          constexpr int TN = decltype(tn)::value;
+          const auto kernel = m.col24 ? coo_tile_kernel<VT, XT, YT, TN, true, false>
+                                      : coo_tile_kernel<VT, XT, YT, TN, false, false>;
+          hipLaunchKernelGGL(kernel, dim3(d.ntiles), dim3(kTileThreads), 0, s, m, x, y, d.segrow.as<int>(), y_off);
         });
       if (d.nlong > 0)
-        hipLaunchKernelGGL((coo_tile_kernel<VT, XT, YT, kTileThreads, true>), dim3(d.nlong), dim3(kTileThreads), 0, s, m, x, y,
+        hipLaunchKernelGGL((coo_tile_kernel<VT, XT, YT, kTileThreads, false, true>), dim3(d.nlong), dim3(kTileThreads), 0, s, m, x, y,
                            d.segrow.as<int>(), y_off);
       break;
     }
@@ -287,6 +306,15 @@ void launch_spmv(const DeviceMatrix &d, const void *x, Dtype xdt, void *y, Dtype
   } else {
     throw std::invalid_argument("tbsla: unsupported value/vector type combination for this format");
   }
+}
+
+void pack_columns(DeviceMatrix &d) {
+  if (d.entries <= 0 || d.x_need > (1L << 24) || (d.vdt == Dtype::F64 && d.entries > (1L << 25))) return;
+  const long groups = (d.entries + 3) / 4;
+  d.col24.reserve(static_cast<std::size_t>(groups) * 12);
+  hipLaunchKernelGGL(pack24_kernel, dim3(static_cast<unsigned>(std::min<long>((groups + 255) / 256, 65536))), dim3(256),
+                     0, nullptr, d.colidx.as<int>(), d.entries, d.f_col, d.col24.as<unsigned>());
+  TBSLA_HIP_CHECK(hipGetLastError());
 }
 
 void launch_fill(void *y, Dtype ydt, long n, double value, hipStream_t s) {

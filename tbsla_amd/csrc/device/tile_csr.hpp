@@ -5,7 +5,8 @@
 // (T = kCsrTileNnz, 3072, or the caller's TN) and owns the rows whose first
 // entry lies in it
 // (tile_row[t] .. tile_row[t+1]).  A tile's entries are read with 16-byte
-// loads at an aligned offset that needs no descriptor load, the products
+// loads (packed columns: 12 bytes) at an aligned offset that needs no
+// descriptor load, the products
 // v * x[c] are rounded and staged in LDS, and each owned row is summed by one
 // thread from 0, left to right, finishing a row that runs past the tile from
 // global memory in the same order.  That reproduces the sequential FP64 row
@@ -123,12 +124,23 @@ struct CsrView {
   const int *long_rows;
   long nnz;
   int rp0, f_col;
+  // the columns minus f_col packed in three bytes each (little endian, four
+  // in three words), or nullptr
+  const unsigned *col24 = nullptr;
+
+  __device__ int col(long e) const {  // local column of entry e
+    typedef unsigned u32_u __attribute__((aligned(1)));
+    if (col24)
+      return static_cast<int>(*reinterpret_cast<const u32_u *>(reinterpret_cast<const char *>(col24) + 3 * e) &
+                              0xFFFFFFu);
+    return colidx[e] - f_col;
+  }
 };
 
 template <typename VT>
 inline CsrView<VT> csr_view(const DeviceMatrix &d) {
   return CsrView<VT>{d.rowptr.as<int>(), d.colidx.as<int>(), d.vals.as<VT>(), d.tiles.as<int>(),
-                     d.long_rows.as<int>(), d.entries, d.rp0, d.f_col};
+                     d.long_rows.as<int>(), d.entries, d.rp0, d.f_col, d.col24.as<unsigned>()};
 }
 
 // A row's sum reads its products from LDS kSumRun at a time, all reads issued
@@ -156,7 +168,7 @@ struct Prod {
   }
   __device__ static AT one(const CsrView<VT> &m, const XT *__restrict__ x, long e) {
     const AT v = Val<VT>::get(m.vals, e);
-    const AT xv = static_cast<AT>(x[m.colidx[e] - m.f_col]);
+    const AT xv = static_cast<AT>(x[m.col(e)]);
     return v * xv;
   }
 };
@@ -174,7 +186,7 @@ struct Prod<Pattern, XT> {
     for (int q = 0; q < 4; q++) p[q] = static_cast<double>(z[c[q]]);
   }
   __device__ static double one(const CsrView<Pattern> &m, const XT *__restrict__ z, long e) {
-    return static_cast<double>(z[m.colidx[e] - m.f_col]);
+    return static_cast<double>(z[m.col(e)]);
   }
 };
 
@@ -195,34 +207,67 @@ __device__ inline AT epi_init(const E &, int, long) {
 // prod[0 .. ne).  FULL (ne == TN, every tile but the matrix's last)
 // reads with no per-entry guard; otherwise entries at or past ne are not read
 // (a caller's value array holds exactly nnz values).
-template <bool FULL, typename VT, typename XT, int TN>
+template <bool FULL, bool PACK, typename VT, typename XT, int TN>
 struct TileEntries {
   using AT = typename Val<VT>::A;
   static constexpr int G = TN / 4 / kTileThreads;  // 4-entry groups per thread
-  int c[G][4];
+  v4i raw[G];  // the groups' columns as loaded: four ints, or three words of packed ones
   AT v[G][4];
 
   __device__ void load(const CsrView<VT> &m, long e0, int ne) {
+    typedef unsigned v3u __attribute__((ext_vector_type(3), aligned(4)));
+    if constexpr (PACK) {
+#pragma unroll
+      for (int k = 0; k < G; k++) {
+        const int g = k * kTileThreads + threadIdx.x;
+        if (FULL || 4 * g < ne) {
+          const v3u w = *reinterpret_cast<const v3u *>(m.col24 + (e0 / 4 + g) * 3);
+          raw[k].x = static_cast<int>(w.x);
+          raw[k].y = static_cast<int>(w.y);
+          raw[k].z = static_cast<int>(w.z);
+        }
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < G; k++) {
+        const int g = k * kTileThreads + threadIdx.x;
+        if (FULL || 4 * g < ne) raw[k] = *reinterpret_cast<const v4i *>(m.colidx + e0 + 4 * g);
+      }
+    }
 #pragma unroll
     for (int k = 0; k < G; k++) {
       const int g = k * kTileThreads + threadIdx.x;
-      if (FULL || 4 * g < ne) {
-        const v4i ci = *reinterpret_cast<const v4i *>(m.colidx + e0 + 4 * g);
-        c[k][0] = ci.x - m.f_col;
-        c[k][1] = ci.y - m.f_col;
-        c[k][2] = ci.z - m.f_col;
-        c[k][3] = ci.w - m.f_col;
-        if (!FULL)  // entries past the matrix end read the zeroed padding: column 0
-          for (int q = 0; q < 4; q++)
-            if (4 * g + q >= ne) c[k][q] = 0;
-      }
       if (FULL || 4 * g + 4 <= ne) Prod<VT, XT>::load4(m, e0 + 4 * g, v[k]);
+    }
+  }
+
+  __device__ void columns(const CsrView<VT> &m, int ne, int (&c)[G][4]) const {
+#pragma unroll
+    for (int k = 0; k < G; k++) {
+      if constexpr (PACK) {
+        const unsigned a = static_cast<unsigned>(raw[k].x), b = static_cast<unsigned>(raw[k].y),
+                       d = static_cast<unsigned>(raw[k].z);
+        c[k][0] = static_cast<int>(a & 0xFFFFFFu);
+        c[k][1] = static_cast<int>(a >> 24 | (b & 0xFFFFu) << 8);
+        c[k][2] = static_cast<int>(b >> 16 | (d & 0xFFu) << 16);
+        c[k][3] = static_cast<int>(d >> 8);
+      } else {
+        c[k][0] = raw[k].x - m.f_col;
+        c[k][1] = raw[k].y - m.f_col;
+        c[k][2] = raw[k].z - m.f_col;
+        c[k][3] = raw[k].w - m.f_col;
+      }
+      if (!FULL)  // entries past the matrix end: column 0
+        for (int q = 0; q < 4; q++)
+          if (4 * (k * kTileThreads + static_cast<int>(threadIdx.x)) + q >= ne) c[k][q] = 0;
     }
   }
 
   // gathers and rounded products into p
   __device__ void products(const CsrView<VT> &m, const XT *__restrict__ x, long e0, int ne, AT (&p)[G][4]) const {
 #pragma clang fp contract(off)
+    int c[G][4];
+    columns(m, ne, c);
 #pragma unroll
     for (int k = 0; k < G; k++) {
       const int g = k * kTileThreads + threadIdx.x;
@@ -257,7 +302,7 @@ struct NoPre {
 // The bounds of the thread's first owned row, then the index/value loads,
 // gathers and products into prod.  (Issuing the row table first measured
 // faster than deferring it behind the tile loads.)
-template <bool FULL, typename VT, typename XT, int TN, typename Pre>
+template <bool FULL, bool PACK, typename VT, typename XT, int TN, typename Pre>
 __device__ inline void csr_tile_stage(const CsrView<VT> &m, const XT *__restrict__ x, typename Val<VT>::A *prod,
                                       long e0, int ne, int rlo, int rhi, int &a, int &b, Pre &pre) {
   // loaded with no branch so they stay in flight under the tile loads
@@ -265,19 +310,22 @@ __device__ inline void csr_tile_stage(const CsrView<VT> &m, const XT *__restrict
   // that owns a row)
   a = m.rowptr[min(rlo + static_cast<int>(threadIdx.x), rhi)] - m.rp0;
   b = m.rowptr[min(rlo + static_cast<int>(threadIdx.x) + 1, rhi)] - m.rp0;
-  TileEntries<FULL, VT, XT, TN> t;
+  TileEntries<FULL, PACK, VT, XT, TN> t;
   t.load(m, e0, ne);
   pre.issue();
-  typename Val<VT>::A p[TileEntries<FULL, VT, XT, TN>::G][4];
+  typename Val<VT>::A p[TileEntries<FULL, PACK, VT, XT, TN>::G][4];
   t.products(m, x, e0, ne, p);
   pre.finish();
-  TileEntries<FULL, VT, XT, TN>::store(p, prod, ne);
+  TileEntries<FULL, PACK, VT, XT, TN>::store(p, prod, ne);
 }
 
 // Rows of entry tile `tile`; epi(row, sum) once per owned row by the thread
 // that sums it, rows longer than LT left to csr_long_row.  The caller
 // synchronises the block before reusing `lds`.
-template <typename VT, typename XT, typename Epi, int TN, int LT, typename Pre = NoPre>
+// COLS: whether the columns are packed (kPacked, kPlain: known to the caller;
+// kEither: looked up in m).
+enum TileCols { kEither, kPlain, kPacked };
+template <typename VT, typename XT, typename Epi, int TN, int LT, TileCols COLS = kEither, typename Pre = NoPre>
 __device__ inline void csr_tile_rows_at(const CsrView<VT> &m, const XT *__restrict__ x,
                                         CsrTileLds<typename Val<VT>::A, TN> &lds, Epi &epi, int tile,
                                         Pre &&pre = Pre()) {
@@ -288,10 +336,15 @@ __device__ inline void csr_tile_rows_at(const CsrView<VT> &m, const XT *__restri
   const int ne = static_cast<int>(min(static_cast<long>(TN), m.nnz - e0));
   const int rlo = m.tile_row[tile], rhi = m.tile_row[tile + 1];
   int a, b;
-  if (ne == TN)
-    csr_tile_stage<true, VT, XT, TN>(m, x, lds.prod, e0, ne, rlo, rhi, a, b, pre);
+  const bool packed = COLS == kPacked || (COLS == kEither && m.col24);
+  if (packed && ne == TN)
+    csr_tile_stage<true, true, VT, XT, TN>(m, x, lds.prod, e0, ne, rlo, rhi, a, b, pre);
+  else if (packed)
+    csr_tile_stage<false, true, VT, XT, TN>(m, x, lds.prod, e0, ne, rlo, rhi, a, b, pre);
+  else if (ne == TN)
+    csr_tile_stage<true, false, VT, XT, TN>(m, x, lds.prod, e0, ne, rlo, rhi, a, b, pre);
   else
-    csr_tile_stage<false, VT, XT, TN>(m, x, lds.prod, e0, ne, rlo, rhi, a, b, pre);
+    csr_tile_stage<false, false, VT, XT, TN>(m, x, lds.prod, e0, ne, rlo, rhi, a, b, pre);
   __syncthreads();
   const long e1 = e0 + ne;
   for (int r = rlo + tid; r < rhi; r += kTileThreads) {
@@ -326,10 +379,10 @@ __device__ inline void csr_tile_rows_at(const CsrView<VT> &m, const XT *__restri
 }
 
 // Rows of entry tile blockIdx.x.
-template <typename VT, typename XT, int TN, typename Epi, typename Pre = NoPre>
+template <typename VT, typename XT, int TN, TileCols COLS = kEither, typename Epi, typename Pre = NoPre>
 __device__ inline void csr_tile_rows(const CsrView<VT> &m, const XT *__restrict__ x,
                                      CsrTileLds<typename Val<VT>::A, TN> &lds, Epi &epi, Pre &&pre = Pre()) {
-  csr_tile_rows_at<VT, XT, Epi, TN, kCsrLongRow>(m, x, lds, epi, blockIdx.x, pre);
+  csr_tile_rows_at<VT, XT, Epi, TN, kCsrLongRow, COLS>(m, x, lds, epi, blockIdx.x, pre);
 }
 
 // One long row (m.long_rows[idx]) per workgroup: chunk products (LC
