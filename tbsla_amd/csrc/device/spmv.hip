@@ -18,7 +18,8 @@
 //                   y[row], so each row is accumulated in entry order
 //                   (MatrixCOO.cpp:113-115 / MatrixSCOO.cpp:120-122 with one
 //                   thread).
-// dense_kernel      four rows per wavefront sharing each x load, butterfly reduction
+// dense_kernel      one row per wavefront, or four sharing each x load, butterfly
+//                   reduction
 //                   (MatrixDENSE.cpp:67-72, different summation order).
 #include <hip/hip_runtime.h>
 
@@ -160,15 +161,15 @@ __global__ __launch_bounds__(kTileThreads) void coo_tile_kernel(dev::CsrView<VT>
     dev::csr_tile_rows<VT, XT, TN, PACK ? dev::kPacked : dev::kPlain>(m, x, lds, epi);
 }
 
-// kDenseRows consecutive rows per wavefront, so each x load serves all of
-// them; per row and lane the columns are summed in the same order as with one
-// row per wavefront (j = 2*lane + 128*k), then a butterfly.
-constexpr int kDenseRows = 4;
-
-template <typename XT, typename YT>
+// R consecutive rows per wavefront, so each x load serves all of them; per row
+// and lane the columns are summed in one order whatever R is (j = 2*lane +
+// 128*k), then a butterfly.  Bound by the HBM reads of A: two steps of R
+// 16-byte loads in flight, non-temporal, and with an odd row length every
+// other row starts 8 bytes off a 16-byte boundary, which the loads allow (8191
+// x 8191: 247 us with 8-byte loads, 83 now; 8192 x 8192 83 in both, 6.5 TB/s).
+template <typename XT, typename YT, int R>
 __global__ __launch_bounds__(256) void dense_kernel(const double *__restrict__ A, const XT *__restrict__ x,
                                                     YT *__restrict__ y, int rows, int cols, long ld) {
-  constexpr int R = kDenseRows;
   const int w = (blockIdx.x * 256 + threadIdx.x) >> 6;
   const int lane = threadIdx.x & 63;
   const long r0 = static_cast<long>(w) * R;
@@ -177,43 +178,34 @@ __global__ __launch_bounds__(256) void dense_kernel(const double *__restrict__ A
   double acc[R];
 #pragma unroll
   for (int r = 0; r < R; r++) acc[r] = 0;
-  if ((ld & 1) == 0) {
-    // 16-byte non-temporal loads, two columns per lane, two steps of R rows in flight
-    int j = 2 * lane;
-    for (; j + 128 + 1 < cols; j += 2 * 128) {
-      dev::v2d av[2][R];
-      double xv[2][2];
+  typedef double v2d_8 __attribute__((ext_vector_type(2), aligned(8)));
+  int j = 2 * lane;
+  for (; j + 128 + 1 < cols; j += 2 * 128) {
+    v2d_8 av[2][R];
+    double xv[2][2];
 #pragma unroll
-      for (int u = 0; u < 2; u++) {
-        xv[u][0] = static_cast<double>(x[j + u * 128]);
-        xv[u][1] = static_cast<double>(x[j + u * 128 + 1]);
-#pragma unroll
-        for (int r = 0; r < R; r++)
-          av[u][r] = r < nr ? __builtin_nontemporal_load(
-                                  reinterpret_cast<const dev::v2d *>(A + (r0 + r) * ld + j + u * 128))
-                            : dev::v2d{0, 0};
-      }
-#pragma unroll
-      for (int u = 0; u < 2; u++)
-#pragma unroll
-        for (int r = 0; r < R; r++) acc[r] += av[u][r].x * xv[u][0] + av[u][r].y * xv[u][1];
-    }
-    for (; j < cols; j += 128)
+    for (int u = 0; u < 2; u++) {
+      xv[u][0] = static_cast<double>(x[j + u * 128]);
+      xv[u][1] = static_cast<double>(x[j + u * 128 + 1]);
 #pragma unroll
       for (int r = 0; r < R; r++)
-        if (r < nr) {
-          const double *a = A + (r0 + r) * ld;
-          acc[r] += __builtin_nontemporal_load(a + j) * static_cast<double>(x[j]);
-          if (j + 1 < cols) acc[r] += __builtin_nontemporal_load(a + j + 1) * static_cast<double>(x[j + 1]);
-        }
-  } else {
+        av[u][r] = r < nr ? __builtin_nontemporal_load(
+                                reinterpret_cast<const v2d_8 *>(A + (r0 + r) * ld + j + u * 128))
+                          : v2d_8{0, 0};
+    }
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+#pragma unroll
+      for (int r = 0; r < R; r++) acc[r] += av[u][r].x * xv[u][0] + av[u][r].y * xv[u][1];
+  }
+  for (; j < cols; j += 128)
 #pragma unroll
     for (int r = 0; r < R; r++)
       if (r < nr) {
         const double *a = A + (r0 + r) * ld;
-        for (int j = lane; j < cols; j += 64) acc[r] += __builtin_nontemporal_load(a + j) * static_cast<double>(x[j]);
+        acc[r] += __builtin_nontemporal_load(a + j) * static_cast<double>(x[j]);
+        if (j + 1 < cols) acc[r] += __builtin_nontemporal_load(a + j + 1) * static_cast<double>(x[j + 1]);
       }
-  }
 #pragma unroll
   for (int r = 0; r < R; r++) {
 #pragma unroll
@@ -244,6 +236,20 @@ __global__ __launch_bounds__(256) void pack24_kernel(const int *__restrict__ col
 }
 
 inline unsigned blocks_for(long n, int per_block) { return static_cast<unsigned>((n + per_block - 1) / per_block); }
+
+// Four rows per wavefront from 7168 rows on, where that still fills the chip
+// (seven wavefronts a CU); one below: 2000 x 2000 10.9 us with four, 8.3 with
+// one, 4096 28.3 and 21.6, 7001 66.2 and 64.4, 8192 83.0 and 85.9.
+constexpr int kDenseRows = 4, kDenseManyRows = 7168;
+
+template <typename XT, typename YT>
+void launch_dense(const DeviceMatrix &d, const XT *x, YT *y, hipStream_t s) {
+  const bool many = d.rows >= kDenseManyRows;
+  const long waves = many ? (static_cast<long>(d.rows) + kDenseRows - 1) / kDenseRows : d.rows;
+  const auto kernel = many ? dense_kernel<XT, YT, kDenseRows> : dense_kernel<XT, YT, 1>;
+  hipLaunchKernelGGL(kernel, dim3(blocks_for(waves * 64, 256)), dim3(256), 0, s, d.dvals.as<double>(), x, y, d.rows,
+                     d.dcols, static_cast<long>(d.dcols));
+}
 
 template <typename VT, typename XT, typename YT>
 void run_typed(const DeviceMatrix &d, const XT *x, YT *y, int vect_incr, hipStream_t s) {
@@ -284,9 +290,7 @@ void run_typed(const DeviceMatrix &d, const XT *x, YT *y, int vect_incr, hipStre
       break;
     }
     case cpp::FORMAT_DENSE:
-      if (d.rows > 0)
-        hipLaunchKernelGGL((dense_kernel<XT, YT>), dim3(blocks_for((static_cast<long>(d.rows) + kDenseRows - 1) / kDenseRows * 64, 256)),
-                           dim3(256), 0, s, d.dvals.as<double>(), x, y, d.rows, d.dcols, static_cast<long>(d.dcols));
+      if (d.rows > 0) launch_dense<XT, YT>(d, x, y, s);
       break;
   }
   TBSLA_HIP_CHECK(hipGetLastError());
