@@ -216,27 +216,19 @@ struct TileEntries {
 
   __device__ void load(const CsrView<VT> &m, long e0, int ne) {
     typedef unsigned v3u __attribute__((ext_vector_type(3), aligned(4)));
-    if constexpr (PACK) {
 #pragma unroll
-      for (int k = 0; k < G; k++) {
-        const int g = k * kTileThreads + threadIdx.x;
-        if (FULL || 4 * g < ne) {
+    for (int k = 0; k < G; k++) {
+      const int g = k * kTileThreads + threadIdx.x;
+      if (FULL || 4 * g < ne) {
+        if constexpr (PACK) {
           const v3u w = *reinterpret_cast<const v3u *>(m.col24 + (e0 / 4 + g) * 3);
           raw[k].x = static_cast<int>(w.x);
           raw[k].y = static_cast<int>(w.y);
           raw[k].z = static_cast<int>(w.z);
+        } else {
+          raw[k] = *reinterpret_cast<const v4i *>(m.colidx + e0 + 4 * g);
         }
       }
-    } else {
-#pragma unroll
-      for (int k = 0; k < G; k++) {
-        const int g = k * kTileThreads + threadIdx.x;
-        if (FULL || 4 * g < ne) raw[k] = *reinterpret_cast<const v4i *>(m.colidx + e0 + 4 * g);
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < G; k++) {
-      const int g = k * kTileThreads + threadIdx.x;
       if (FULL || 4 * g + 4 <= ne) Prod<VT, XT>::load4(m, e0 + 4 * g, v[k]);
     }
   }
@@ -326,10 +318,12 @@ __device__ inline void csr_tile_stage(const CsrView<VT> &m, const XT *__restrict
 // kEither: looked up in m).
 enum TileCols { kEither, kPlain, kPacked };
 template <typename VT, typename XT, typename Epi, int TN, int LT, TileCols COLS = kEither, typename Pre = NoPre>
-__device__ inline void csr_tile_rows_at(const CsrView<VT> &m, const XT *__restrict__ x,
+__device__ inline void csr_tile_rows_at(const CsrView<VT> &mat, const XT *__restrict__ x,
                                         CsrTileLds<typename Val<VT>::A, TN> &lds, Epi &epi, int tile,
                                         Pre &&pre = Pre()) {
 #pragma clang fp contract(off)
+  CsrView<VT> m = mat;
+  if (COLS == kPlain) m.col24 = nullptr;
   using AT = typename Val<VT>::A;
   const int tid = threadIdx.x;
   const long e0 = static_cast<long>(tile) * TN;
