@@ -79,6 +79,19 @@ class DevBuf {
     TBSLA_HIP_CHECK(hipMalloc(&p_, padded));
     bytes_ = padded - 256;
   }
+  // reserve for memory that can be done without: false if there is none
+  bool try_reserve(std::size_t bytes) {
+    if (bytes <= bytes_ && p_) return true;
+    release();
+    std::size_t padded = ((bytes ? bytes : 1) + 255 + 256) & ~std::size_t(255);
+    if (hipMalloc(&p_, padded) != hipSuccess) {
+      (void)hipGetLastError();
+      p_ = nullptr;
+      return false;
+    }
+    bytes_ = padded - 256;
+    return true;
+  }
   void upload(const void *src, std::size_t bytes, hipStream_t s = nullptr) {
     alloc(bytes);
     if (bytes) TBSLA_HIP_CHECK(hipMemcpyAsync(p_, src, bytes, hipMemcpyHostToDevice, s));

@@ -170,6 +170,7 @@ void build_ell(DeviceMatrix &d, const cpp::MatrixELL &m, Dtype vdt) {
   });
   d.x_need = hi + 1;
   d.ecols.upload(ccm.data(), ccm.size() * sizeof(int));
+  pack_ell_columns(d);
   upload_values(d.evals, vcm.data(), vcm.size(), vdt);
 }
 

@@ -60,7 +60,11 @@ struct DeviceMatrix {
   int tile_nnz = kCsrTileNnz;  // entries per tile of the table in `tiles`
   // ELL (sliced column-major)
   int K = 0;
+  // ecols with epacked: slots in groups of four, the columns of slots j..j+3 of
+  // row i in three words at 3 * (((i / kEllSlice) * ceil(K / 4) + j / 4) *
+  // kEllSlice + i % kEllSlice)
   DevBuf ecols, evals;
+  bool epacked = false;
   // COO / SCOO: segments of the row-sorted view (rowptr, colidx, vals, tiles
   // and long_rows above hold the segment CSR)
   DevBuf segrow;

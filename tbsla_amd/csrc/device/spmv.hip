@@ -68,7 +68,8 @@ __global__ __launch_bounds__(kTileThreads) void csr_long_kernel(dev::CsrView<VT>
 // is one coalesced load per wavefront.  Slots go in groups of kEllGroup; the
 // next group's loads are issued before this group's gathers (two register
 // sets, alternating), so each group waits on one round trip.  Each row still
-// sums its slots in order 0..K-1.
+// sums its slots in order 0..K-1.  Bound by the HBM reads of the slots: columns
+// are read packed in three bytes where they fit (pack_ell_columns).
 constexpr int kEllGroup = 8;
 
 __device__ inline double ell_value(const double *p, long i) { return __builtin_nontemporal_load(p + i); }
@@ -77,20 +78,40 @@ __device__ inline float ell_value(const bf16 *p, long i) {
   return Val<bf16>::cvt(__builtin_nontemporal_load(reinterpret_cast<const unsigned short *>(p) + i));
 }
 
-template <typename VT>
+// Columns of N slots from slot j of the slice: `cols` points at the thread's
+// first slot (plain) or its first group's words (packed; j a multiple of 4).
+template <bool PACK, int N>
+__device__ inline void ell_columns(const int *__restrict__ cols, int j, int (&c)[kEllGroup]) {
+  if constexpr (PACK) {
+#pragma unroll
+    for (int g = 0; g < (N + 3) / 4; g++) {
+      const int *w = cols + static_cast<long>(j / 4 + g) * kEllSlice * 3;
+      const unsigned a = static_cast<unsigned>(__builtin_nontemporal_load(w)),
+                     b = static_cast<unsigned>(__builtin_nontemporal_load(w + 1)),
+                     d = static_cast<unsigned>(__builtin_nontemporal_load(w + 2));
+      c[4 * g] = static_cast<int>(a & 0xFFFFFFu);
+      c[4 * g + 1] = static_cast<int>(a >> 24 | (b & 0xFFFFu) << 8);
+      c[4 * g + 2] = static_cast<int>(b >> 16 | (d & 0xFFu) << 16);
+      c[4 * g + 3] = static_cast<int>(d >> 8);
+    }
+  } else {
+#pragma unroll
+    for (int u = 0; u < N; u++) c[u] = nt_load(cols, static_cast<long>(j + u) * kEllSlice);
+  }
+}
+
+template <typename VT, bool PACK>
 struct EllGroup {
   using AT = typename Val<VT>::A;
   int c[kEllGroup];
   AT v[kEllGroup];
 
-  // slots o, o + kEllSlice, ... (N of them)
+  // slots j, j + 1, ... (N of them)
   template <int N>
-  __device__ void load(const int *__restrict__ cols, const VT *__restrict__ vals, long o) {
+  __device__ void load(const int *__restrict__ cols, const VT *__restrict__ vals, int j) {
+    ell_columns<PACK, N>(cols, j, c);
 #pragma unroll
-    for (int u = 0; u < N; u++) {
-      c[u] = nt_load(cols, o + u * kEllSlice);
-      v[u] = ell_value(vals, o + u * kEllSlice);
-    }
+    for (int u = 0; u < N; u++) v[u] = ell_value(vals, static_cast<long>(j + u) * kEllSlice);
   }
   template <int N, typename XT>
   __device__ void accumulate(const XT *__restrict__ x, AT &acc) const {
@@ -103,30 +124,44 @@ struct EllGroup {
   }
 };
 
-template <typename VT, typename XT, typename YT>
+template <typename VT, typename XT, typename YT, bool PACK>
 __global__ __launch_bounds__(kEllSlice) void ell_kernel(const int *__restrict__ cols, const VT *__restrict__ vals,
                                                         const XT *__restrict__ x, YT *__restrict__ y, int rows,
                                                         int K) {
   using AT = typename Val<VT>::A;
   const long i = static_cast<long>(blockIdx.x) * kEllSlice + threadIdx.x;
   if (i >= rows) return;
-  const long base = static_cast<long>(blockIdx.x) * K * kEllSlice + threadIdx.x;
+  vals += static_cast<long>(blockIdx.x) * K * kEllSlice + threadIdx.x;
+  cols += PACK ? (static_cast<long>(blockIdx.x) * ((K + 3) / 4) * kEllSlice + threadIdx.x) * 3
+               : static_cast<long>(blockIdx.x) * K * kEllSlice + threadIdx.x;
   const int KG = K - K % kEllGroup;  // slots in whole groups
   AT acc = 0;
-  EllGroup<VT> A, B;
+  EllGroup<VT, PACK> A, B;
   int j = 0;
-  if (KG > 0) A.template load<kEllGroup>(cols, vals, base);
+  if (KG > 0) A.template load<kEllGroup>(cols, vals, 0);
   while (j < KG) {
-    if (j + kEllGroup < KG) B.template load<kEllGroup>(cols, vals, base + static_cast<long>(j + kEllGroup) * kEllSlice);
+    if (j + kEllGroup < KG) B.template load<kEllGroup>(cols, vals, j + kEllGroup);
     A.template accumulate<kEllGroup>(x, acc);
     j += kEllGroup;
     if (j >= KG) break;
-    if (j + kEllGroup < KG) A.template load<kEllGroup>(cols, vals, base + static_cast<long>(j + kEllGroup) * kEllSlice);
+    if (j + kEllGroup < KG) A.template load<kEllGroup>(cols, vals, j + kEllGroup);
     B.template accumulate<kEllGroup>(x, acc);
     j += kEllGroup;
   }
-  for (; j < K; j++) {  // the last K % kEllGroup slots
-    A.template load<1>(cols, vals, base + static_cast<long>(j) * kEllSlice);
+  // the last K % kEllGroup slots: four together, then one to three
+  if (K - j >= 4) {
+    A.template load<4>(cols, vals, j);
+    A.template accumulate<4>(x, acc);
+    j += 4;
+  }
+  if (K - j == 3) {
+    A.template load<3>(cols, vals, j);
+    A.template accumulate<3>(x, acc);
+  } else if (K - j == 2) {
+    A.template load<2>(cols, vals, j);
+    A.template accumulate<2>(x, acc);
+  } else if (K - j == 1) {
+    A.template load<1>(cols, vals, j);
     A.template accumulate<1>(x, acc);
   }
   y[i] = static_cast<YT>(acc);
@@ -235,6 +270,24 @@ __global__ __launch_bounds__(256) void pack24_kernel(const int *__restrict__ col
   }
 }
 
+// the columns of slot group j / 4 of every row of every slice (plain layout
+// `in`, K slots; slots past K: column 0), as DeviceMatrix::ecols packed
+__global__ __launch_bounds__(kEllSlice) void pack_ell_kernel(const int *__restrict__ in, int K,
+                                                             unsigned *__restrict__ out) {
+  const int KQ = (K + 3) / 4;
+  for (int g = 0; g < KQ; g++) {
+    unsigned c[4];
+    for (int q = 0; q < 4; q++)
+      c[q] = 4 * g + q < K ? static_cast<unsigned>(in[(static_cast<long>(blockIdx.x) * K + 4 * g + q) * kEllSlice +
+                                                      threadIdx.x])
+                           : 0u;
+    unsigned *o = out + ((static_cast<long>(blockIdx.x) * KQ + g) * kEllSlice + threadIdx.x) * 3;
+    o[0] = c[0] | c[1] << 24;
+    o[1] = c[1] >> 8 | c[2] << 16;
+    o[2] = c[2] >> 16 | c[3] << 8;
+  }
+}
+
 inline unsigned blocks_for(long n, int per_block) { return static_cast<unsigned>((n + per_block - 1) / per_block); }
 
 // Four rows per wavefront from 7168 rows on, where that still fills the chip
@@ -268,8 +321,9 @@ void run_typed(const DeviceMatrix &d, const XT *x, YT *y, int vect_incr, hipStre
     }
     case cpp::FORMAT_ELL:
       if (d.rows > 0)
-        hipLaunchKernelGGL((ell_kernel<VT, XT, YT>), dim3(blocks_for(d.rows, kEllSlice)), dim3(kEllSlice), 0, s,
-                           d.ecols.as<int>(), d.evals.as<VT>(), x, y, d.rows, d.K);
+        hipLaunchKernelGGL((d.epacked ? ell_kernel<VT, XT, YT, true> : ell_kernel<VT, XT, YT, false>),
+                           dim3(blocks_for(d.rows, kEllSlice)), dim3(kEllSlice), 0, s, d.ecols.as<int>(),
+                           d.evals.as<VT>(), x, y, d.rows, d.K);
       break;
     case cpp::FORMAT_COO:
     case cpp::FORMAT_SCOO: {
@@ -315,10 +369,24 @@ void launch_spmv(const DeviceMatrix &d, const void *x, Dtype xdt, void *y, Dtype
 void pack_columns(DeviceMatrix &d) {
   if (d.entries <= 0 || d.x_need > (1L << 24) || (d.vdt == Dtype::F64 && d.entries > (1L << 25))) return;
   const long groups = (d.entries + 3) / 4;
-  d.col24.reserve(static_cast<std::size_t>(groups) * 12);
+  if (!d.col24.try_reserve(static_cast<std::size_t>(groups) * 12)) return;
   hipLaunchKernelGGL(pack24_kernel, dim3(static_cast<unsigned>(std::min<long>((groups + 255) / 256, 65536))), dim3(256),
                      0, nullptr, d.colidx.as<int>(), d.entries, d.f_col, d.col24.as<unsigned>());
   TBSLA_HIP_CHECK(hipGetLastError());
+}
+
+void pack_ell_columns(DeviceMatrix &d) {
+  if (d.rows <= 0 || d.x_need > (1L << 24)) return;
+  const unsigned slices = blocks_for(d.rows, kEllSlice);
+  DevBuf out;
+  if (!out.try_reserve(static_cast<std::size_t>(slices) * static_cast<std::size_t>((d.K + 3) / 4) * kEllSlice * 12))
+    return;
+  hipLaunchKernelGGL(pack_ell_kernel, dim3(slices), dim3(kEllSlice), 0, nullptr, d.ecols.as<int>(), d.K,
+                     out.as<unsigned>());
+  TBSLA_HIP_CHECK(hipGetLastError());
+  TBSLA_HIP_CHECK(hipDeviceSynchronize());
+  d.ecols = std::move(out);
+  d.epacked = true;
 }
 
 void launch_fill(void *y, Dtype ydt, long n, double value, hipStream_t s) {
