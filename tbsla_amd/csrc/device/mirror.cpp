@@ -80,17 +80,19 @@ MinMax minmax_offset(const int *a, std::size_t n, long off) {
 }
 
 // Entries per tile.  A CU holds six workgroups with 3072-entry tiles (LDS) and
-// eight with smaller ones, so up to two rounds of them (9.4 M entries) 2048
-// fills the last round better (500,009 rows of 16: 30.8 -> 26.7 us; 300,007
-// of 12: 14.0 -> 13.1; 1,000,003 of 16, past the line: 51.8 against 53.9).  Up
-// to a tile of 1024 per workgroup slot's half, PageRank's updates are latency
-// alone and take the smallest (a row per thread, and the step decision merged
-// in).  A row that runs past its tile is finished by one thread from memory:
-// with rows over 256 entries the large tiles stay.
+// eight with smaller ones, so matrices that the caches hold run faster with
+// 2048 (500,009 rows of 16: 25.8 -> 25.2 us; 1,000,003: 49.8 -> 46.5, FP32 32.3
+// -> 29.6; 1,500,003: 73.4 -> 72.4) and those that stream from HBM with 3072
+// (3,000,003: 158.5 -> 152.4; 700,001 of 37: 90.2 -> 86.7).  Up to a tile of
+// 1024 per workgroup slot's half, PageRank's updates are latency alone and
+// take the smallest (a row per thread, and the step decision merged in).  A
+// row that runs past its tile is finished by one thread from memory: with rows
+// over 256 entries the large tiles stay.
+constexpr long kLargeTiles = 3L << 23;  // more entries than this: 3072
 int tile_size(long nnz, const int *rowptr, int rows) {
   int longest = 0;
   for (int i = 0; i < rows; i++) longest = std::max(longest, rowptr[i + 1] - rowptr[i]);
-  if (longest > 256 || nnz > 2L * 1536 * kCsrTileNnz) return kCsrTileNnz;
+  if (longest > 256 || nnz > kLargeTiles) return kCsrTileNnz;
   return nnz <= (1L << 20) ? 1024 : 2048;
 }
 
