@@ -362,7 +362,7 @@ template <typename VT, typename XT, int UNR, int TN>
 __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(UNR == 16 ? 2 : 1)))
 void batch_step(BatchDev<VT, XT> d, int par) {
   using AT = typename dev::Val<VT>::A;
-  __shared__ dev::CsrTileLds<AT, TN> lds;
+  __shared__ dev::CsrTileLds<AT, TN, 0> lds;
   __shared__ double red[kTileThreads];
   {  // nothing left to do once every set is done (a replay may run on past it)
     int active = 0;
@@ -401,9 +401,9 @@ void batch_step(BatchDev<VT, XT> d, int par) {
       TileEpi<XT> epi{xa_out, d.row_graph, d.rs, d.a_member, d.slots, d.beta, gA, gB, w % kSlots,
                       -INFINITY, -INFINITY};
       if (tile)
-        dev::csr_tile_rows_at<VT, XT, TileEpi<XT>, TN, kBatchLongRow, dev::kPlain>(d.a, xa_in, lds, epi, w);
+        dev::csr_tile_rows_at<VT, XT, TileEpi<XT>, TN, kBatchLongRow, dev::kPlain, 0>(d.a, xa_in, lds, epi, w);
       else
-        dev::csr_long_row_at<VT, XT, TileEpi<XT>, TN, kBatchLongChunk>(d.a, xa_in, lds, epi, w - d.a_ntiles);
+        dev::csr_long_row_at<VT, XT, TileEpi<XT>, TN, kBatchLongChunk, 0>(d.a, xa_in, lds, epi, w - d.a_ntiles);
       const double bA = dev::block_tree_max<double>(epi.mA, red);
       const double bB = dev::block_tree_max<double>(epi.mB, red);
       if (threadIdx.x == 0) {

@@ -8,8 +8,8 @@
 // loads (packed columns: 12 bytes) at an aligned offset that needs no
 // descriptor load, the products
 // v * x[c] are rounded and staged in LDS, and each owned row is summed by one
-// thread from 0, left to right, finishing a row that runs past the tile from
-// global memory in the same order.  That reproduces the sequential FP64 row
+// thread from 0, left to right; of a row that runs past the tile the rest is
+// staged too (kTileTail).  That reproduces the sequential FP64 row
 // sum of MatrixCSR.cpp:133-139 exactly.  Rows longer than T / 2 entries are
 // left to csr_long_row (one workgroup per row, fixed-order tree).
 #pragma once
@@ -148,6 +148,13 @@ inline CsrView<VT> csr_view(const DeviceMatrix &d) {
 // (their contents are never added).
 constexpr int kSumRun = 16;
 
+// Entries past the tile's end that are staged after the tile's, one a thread,
+// for the tile's last row where it goes on: loaded beside the tile's own, where
+// one thread fetching them after the barrier was a chain of memory round trips
+// in every tile (50,000 rows of 100 FP64 35.9 -> 13.4 us, 200,001 of 37 27.1 ->
+// 18.0, 300,007 of 12 13.0 -> 11.8, 62 million entries 146.2 -> 144.8).
+constexpr int kTileTail = kTileThreads;
+
 // TN: entries per tile (kCsrTileNnz unless a caller builds its own tile
 // table with another size); rows longer than TN / 2 go to csr_long_row.
 // Product i of the tile is at slot(i): a free slot after every 16, so that the
@@ -156,11 +163,15 @@ constexpr int kSumRun = 16;
 // 27.0 -> 25.1 us, 1,000,003 52.2 -> 49.8 and FP32 32.4 -> 31.2.  FP32 in the
 // largest tiles, which stream from HBM, stays packed (62 million entries 100.8
 // us, 101.6 spread; FP64 146.2 and 146.0).
-template <typename AT, int TN>
+// TAIL: kTileTail, or 0 where the staging does not pay: a persistent kernel's
+// registers (batch_step: 20.3 -> 21.9 ms for the mixed-size batch with it); one
+// thread then finishes the last row.
+template <typename AT, int TN, int TAIL = kTileTail>
 struct CsrTileLds {
   static constexpr bool kSpread = sizeof(AT) == 8 || TN < kCsrTileNnz;
   __device__ static constexpr int slot(int i) { return kSpread ? i + (i >> 4) : i; }
-  AT prod[TN + kSumRun + (kSpread ? (TN + kSumRun) / 16 : 0)];
+  static constexpr int kEnd = TN + TAIL + kSumRun;
+  AT prod[kEnd + (kSpread ? kEnd / 16 : 0)];
 };
 
 // Value source: stored values (VT) or value-free (every product is z[c]).
@@ -174,10 +185,11 @@ struct Prod {
 #pragma unroll
     for (int q = 0; q < 4; q++) p[q] = v[q] * static_cast<AT>(x[c[q]]);
   }
+  __device__ static AT load1(const CsrView<VT> &m, long e) { return Val<VT>::get(m.vals, e); }
+  __device__ static AT apply1(AT v, const XT *__restrict__ x, int c) { return v * static_cast<AT>(x[c]); }
   __device__ static AT one(const CsrView<VT> &m, const XT *__restrict__ x, long e) {
-    const AT v = Val<VT>::get(m.vals, e);
-    const AT xv = static_cast<AT>(x[m.col(e)]);
-    return v * xv;
+    const AT v = load1(m, e);
+    return apply1(v, x, m.col(e));
   }
 };
 struct Pattern {};
@@ -193,6 +205,8 @@ struct Prod<Pattern, XT> {
 #pragma unroll
     for (int q = 0; q < 4; q++) p[q] = static_cast<double>(z[c[q]]);
   }
+  __device__ static double load1(const CsrView<Pattern> &, long) { return 1.0; }
+  __device__ static double apply1(double, const XT *__restrict__ z, int c) { return static_cast<double>(z[c]); }
   __device__ static double one(const CsrView<Pattern> &m, const XT *__restrict__ z, long e) {
     return static_cast<double>(z[m.col(e)]);
   }
@@ -302,21 +316,47 @@ struct NoPre {
 // The bounds of the thread's first owned row, then the index/value loads,
 // gathers and products into prod.  (Issuing the row table first measured
 // faster than deferring it behind the tile loads.)
-template <bool FULL, bool PACK, typename VT, typename XT, int TN, typename Pre>
+template <bool FULL, bool PACK, int TAIL, typename VT, typename XT, int TN, typename Pre>
 __device__ inline void csr_tile_stage(const CsrView<VT> &m, const XT *__restrict__ x, typename Val<VT>::A *prod,
-                                      long e0, int ne, int rlo, int rhi, int &a, int &b, Pre &pre) {
+                                      long e0, int ne, int rlo, int rhi, int &a, int &b, int &last, Pre &pre) {
   // loaded with no branch so they stay in flight under the tile loads
   // (indices clamped to rhi <= rows: in bounds, and exact for every thread
   // that owns a row)
   a = m.rowptr[min(rlo + static_cast<int>(threadIdx.x), rhi)] - m.rp0;
   b = m.rowptr[min(rlo + static_cast<int>(threadIdx.x) + 1, rhi)] - m.rp0;
+  using AT = typename Val<VT>::A;
   TileEntries<FULL, PACK, VT, XT, TN> t;
   t.load(m, e0, ne);
+  last = TAIL > 0 && FULL && rlo < rhi ? m.rowptr[rhi] - m.rp0 : 0;
+  const int tail = min(max(last - static_cast<int>(e0) - ne, 0), TAIL);
+  int tc = 0;
+  AT tv = 0;
+  if (static_cast<int>(threadIdx.x) < tail) {
+    tc = m.col(e0 + ne + threadIdx.x);
+    tv = Prod<VT, XT>::load1(m, e0 + ne + threadIdx.x);
+  }
   pre.issue();
-  typename Val<VT>::A p[TileEntries<FULL, PACK, VT, XT, TN>::G][4];
+  AT p[TileEntries<FULL, PACK, VT, XT, TN>::G][4];
   t.products(m, x, e0, ne, p);
+  AT tp = 0;
+  if (static_cast<int>(threadIdx.x) < tail) tp = Prod<VT, XT>::apply1(tv, x, tc);
   pre.finish();
   TileEntries<FULL, PACK, VT, XT, TN>::store(p, prod, ne);
+  if (static_cast<int>(threadIdx.x) < tail) prod[CsrTileLds<AT, TN>::slot(ne + static_cast<int>(threadIdx.x))] = tp;
+}
+
+// s + the products [e, end) of the tile, in order.
+template <typename AT, int TN, int TAIL>
+__device__ inline AT sum_staged(const CsrTileLds<AT, TN, TAIL> &lds, int e, int end, AT s) {
+#pragma clang fp contract(off)
+  for (; e < end; e += kSumRun) {
+    AT v[kSumRun];
+#pragma unroll
+    for (int u = 0; u < kSumRun; u++) v[u] = lds.prod[lds.slot(e + u)];
+#pragma unroll
+    for (int u = 0; u < kSumRun; u++) s = e + u < end ? s + v[u] : s;
+  }
+  return s;
 }
 
 // Rows of entry tile `tile`; epi(row, sum) once per owned row by the thread
@@ -325,9 +365,10 @@ __device__ inline void csr_tile_stage(const CsrView<VT> &m, const XT *__restrict
 // COLS: whether the columns are packed (kPacked, kPlain: known to the caller;
 // kEither: looked up in m).
 enum TileCols { kEither, kPlain, kPacked };
-template <typename VT, typename XT, typename Epi, int TN, int LT, TileCols COLS = kEither, typename Pre = NoPre>
+template <typename VT, typename XT, typename Epi, int TN, int LT, TileCols COLS = kEither, int TAIL = kTileTail,
+          typename Pre = NoPre>
 __device__ inline void csr_tile_rows_at(const CsrView<VT> &mat, const XT *__restrict__ x,
-                                        CsrTileLds<typename Val<VT>::A, TN> &lds, Epi &epi, int tile,
+                                        CsrTileLds<typename Val<VT>::A, TN, TAIL> &lds, Epi &epi, int tile,
                                         Pre &&pre = Pre()) {
 #pragma clang fp contract(off)
   CsrView<VT> m = mat;
@@ -337,37 +378,34 @@ __device__ inline void csr_tile_rows_at(const CsrView<VT> &mat, const XT *__rest
   const long e0 = static_cast<long>(tile) * TN;
   const int ne = static_cast<int>(min(static_cast<long>(TN), m.nnz - e0));
   const int rlo = m.tile_row[tile], rhi = m.tile_row[tile + 1];
-  int a, b;
+  int a, b, last;  // last: end of the last owned row (0 in the matrix's last tile)
   const bool packed = COLS == kPacked || (COLS == kEither && m.col24);
   if (packed && ne == TN)
-    csr_tile_stage<true, true, VT, XT, TN>(m, x, lds.prod, e0, ne, rlo, rhi, a, b, pre);
+    csr_tile_stage<true, true, TAIL, VT, XT, TN>(m, x, lds.prod, e0, ne, rlo, rhi, a, b, last, pre);
   else if (packed)
-    csr_tile_stage<false, true, VT, XT, TN>(m, x, lds.prod, e0, ne, rlo, rhi, a, b, pre);
+    csr_tile_stage<false, true, TAIL, VT, XT, TN>(m, x, lds.prod, e0, ne, rlo, rhi, a, b, last, pre);
   else if (ne == TN)
-    csr_tile_stage<true, false, VT, XT, TN>(m, x, lds.prod, e0, ne, rlo, rhi, a, b, pre);
+    csr_tile_stage<true, false, TAIL, VT, XT, TN>(m, x, lds.prod, e0, ne, rlo, rhi, a, b, last, pre);
   else
-    csr_tile_stage<false, false, VT, XT, TN>(m, x, lds.prod, e0, ne, rlo, rhi, a, b, pre);
+    csr_tile_stage<false, false, TAIL, VT, XT, TN>(m, x, lds.prod, e0, ne, rlo, rhi, a, b, last, pre);
   __syncthreads();
-  const long e1 = e0 + ne;
-  for (int r = rlo + tid; r < rhi; r += kTileThreads) {
+  const int t0 = static_cast<int>(e0);
+  const int e1 = t0 + ne + min(max(last - t0 - ne, 0), TAIL);  // end of what is staged
+  AT s = 0;
+  int r = rlo + tid;
+  for (; r < rhi; r += kTileThreads) {
     if (r != rlo + tid) {
       a = m.rowptr[r] - m.rp0;
       b = m.rowptr[r + 1] - m.rp0;
     }
     if (b - a > LT) continue;  // summed by csr_long_row
-    AT s = epi_init<AT>(epi, r, 0);
-    // a row owned by the tile starts in it: 0 <= a - e0 < TN, so the reads
-    // below stay under slot(TN + kSumRun)
-    const int lend = static_cast<int>(min(static_cast<long>(b), e1) - e0);
-    for (int e = a - static_cast<int>(e0); e < lend; e += kSumRun) {
-      AT v[kSumRun];
-#pragma unroll
-      for (int u = 0; u < kSumRun; u++) v[u] = lds.prod[lds.slot(e + u)];
-#pragma unroll
-      for (int u = 0; u < kSumRun; u++) s = e + u < lend ? s + v[u] : s;
-    }
-    // the rest of a row that runs past the tile, same order, 8 loads in flight
-    for (long e = e1; e < b; e += 8) {
+    s = epi_init<AT>(epi, r, 0);
+    // a row owned by the tile starts in it and what is staged of it ends by
+    // TN + kTileTail, so the reads below stay under slot(kEnd)
+    s = sum_staged(lds, a - t0, min(b, e1) - t0, s);
+    if (TAIL > 0 && b > e1) break;  // the last row, below
+    // (no staging) the rest of the last row, same order, 8 loads in flight
+    for (int e = e1; TAIL == 0 && e < b; e += 8) {
       AT q8[8];
 #pragma unroll
       for (int u = 0; u < 8; u++)
@@ -378,6 +416,19 @@ __device__ inline void csr_tile_rows_at(const CsrView<VT> &mat, const XT *__rest
     }
     epi(r, s);
   }
+  if (TAIL == 0 || last <= e1) return;
+  // the last row runs past what is staged: the whole block stages the rest,
+  // kTileThreads entries at a time, for the thread that sums it
+  if (last - (m.rowptr[rhi - 1] - m.rp0) > LT) return;
+  const bool mine = r == rhi - 1;
+  for (int e = e1; e < last; e += kTileThreads) {
+    const int n = min(last - e, kTileThreads);
+    __syncthreads();
+    if (tid < n) lds.prod[lds.slot(tid)] = Prod<VT, XT>::one(m, x, e + tid);
+    __syncthreads();
+    if (mine) s = sum_staged(lds, 0, n, s);
+  }
+  if (mine) epi(rhi - 1, s);
 }
 
 // Rows of entry tile blockIdx.x.
@@ -390,9 +441,9 @@ __device__ inline void csr_tile_rows(const CsrView<VT> &m, const XT *__restrict_
 // One long row (m.long_rows[idx]) per workgroup: chunk products (LC
 // entries per chunk), a fixed-order tree per chunk, chunk totals added in
 // order.  epi by thread 0.
-template <typename VT, typename XT, typename Epi, int TN, int LC>
+template <typename VT, typename XT, typename Epi, int TN, int LC, int TAIL>
 __device__ inline void csr_long_row_at(const CsrView<VT> &m, const XT *__restrict__ x,
-                                       CsrTileLds<typename Val<VT>::A, TN> &lds, Epi &epi, int idx) {
+                                       CsrTileLds<typename Val<VT>::A, TN, TAIL> &lds, Epi &epi, int idx) {
   using AT = typename Val<VT>::A;
   const int r = m.long_rows[idx];
   const long a = m.rowptr[r] - m.rp0, b = m.rowptr[r + 1] - m.rp0;
@@ -409,7 +460,7 @@ __device__ inline void csr_long_row_at(const CsrView<VT> &m, const XT *__restric
 template <typename VT, typename XT, int TN, typename Epi>
 __device__ inline void csr_long_row(const CsrView<VT> &m, const XT *__restrict__ x,
                                     CsrTileLds<typename Val<VT>::A, TN> &lds, Epi &epi) {
-  csr_long_row_at<VT, XT, Epi, TN, kCsrTileNnz>(m, x, lds, epi, blockIdx.x);
+  csr_long_row_at<VT, XT, Epi, TN, kCsrTileNnz, kTileTail>(m, x, lds, epi, blockIdx.x);
 }
 
 }  // namespace dev

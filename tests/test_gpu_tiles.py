@@ -32,3 +32,27 @@ def test_rows_over_small_tiles_exact(tb, gpu, longest):
         for k in range(ptr[r], ptr[r + 1]):
             s += float(val[k]) * float(x[col[k]])
         assert y[r] == s, r
+
+
+@pytest.mark.parametrize("fmt", ["CSR", "COO"])
+@pytest.mark.parametrize("shortest,longest,rows", [(0, 40, 9000), (100, 256, 1500), (256, 257, 900), (200, 600, 400),
+                                                   (1100, 1536, 130), (1500, 1540, 40)])
+def test_rows_past_their_tile_exact(tb, oracle, gpu, fmt, shortest, longest, rows):
+    """Rows of every offset from their tile's end: what is staged of them beside
+    the tile, and what the block stages after it.  Rows over 1536 entries are
+    tree sums, within 1e-13 of sum |a||x| (fewer than 30 roundings a product)."""
+    rng = np.random.default_rng(longest)
+    lens = rng.integers(shortest, longest + 1, rows)
+    n = max(rows, 1600)
+    row = np.repeat(np.arange(rows, dtype=np.int32), lens)
+    col = rng.integers(0, n, row.size).astype(np.int32)
+    val, x = rng.random(row.size) - 0.5, rng.random(n) - 0.5
+    # (both hold the entries in this order; a conversion would sort the columns)
+    ptr = np.concatenate([[0], np.cumsum(lens), np.full(n - rows, row.size)]).astype(np.int32)
+    m = tb.MatrixCOO(n, n, val, row, col) if fmt == "COO" else tb.MatrixCSR(n, n, val, ptr, col)
+    o = oracle.from_arrays("COO", n, n, val, row, col)
+    y, yo = m.spmv(x), o.spmv(x)
+    exact = np.concatenate([lens <= 1536, np.ones(n - rows, bool)])
+    assert np.array_equal(y[exact], yo[exact])
+    absy = oracle.from_arrays("COO", n, n, np.abs(val), row, col).spmv(np.abs(x))
+    assert np.all(np.abs(y - yo) <= 1e-13 * absy)
