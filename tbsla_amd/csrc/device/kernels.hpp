@@ -15,15 +15,13 @@ namespace hip {
 void launch_spmv(const DeviceMatrix &d, const void *x, Dtype xdt, void *y, Dtype ydt, int vect_incr,
                  hipStream_t s);
 
-// d.col24 from d.colidx, if every local column (x_need of them) fits 24 bits:
-// the tile products then read 11 instead of 12 bytes an entry in FP64, 7
-// instead of 8 in FP32.  FP64 mirrors of over 2^25 entries, which stream from
-// HBM and are bound by the tile's chain of waits, keep the 32-bit columns (62
-// million entries: CSR 146.7 us with them, 147.2 packed, SCOO 154 and 162).
-// Packed against not: CSR FP32 105.7 -> 100.3 us and BF16 90.5 -> 84.3 on
-// those 62 million, FP64 56.1 -> 53.8 and FP32 34.9 -> 32.5 on 1,000,003 rows
-// of 16, 28.0 -> 26.7 on 500,009.
-void pack_columns(DeviceMatrix &d);
+// d.col24 (pairs: d.col24_pairs) from d.colidx, if every local column (x_need
+// of them) fits 24 bits and the memory is there: the tile products then read
+// 11 instead of 12 bytes an entry in FP64, 7 instead of 8 in FP32.  Packed
+// against not: 62 million entries CSR FP64 141.5 -> 132.7 us, SCOO 148.0 ->
+// 140.0, CSR FP32 105.7 -> 100.3; 1,000,003 rows of 16 FP64 56.1 -> 53.8 and
+// FP32 34.9 -> 32.5, 500,009 FP64 28.0 -> 26.7.
+void pack_columns(DeviceMatrix &d, bool pairs);
 
 // The same for an ELL mirror, whose slots' columns are replaced (groups of
 // four; plain if the memory for both during the change is not there): 4194304

@@ -123,7 +123,7 @@ void build_csr(DeviceMatrix &d, const cpp::MatrixCSR &m, Dtype vdt) {
   d.rowptr.upload(rp.data(), rp.size() * sizeof(int));
   // entry j of row i is values[rowptr[i] - rowptr[0] + k] (MatrixCSR.cpp:135)
   d.colidx.upload(ci.data(), static_cast<std::size_t>(used) * sizeof(int));
-  pack_columns(d);
+  pack_columns(d, vdt == Dtype::F64);
   upload_values(d.vals, vals.data(), static_cast<std::size_t>(used), vdt);
   d.tile_nnz = tile_size(used, rp.data(), d.rows);
   std::vector<int> t = csr_entry_tiles(rp.data(), d.rows, d.tile_nnz);
@@ -236,7 +236,7 @@ void build_coo_like(DeviceMatrix &d, const M &m, Dtype vdt, bool scoo) {
   d.rowptr.upload(segptr.data(), segptr.size() * sizeof(int));
   d.segrow.upload(segrow.data(), segrow.size() * sizeof(int));
   d.colidx.upload(pcol, n * sizeof(int));
-  pack_columns(d);
+  pack_columns(d, vdt == Dtype::F64);
   upload_values(d.vals, pval, n, vdt);
   d.tile_nnz = tile_size(static_cast<long>(n), segptr.data(), d.nseg);
   std::vector<int> t = csr_entry_tiles(segptr.data(), d.nseg, d.tile_nnz);
@@ -340,7 +340,8 @@ const DeviceMatrix &transpose_mirror(const cpp::Matrix &m) {
   d->x_need = rows;
   d->rowptr.upload(ptr.data(), ptr.size() * sizeof(int));
   d->colidx.upload(ridx.data(), ridx.size() * sizeof(int));
-  pack_columns(*d);
+  pack_columns(*d, false);
+  pack_columns(*d, true);  // (read with the run's FP32 or FP64 values)
   d->perm.upload(perm.data(), perm.size() * sizeof(int));
   d->tile_nnz = tile_size(used, ptr.data(), cols);
   std::vector<int> t = csr_entry_tiles(ptr.data(), cols, d->tile_nnz);

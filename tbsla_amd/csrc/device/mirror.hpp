@@ -55,7 +55,9 @@ struct DeviceMatrix {
   long y_lo = 0, y_hi = 0; // COO/SCOO: rows touched are [y_lo, y_hi) before vect_incr
   // CSR
   DevBuf rowptr, colidx, vals, tiles, long_rows;
-  DevBuf col24;  // the tile products' columns (CsrView::col24), where they fit
+  // the tile products' columns (CsrView::col24) where they fit: for values of up
+  // to four bytes, and for eight
+  DevBuf col24, col24_pairs;
   int ntiles = 0, nlong = 0, rp0 = 0;
   int tile_nnz = kCsrTileNnz;  // entries per tile of the table in `tiles`
   // ELL (sliced column-major)

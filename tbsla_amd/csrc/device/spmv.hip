@@ -46,12 +46,12 @@ struct StoreRow {
   }
 };
 
-template <typename VT, typename XT, typename YT, int TN, bool PACK>
+template <typename VT, typename XT, typename YT, int TN, int LOADS>
 __global__ __launch_bounds__(kTileThreads) void csr_tile_kernel(dev::CsrView<VT> m, const XT *__restrict__ x,
                                                                 YT *__restrict__ y) {
   __shared__ dev::CsrTileLds<typename Val<VT>::A, TN> lds;
   StoreRow<YT> epi{y};
-  dev::csr_tile_rows<VT, XT, TN, PACK ? dev::kPacked : dev::kPlain>(m, x, lds, epi);
+  dev::csr_tile_rows<VT, XT, TN, static_cast<dev::TileLoads>(LOADS)>(m, x, lds, epi);
 }
 
 template <typename VT, typename XT, typename YT>
@@ -184,7 +184,7 @@ struct AccRow {
   }
 };
 
-template <typename VT, typename XT, typename YT, int TN, bool PACK, bool LONG>
+template <typename VT, typename XT, typename YT, int TN, int LOADS, bool LONG>
 __global__ __launch_bounds__(kTileThreads) void coo_tile_kernel(dev::CsrView<VT> m, const XT *__restrict__ x,
                                                                 YT *__restrict__ y, const int *__restrict__ segrow,
                                                                 long y_off) {
@@ -193,7 +193,7 @@ __global__ __launch_bounds__(kTileThreads) void coo_tile_kernel(dev::CsrView<VT>
   if constexpr (LONG)
     dev::csr_long_row<VT, XT, TN>(m, x, lds, epi);
   else
-    dev::csr_tile_rows<VT, XT, TN, PACK ? dev::kPacked : dev::kPlain>(m, x, lds, epi);
+    dev::csr_tile_rows<VT, XT, TN, static_cast<dev::TileLoads>(LOADS)>(m, x, lds, epi);
 }
 
 // R consecutive rows per wavefront, so each x load serves all of them; per row
@@ -257,13 +257,16 @@ __global__ void fill_kernel(T *y, long n, T v) {
   for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += static_cast<long>(gridDim.x) * 256) y[i] = v;
 }
 
-// three words of packed columns for entries 4g .. 4g + 3 (0 past the end)
-__global__ __launch_bounds__(256) void pack24_kernel(const int *__restrict__ colidx, long nnz, int f_col,
+// three words of packed columns for the four entries of group g (0 past the end)
+__global__ __launch_bounds__(256) void pack24_kernel(const int *__restrict__ colidx, long nnz, int f_col, bool pairs,
                                                      unsigned *__restrict__ out) {
-  const long groups = (nnz + 3) / 4;
+  const long groups = (nnz + 255) / 256 * 64;
   for (long g = blockIdx.x * 256L + threadIdx.x; g < groups; g += static_cast<long>(gridDim.x) * 256) {
     unsigned c[4];
-    for (int q = 0; q < 4; q++) c[q] = 4 * g + q < nnz ? static_cast<unsigned>(colidx[4 * g + q] - f_col) : 0u;
+    for (int q = 0; q < 4; q++) {
+      const long e = pairs ? (g & ~63L) * 4 + 2 * (g & 63) + (q >> 1) * 128 + (q & 1) : 4 * g + q;
+      c[q] = e < nnz ? static_cast<unsigned>(colidx[e] - f_col) : 0u;
+    }
     out[3 * g] = c[0] | c[1] << 24;
     out[3 * g + 1] = c[1] >> 8 | c[2] << 16;
     out[3 * g + 2] = c[2] >> 16 | c[3] << 8;
@@ -304,6 +307,18 @@ void launch_dense(const DeviceMatrix &d, const XT *x, YT *y, hipStream_t s) {
                      d.dcols, static_cast<long>(d.dcols));
 }
 
+template <typename VT, typename F>
+void with_loads(const dev::CsrView<VT> &m, F f) {
+  if (m.col24 && m.stream)
+    f(std::integral_constant<int, dev::kPackedStream>());
+  else if (m.col24)
+    f(std::integral_constant<int, dev::kPacked>());
+  else if (m.stream)
+    f(std::integral_constant<int, dev::kStream>());
+  else
+    f(std::integral_constant<int, dev::kPlain>());
+}
+
 template <typename VT, typename XT, typename YT>
 void run_typed(const DeviceMatrix &d, const XT *x, YT *y, int vect_incr, hipStream_t s) {
   switch (d.format) {
@@ -312,8 +327,10 @@ void run_typed(const DeviceMatrix &d, const XT *x, YT *y, int vect_incr, hipStre
       if (d.ntiles > 0)
         with_tile_size(d, [&](auto tn) {
           constexpr int TN = decltype(tn)::value;
-          const auto kernel = m.col24 ? csr_tile_kernel<VT, XT, YT, TN, true> : csr_tile_kernel<VT, XT, YT, TN, false>;
-          hipLaunchKernelGGL(kernel, dim3(d.ntiles), dim3(kTileThreads), 0, s, m, x, y);
+          with_loads(m, [&](auto loads) {
+            hipLaunchKernelGGL((csr_tile_kernel<VT, XT, YT, TN, decltype(loads)::value>), dim3(d.ntiles),
+                               dim3(kTileThreads), 0, s, m, x, y);
+          });
         });
       if (d.nlong > 0)
         hipLaunchKernelGGL((csr_long_kernel<VT, XT, YT>), dim3(d.nlong), dim3(kTileThreads), 0, s, m, x, y);
@@ -334,12 +351,13 @@ void run_typed(const DeviceMatrix &d, const XT *x, YT *y, int vect_incr, hipStre
       if (d.ntiles > 0)
         with_tile_size(d, [&](auto tn) {
           constexpr int TN = decltype(tn)::value;
-          const auto kernel = m.col24 ? coo_tile_kernel<VT, XT, YT, TN, true, false>
-                                      : coo_tile_kernel<VT, XT, YT, TN, false, false>;
-          hipLaunchKernelGGL(kernel, dim3(d.ntiles), dim3(kTileThreads), 0, s, m, x, y, d.segrow.as<int>(), y_off);
+          with_loads(m, [&](auto loads) {
+            hipLaunchKernelGGL((coo_tile_kernel<VT, XT, YT, TN, decltype(loads)::value, false>), dim3(d.ntiles),
+                               dim3(kTileThreads), 0, s, m, x, y, d.segrow.as<int>(), y_off);
+          });
         });
       if (d.nlong > 0)
-        hipLaunchKernelGGL((coo_tile_kernel<VT, XT, YT, kTileThreads, false, true>), dim3(d.nlong), dim3(kTileThreads), 0, s, m, x, y,
+        hipLaunchKernelGGL((coo_tile_kernel<VT, XT, YT, kTileThreads, dev::kPlain, true>), dim3(d.nlong), dim3(kTileThreads), 0, s, m, x, y,
                            d.segrow.as<int>(), y_off);
       break;
     }
@@ -366,12 +384,13 @@ void launch_spmv(const DeviceMatrix &d, const void *x, Dtype xdt, void *y, Dtype
   }
 }
 
-void pack_columns(DeviceMatrix &d) {
-  if (d.entries <= 0 || d.x_need > (1L << 24) || (d.vdt == Dtype::F64 && d.entries > (1L << 25))) return;
-  const long groups = (d.entries + 3) / 4;
-  if (!d.col24.try_reserve(static_cast<std::size_t>(groups) * 12)) return;
+void pack_columns(DeviceMatrix &d, bool pairs) {
+  if (d.entries <= 0 || d.x_need > (1L << 24)) return;
+  DevBuf &out = pairs ? d.col24_pairs : d.col24;
+  const long groups = (d.entries + 255) / 256 * 64;
+  if (!out.try_reserve(static_cast<std::size_t>(groups) * 12)) return;
   hipLaunchKernelGGL(pack24_kernel, dim3(static_cast<unsigned>(std::min<long>((groups + 255) / 256, 65536))), dim3(256),
-                     0, nullptr, d.colidx.as<int>(), d.entries, d.f_col, d.col24.as<unsigned>());
+                     0, nullptr, d.colidx.as<int>(), d.entries, d.f_col, pairs, out.as<unsigned>());
   TBSLA_HIP_CHECK(hipGetLastError());
 }
 

@@ -16,6 +16,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "mirror.hpp"
 
 namespace tbsla {
@@ -40,16 +42,27 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef unsigned short v4us __attribute__((ext_vector_type(4)));
 
+// A load, non-temporal or plain.
+template <bool NT, typename V>
+__device__ inline V vec_load(const V *p) {
+  if constexpr (NT) return __builtin_nontemporal_load(p);
+  return *p;
+}
+
 template <typename T>
 struct Val;
 template <>
 struct Val<double> {
   using A = double;
+  static constexpr int kXBytes = 8;
   __device__ static double get(const double *p, long i) { return p[i]; }
   // four consecutive values starting at a multiple of 4
-  __device__ static void get4(const double *p, long i, double (&v)[4]) {
-    const v2d a = *reinterpret_cast<const v2d *>(p + i);
-    const v2d b = *reinterpret_cast<const v2d *>(p + i + 2);
+  __device__ static void get4(const double *p, long i, double (&v)[4]) { get22<false>(p, i, i + 2, v); }
+  // two from i, two from j
+  template <bool NT>
+  __device__ static void get22(const double *p, long i, long j, double (&v)[4]) {
+    const v2d a = vec_load<NT>(reinterpret_cast<const v2d *>(p + i));
+    const v2d b = vec_load<NT>(reinterpret_cast<const v2d *>(p + j));
     v[0] = a.x;
     v[1] = a.y;
     v[2] = b.x;
@@ -59,9 +72,11 @@ struct Val<double> {
 template <>
 struct Val<float> {
   using A = float;
+  static constexpr int kXBytes = 4;
   __device__ static float get(const float *p, long i) { return p[i]; }
+  template <bool NT = false>
   __device__ static void get4(const float *p, long i, float (&v)[4]) {
-    const v4f a = *reinterpret_cast<const v4f *>(p + i);
+    const v4f a = vec_load<NT>(reinterpret_cast<const v4f *>(p + i));
     v[0] = a.x;
     v[1] = a.y;
     v[2] = a.z;
@@ -71,10 +86,12 @@ struct Val<float> {
 template <>
 struct Val<bf16> {
   using A = float;
+  static constexpr int kXBytes = 4;
   __device__ static float cvt(unsigned short b) { return __uint_as_float(static_cast<unsigned>(b) << 16); }
   __device__ static float get(const bf16 *p, long i) { return cvt(reinterpret_cast<const unsigned short *>(p)[i]); }
+  template <bool NT = false>
   __device__ static void get4(const bf16 *p, long i, float (&v)[4]) {
-    const v4us a = *reinterpret_cast<const v4us *>(reinterpret_cast<const unsigned short *>(p) + i);
+    const v4us a = vec_load<NT>(reinterpret_cast<const v4us *>(reinterpret_cast<const unsigned short *>(p) + i));
     v[0] = cvt(a.x);
     v[1] = cvt(a.y);
     v[2] = cvt(a.z);
@@ -111,6 +128,21 @@ __device__ inline AT block_tree_max(AT v, AT *part) {
   return r;
 }
 
+// The four entries of a tile's group in a thread: eight-byte values go two and
+// two (lane l of the wavefront's 256 entries has 2l, 2l + 1, 128 + 2l, 129 +
+// 2l), so that each 16-byte load of a wavefront is one run of 1 KB (with 32
+// bytes a lane, read in halves, non-temporal loads fetched lines twice: 62
+// million entries 161.8 us, 142.5 so); smaller values four in a row.
+template <typename VT>
+__host__ __device__ constexpr bool tile_pairs() {
+  return sizeof(typename Val<VT>::A) == 8;
+}
+// Place of entry e in the order of the groups' threads.
+template <typename VT>
+__device__ inline long tile_place(long e) {
+  return tile_pairs<VT>() ? (e & ~255L) + 4 * ((e & 127) >> 1) + ((e & 128) >> 6) + (e & 1) : e;
+}
+
 // Device view of a CSR mirror (entry j of the matrix is colidx[j], vals[j],
 // with j = rowptr[i] - rp0 + k for the k-th entry of row i).  colidx is the
 // mirror's padded buffer; vals may be a caller's array of exactly nnz
@@ -125,22 +157,34 @@ struct CsrView {
   long nnz;
   int rp0, f_col;
   // the columns minus f_col packed in three bytes each (little endian, four
-  // in three words), or nullptr
+  // in three words; column of entry e at 3 * tile_place<VT>(e)), or nullptr
   const unsigned *col24 = nullptr;
+  bool stream = false;  // the entries are read non-temporally (stream_entries)
 
-  __device__ int col(long e) const {  // local column of entry e
+  // the local column of entry e, in a load and what is done with its word
+  __device__ unsigned col_word(long e) const {
     typedef unsigned u32_u __attribute__((aligned(1)));
     if (col24)
-      return static_cast<int>(*reinterpret_cast<const u32_u *>(reinterpret_cast<const char *>(col24) + 3 * e) &
-                              0xFFFFFFu);
-    return colidx[e] - f_col;
+      return *reinterpret_cast<const u32_u *>(reinterpret_cast<const char *>(col24) + 3 * tile_place<VT>(e));
+    return static_cast<unsigned>(colidx[e]);
   }
+  __device__ int col_of(unsigned w) const { return col24 ? static_cast<int>(w & 0xFFFFFFu) : static_cast<int>(w) - f_col; }
+  __device__ int col(long e) const { return col_of(col_word(e)); }
 };
+
+// Entries are read non-temporally where x does not stay in an L2 (4 MB) beside
+// them otherwise: 1,000,003 rows of 16 FP64 46.3 -> 42.6 us, 3,000,003 FP32 110
+// -> 98, 600,007 of 8 FP64 (4.8 MB of x) 16.5 -> 15.4; a smaller x stays, and
+// then the caches' share of the entries counts: 800,003 of 16 FP32 (3.2 MB)
+// 23.9 plain and 27.6 so, 300,007 of 31 FP64 (2.4 MB) 22.1 and 23.7.
+inline bool stream_entries(long x_bytes) { return x_bytes > (7L << 19); }
 
 template <typename VT>
 inline CsrView<VT> csr_view(const DeviceMatrix &d) {
+  const unsigned *col24 = (tile_pairs<VT>() ? d.col24_pairs : d.col24).template as<unsigned>();
   return CsrView<VT>{d.rowptr.as<int>(), d.colidx.as<int>(), d.vals.as<VT>(), d.tiles.as<int>(),
-                     d.long_rows.as<int>(), d.entries, d.rp0, d.f_col, d.col24.as<unsigned>()};
+                     d.long_rows.as<int>(), d.entries, d.rp0, d.f_col, col24,
+                     stream_entries(d.x_need * Val<VT>::kXBytes)};
 }
 
 // A row's sum reads its products from LDS kSumRun at a time, all reads issued
@@ -175,12 +219,18 @@ struct CsrTileLds {
 };
 
 // Value source: stored values (VT) or value-free (every product is z[c]).
-// load4 reads four consecutive values (issued before the gathers that need
+// load4 reads the four values of a group (issued before the gathers that need
 // the column indices), apply4 gathers x and forms the rounded products.
 template <typename VT, typename XT>
 struct Prod {
   using AT = typename Val<VT>::A;
-  __device__ static void load4(const CsrView<VT> &m, long e, AT (&v)[4]) { Val<VT>::get4(m.vals, e, v); }
+  template <bool NT>
+  __device__ static void load4(const CsrView<VT> &m, long e, AT (&v)[4]) {
+    if constexpr (tile_pairs<VT>())
+      Val<VT>::template get22<NT>(m.vals, e, e + 128, v);
+    else
+      Val<VT>::template get4<NT>(m.vals, e, v);
+  }
   __device__ static void apply4(const AT (&v)[4], const XT *__restrict__ x, const int (&c)[4], AT (&p)[4]) {
 #pragma unroll
     for (int q = 0; q < 4; q++) p[q] = v[q] * static_cast<AT>(x[c[q]]);
@@ -196,10 +246,12 @@ struct Pattern {};
 template <>
 struct Val<Pattern> {
   using A = double;
+  static constexpr int kXBytes = 8;
 };
 template <typename XT>
 struct Prod<Pattern, XT> {
   using AT = double;
+  template <bool NT>
   __device__ static void load4(const CsrView<Pattern> &, long, double (&)[4]) {}
   __device__ static void apply4(const double (&)[4], const XT *__restrict__ z, const int (&c)[4], double (&p)[4]) {
 #pragma unroll
@@ -223,36 +275,56 @@ __device__ inline AT epi_init(const E &, int, long) {
   return AT(0);
 }
 
-// The entries [e0, e0 + ne) of one tile held by the calling thread: groups
-// of four at 4 * (k * kTileThreads + threadIdx.x).  load() issues the index and
-// value loads; products() gathers x and writes the rounded products to
-// slots 0 .. ne of prod.  FULL (ne == TN, every tile but the matrix's last)
-// reads with no per-entry guard; otherwise entries at or past ne are not read
-// (a caller's value array holds exactly nnz values).
-template <bool FULL, bool PACK, typename VT, typename XT, int TN>
+// The entries [e0, e0 + ne) of one tile held by the calling thread, in groups
+// of four (at(k, q): place of group k's entry q in the tile).  load() issues
+// the index and value loads; products() gathers x and forms the rounded
+// products, store() writes them to the slots of prod.  FULL (ne == TN, every
+// tile but the matrix's last) reads with no per-entry guard; otherwise entries
+// at or past ne are not read (a caller's value array holds exactly nnz values).
+template <bool FULL, bool PACK, bool NT, typename VT, typename XT, int TN>
 struct TileEntries {
   using AT = typename Val<VT>::A;
   static constexpr int G = TN / 4 / kTileThreads;  // 4-entry groups per thread
+  static constexpr bool PAIRS = tile_pairs<VT>();
   v4i raw[G];  // the groups' columns as loaded: four ints, or three words of packed ones
   AT v[G][4];
 
+  __device__ static int at(int k, int q) {
+    const int t = static_cast<int>(threadIdx.x);
+    return PAIRS ? 4 * (k * kTileThreads + (t & ~63)) + 2 * (t & 63) + (q >> 1) * 128 + (q & 1)
+                 : 4 * (k * kTileThreads + t) + q;
+  }
+
   __device__ void load(const CsrView<VT> &m, long e0, int ne) {
     typedef unsigned v3u __attribute__((ext_vector_type(3), aligned(4)));
+    typedef int v2i __attribute__((ext_vector_type(2)));
 #pragma unroll
     for (int k = 0; k < G; k++) {
-      const int g = k * kTileThreads + threadIdx.x;
-      if (FULL || 4 * g < ne) {
+      if (FULL || at(k, 0) < ne) {
         if constexpr (PACK) {
-          const v3u w = *reinterpret_cast<const v3u *>(m.col24 + (e0 / 4 + g) * 3);
+          const int g = k * kTileThreads + threadIdx.x;
+          const v3u w = vec_load<NT>(reinterpret_cast<const v3u *>(m.col24 + (e0 / 4 + g) * 3));
           raw[k].x = static_cast<int>(w.x);
           raw[k].y = static_cast<int>(w.y);
           raw[k].z = static_cast<int>(w.z);
+        } else if constexpr (PAIRS) {
+          const v2i c01 = vec_load<NT>(reinterpret_cast<const v2i *>(m.colidx + e0 + at(k, 0)));
+          raw[k].x = c01.x;
+          raw[k].y = c01.y;
+          if (FULL || at(k, 2) < ne) {
+            const v2i c23 = vec_load<NT>(reinterpret_cast<const v2i *>(m.colidx + e0 + at(k, 2)));
+            raw[k].z = c23.x;
+            raw[k].w = c23.y;
+          }
         } else {
-          raw[k] = *reinterpret_cast<const v4i *>(m.colidx + e0 + 4 * g);
+          raw[k] = vec_load<NT>(reinterpret_cast<const v4i *>(m.colidx + e0 + at(k, 0)));
         }
       }
-      if (FULL || 4 * g + 4 <= ne) Prod<VT, XT>::load4(m, e0 + 4 * g, v[k]);
     }
+    // (after every group's columns: the gathers wait for those alone)
+#pragma unroll
+    for (int k = 0; k < G; k++)
+      if (FULL || at(k, 3) < ne) Prod<VT, XT>::template load4<NT>(m, e0 + at(k, 0), v[k]);
   }
 
   __device__ void columns(const CsrView<VT> &m, int ne, int (&c)[G][4]) const {
@@ -273,7 +345,7 @@ struct TileEntries {
       }
       if (!FULL)  // entries past the matrix end: column 0
         for (int q = 0; q < 4; q++)
-          if (4 * (k * kTileThreads + static_cast<int>(threadIdx.x)) + q >= ne) c[k][q] = 0;
+          if (at(k, q) >= ne) c[k][q] = 0;
     }
   }
 
@@ -284,23 +356,23 @@ struct TileEntries {
     columns(m, ne, c);
 #pragma unroll
     for (int k = 0; k < G; k++) {
-      const int g = k * kTileThreads + threadIdx.x;
-      if (FULL || 4 * g + 4 <= ne)
+      if (FULL || at(k, 3) < ne)
         Prod<VT, XT>::apply4(v[k], x, c[k], p[k]);
-      else if (4 * g < ne)  // the matrix's last entries: no value read past nnz
+      else  // the matrix's last entries: no value read past nnz
 #pragma unroll
-        for (int q = 0; q < 4; q++)
-          if (4 * g + q < ne) p[k][q] = Prod<VT, XT>::one(m, x, e0 + 4 * g + q);
+        for (int q = 0; q < 4; q++) p[k][q] = at(k, q) < ne ? Prod<VT, XT>::one(m, x, e0 + at(k, q)) : AT(0);
     }
   }
 
   static __device__ void store(const AT (&p)[G][4], AT *prod, int ne) {
 #pragma unroll
     for (int k = 0; k < G; k++) {
-      const int g = k * kTileThreads + threadIdx.x;
 #pragma unroll
-      for (int q = 0; q < 4; q++)
-        if (FULL || 4 * g + q < ne) prod[CsrTileLds<AT, TN>::slot(4 * g) + q] = p[k][q];
+      for (int q = 0; q < 4; q += 2) {  // (entries q and q + 1 are neighbours, in one run of 16)
+        AT *o = prod + CsrTileLds<AT, TN>::slot(at(k, q));
+        if (FULL || at(k, q) < ne) o[0] = p[k][q];
+        if (FULL || at(k, q + 1) < ne) o[1] = p[k][q + 1];
+      }
     }
   }
 };
@@ -316,7 +388,7 @@ struct NoPre {
 // The bounds of the thread's first owned row, then the index/value loads,
 // gathers and products into prod.  (Issuing the row table first measured
 // faster than deferring it behind the tile loads.)
-template <bool FULL, bool PACK, int TAIL, typename VT, typename XT, int TN, typename Pre>
+template <bool FULL, bool PACK, bool NT, int TAIL, typename VT, typename XT, int TN, typename Pre>
 __device__ inline void csr_tile_stage(const CsrView<VT> &m, const XT *__restrict__ x, typename Val<VT>::A *prod,
                                       long e0, int ne, int rlo, int rhi, int &a, int &b, int &last, Pre &pre) {
   // loaded with no branch so they stay in flight under the tile loads
@@ -325,23 +397,23 @@ __device__ inline void csr_tile_stage(const CsrView<VT> &m, const XT *__restrict
   a = m.rowptr[min(rlo + static_cast<int>(threadIdx.x), rhi)] - m.rp0;
   b = m.rowptr[min(rlo + static_cast<int>(threadIdx.x) + 1, rhi)] - m.rp0;
   using AT = typename Val<VT>::A;
-  TileEntries<FULL, PACK, VT, XT, TN> t;
+  TileEntries<FULL, PACK, NT, VT, XT, TN> t;
   t.load(m, e0, ne);
   last = TAIL > 0 && FULL && rlo < rhi ? m.rowptr[rhi] - m.rp0 : 0;
   const int tail = min(max(last - static_cast<int>(e0) - ne, 0), TAIL);
-  int tc = 0;
+  unsigned tc = 0;
   AT tv = 0;
   if (static_cast<int>(threadIdx.x) < tail) {
-    tc = m.col(e0 + ne + threadIdx.x);
+    tc = m.col_word(e0 + ne + threadIdx.x);
     tv = Prod<VT, XT>::load1(m, e0 + ne + threadIdx.x);
   }
   pre.issue();
-  AT p[TileEntries<FULL, PACK, VT, XT, TN>::G][4];
+  AT p[TileEntries<FULL, PACK, NT, VT, XT, TN>::G][4];
   t.products(m, x, e0, ne, p);
   AT tp = 0;
-  if (static_cast<int>(threadIdx.x) < tail) tp = Prod<VT, XT>::apply1(tv, x, tc);
+  if (static_cast<int>(threadIdx.x) < tail) tp = Prod<VT, XT>::apply1(tv, x, m.col_of(tc));
   pre.finish();
-  TileEntries<FULL, PACK, VT, XT, TN>::store(p, prod, ne);
+  TileEntries<FULL, PACK, NT, VT, XT, TN>::store(p, prod, ne);
   if (static_cast<int>(threadIdx.x) < tail) prod[CsrTileLds<AT, TN>::slot(ne + static_cast<int>(threadIdx.x))] = tp;
 }
 
@@ -362,32 +434,46 @@ __device__ inline AT sum_staged(const CsrTileLds<AT, TN, TAIL> &lds, int e, int 
 // Rows of entry tile `tile`; epi(row, sum) once per owned row by the thread
 // that sums it, rows longer than LT left to csr_long_row.  The caller
 // synchronises the block before reusing `lds`.
-// COLS: whether the columns are packed (kPacked, kPlain: known to the caller;
-// kEither: looked up in m).
-enum TileCols { kEither, kPlain, kPacked };
-template <typename VT, typename XT, typename Epi, int TN, int LT, TileCols COLS = kEither, int TAIL = kTileTail,
+// LOADS: what is known of m where the kernel is compiled: nothing (kEither), or
+// whether the columns are packed and the entries stream.
+enum TileLoads { kEither = -1, kPlain = 0, kPacked = 1, kStream = 2, kPackedStream = 3 };
+template <typename VT, typename XT, typename Epi, int TN, int LT, TileLoads LOADS = kEither, int TAIL = kTileTail,
           typename Pre = NoPre>
 __device__ inline void csr_tile_rows_at(const CsrView<VT> &mat, const XT *__restrict__ x,
                                         CsrTileLds<typename Val<VT>::A, TN, TAIL> &lds, Epi &epi, int tile,
                                         Pre &&pre = Pre()) {
 #pragma clang fp contract(off)
   CsrView<VT> m = mat;
-  if (COLS == kPlain) m.col24 = nullptr;
+  if (LOADS == kPlain || LOADS == kStream) m.col24 = nullptr;
   using AT = typename Val<VT>::A;
   const int tid = threadIdx.x;
   const long e0 = static_cast<long>(tile) * TN;
   const int ne = static_cast<int>(min(static_cast<long>(TN), m.nnz - e0));
   const int rlo = m.tile_row[tile], rhi = m.tile_row[tile + 1];
   int a, b, last;  // last: end of the last owned row (0 in the matrix's last tile)
-  const bool packed = COLS == kPacked || (COLS == kEither && m.col24);
-  if (packed && ne == TN)
-    csr_tile_stage<true, true, TAIL, VT, XT, TN>(m, x, lds.prod, e0, ne, rlo, rhi, a, b, last, pre);
-  else if (packed)
-    csr_tile_stage<false, true, TAIL, VT, XT, TN>(m, x, lds.prod, e0, ne, rlo, rhi, a, b, last, pre);
-  else if (ne == TN)
-    csr_tile_stage<true, false, TAIL, VT, XT, TN>(m, x, lds.prod, e0, ne, rlo, rhi, a, b, last, pre);
-  else
-    csr_tile_stage<false, false, TAIL, VT, XT, TN>(m, x, lds.prod, e0, ne, rlo, rhi, a, b, last, pre);
+  const bool packed = LOADS == kEither ? m.col24 != nullptr : LOADS & 1;
+  const bool stream = LOADS == kEither ? m.stream : LOADS & 2;
+  const auto stage = [&](auto full, auto pack, auto nt) {
+    csr_tile_stage<decltype(full)::value, decltype(pack)::value, decltype(nt)::value, TAIL, VT, XT, TN>(
+        m, x, lds.prod, e0, ne, rlo, rhi, a, b, last, pre);
+  };
+  constexpr std::true_type yes{};
+  constexpr std::false_type no{};
+  if (ne == TN) {
+    if (packed && stream)
+      stage(yes, yes, yes);
+    else if (packed)
+      stage(yes, yes, no);
+    else if (stream)
+      stage(yes, no, yes);
+    else
+      stage(yes, no, no);
+  } else {  // the matrix's last tile
+    if (packed)
+      stage(no, yes, no);
+    else
+      stage(no, no, no);
+  }
   __syncthreads();
   const int t0 = static_cast<int>(e0);
   const int e1 = t0 + ne + min(max(last - t0 - ne, 0), TAIL);  // end of what is staged
@@ -432,10 +518,10 @@ __device__ inline void csr_tile_rows_at(const CsrView<VT> &mat, const XT *__rest
 }
 
 // Rows of entry tile blockIdx.x.
-template <typename VT, typename XT, int TN, TileCols COLS = kEither, typename Epi, typename Pre = NoPre>
+template <typename VT, typename XT, int TN, TileLoads LOADS = kEither, typename Epi, typename Pre = NoPre>
 __device__ inline void csr_tile_rows(const CsrView<VT> &m, const XT *__restrict__ x,
                                      CsrTileLds<typename Val<VT>::A, TN> &lds, Epi &epi, Pre &&pre = Pre()) {
-  csr_tile_rows_at<VT, XT, Epi, TN, kCsrLongRow, COLS>(m, x, lds, epi, blockIdx.x, pre);
+  csr_tile_rows_at<VT, XT, Epi, TN, kCsrLongRow, LOADS>(m, x, lds, epi, blockIdx.x, pre);
 }
 
 // One long row (m.long_rows[idx]) per workgroup: chunk products (LC

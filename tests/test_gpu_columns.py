@@ -29,6 +29,23 @@ def test_columns_at_the_packed_limit(tb, gpu, fmt, last):
     assert np.array_equal(m.spmv(x), row_sums(n, row, col.ravel(), val, x))
 
 
+@pytest.mark.parametrize("fmt", ["CSR", "SCOO"])
+@pytest.mark.parametrize("rows", [146, 147, 1000])
+@pytest.mark.parametrize("n_col", [450_000, 600_001, (1 << 24) + 9])
+def test_whole_tiles_against_a_large_x(tb, gpu, fmt, rows, n_col):
+    """1022, 1029 and 7000 entries: no, one and several whole tiles, with an x
+    that stays in an L2 and with ones that do not."""
+    k = 7
+    rng = np.random.default_rng(rows)
+    col = np.sort(rng.integers(0, n_col, (rows, k)), axis=1).astype(np.int32)
+    col[rows // 2, k - 1] = n_col - 1
+    row = np.repeat(np.arange(rows, dtype=np.int32), k)
+    val = rng.random(rows * k)
+    x = rng.random(n_col)
+    m = tb.FORMATS[fmt](tb.MatrixCOO(rows, n_col, val, row, col.ravel()))
+    assert np.array_equal(m.spmv(x), row_sums(rows, row, col.ravel(), val, x))
+
+
 @pytest.mark.parametrize("fmt", ["CSR", "SCOO", "ELL"])
 @pytest.mark.parametrize("k", list(range(1, 10)) + [16, 19])
 @pytest.mark.parametrize("n", [19, 64, 255, 257, 1000])
