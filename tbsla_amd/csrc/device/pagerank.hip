@@ -1210,7 +1210,20 @@ struct PbView {
   const int *bp, *lp;
   const unsigned short *frow, *lkey, *lbase;
   int n, rows;  // rows per bin
+  long n_far;
 };
+
+// Far products are read non-temporally where they are past the L2s but partly
+// in the 256 MB memory-side cache, whose lines the next scatter writes again
+// (per iteration, graphs of 8 entries a row, half of them random: 3,000,003
+// nodes FP64 82 -> 75 us, 5,000,011 150 -> 142.6 and FP32 112.3 -> 108.5,
+// 8,000,009 241 -> 226).  Fewer are read sooner plain (2,000,003 nodes 51.3
+// against 52.5; 3,000,003 in FP32, half the bytes, 58.1 and 59.3), more come
+// from HBM either way (2^24 nodes 528 and 529).
+template <typename AT>
+__device__ inline bool pb_stream(long n_far) {
+  return n_far > (sizeof(AT) == 8 ? 10L << 20 : 16L << 20) && n_far <= 48L << 20;
+}
 
 // Two products of type T in one vector load.
 template <typename T>
@@ -1254,7 +1267,8 @@ __device__ inline void pb_accumulate(const PbView &v, const VT *__restrict__ lva
     if (tid == 1023) atomicAdd(&ybin[v.frow[fe - 1]], static_cast<double>(prod[fe - 1]));
     fe--;
   }
-  {
+  const auto far = [&](auto nt) {
+    constexpr bool NT = decltype(nt)::value;
     using AT2 = typename PbPair<AT>::type;
     const unsigned *__restrict__ frow2 = reinterpret_cast<const unsigned *>(v.frow);
     const AT2 *__restrict__ prod2 = reinterpret_cast<const AT2 *>(prod);
@@ -1269,7 +1283,7 @@ __device__ inline void pb_accumulate(const PbView &v, const VT *__restrict__ lva
       unsigned rA[U];
       AT2 pA[U];
 #pragma unroll
-      for (int u = 0; u < U; u++) rA[u] = frow2[kp + u * 1024], pA[u] = prod2[kp + u * 1024];
+      for (int u = 0; u < U; u++) rA[u] = dev::vec_load<NT>(frow2 + kp + u * 1024), pA[u] = dev::vec_load<NT>(prod2 + kp + u * 1024);
       for (;;) {
         const int kn = kp + U * 1024;
         const bool more = kn + (U - 1) * 1024 < p1;
@@ -1277,7 +1291,8 @@ __device__ inline void pb_accumulate(const PbView &v, const VT *__restrict__ lva
         AT2 pB[U];
         if (more)
 #pragma unroll
-          for (int u = 0; u < U; u++) rB[u] = frow2[kn + u * 1024], pB[u] = prod2[kn + u * 1024];
+          for (int u = 0; u < U; u++)
+            rB[u] = dev::vec_load<NT>(frow2 + kn + u * 1024), pB[u] = dev::vec_load<NT>(prod2 + kn + u * 1024);
 #pragma unroll
         for (int u = 0; u < U; u++) add(rA[u], pA[u]);
         kp = kn;
@@ -1299,7 +1314,11 @@ __device__ inline void pb_accumulate(const PbView &v, const VT *__restrict__ lva
       for (int u = 0; u < U; u++)
         if (kp + u * 1024 < p1) add(r[u], pv[u]);
     }
-  }
+  };
+  if (pb_stream<AT>(v.n_far))
+    far(std::true_type{});
+  else
+    far(std::false_type{});
   // local entries: one group of four per thread (a 2-byte base row, one
   // 8-byte key load, aligned value loads), rows decoded from the keys; runs
   // of one row summed and added once
@@ -1506,7 +1525,7 @@ __global__ __launch_bounds__(1024) void pb_gather_mx(PbView v, const VA *__restr
 
 PbView pb_view(const PbMatrix &pb) {
   return PbView{pb.bp.as<int>(), pb.lp.as<int>(), pb.frow.as<unsigned short>(), pb.lkey.as<unsigned short>(),
-                pb.lbase.as<unsigned short>(), pb.n, pb.rows};
+                pb.lbase.as<unsigned short>(), pb.n, pb.rows, pb.n_far};
 }
 
 PbScatterArgs pb_args(const PbMatrix &pb) {
