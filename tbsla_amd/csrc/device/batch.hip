@@ -357,9 +357,11 @@ __device__ void spmm_item(const BatchDev<VT, XT> &d, const SpmmGroup<VT> &G, int
 // Persistent step: every workgroup walks its queue with a static stride
 // (queue = XCD of the workgroup when xcd_map is set, else one shared list).
 // (sixteen gathers in flight fit two waves per SIMD in FP32 only with the
-// register budget held to 256)
+// register budget held to 256; four fit four waves in FP32 and three in FP64,
+// held to 128 and 168: without that the 3072-entry tiles took 153 registers and
+// the 320-set batch 157.0 ms, 151.0 with)
 template <typename VT, typename XT, int UNR, int TN>
-__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(UNR == 16 ? 2 : 1)))
+__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(UNR == 16 ? 2 : UNR == 4 ? (sizeof(VT) == 4 ? 4 : 3) : 1)))
 void batch_step(BatchDev<VT, XT> d, int par) {
   using AT = typename dev::Val<VT>::A;
   __shared__ dev::CsrTileLds<AT, TN, 0> lds;
