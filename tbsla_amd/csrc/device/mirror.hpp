@@ -90,7 +90,8 @@ struct DeviceMatrix {
 //          value and the slot of its product (sp: superblock boundaries), and
 //          in bin-grouped order -- by (row bin, column) -- with the row offset
 //          in the bin (bp: bin boundaries).  Within a bin the products of one
-//          superblock are contiguous, so the scatter pass writes runs.
+//          superblock are contiguous, so the scatter pass writes runs.  (The
+//          products are a run's own memory: runs share the layout.)
 //   local  bin-grouped in row order (lp: bin boundaries), summed by the
 //          gather pass with x read from the bin's own slice, in groups of
 //          kPbLocalGroup entries: each group has a base row (lbase, offset in
@@ -170,8 +171,6 @@ struct PbMatrix {
   // both and these stay empty.
   int nsb_w = 0;
   DevBuf sp_w, fkey_w, rp_w, rdelta_w, cbase_w, cp_w;
-  DevBuf prod;              // 8-byte product slots, n_far + kPbChunk (spare slots that
-                            // the scatter's lanes past a superblock's end write)
   // CSR entry of each far entry (narrow and wide scatter order) and of each
   // local slot (-1: padding), int, on the device (the value builds read them)
   DevBuf far_src, far_src_w, loc_src;

@@ -1579,17 +1579,16 @@ struct SnPartials {
 };
 
 // One FP64 iteration on the blocked products (values VT; dev::Pattern: value-
-// free, cs the column values): scatter and gather.  sp == nullptr: the
-// reference-rule update, block maxima into the slots; else the sum-normalised
-// one with its partials.  pp: the partials of the iteration before, whose step
+// free, cs the column values): scatter and gather, through the run's product
+// slots prod.  sp == nullptr: the reference-rule update, block maxima into the
+// slots; else the sum-normalised one with its partials.  pp: the partials of the iteration before, whose step
 // decision the scatter takes (pp.n = 0: taken already).
 template <typename VT, int TM>
-void launch_pb_tm(const PbMatrix &pb, const double *cs, const double *x, const Teleport &tp, double *out, PrState *st,
-                  unsigned long long *slots, const SnPartials *sp, const Partials &pp, hipStream_t s) {
+void launch_pb_tm(const PbMatrix &pb, const double *cs, const double *x, double *prod, const Teleport &tp, double *out,
+                  PrState *st, unsigned long long *slots, const SnPartials *sp, const Partials &pp, hipStream_t s) {
   constexpr int slot = static_cast<int>(Dtype::F64);
   const VT *fval = pb_value_free<VT>() ? nullptr : pb.fval[slot].as<VT>();
   const VT *lval = pb_value_free<VT>() ? nullptr : pb.lval[slot].as<VT>();
-  double *prod = pb.prod.as<double>();
   launch_pb_scatter<VT>(pb, fval, cs, x, prod, st, pp, s);
   if (sp)
     hipLaunchKernelGGL((pb_gather_sn<VT, TM>), dim3(pb.nbins), dim3(1024), 0, s, pb_view(pb), lval, cs, x, prod, tp,
@@ -1599,16 +1598,17 @@ void launch_pb_tm(const PbMatrix &pb, const double *cs, const double *x, const T
                        st, slots);
 }
 
-void launch_pb(int tmode, const PbMatrix &pb, const double *cs, const double *x, const Teleport &tp, double *out,
-               PrState *st, unsigned long long *slots, const SnPartials *sp, const Partials &pp, hipStream_t s) {
+void launch_pb(int tmode, const PbMatrix &pb, const double *cs, const double *x, double *prod, const Teleport &tp,
+               double *out, PrState *st, unsigned long long *slots, const SnPartials *sp, const Partials &pp,
+               hipStream_t s) {
   const auto go = [&](auto tag) {
     using VT = decltype(tag);
     if (tmode == 1)
-      launch_pb_tm<VT, 1>(pb, cs, x, tp, out, st, slots, sp, pp, s);
+      launch_pb_tm<VT, 1>(pb, cs, x, prod, tp, out, st, slots, sp, pp, s);
     else if (tmode == 2)
-      launch_pb_tm<VT, 2>(pb, cs, x, tp, out, st, slots, sp, pp, s);
+      launch_pb_tm<VT, 2>(pb, cs, x, prod, tp, out, st, slots, sp, pp, s);
     else
-      launch_pb_tm<VT, 0>(pb, cs, x, tp, out, st, slots, sp, pp, s);
+      launch_pb_tm<VT, 0>(pb, cs, x, prod, tp, out, st, slots, sp, pp, s);
   };
   if (cs)
     go(dev::Pattern());
@@ -1620,6 +1620,7 @@ void launch_pb(int tmode, const PbMatrix &pb, const double *cs, const double *x,
 struct MxBufs {
   AnchorMove am;           // anchor xhat (and 1/count, value-free) with the scatter's sum partials
   const void *xd;          // the delta product's input: delta (F32/BF16) or zd (PATTERN_F32)
+  void *prod;              // the run's product slots
   float *w;                // FP32 one-step change of the anchor
   const float *dold;       // delta of the current iterate
   float *dnew, *zdnew;     // delta (and zd) of the next
@@ -1646,10 +1647,10 @@ void launch_pb_mx_tm(const PbMatrix &pb, int va, int vd, const MxBufs &b, const 
   constexpr bool awide = pb_anchor_wide<VA>();
   hipLaunchKernelGGL((pb_scatter_mx<VA, VD, XD, float, wide ? kPbColsWide : kPbCols>), pb_scatter_grid(pb),
                      dim3(kPbScatterThreads), awide ? 0 : kPbScatterLdsPad, s, awide ? pb_args_wide(pb) : pb_args(pb),
-                     wide ? pb_args_wide(pb) : pb_args(pb), fa, fd, xd, pb.prod.get(), b.am, st);
+                     wide ? pb_args_wide(pb) : pb_args(pb), fa, fd, xd, b.prod, b.am, st);
   hipLaunchKernelGGL((pb_gather_mx<VA, VD, XD, float, TM, PAT32>), dim3(pb.nbins), dim3(1024), 0, s, pb_view(pb), la,
-                     b.am.colscale, ld, xd, pb.prod.get(), tp, b.am.xhat, b.am.xhat32, b.w, b.dold, b.dnew, b.zdnew, b.colscale32, st,
-                     sp.perr, sp.ps, sp.pc);
+                     b.am.colscale, ld, xd, b.prod, tp, b.am.xhat, b.am.xhat32, b.w, b.dold, b.dnew, b.zdnew,
+                     b.colscale32, st, sp.perr, sp.ps, sp.pc);
 }
 
 template <typename VA, typename VD, typename XD, bool PAT32>
@@ -1719,7 +1720,7 @@ void launch_anchor(const DeviceMatrix &d, const double *x, double *yhat, const P
 
 struct Scratch {
   WsBuf st, slots, perr, ps, pc, member, nodes, hsum, hcomp;
-  WsBuf X0, X1, Z, yhat, xhat, xhat32, D0, D1, ZD0, ZD1, W, out, cs, flag;
+  WsBuf X0, X1, Z, yhat, xhat, xhat32, D0, D1, ZD0, ZD1, W, out, cs, flag, prod;
 };
 
 // One block: the step decision of a sum-normalised propagation-blocked
@@ -1894,6 +1895,10 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
     ws.alloc(w.X0, sizeof(double) * n);
     ws.alloc(w.X1, sizeof(double) * n);
   }
+  // blocked products: 8 bytes per far entry, and kPbChunk spare slots that the
+  // scatter's idle lanes write (the run's own: the layout is shared between
+  // the runs of a matrix)
+  if (pbm) ws.alloc(w.prod, sizeof(double) * (static_cast<std::size_t>(pbm->n_far) + kPbChunk));
   // teleport mode: 0 uniform, 1 node set (Matrix.cpp:63-114), 2 distribution vector
   const int tmode = p.teleport ? 2 : (p.personalized ? 1 : 0);
   Teleport tp{nullptr, p.teleport};
@@ -2109,6 +2114,7 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
           b.am = AnchorMove{w.xhat.as<double>(), w.xhat32.as<float>(), D[it & 1], colscale, w.hsum.as<double>(),
                             w.hcomp.as<double>(), 0};
           b.xd = vfree ? static_cast<const void *>(ZD[it & 1]) : static_cast<const void *>(D[it & 1]);
+          b.prod = w.prod.p;
           b.w = w.W.as<float>();
           b.dold = D[it & 1];
           b.dnew = D[(it + 1) & 1];
@@ -2121,7 +2127,7 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
           else
             launch_pb_mx<double, dev::bf16, float, false>(tmode, *pbm, 0, 2, b, tp, st, sp, s);
         } else {
-          launch_pb(tmode, *pbm, colscale, xin, tp, xout, st, nullptr, &sp, pp, s);
+          launch_pb(tmode, *pbm, colscale, xin, w.prod.as<double>(), tp, xout, st, nullptr, &sp, pp, s);
         }
         // (the anchor move's sum partials: one per superblock of the anchor
         // product's scatter order)
@@ -2157,7 +2163,7 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
             normalize(integral_constant<int, 1>(), xout, nullptr, dcur, dnext, nullptr, nullptr, it);
           decide(st);
         } else if (pbm) {
-          launch_pb(tmode, *pbm, colscale, xin, tp, xout, st, slot, nullptr, pp, s);
+          launch_pb(tmode, *pbm, colscale, xin, w.prod.as<double>(), tp, xout, st, slot, nullptr, pp, s);
           normalize(integral_constant<int, 4>(), xout, xin, nullptr, nullptr, nullptr, nullptr, it);
           if (k == batch - 1) decide(st);
         } else {
