@@ -204,10 +204,16 @@ __global__ __launch_bounds__(kTileThreads) void coo_tile_kernel(dev::CsrView<VT>
 
 // R consecutive rows per wavefront, so each x load serves all of them; per row
 // and lane the columns are summed in one order whatever R is (j = 2*lane +
-// 128*k), then a butterfly.  Bound by the HBM reads of A: two steps of R
-// 16-byte loads in flight, non-temporal, and with an odd row length every
-// other row starts 8 bytes off a 16-byte boundary, which the loads allow (8191
-// x 8191: 247 us with 8-byte loads, 83 now; 8192 x 8192 83 in both, 6.5 TB/s).
+// 128*k; short rows lane + 64*k), then a butterfly.  Bound by the HBM reads of
+// A: two steps of R 16-byte loads in flight, non-temporal, and with an odd row
+// length every other row starts 8 bytes off a 16-byte boundary, which the loads
+// allow (8191 x 8191: 247 us with 8-byte loads, 83 now; 8192 x 8192 83 in both,
+// 6.5 TB/s).
+// Rows of at most kDenseShortRow columns take a column a lane: two columns a
+// lane leave half the lanes of a short row idle (1,000,000 x 15 224.5 us, 173.7
+// so; x 16 216 and 172; x 63 260 and 198; 300,000 x 161 142 and 116; x 192 114.5
+// and 115.7; x 208 117 and 141).
+constexpr int kDenseShortRow = 192;
 template <typename XT, typename YT, int R>
 __global__ __launch_bounds__(256) void dense_kernel(const double *__restrict__ A, const XT *__restrict__ x,
                                                     YT *__restrict__ y, int rows, int cols, long ld) {
@@ -220,7 +226,14 @@ __global__ __launch_bounds__(256) void dense_kernel(const double *__restrict__ A
 #pragma unroll
   for (int r = 0; r < R; r++) acc[r] = 0;
   typedef double v2d_8 __attribute__((ext_vector_type(2), aligned(8)));
-  int j = 2 * lane;
+  if (cols <= kDenseShortRow) {
+#pragma unroll
+    for (int r = 0; r < R; r++)
+      if (r < nr)
+        for (int k = lane; k < cols; k += 64)
+          acc[r] += __builtin_nontemporal_load(A + (r0 + r) * ld + k) * static_cast<double>(x[k]);
+  }
+  int j = cols <= kDenseShortRow ? cols : 2 * lane;
   for (; j + 128 + 1 < cols; j += 2 * 128) {
     v2d_8 av[2][R];
     double xv[2][2];
