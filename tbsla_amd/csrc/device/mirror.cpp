@@ -533,6 +533,7 @@ std::unique_ptr<PbMatrix> pb_build_host(const cpp::MatrixCSR &c) {
   pb->bp.upload(bincnt.data(), bincnt.size() * sizeof(int));
   pb->lp.upload(loccnt.data(), loccnt.size() * sizeof(int));
   pb->lkey.upload(lkey.data(), lkey.size() * sizeof(unsigned short));
+  for (std::size_t k = 0; k + kPbLocalGroup <= lkey.size(); k += kPbLocalGroup) pb->loc_lines += pb_group_lines(&lkey[k]);
   pb->lbase.upload(lbase.data(), lbase.size() * sizeof(unsigned short));
   pb->far_src.upload(far_src_h.data(), far_src_h.size() * sizeof(int));
   pb->far_src_w.upload(far_src_w_h.data(), far_src_w_h.size() * sizeof(int));
@@ -543,7 +544,8 @@ std::unique_ptr<PbMatrix> pb_build_host(const cpp::MatrixCSR &c) {
 
 std::string pb_layout_compare(const PbMatrix &a, const PbMatrix &b) {
   if (a.n != b.n || a.nbins != b.nbins || a.nsb != b.nsb || a.nsb_w != b.nsb_w || a.rows != b.rows ||
-      a.cols != b.cols || a.cols_w != b.cols_w || a.n_far != b.n_far || a.n_loc != b.n_loc)
+      a.cols != b.cols || a.cols_w != b.cols_w || a.n_far != b.n_far || a.n_loc != b.n_loc ||
+      a.loc_lines != b.loc_lines)
     return "sizes";
   const bool wide = a.cols_w != a.cols;  // (else there is no separate wide order)
   auto dl = [](const DevBuf &d, std::size_t bytes) {

@@ -140,6 +140,17 @@ inline int pb_width(int n, int cap) {
   return static_cast<int>(std::min<long>(cap, std::max<long>(kPbMinWidth, w)));
 }
 
+// Cache lines of x (16 doubles) that one local group's keys read in turn.
+__host__ __device__ inline int pb_group_lines(const unsigned short *key) {
+  int lines = 0, last = -1;
+  for (int u = 0; u < kPbLocalGroup && key[u] >> kPbShift != kPbLocalPad; u++) {
+    const int line = (key[u] & (kPbRows - 1)) >> 4;
+    lines += line != last;
+    last = line;
+  }
+  return lines;
+}
+
 struct PbMatrix {
   int n = 0, nbins = 0, nsb = 0;
   int rows = 0, cols = 0, cols_w = 0;  // rows per bin, columns per superblock (narrow and wide order)
@@ -154,6 +165,13 @@ struct PbMatrix {
     nsb_w = (n + cols_w - 1) / cols_w;
   }
   long n_far = 0, n_loc = 0;  // n_loc counts the padding entries too
+  long loc_lines = 0;         // sum of pb_group_lines over the local groups
+  // whether the gather of a value-free FP64 product stages the bin's slice of
+  // the scaled x in LDS (see pb_accumulate)
+  bool stage_local() const {
+    const bool scattered = 8 * loc_lines > 5 * n_loc;  // over 2.5 lines a group
+    return scattered ? 4 * n_loc > n_far : 3 * n_loc > 4 * n_far;
+  }
   // far entries in scatter order: fkey (16 bits) = column within the
   // superblock, | kPbRunStart on the first entry of a run. A run is the far
   // entries of one superblock that go to one bin; entry o of run r of

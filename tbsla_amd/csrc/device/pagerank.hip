@@ -1240,15 +1240,30 @@ struct PbPair<double> {
 // The row sums of one bin (blockIdx) into the FP64 LDS accumulator ybin
 // (v.rows <= kPbRows entries): the bin's far products and its local products, x read
 // from the bin's own slice, scaled by xsc (XCS: and by xcs[j], the column
-// values of a value-free FP64 product).  Ends with a barrier.
-template <typename VT, typename XT, typename AT, bool XCS = false>
+// values of a value-free FP64 product, where they are read or once per column
+// into zbin, in LDS).  Ends with a barrier.
+//
+// Local entries whose columns lie apart are bound by the lines that their loads
+// touch, and two arrays are twice the lines, and more than an L1: 2^22 nodes of
+// 12, columns within 4000 of the row's, 499 us an iteration with x and xcs read
+// per entry, 316 with stored values, 114 staged; within 16000 (a quarter of the
+// entries local) 351, 334 and 212.  zbin leaves a CU one workgroup instead of
+// two, which far entries feel (2^24 nodes of 8, half of them far and the others
+// beside each other: 530 us read, 541 staged; 40% far 489 and 483), and costs a
+// pass over the slice (300,007 nodes of 12, 15% local: 24.5 and 25.4).  Hence
+// PbMatrix::stage_local: scattered local entries are staged from a quarter of
+// the far ones on, the others where they are 4/3 of them.
+enum PbColumnValues { kNoColumnValues, kReadColumnValues, kStagedColumnValues };
+template <typename VT, typename XT, typename AT, PbColumnValues XCS = kNoColumnValues>
 __device__ inline void pb_accumulate(const PbView &v, const VT *__restrict__ lval, const XT *__restrict__ x,
                                      const AT *__restrict__ prod, double *ybin, XT xsc = XT(1),
-                                     const double *__restrict__ xcs = nullptr) {
+                                     const double *__restrict__ xcs = nullptr, double *zbin = nullptr) {
 #pragma clang fp contract(off)
   const int bin = blockIdx.x, tid = threadIdx.x;
   const int base = bin * v.rows;
   for (int i = tid; i < v.rows; i += 1024) ybin[i] = 0.0;
+  if constexpr (XCS == kStagedColumnValues)
+    for (int i = tid; i < min(v.rows, v.n - base); i += 1024) zbin[i] = xcs[base + i] * (x[base + i] * xsc);
   __syncthreads();
   const int f1 = v.bp[bin + 1], l1 = v.lp[bin + 1];
   // far products in pairs: one 4-byte load of two rows and one 8- or
@@ -1351,7 +1366,12 @@ __device__ inline void pb_accumulate(const PbView &v, const VT *__restrict__ lva
 #pragma unroll
       for (int u = 0; u < 4; u++) {
         const int j = base + c[g][u];
-        xv[g][u] = static_cast<AT>(XCS ? xcs[j] * (x[j] * xsc) : x[j] * xsc);
+        if constexpr (XCS == kStagedColumnValues)
+          xv[g][u] = zbin[c[g][u]];
+        else if constexpr (XCS == kReadColumnValues)
+          xv[g][u] = xcs[j] * (x[j] * xsc);
+        else
+          xv[g][u] = static_cast<AT>(x[j] * xsc);
       }
 #pragma unroll
     for (int g = 0; g < LU; g++) {
@@ -1373,9 +1393,14 @@ __device__ inline void pb_accumulate(const PbView &v, const VT *__restrict__ lva
   __syncthreads();
 }
 
+template <typename VT, bool STAGE>
+constexpr PbColumnValues pb_columns() {
+  return !pb_value_free<VT>() ? kNoColumnValues : STAGE ? kStagedColumnValues : kReadColumnValues;
+}
+
 // FP64 runs under the reference rule: b = beta*(A x) + t into out, block
 // max into the slots (normalised by a separate pass).
-template <typename VT, int TM>
+template <typename VT, int TM, bool STAGE>
 __global__ __launch_bounds__(1024) void pb_gather(PbView v, const VT *__restrict__ lval, const double *__restrict__ cs,
                                                   const double *__restrict__ x, const double *__restrict__ prod,
                                                   Teleport tp, double *__restrict__ out, PrState *st,
@@ -1384,7 +1409,8 @@ __global__ __launch_bounds__(1024) void pb_gather(PbView v, const VT *__restrict
   if (st->done) return;
   __shared__ double ybin[kPbRows];
   __shared__ double red[16];
-  pb_accumulate<VT, double, double, pb_value_free<VT>()>(v, lval, x, prod, ybin, st->xnext, cs);
+  __shared__ double zbin[STAGE ? kPbRows : 1];
+  pb_accumulate<VT, double, double, pb_columns<VT, STAGE>()>(v, lval, x, prod, ybin, st->xnext, cs, zbin);
   const int bin = blockIdx.x, tid = threadIdx.x;
   const int base = bin * v.rows;
   const int rows = min(v.rows, v.n - base);
@@ -1412,7 +1438,7 @@ __global__ __launch_bounds__(1024) void pb_gather(PbView v, const VT *__restrict
 // sum-normalised iterate does not depend on the scale, so the scale of the
 // last iterate serves), with sum|x' - x| and the compensated sum of x' as
 // per-bin partials.
-template <typename VT, int TM>
+template <typename VT, int TM, bool STAGE>
 __global__ __launch_bounds__(1024) void pb_gather_sn(PbView v, const VT *__restrict__ lval,
                                                      const double *__restrict__ colscale,
                                                      const double *__restrict__ x, const double *__restrict__ prod,
@@ -1423,7 +1449,8 @@ __global__ __launch_bounds__(1024) void pb_gather_sn(PbView v, const VT *__restr
   if (st->done) return;
   __shared__ double ybin[kPbRows];
   __shared__ double red[48];
-  pb_accumulate<VT, double, double, pb_value_free<VT>()>(v, lval, x, prod, ybin, 1.0, colscale);
+  __shared__ double zbin[STAGE ? kPbRows : 1];
+  pb_accumulate<VT, double, double, pb_columns<VT, STAGE>()>(v, lval, x, prod, ybin, 1.0, colscale, zbin);
   const int bin = blockIdx.x, tid = threadIdx.x;
   const int base = bin * v.rows;
   const int rows = min(v.rows, v.n - base);
@@ -1479,8 +1506,8 @@ __global__ __launch_bounds__(1024) void pb_gather_mx(PbView v, const VA *__restr
   __shared__ double red[48];
   const bool anchor = st->need_anchor != 0;
   if (anchor)
-    pb_accumulate<VA, double, double, pb_value_free<VA>()>(v, lvala, xhat, static_cast<const double *>(prod), ybin,
-                                                          1.0, acs);
+    pb_accumulate<VA, double, double, pb_columns<VA, false>()>(v, lvala, xhat, static_cast<const double *>(prod), ybin,
+                                                              1.0, acs);
   else
     pb_accumulate<VD, XD, AD>(v, lvald, xd, static_cast<const AD *>(prod), ybin);
   const int bin = blockIdx.x, tid = threadIdx.x;
@@ -1590,12 +1617,19 @@ void launch_pb_tm(const PbMatrix &pb, const double *cs, const double *x, double 
   const VT *fval = pb_value_free<VT>() ? nullptr : pb.fval[slot].as<VT>();
   const VT *lval = pb_value_free<VT>() ? nullptr : pb.lval[slot].as<VT>();
   launch_pb_scatter<VT>(pb, fval, cs, x, prod, st, pp, s);
-  if (sp)
-    hipLaunchKernelGGL((pb_gather_sn<VT, TM>), dim3(pb.nbins), dim3(1024), 0, s, pb_view(pb), lval, cs, x, prod, tp,
-                       out, st, sp->perr, sp->ps, sp->pc);
-  else
-    hipLaunchKernelGGL((pb_gather<VT, TM>), dim3(pb.nbins), dim3(1024), 0, s, pb_view(pb), lval, cs, x, prod, tp, out,
-                       st, slots);
+  const auto gather = [&](auto stage) {
+    constexpr bool STAGE = decltype(stage)::value;
+    if (sp)
+      hipLaunchKernelGGL((pb_gather_sn<VT, TM, STAGE>), dim3(pb.nbins), dim3(1024), 0, s, pb_view(pb), lval, cs, x,
+                         prod, tp, out, st, sp->perr, sp->ps, sp->pc);
+    else
+      hipLaunchKernelGGL((pb_gather<VT, TM, STAGE>), dim3(pb.nbins), dim3(1024), 0, s, pb_view(pb), lval, cs, x, prod,
+                         tp, out, st, slots);
+  };
+  if constexpr (pb_value_free<VT>()) {
+    if (pb.stage_local()) return gather(std::true_type());
+  }
+  gather(std::false_type());
 }
 
 void launch_pb(int tmode, const PbMatrix &pb, const double *cs, const double *x, double *prod, const Teleport &tp,

@@ -269,6 +269,18 @@ __global__ __launch_bounds__(kT) void pbb_local_place(const int *__restrict__ re
 __global__ __launch_bounds__(kT) void pbb_fill_u16(unsigned short *__restrict__ a, long n, unsigned short v) {
   for (long i = blockIdx.x * static_cast<long>(kT) + threadIdx.x; i < n; i += static_cast<long>(gridDim.x) * kT) a[i] = v;
 }
+// *out += the cache lines of x (16 doubles) that the local groups read, a line
+// again where the entry before in its group read another
+__global__ __launch_bounds__(kT) void pbb_local_lines(const unsigned short *__restrict__ lkey, long groups,
+                                                      unsigned long long *__restrict__ out) {
+  int lines = 0;
+  for (long g = blockIdx.x * static_cast<long>(kT) + threadIdx.x; g < groups; g += static_cast<long>(gridDim.x) * kT)
+    lines += pb_group_lines(lkey + g * kPbLocalGroup);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) lines += __shfl_xor(lines, off, 64);
+  if ((threadIdx.x & 63) == 0) atomicAdd(out, static_cast<unsigned long long>(lines));
+}
+
 __global__ __launch_bounds__(kT) void pbb_fill_i32(int *__restrict__ a, long n, int v) {
   for (long i = blockIdx.x * static_cast<long>(kT) + threadIdx.x; i < n; i += static_cast<long>(gridDim.x) * kT) a[i] = v;
 }
@@ -495,6 +507,13 @@ std::unique_ptr<PbMatrix> pb_build_gpu(const DeviceMatrix &d, int n) {
     hipLaunchKernelGGL(pbb_local_place, dim3(blocks_for(nloc)), dim3(kT), 0, s, rel.as<int>(), lrow.as<int>(),
                        lcol.as<int>(), le.as<int>(), pb->lp.as<int>(), nloc, rows, pb->lkey.as<unsigned short>(),
                        pb->lbase.as<unsigned short>(), pb->loc_src.as<int>());
+    DevBuf lines;
+    lines.alloc(sizeof(unsigned long long));
+    hipLaunchKernelGGL(pbb_local_lines, dim3(blocks_for(nl / kPbLocalGroup)), dim3(kT), 0, s,
+                       pb->lkey.as<unsigned short>(), nl / kPbLocalGroup, lines.as<unsigned long long>());
+    unsigned long long v = 0;
+    TBSLA_HIP_CHECK(hipMemcpy(&v, lines.get(), sizeof(v), hipMemcpyDeviceToHost));
+    pb->loc_lines = static_cast<long>(v);
   }
   TBSLA_HIP_CHECK(hipGetLastError());
   TBSLA_HIP_CHECK(hipDeviceSynchronize());
