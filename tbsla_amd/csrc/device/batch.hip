@@ -89,6 +89,7 @@ struct BatchDev {
   const SpmmGroup<VT> *g;     // n_groups descriptors (device memory)
   RhsState *rs;
   int n_rhs_total;
+  const int *n_active;        // sets not done yet
   unsigned long long *slots;  // kSlots per RHS, two sets (by parity)
   const int *q_items;
   const int *q_off;           // kQueues + 1 queue boundaries in q_items
@@ -366,11 +367,7 @@ void batch_step(BatchDev<VT, XT> d, int par) {
   using AT = typename dev::Val<VT>::A;
   __shared__ dev::CsrTileLds<AT, TN, 0> lds;
   __shared__ double red[kTileThreads];
-  {  // nothing left to do once every set is done (a replay may run on past it)
-    int active = 0;
-    for (int r = threadIdx.x; r < d.n_rhs_total; r += kTileThreads) active |= !d.rs[r].done;
-    if (!__syncthreads_or(active)) return;
-  }
+  if (*d.n_active == 0) return;  // (a replay may run on past the last set's end)
   d.slots += static_cast<long>(par) * kSlots * d.n_rhs_total;
   const XT *xa_in = par ? d.xa1 : d.xa0, *xb_in = par ? d.xb1 : d.xb0;
   XT *xa_out = par ? d.xa0 : d.xa1, *xb_out = par ? d.xb0 : d.xb1;
@@ -646,7 +643,8 @@ __global__ __launch_bounds__(kTileThreads) void batch_output(BatchDev<VT, XT> d,
 // One wavefront per RHS: merge its partials in a fixed order, then the step
 // decision (reference residual or sum-normalised bound) and the next teleport
 // term.
-__global__ __launch_bounds__(64) void batch_finalize_norm(RhsState *rs, const RhsInfo *__restrict__ info,
+__global__ __launch_bounds__(64) void batch_finalize_norm(RhsState *rs, int *n_active,
+                                                          const RhsInfo *__restrict__ info,
                                                           const PassPart *__restrict__ part, double eps,
                                                           double bound_target, int rule, int max_it) {
   const int r = blockIdx.x, l = threadIdx.x;
@@ -683,6 +681,7 @@ __global__ __launch_bounds__(64) void batch_finalize_norm(RhsState *rs, const Rh
   st.bound = e / S + fabs(st.sum_prev / S - 1.0);
   const bool converged = rule == 0 ? (e < eps) : (st.bound <= bound_target);
   st.done = (converged || st.it >= max_it) ? 1 : 0;
+  if (st.done) atomicSub(n_active, 1);
   st.tele = S * st.tele_scale;
 }
 
@@ -738,7 +737,7 @@ struct PageRankBatch::Impl {
   std::vector<int> user_to_dev;      // device RHS id of each user RHS
   std::vector<int> dev_rows;         // rows of each device RHS's graph
   std::vector<double> dev_nodes;     // |nodes| of each device RHS
-  DevBuf rs, slots, info, parts, items, out_off;
+  DevBuf rs, n_active, slots, info, parts, items, out_off;
   int n_items = 0;
   long n_parts = 0;
   // The work items of one step for one (tile size, SpMM rows per wavefront):
@@ -1126,6 +1125,7 @@ void PageRankBatch::Impl::build() {
   parts.alloc(sizeof(PassPart) * static_cast<std::size_t>(std::max(1L, np)));
   out_off.upload(dev_out.data(), dev_out.size() * sizeof(long));
   rs.alloc(sizeof(RhsState) * static_cast<std::size_t>(std::max(1, n_rhs_total)));
+  n_active.alloc(sizeof(int));
   slots.alloc(sizeof(unsigned long long) * 2 * kSlots * static_cast<std::size_t>(std::max(1, n_rhs_total)));
 
   // ---- work items and queues of every (tile size, SpMM rows) layout
@@ -1176,6 +1176,7 @@ BatchDev<VT, XT> PageRankBatch::Impl::dev_view(const BatchConfig &c, double beta
   d.g = w.group_desc.as<SpmmGroup<VT>>();
   d.rs = rs.as<RhsState>();
   d.n_rhs_total = n_rhs_total;
+  d.n_active = n_active.as<int>();
   d.slots = slots.as<unsigned long long>();
   d.q_items = w.q_items[xcd_map].as<int>();
   d.q_off = w.q_off_dev[xcd_map].as<int>();
@@ -1224,8 +1225,8 @@ void PageRankBatch::Impl::enqueue_rest(const BatchDev<VT, XT> &d, int par, const
   if (n_items)
     hipLaunchKernelGGL((batch_normalize<VT, XT>), dim3(n_items), dim3(kTileThreads), 0, s, d, items.as<PassItem>(),
                        parts.as<PassPart>(), par);
-  hipLaunchKernelGGL(batch_finalize_norm, dim3(n_rhs_total), dim3(64), 0, s, d.rs, info.as<RhsInfo>(),
-                     parts.as<PassPart>(), p.epsilon, p.epsilon * (1.0 - p.beta) / p.beta, static_cast<int>(p.rule),
+  hipLaunchKernelGGL(batch_finalize_norm, dim3(n_rhs_total), dim3(64), 0, s, d.rs, n_active.as<int>(),
+                     info.as<RhsInfo>(), parts.as<PassPart>(), p.epsilon, p.epsilon * (1.0 - p.beta) / p.beta, static_cast<int>(p.rule),
                      p.max_iteration);
 }
 
@@ -1248,6 +1249,8 @@ void PageRankBatch::Impl::init_state(const BatchParams &p, hipStream_t s) {
     if (a_rows) hipLaunchKernelGGL(batch_fill<float>, dim3(fill_grid(a_rows)), dim3(256), 0, s, xa[0].as<float>(), static_cast<long>(a_rows), 0.25f);
     if (xb_len) hipLaunchKernelGGL(batch_fill<float>, dim3(fill_grid(xb_len)), dim3(256), 0, s, xb[0].as<float>(), xb_len, 0.25f);
   }
+  hipLaunchKernelGGL(batch_fill<int>, dim3(1), dim3(256), 0, s, n_active.as<int>(), 1L,
+                     p.max_iteration <= 0 ? 0 : n_rhs_total);
   const long ns = 2L * kSlots * n_rhs_total;
   hipLaunchKernelGGL(batch_fill<unsigned long long>, dim3(fill_grid(ns)), dim3(256), 0, s, slots.as<unsigned long long>(), ns, 0ull);
   TBSLA_HIP_CHECK(hipGetLastError());
