@@ -44,6 +44,9 @@ constexpr int kBatchLongChunk = 1024;
 int spmm_chunk_rows(int rows) { return std::max(64, std::min(1024, (rows / 2048 + 63) / 64 * 64)); }
 constexpr int kMaxGroups = 64;
 constexpr int kQueues = 8;           // one per XCD
+// more pass items of single-set graphs than this (two rounds of what the chip
+// holds of the pass with SpMM code, four workgroups a CU) go in a launch of their own
+constexpr int kManySingleItems = 2048;
 
 int tile_index(int tile_nnz) { return tile_nnz == 1024 ? 0 : (tile_nnz == 3072 ? 2 : 1); }
 int rpw_index(int spmm_rows) { return spmm_rows == 32 ? 0 : (spmm_rows == 128 ? 2 : 1); }
@@ -427,7 +430,10 @@ void batch_step(BatchDev<VT, XT> d, int par) {
 // rows per lane loaded before any is used.  With one RHS per lane and one row
 // at a time the pass over 2^20 rows x 64 FP32 sets and 48 single graphs took
 // 296 us; 173 us now, 4.7 TB/s.
-template <typename VT, typename XT>
+// SPMM = false: single-set items only.  Items of few rows are bound by the
+// workgroups in flight, and the registers of the SpMM items (118 in FP32) halve
+// them: 16,384 graphs of 200 rows 33 us with them, 19 without.
+template <typename VT, typename XT, bool SPMM>
 __global__ __launch_bounds__(kTileThreads) void batch_normalize(BatchDev<VT, XT> d, const PassItem *__restrict__ items,
                                                                 PassPart *__restrict__ part, int par) {
 #pragma clang fp contract(off)
@@ -437,7 +443,7 @@ __global__ __launch_bounds__(kTileThreads) void batch_normalize(BatchDev<VT, XT>
   const long set = static_cast<long>(kSlots) * d.n_rhs_total;
   const unsigned long long *slots = d.slots + par * set;
   unsigned long long *next = d.slots + (1 - par) * set;
-  if (it.kind == 0) {
+  if (!SPMM || it.kind == 0) {
     const int g = it.id;
     const RhsState &st = d.rs[g];
     if (st.done) return;
@@ -738,7 +744,7 @@ struct PageRankBatch::Impl {
   std::vector<int> dev_rows;         // rows of each device RHS's graph
   std::vector<double> dev_nodes;     // |nodes| of each device RHS
   DevBuf rs, n_active, slots, info, parts, items, out_off;
-  int n_items = 0;
+  int n_items = 0, n_single_items = 0;
   long n_parts = 0;
   // The work items of one step for one (tile size, SpMM rows per wavefront):
   // the tiles, then the long rows, then each group's SpMM items; queued in
@@ -1104,6 +1110,7 @@ void PageRankBatch::Impl::build() {
       }
       base += rows;
     }
+    n_single_items = static_cast<int>(it.size());
     for (std::size_t s = 0; s < groups.size(); s++) {
       const Group &gr = *groups[s];
       const int rows = sgraphs[static_cast<std::size_t>(gr.sgraph)]->rows;
@@ -1222,9 +1229,14 @@ void PageRankBatch::Impl::enqueue_iteration(const BatchDev<VT, XT> &d, int par, 
 template <typename VT, typename XT>
 void PageRankBatch::Impl::enqueue_rest(const BatchDev<VT, XT> &d, int par, const BatchParams &p,
                                        hipStream_t s) const {
-  if (n_items)
-    hipLaunchKernelGGL((batch_normalize<VT, XT>), dim3(n_items), dim3(kTileThreads), 0, s, d, items.as<PassItem>(),
-                       parts.as<PassPart>(), par);
+  // (the single-set graphs' items are the first)
+  const int alone = groups.empty() || n_single_items > kManySingleItems ? n_single_items : 0;
+  if (alone)
+    hipLaunchKernelGGL((batch_normalize<VT, XT, false>), dim3(alone), dim3(kTileThreads), 0, s, d,
+                       items.as<PassItem>(), parts.as<PassPart>(), par);
+  if (n_items > alone)
+    hipLaunchKernelGGL((batch_normalize<VT, XT, true>), dim3(n_items - alone), dim3(kTileThreads), 0, s, d,
+                       items.as<PassItem>() + alone, parts.as<PassPart>(), par);
   hipLaunchKernelGGL(batch_finalize_norm, dim3(n_rhs_total), dim3(64), 0, s, d.rs, n_active.as<int>(),
                      info.as<RhsInfo>(), parts.as<PassPart>(), p.epsilon, p.epsilon * (1.0 - p.beta) / p.beta, static_cast<int>(p.rule),
                      p.max_iteration);
