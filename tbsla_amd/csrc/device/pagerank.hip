@@ -760,26 +760,40 @@ __global__ __launch_bounds__(kTileThreads) void pr_anchor_spmv(dev::CsrView<VT> 
     dev::csr_tile_rows<VT, double, TN>(m, x, lds, epi);
 }
 
-// Mixed runs on the tile products: the state's sum becomes the compensated
-// sum of the anchor plus the FP32 delta (one block; once per run).
+// Mixed runs on the tile products, once per run: the state's sum becomes the
+// compensated sum of the anchor plus the FP32 delta, from one partial per block
+// (2^24 nodes: 3.8 ms in one workgroup, 39 us so).
 __global__ __launch_bounds__(1024) void pr_sum_rounded(const double *__restrict__ a, const float *__restrict__ d,
-                                                       long n, PrState *st) {
+                                                       long n, double *__restrict__ ps, double *__restrict__ pc) {
 #pragma clang fp contract(off)
   __shared__ double red[48];
+  const long stride = static_cast<long>(gridDim.x) * 1024;
   CSum cs{0, 0}, t;
-  for (long i0 = threadIdx.x; i0 < n; i0 += 8 * 1024) {
+  for (long i0 = blockIdx.x * 1024L + threadIdx.x; i0 < n; i0 += 8 * stride) {
     double v[8];
 #pragma unroll
     for (int u = 0; u < 8; u++) {
-      const long i = min(i0 + u * 1024, n - 1);
+      const long i = min(i0 + u * stride, n - 1);
       v[u] = a[i] + static_cast<double>(d[i]);
     }
 #pragma unroll
     for (int u = 0; u < 8; u++)
-      if (i0 + u * 1024 < n) csum_add(cs, v[u]);
+      if (i0 + u * stride < n) csum_add(cs, v[u]);
   }
   double unused;
   block1024_err_csum(0.0, cs, red, unused, t);
+  if (threadIdx.x == 0) {
+    ps[blockIdx.x] = t.s;
+    pc[blockIdx.x] = t.c;
+  }
+}
+__global__ __launch_bounds__(kTileThreads) void pr_sum_merge(const double *__restrict__ ps,
+                                                             const double *__restrict__ pc, int nb, PrState *st) {
+  __shared__ double red_s[kTileThreads], red_c[kTileThreads];
+  double unused = 0;
+  CSum t{0, 0};
+  sum_partials(nullptr, ps, pc, nb, unused, t);
+  t = block_csum(t, red_s, red_c);
   if (threadIdx.x == 0) st->sum = t.s + t.c;
 }
 
@@ -2280,8 +2294,10 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
   // final sum normalisation (Matrix.cpp:52-59), compensated
   const double *a = mixed ? w.xhat.as<double>() : X[it & 1];
   const float *dd = mixed ? D[it & 1] : nullptr;
-  if (mixed && !sn)  // the state's sum is that of the FP64 update; the result's elements are rounded
-    hipLaunchKernelGGL(pr_sum_rounded, dim3(1), dim3(1024), 0, s, a, dd, n, st);
+  if (mixed && !sn) {  // the state's sum is that of the FP64 update; the result's elements are rounded
+    hipLaunchKernelGGL(pr_sum_rounded, dim3(gM), dim3(1024), 0, s, a, dd, n, sp.ps, sp.pc);
+    hipLaunchKernelGGL(pr_sum_merge, dim3(1), dim3(kTileThreads), 0, s, sp.ps, sp.pc, static_cast<int>(gM), st);
+  }
   if (!one_block)  // (which wrote the result)
     hipLaunchKernelGGL(pr_scale_kernel, dim3(gN), dim3(256), 0, s, a, dd, n, state(launched), out_dev);
   TBSLA_HIP_CHECK(hipGetLastError());
