@@ -96,6 +96,17 @@ int tile_size(long nnz, const int *rowptr, int rows) {
   return nnz <= (1L << 20) ? 1024 : 2048;
 }
 
+int one_block_chain(const int *rowptr, int rows) {
+  if (rows > kOneBlockRows) return 0;
+  int waves[16] = {};
+  for (int r0 = 0; r0 < rows; r0 += 64) {
+    int most = 0;
+    for (int r = r0; r < std::min(rows, r0 + 64); r++) most = std::max(most, (rowptr[r + 1] - rowptr[r] + 7) / 8);
+    waves[r0 / 64 % 16] += most;
+  }
+  return *std::max_element(waves, waves + 16);
+}
+
 [[noreturn]] void bad(const char *what) { throw std::invalid_argument(std::string("tbsla: ") + what); }
 
 void build_csr(DeviceMatrix &d, const cpp::MatrixCSR &m, Dtype vdt) {
@@ -126,6 +137,7 @@ void build_csr(DeviceMatrix &d, const cpp::MatrixCSR &m, Dtype vdt) {
   pack_columns(d, vdt == Dtype::F64);
   upload_values(d.vals, vals.data(), static_cast<std::size_t>(used), vdt);
   d.tile_nnz = tile_size(used, rp.data(), d.rows);
+  d.one_block_chain = one_block_chain(rp.data(), d.rows);
   std::vector<int> t = csr_entry_tiles(rp.data(), d.rows, d.tile_nnz);
   d.ntiles = static_cast<int>(t.size()) - 1;
   d.tiles.upload(t.data(), t.size() * sizeof(int));

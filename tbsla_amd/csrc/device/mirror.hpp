@@ -44,6 +44,8 @@ constexpr int kCsrTileNnz = kTileThreads * kTilePer;  // entries staged in LDS p
 constexpr int kCsrLongRow = kCsrTileNnz / 2;          // longer rows: one workgroup each
 constexpr int kEllSlice = 128;  // ELL rows per slice (one row per thread, one workgroup per slice)
 
+constexpr int kOneBlockRows = 5632;  // rows of a PageRank graph that one workgroup runs (pr_one_block)
+
 struct DeviceMatrix {
   cpp::Format format = cpp::FORMAT_CSR;
   Dtype vdt = Dtype::F64;
@@ -60,6 +62,10 @@ struct DeviceMatrix {
   DevBuf col24, col24_pairs;
   int ntiles = 0, nlong = 0, rp0 = 0;
   int tile_nnz = kCsrTileNnz;  // entries per tile of the table in `tiles`
+  // CSR of at most kOneBlockRows rows: the most eight-entry loads that a
+  // wavefront of one 1024-thread workgroup, a row per thread, makes in turn
+  // (in each round of 1024 rows those of its longest row)
+  int one_block_chain = 0;
   // ELL (sliced column-major)
   int K = 0;
   // ecols with epacked: slots in groups of four, the columns of slots j..j+3 of

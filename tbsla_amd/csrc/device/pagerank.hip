@@ -606,7 +606,14 @@ __global__ __launch_bounds__(256) void pr_anchor_move(double *__restrict__ xhat,
 // of 16 12.4 -> 8.1.  With stored values (three times the bytes, and most of
 // each line another lane's) 2,500 of 8 took 6.2 and 5,003 9.5, 3,000 of 16
 // 16.3: the lines kOneBlockEntries* draw.
-constexpr int kOneBlockRows = 5632;  // 28 bytes a row: 154 KB of LDS
+// A long row is one thread's, a load of a chunk after the other, 0.2 us each:
+// past kOneBlockChain of them (DeviceMatrix::one_block_chain) in a wavefront the
+// tiles are sooner.  4,000 nodes of 4 (us an iteration, value-free, here and
+// tiles): one row of 400 (53 loads) 14.0 and 19.0, one of 800 (103) 22.9 and
+// 21.7, one of 1500 39.6 and 26.3, 40 rows of 100 (52) 16.4 and 13.6, 40 of 200
+// (100) 30.9 and 14.0; with stored values 12 rows of 400 (102) 35.3 and 22.3.
+static_assert(kOneBlockRows * 28 <= 158 << 10, "28 bytes of LDS a row");
+constexpr int kOneBlockChain = 64;
 constexpr long kOneBlockEntries = 65536;       // value-free
 constexpr long kOneBlockEntriesVal = 24576;    // with stored values
 constexpr int kOneBlockLenBits = 11;
@@ -1896,11 +1903,11 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
   // products, whose sums are the reference's)
   const bool use_pb = fused && !p.values && (p.gather == 2 || (p.gather == 0 && n >= (1L << 16)));
   const PbMatrix *pbm = nullptr;
-  // small graphs with no long row: the whole run in one workgroup.  (The
+  // small graphs with few long rows: the whole run in one workgroup.  (The
   // stored values' padding is read, so explicit ones take the tiles; f_col is
   // 0 in a matrix of one block.)
   const bool small = fused && !use_pb && !mixed && !p.values && n <= kOneBlockRows && d64.nlong == 0 &&
-                     d64.f_col == 0 && p.max_iteration > 0;
+                     d64.one_block_chain <= kOneBlockChain && d64.f_col == 0 && p.max_iteration > 0;
   // Blocked products of a matrix whose stored entries agree within every
   // column (a link graph: 1/out-degree) read no values: the input is scaled
   // by the column's value once, which gives the same rounded products.  (On
