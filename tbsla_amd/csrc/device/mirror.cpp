@@ -134,7 +134,6 @@ void build_csr(DeviceMatrix &d, const cpp::MatrixCSR &m, Dtype vdt) {
   d.rowptr.upload(rp.data(), rp.size() * sizeof(int));
   // entry j of row i is values[rowptr[i] - rowptr[0] + k] (MatrixCSR.cpp:135)
   d.colidx.upload(ci.data(), static_cast<std::size_t>(used) * sizeof(int));
-  pack_columns(d, vdt == Dtype::F64);
   upload_values(d.vals, vals.data(), static_cast<std::size_t>(used), vdt);
   d.tile_nnz = tile_size(used, rp.data(), d.rows);
   d.one_block_chain = one_block_chain(rp.data(), d.rows);
@@ -146,6 +145,7 @@ void build_csr(DeviceMatrix &d, const cpp::MatrixCSR &m, Dtype vdt) {
     if (rp[static_cast<std::size_t>(i) + 1] - rp[static_cast<std::size_t>(i)] > kCsrLongRow) lr.push_back(i);
   d.nlong = static_cast<int>(lr.size());
   if (d.nlong) d.long_rows.upload(lr.data(), lr.size() * sizeof(int));
+  pack_columns(d, vdt == Dtype::F64);  // (after all that the mirror cannot do without)
 }
 
 void build_ell(DeviceMatrix &d, const cpp::MatrixELL &m, Dtype vdt) {
@@ -248,7 +248,6 @@ void build_coo_like(DeviceMatrix &d, const M &m, Dtype vdt, bool scoo) {
   d.rowptr.upload(segptr.data(), segptr.size() * sizeof(int));
   d.segrow.upload(segrow.data(), segrow.size() * sizeof(int));
   d.colidx.upload(pcol, n * sizeof(int));
-  pack_columns(d, vdt == Dtype::F64);
   upload_values(d.vals, pval, n, vdt);
   d.tile_nnz = tile_size(static_cast<long>(n), segptr.data(), d.nseg);
   std::vector<int> t = csr_entry_tiles(segptr.data(), d.nseg, d.tile_nnz);
@@ -259,6 +258,7 @@ void build_coo_like(DeviceMatrix &d, const M &m, Dtype vdt, bool scoo) {
     if (segptr[static_cast<std::size_t>(sidx) + 1] - segptr[static_cast<std::size_t>(sidx)] > kCsrLongRow) lr.push_back(sidx);
   d.nlong = static_cast<int>(lr.size());
   if (d.nlong) d.long_rows.upload(lr.data(), lr.size() * sizeof(int));
+  pack_columns(d, vdt == Dtype::F64);  // (after all that the mirror cannot do without)
 }
 
 void build_dense(DeviceMatrix &d, const cpp::MatrixDENSE &m, Dtype vdt) {
@@ -352,8 +352,6 @@ const DeviceMatrix &transpose_mirror(const cpp::Matrix &m) {
   d->x_need = rows;
   d->rowptr.upload(ptr.data(), ptr.size() * sizeof(int));
   d->colidx.upload(ridx.data(), ridx.size() * sizeof(int));
-  pack_columns(*d, false);
-  pack_columns(*d, true);  // (read with the run's FP32 or FP64 values)
   d->perm.upload(perm.data(), perm.size() * sizeof(int));
   d->tile_nnz = tile_size(used, ptr.data(), cols);
   std::vector<int> t = csr_entry_tiles(ptr.data(), cols, d->tile_nnz);
@@ -364,6 +362,8 @@ const DeviceMatrix &transpose_mirror(const cpp::Matrix &m) {
     if (ptr[static_cast<std::size_t>(j) + 1] - ptr[static_cast<std::size_t>(j)] > kCsrLongRow) lr.push_back(j);
   d->nlong = static_cast<int>(lr.size());
   if (d->nlong) d->long_rows.upload(lr.data(), lr.size() * sizeof(int));
+  pack_columns(*d, false);
+  pack_columns(*d, true);  // (read with the run's FP32 or FP64 values)
   TBSLA_HIP_CHECK(hipDeviceSynchronize());
   cache.transposed = std::move(d);
   return *cache.transposed;
