@@ -43,6 +43,10 @@ struct HipError : std::runtime_error {
                                            __FILE__ + ":" + std::to_string(__LINE__));               \
   } while (0)
 
+// Frees the device memory that is kept between runs (runspace.hpp); whether
+// there was any.
+bool drop_idle_memory();
+
 // Owning device allocation, padded to 256 bytes so vector loads that round
 // an index range up never leave the allocation.
 class DevBuf {
@@ -76,7 +80,16 @@ class DevBuf {
     if (bytes <= bytes_ && p_) return;
     release();
     std::size_t padded = ((bytes ? bytes : 1) + 255 + 256) & ~std::size_t(255);
-    TBSLA_HIP_CHECK(hipMalloc(&p_, padded));
+    hipError_t e = hipMalloc(&p_, padded);
+    if (e != hipSuccess) (void)hipGetLastError();  // (the caller's launches check it)
+    if (e == hipErrorOutOfMemory && drop_idle_memory()) {
+      e = hipMalloc(&p_, padded);
+      if (e != hipSuccess) (void)hipGetLastError();
+    }
+    if (e != hipSuccess) {
+      p_ = nullptr;
+      throw HipError(e, "hipMalloc of " + std::to_string(padded) + " bytes: " + hipGetErrorString(e));
+    }
     bytes_ = padded - 256;
   }
   // reserve for memory that can be done without: false if there is none

@@ -5,13 +5,14 @@
 // A run leases a RunSpace for itself alone and gives it back once its stream
 // has drained, so runs on other streams and threads never share one; a run
 // that fails does not give it back (the memory is freed instead).  At most
-// kIdleSpaces are kept per matrix, and they go when the matrix's device data
-// goes (destruction or a mutating call).
+// kIdleSpaces are kept per matrix and kIdleBytes over all matrices (the one
+// given back longest ago goes first), and they go when the matrix's device data
+// goes (destruction or a mutating call) or when an allocation of this library
+// finds no memory (drop_idle_memory, common.hpp).
 #pragma once
 
 #include <cstddef>
 #include <memory>
-#include <mutex>
 #include <vector>
 
 #include "common.hpp"
@@ -20,6 +21,9 @@ namespace tbsla {
 namespace hip {
 
 constexpr std::size_t kIdleSpaces = 2;  // a forward's and a backward's
+// 2^24 nodes of 8 edges take 0.8 GB a run, so graphs of up to 2^28 keep theirs;
+// 6% of the card's memory
+constexpr std::size_t kIdleBytes = std::size_t(16) << 30;
 constexpr std::size_t kReadBackBytes = 1024;
 
 struct RunSpace {
@@ -53,42 +57,16 @@ struct RunSpace {
   }
 };
 
-// The idle spaces of one matrix.
+// The run memory of one matrix.
 class RunSpaces {
  public:
+  RunSpaces() = default;
+  ~RunSpaces();
+  RunSpaces(const RunSpaces &) = delete;
+  RunSpaces &operator=(const RunSpaces &) = delete;
   // the smallest idle space of at least `bytes`, or a new one
-  std::unique_ptr<RunSpace> take(std::size_t bytes) {
-    std::unique_ptr<RunSpace> s;
-    {
-      std::lock_guard<std::mutex> g(mu_);
-      std::size_t best = idle_.size();
-      for (std::size_t k = 0; k < idle_.size(); k++)
-        if (idle_[k]->mem.bytes() >= bytes && (best == idle_.size() || idle_[k]->mem.bytes() < idle_[best]->mem.bytes()))
-          best = k;
-      if (best < idle_.size()) {
-        s = std::move(idle_[best]);
-        idle_.erase(idle_.begin() + static_cast<std::ptrdiff_t>(best));
-      }
-    }
-    if (!s) s.reset(new RunSpace());
-    s->mem.reserve(bytes);
-    return s;
-  }
-  void give(std::unique_ptr<RunSpace> s) {
-    std::unique_ptr<RunSpace> drop;  // (freed outside the lock)
-    std::lock_guard<std::mutex> g(mu_);
-    idle_.push_back(std::move(s));
-    if (idle_.size() <= kIdleSpaces) return;
-    std::size_t least = 0;
-    for (std::size_t k = 1; k < idle_.size(); k++)
-      if (idle_[k]->mem.bytes() < idle_[least]->mem.bytes()) least = k;
-    drop = std::move(idle_[least]);
-    idle_.erase(idle_.begin() + static_cast<std::ptrdiff_t>(least));
-  }
-
- private:
-  std::mutex mu_;
-  std::vector<std::unique_ptr<RunSpace>> idle_;
+  std::unique_ptr<RunSpace> take(std::size_t bytes);
+  void give(std::unique_ptr<RunSpace> s);
 };
 
 // One device buffer of a run: a slice of its memory.

@@ -1,7 +1,9 @@
-// Device memory under a small limit, on the CPU: the mirrors (mirror.cpp)
-// against HIP calls that only count bytes.
+// Device memory under a small limit, on the CPU: the mirrors (mirror.cpp) and
+// the run memory (runspace.hpp) against HIP calls that only count bytes.
 //   device_memory mirror  a matrix whose mirror fits without its packed columns
 //                         is mirrored, and packed where there is room
+//   device_memory spaces  memory kept between runs gives way to what is needed,
+//                         and is bounded over all matrices
 #include <hip/hip_runtime.h>
 
 #include <cstdio>
@@ -19,10 +21,11 @@
 
 static std::size_t g_limit = ~std::size_t(0), g_used = 0;
 static std::map<void *, std::size_t> g_live;
+static hipError_t g_last = hipSuccess;
 
 extern "C" {
 hipError_t hipMalloc(void **p, size_t n) {
-  if (n > g_limit || g_used > g_limit - n) return hipErrorOutOfMemory;
+  if (n > g_limit || g_used > g_limit - n) return g_last = hipErrorOutOfMemory;
   *p = std::malloc(n > (1u << 20) ? 1 : n);  // (large blocks are never touched)
   g_live[*p] = n;
   g_used += n;
@@ -62,7 +65,11 @@ hipError_t hipEventDestroy(hipEvent_t e) {
   std::free(e);
   return hipSuccess;
 }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError() {
+  const hipError_t e = g_last;
+  g_last = hipSuccess;
+  return e;
+}
 const char *hipGetErrorString(hipError_t) { return "error"; }
 }
 
@@ -139,7 +146,55 @@ static void mirrors() {
   CHECK(g_used == 0);
 }
 
+static void spaces() {
+  const std::size_t MB = 1 << 20;
+  {
+    hip::RunSpaces a, b;
+    g_limit = 100 * MB;
+    a.give(a.take(60 * MB));
+    CHECK(g_used > 60 * MB);       // kept
+    auto s = a.take(50 * MB);      // the idle one serves
+    CHECK(g_used < 61 * MB);
+    a.give(std::move(s));
+    s = a.take(80 * MB);           // too small: it gives way
+    CHECK(s && s->mem.bytes() >= 80 * MB);
+    a.give(std::move(s));
+    s = b.take(70 * MB);           // another matrix's gives way
+    CHECK(s && g_used < 71 * MB);
+    b.give(std::move(s));
+    hip::DevBuf buf;               // and so it does to any other buffer
+    buf.alloc(60 * MB);
+    CHECK(g_used < 61 * MB);
+    CHECK(throws([&] { (void)a.take(50 * MB); }));  // held memory does not
+    CHECK(hipGetLastError() == hipSuccess);        // and no failure is left for a later check
+    g_limit = ~std::size_t(0);
+    a.give(a.take(10 * MB));
+    a.give(a.take(20 * MB));
+  }
+  CHECK(g_used == 0);
+  {  // bounded over all matrices, the oldest goes first
+    std::vector<std::unique_ptr<hip::RunSpaces>> all;
+    const std::size_t some = hip::kIdleBytes / 16;
+    for (int k = 0; k < 40; k++) {
+      all.emplace_back(new hip::RunSpaces());
+      all.back()->give(all.back()->take(some));
+    }
+    CHECK(g_used <= hip::kIdleBytes + MB);
+    CHECK(g_used > hip::kIdleBytes - 2 * some);
+    const std::size_t before = g_used;
+    all.back()->give(all.back()->take(some));  // the youngest is there
+    CHECK(g_used == before);
+    all.front()->give(all.front()->take(some));  // the oldest is not, and takes another's place
+    CHECK(g_used == before);
+    hip::RunSpaces big;  // more than the bound is not kept, and the others stay
+    big.give(big.take(hip::kIdleBytes + MB));
+    CHECK(g_used == before);
+  }
+  CHECK(g_used == 0);
+}
+
 int main(int argc, char **argv) {
   if (argc > 1 && !std::strcmp(argv[1], "mirror")) mirrors();
+  if (argc > 1 && !std::strcmp(argv[1], "spaces")) spaces();
   return fails ? 1 : 0;
 }
