@@ -540,7 +540,7 @@ int tbsla_hip_mirror_info(tbsla_matrix *m, int value_dtype, long *out) {
     const std::size_t xe = d.vdt == hip::Dtype::F64 ? 8 : 4;
     std::size_t bytes = d.rowptr.bytes() + d.colidx.bytes() + d.vals.bytes() + d.tiles.bytes() + d.ecols.bytes() +
                         d.evals.bytes() + d.segrow.bytes() + d.long_rows.bytes() +
-                        d.dvals.bytes();
+                        d.dvals.bytes() + d.col24.bytes() + d.col24_pairs.bytes();
     const long v[8] = {d.rows, d.entries, d.x_need, d.y_lo, d.y_hi,
                        d.ntiles, static_cast<long>(bytes),
                        d.noop ? 0L : static_cast<long>(d.algorithmic_bytes(xe, xe))};
