@@ -528,6 +528,9 @@ std::unique_ptr<PbMatrix> pb_build_host(const cpp::MatrixCSR &c) {
       }
       chp[static_cast<std::size_t>(s2) + 1] = chp[static_cast<std::size_t>(s2)] + nck;
     }
+    pb->top_w = 0;  // (the last order built is the wide one, or the only one)
+    for (int s2 = 0; s2 < ns2; s2++)
+      pb->top_w = std::max(pb->top_w, spc[static_cast<std::size_t>(s2) + 1] - spc[static_cast<std::size_t>(s2)]);
     sp_d.upload(spc.data(), spc.size() * sizeof(int));
     fkey_d.upload(fkey.data(), fkey.size() * sizeof(unsigned short));
     rp_d.upload(runp.data(), runp.size() * sizeof(int));
@@ -557,7 +560,7 @@ std::unique_ptr<PbMatrix> pb_build_host(const cpp::MatrixCSR &c) {
 std::string pb_layout_compare(const PbMatrix &a, const PbMatrix &b) {
   if (a.n != b.n || a.nbins != b.nbins || a.nsb != b.nsb || a.nsb_w != b.nsb_w || a.rows != b.rows ||
       a.cols != b.cols || a.cols_w != b.cols_w || a.n_far != b.n_far || a.n_loc != b.n_loc ||
-      a.loc_lines != b.loc_lines)
+      a.loc_lines != b.loc_lines || a.top_w != b.top_w)
     return "sizes";
   const bool wide = a.cols_w != a.cols;  // (else there is no separate wide order)
   auto dl = [](const DevBuf &d, std::size_t bytes) {

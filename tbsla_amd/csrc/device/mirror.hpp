@@ -171,6 +171,15 @@ struct PbMatrix {
     nsb_w = (n + cols_w - 1) / cols_w;
   }
   long n_far = 0, n_loc = 0;  // n_loc counts the padding entries too
+  int top_w = 0;              // far entries of the wide order's largest superblock
+  // whether value-free products take the wide order.  A superblock is one
+  // workgroup's, so the scatter waits for one that holds more than a CU's share
+  // (1 / 256) of the entries, and the narrow order halves it.  20 iterations in
+  // ms, wide and narrow, FP64 and FP32 deltas, by the largest in shares: 2^22
+  // nodes of 12, 1.0 5.06 5.20 3.72 3.76, 1.3 5.39 5.40 3.93 3.97, 1.7 5.77 5.65
+  // 4.21 4.11, 3.6 7.96 6.56 6.01 4.83; 2^24 of 8, 0.25 16.2 16.2 11.7 12.5, 1.8
+  // 19.3 19.1 14.2 14.3, 3.4 22.2 20.4 16.3 15.2, 8.0 36.1 29.1 27.6 21.6.
+  bool wide_free() const { return 2L * kPbSlots * top_w <= 3 * n_far; }
   long loc_lines = 0;         // sum of pb_group_lines over the local groups
   // whether the gather of a value-free FP64 product stages the bin's slice of
   // the scaled x in LDS (see pb_accumulate)

@@ -1596,8 +1596,10 @@ PbScatterArgs pb_args_wide(const PbMatrix &pb) {
                        pb.cols_w,            pb.n_far};
 }
 
-dim3 pb_scatter_grid(const PbMatrix &pb) { return dim3((pb.nsb + 7) / 8 * 8); }
-dim3 pb_scatter_grid_wide(const PbMatrix &pb) { return dim3((pb.nsb_w + 7) / 8 * 8); }
+// The scatter order of value-free products.
+PbScatterArgs pb_args_free(const PbMatrix &pb) { return pb.wide_free() ? pb_args_wide(pb) : pb_args(pb); }
+
+dim3 pb_scatter_grid(int nsb) { return dim3((nsb + 7) / 8 * 8); }
 
 // Dynamic LDS added to the scatter launches whose static LDS (a 64 KB x
 // slice) would let two blocks share a CU: one scatter block per CU writes
@@ -1613,12 +1615,14 @@ constexpr unsigned kPbScatterLdsPad = 24 * 1024;
 template <typename VT>
 void launch_pb_scatter(const PbMatrix &pb, const VT *fval, const double *cs, const double *x, double *prod,
                        PrState *st, const Partials &pp, hipStream_t s) {
-  if constexpr (pb_value_free<VT>())
-    hipLaunchKernelGGL((pb_scatter<VT, kPbColsWide>), dim3(pb_scatter_grid_wide(pb).x + 1), dim3(kPbScatterThreads),
-                       0, s, pb_args_wide(pb), fval, cs, x, prod, st, pp);
-  else
-    hipLaunchKernelGGL((pb_scatter<VT, kPbCols>), dim3(pb_scatter_grid(pb).x + 1), dim3(kPbScatterThreads),
+  if constexpr (pb_value_free<VT>()) {
+    const PbScatterArgs a = pb_args_free(pb);
+    hipLaunchKernelGGL((pb_scatter<VT, kPbColsWide>), dim3(pb_scatter_grid(a.nsb).x + 1), dim3(kPbScatterThreads),
+                       0, s, a, fval, cs, x, prod, st, pp);
+  } else {
+    hipLaunchKernelGGL((pb_scatter<VT, kPbCols>), dim3(pb_scatter_grid(pb.nsb).x + 1), dim3(kPbScatterThreads),
                        kPbScatterLdsPad, s, pb_args(pb), fval, cs, x, prod, st, pp);
+  }
 }
 
 // The per-bin partials of a sum-normalised iteration.
@@ -1700,9 +1704,11 @@ void launch_pb_mx_tm(const PbMatrix &pb, int va, int vd, const MxBufs &b, const 
   // (a wide anchor's 128 KB slice leaves room for one block per CU without
   // the LDS pad)
   constexpr bool awide = pb_anchor_wide<VA>();
-  hipLaunchKernelGGL((pb_scatter_mx<VA, VD, XD, float, wide ? kPbColsWide : kPbCols>), pb_scatter_grid(pb),
-                     dim3(kPbScatterThreads), awide ? 0 : kPbScatterLdsPad, s, awide ? pb_args_wide(pb) : pb_args(pb),
-                     wide ? pb_args_wide(pb) : pb_args(pb), fa, fd, xd, b.prod, b.am, st);
+  const PbScatterArgs aa = awide ? pb_args_free(pb) : pb_args(pb);
+  const PbScatterArgs ad = pb_value_free<VD>() ? pb_args_free(pb) : wide ? pb_args_wide(pb) : pb_args(pb);
+  hipLaunchKernelGGL((pb_scatter_mx<VA, VD, XD, float, wide ? kPbColsWide : kPbCols>),
+                     pb_scatter_grid(std::max(aa.nsb, ad.nsb)), dim3(kPbScatterThreads),
+                     awide ? 0 : kPbScatterLdsPad, s, aa, ad, fa, fd, xd, b.prod, b.am, st);
   hipLaunchKernelGGL((pb_gather_mx<VA, VD, XD, float, TM, PAT32>), dim3(pb.nbins), dim3(1024), 0, s, pb_view(pb), la,
                      b.am.colscale, ld, xd, b.prod, tp, b.am.xhat, b.am.xhat32, b.w, b.dold, b.dnew, b.zdnew,
                      b.colscale32, st, sp.perr, sp.ps, sp.pc);
@@ -2186,7 +2192,7 @@ PageRankReport run_page_rank(const cpp::Matrix &m, const PageRankParams &p, doub
         }
         // (the anchor move's sum partials: one per superblock of the anchor
         // product's scatter order)
-        const int nsb_anchor = vfree ? pbm->nsb_w : pbm->nsb;
+        const int nsb_anchor = vfree ? pb_args_free(*pbm).nsb : pbm->nsb;
         if (mixed || k == batch - 1)
           hipLaunchKernelGGL(pr_finalize_sn, dim3(1), dim3(kTileThreads), 0, s, sp.perr, sp.ps, sp.pc, pbm->nbins,
                              mixed ? w.hsum.as<double>() : nullptr, mixed ? w.hcomp.as<double>() : nullptr,

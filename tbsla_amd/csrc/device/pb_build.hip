@@ -323,10 +323,11 @@ std::vector<T> download(const DevBuf &b, std::size_t n) {
 }
 
 // One scatter order (superblocks of `cols` columns) of the CSC-ordered far
-// entries: sp, fkey, rp, rdelta, cbase, cp and far_src.
-void scatter_order(int cols, int rows, int nb, long nf, const DevBuf &csc_col, const DevBuf &csc_e, const DevBuf &row_of,
-                   const DevBuf &slot_of, int ns, DevBuf &sp_d, DevBuf &fkey_d, DevBuf &rp_d, DevBuf &rdelta_d,
-                   DevBuf &cbase_d, DevBuf &cp_d, DevBuf &far_src_d, DevBuf &err) {
+// entries: sp, fkey, rp, rdelta, cbase, cp and far_src.  Returns the entries of
+// the largest superblock.
+int scatter_order(int cols, int rows, int nb, long nf, const DevBuf &csc_col, const DevBuf &csc_e, const DevBuf &row_of,
+                  const DevBuf &slot_of, int ns, DevBuf &sp_d, DevBuf &fkey_d, DevBuf &rp_d, DevBuf &rdelta_d,
+                  DevBuf &cbase_d, DevBuf &cp_d, DevBuf &far_src_d, DevBuf &err) {
   const hipStream_t s = nullptr;
   const int binbits = bits_for(nb - 1), sbbits = bits_for(ns - 1);
   DevBuf key, val, k2, v2, spb;
@@ -364,6 +365,9 @@ void scatter_order(int cols, int rows, int nb, long nf, const DevBuf &csc_col, c
     cp[static_cast<std::size_t>(b) + 1] =
         cp[static_cast<std::size_t>(b)] +
         (sp[static_cast<std::size_t>(b) + 1] - sp[static_cast<std::size_t>(b)] + kPbChunk - 1) / kPbChunk;
+  int top = 0;
+  for (int b = 0; b < ns; b++)
+    top = std::max(top, sp[static_cast<std::size_t>(b) + 1] - sp[static_cast<std::size_t>(b)]);
   sp_d.upload(sp.data(), sp.size() * sizeof(int));
   cp_d.upload(cp.data(), cp.size() * sizeof(int));
   std::vector<int> rp(static_cast<std::size_t>(ns) + 1, runs);
@@ -392,6 +396,7 @@ void scatter_order(int cols, int rows, int nb, long nf, const DevBuf &csc_col, c
   }
   TBSLA_HIP_CHECK(hipGetLastError());
   TBSLA_HIP_CHECK(hipDeviceSynchronize());
+  return top;
 }
 
 }  // namespace
@@ -469,11 +474,11 @@ std::unique_ptr<PbMatrix> pb_build_gpu(const DeviceMatrix &d, int n) {
   bkey.release();
   slot_list.release();
   // the two scatter orders (one where both have the same width)
-  scatter_order(pb->cols, rows, nb, nf, csc_col, csc_e, row_of, slot_of, pb->nsb, pb->sp, pb->fkey, pb->rp, pb->rdelta,
-                pb->cbase, pb->cp, pb->far_src, err);
+  pb->top_w = scatter_order(pb->cols, rows, nb, nf, csc_col, csc_e, row_of, slot_of, pb->nsb, pb->sp, pb->fkey, pb->rp,
+                            pb->rdelta, pb->cbase, pb->cp, pb->far_src, err);
   if (pb->cols_w != pb->cols)
-    scatter_order(pb->cols_w, rows, nb, nf, csc_col, csc_e, row_of, slot_of, pb->nsb_w, pb->sp_w, pb->fkey_w, pb->rp_w,
-                  pb->rdelta_w, pb->cbase_w, pb->cp_w, pb->far_src_w, err);
+    pb->top_w = scatter_order(pb->cols_w, rows, nb, nf, csc_col, csc_e, row_of, slot_of, pb->nsb_w, pb->sp_w,
+                              pb->fkey_w, pb->rp_w, pb->rdelta_w, pb->cbase_w, pb->cp_w, pb->far_src_w, err);
   if (read_int(err.as<int>() + 1)) bad("propagation-blocked layout: run slots are not consecutive");
   // local groups
   DevBuf lbeg, ngroups, rel;
