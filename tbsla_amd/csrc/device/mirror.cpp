@@ -79,22 +79,21 @@ MinMax minmax_offset(const int *a, std::size_t n, long off) {
   return out;
 }
 
-// Entries per tile.  A CU holds six workgroups with 3072-entry tiles (LDS) and
-// eight with smaller ones, so matrices that the caches hold run faster with
+// Entries per tile.  A CU holds five FP64 workgroups with 3072-entry tiles (LDS)
+// and eight with smaller ones, so matrices that the caches hold run faster with
 // 2048 (500,009 rows of 16: 25.8 -> 25.2 us; 1,000,003: 49.8 -> 46.5, FP32 32.3
 // -> 29.6; 1,500,003: 73.4 -> 72.4) and those that stream from HBM with 3072
 // (3,000,003: 158.5 -> 152.4; 700,001 of 37: 90.2 -> 86.7).  Up to a tile of
 // 1024 per workgroup slot's half, PageRank's updates are latency alone and
-// take the smallest (a row per thread, and the step decision merged in).  A
-// row that runs past its tile is finished by one thread from memory: with rows
-// over 256 entries the large tiles stay.
+// take the smallest (a row per thread, and the step decision merged in).  Rows
+// that run past a small tile are staged by their block (csr_tile_rows_at): the
+// large tiles are slower beside long rows too (200 rows of 600 among 20,000 of 8
+// 13.2 us and 10.0 with 1024, one of 257 among 1,000,003 50.4 and 46.8 in FP32
+// with 2048), but for a lone row near the longest (1500 among 20,000 FP32 11.5
+// and 13.6) and rows of all lengths beside longer ones (100,003 of 17, one of
+// 12,500, FP32 37 and 42).
 constexpr long kLargeTiles = 3L << 23;  // more entries than this: 3072
-int tile_size(long nnz, const int *rowptr, int rows) {
-  int longest = 0;
-  for (int i = 0; i < rows; i++) longest = std::max(longest, rowptr[i + 1] - rowptr[i]);
-  if (longest > 256 || nnz > kLargeTiles) return kCsrTileNnz;
-  return nnz <= (1L << 20) ? 1024 : 2048;
-}
+int tile_size(long nnz) { return nnz > kLargeTiles ? kCsrTileNnz : nnz <= (1L << 20) ? 1024 : 2048; }
 
 int one_block_chain(const int *rowptr, int rows) {
   if (rows > kOneBlockRows) return 0;
@@ -135,7 +134,7 @@ void build_csr(DeviceMatrix &d, const cpp::MatrixCSR &m, Dtype vdt) {
   // entry j of row i is values[rowptr[i] - rowptr[0] + k] (MatrixCSR.cpp:135)
   d.colidx.upload(ci.data(), static_cast<std::size_t>(used) * sizeof(int));
   upload_values(d.vals, vals.data(), static_cast<std::size_t>(used), vdt);
-  d.tile_nnz = tile_size(used, rp.data(), d.rows);
+  d.tile_nnz = tile_size(used);
   d.one_block_chain = one_block_chain(rp.data(), d.rows);
   std::vector<int> t = csr_entry_tiles(rp.data(), d.rows, d.tile_nnz);
   d.ntiles = static_cast<int>(t.size()) - 1;
@@ -249,7 +248,7 @@ void build_coo_like(DeviceMatrix &d, const M &m, Dtype vdt, bool scoo) {
   d.segrow.upload(segrow.data(), segrow.size() * sizeof(int));
   d.colidx.upload(pcol, n * sizeof(int));
   upload_values(d.vals, pval, n, vdt);
-  d.tile_nnz = tile_size(static_cast<long>(n), segptr.data(), d.nseg);
+  d.tile_nnz = tile_size(static_cast<long>(n));
   std::vector<int> t = csr_entry_tiles(segptr.data(), d.nseg, d.tile_nnz);
   d.ntiles = static_cast<int>(t.size()) - 1;
   d.tiles.upload(t.data(), t.size() * sizeof(int));
@@ -353,7 +352,7 @@ const DeviceMatrix &transpose_mirror(const cpp::Matrix &m) {
   d->rowptr.upload(ptr.data(), ptr.size() * sizeof(int));
   d->colidx.upload(ridx.data(), ridx.size() * sizeof(int));
   d->perm.upload(perm.data(), perm.size() * sizeof(int));
-  d->tile_nnz = tile_size(used, ptr.data(), cols);
+  d->tile_nnz = tile_size(used);
   std::vector<int> t = csr_entry_tiles(ptr.data(), cols, d->tile_nnz);
   d->ntiles = static_cast<int>(t.size()) - 1;
   d->tiles.upload(t.data(), t.size() * sizeof(int));

@@ -609,9 +609,10 @@ __global__ __launch_bounds__(256) void pr_anchor_move(double *__restrict__ xhat,
 // A long row is one thread's, a load of a chunk after the other, 0.2 us each:
 // past kOneBlockChain of them (DeviceMatrix::one_block_chain) in a wavefront the
 // tiles are sooner.  4,000 nodes of 4 (us an iteration, value-free, here and
-// tiles): one row of 400 (53 loads) 14.0 and 19.0, one of 800 (103) 22.9 and
-// 21.7, one of 1500 39.6 and 26.3, 40 rows of 100 (52) 16.4 and 13.6, 40 of 200
-// (100) 30.9 and 14.0; with stored values 12 rows of 400 (102) 35.3 and 22.3.
+// tiles): one row of 400 (53 loads) 13.7 and 14.8, 12 of 200 (52) 13.9 and 14.0,
+// 40 of 100 (52) 16.4 and 13.3, one of 800 (103) 23.5 and 17.6, one of 1500 39.4
+// and 24.0, 40 of 200 (100) 28.5 and 14.4; with stored values one of 400 15.6
+// and 14.9, 12 of 400 (102) 37.2 and 17.1.
 static_assert(kOneBlockRows * 28 <= 158 << 10, "28 bytes of LDS a row");
 constexpr int kOneBlockChain = 64;
 constexpr long kOneBlockEntries = 65536;       // value-free
