@@ -31,6 +31,7 @@ namespace hip {
 namespace {
 
 constexpr int kT = 256;
+static_assert(kT == kTileThreads, "block_tree_sum adds over kTileThreads");
 
 unsigned blocks_for(long n) { return static_cast<unsigned>(std::max<long>(1, std::min<long>(1L << 16, (n + kT - 1) / kT))); }
 
@@ -270,15 +271,16 @@ __global__ __launch_bounds__(kT) void pbb_fill_u16(unsigned short *__restrict__ 
   for (long i = blockIdx.x * static_cast<long>(kT) + threadIdx.x; i < n; i += static_cast<long>(gridDim.x) * kT) a[i] = v;
 }
 // *out += the cache lines of x (16 doubles) that the local groups read, a line
-// again where the entry before in its group read another
+// again where the entry before in its group read another (one atomic a block,
+// of at most 1024: 262,144 of them took 1.2 ms of a first call on 2^24 nodes)
 __global__ __launch_bounds__(kT) void pbb_local_lines(const unsigned short *__restrict__ lkey, long groups,
                                                       unsigned long long *__restrict__ out) {
   int lines = 0;
   for (long g = blockIdx.x * static_cast<long>(kT) + threadIdx.x; g < groups; g += static_cast<long>(gridDim.x) * kT)
     lines += pb_group_lines(lkey + g * kPbLocalGroup);
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) lines += __shfl_xor(lines, off, 64);
-  if ((threadIdx.x & 63) == 0) atomicAdd(out, static_cast<unsigned long long>(lines));
+  __shared__ int part[kT];
+  lines = dev::block_tree_sum<int>(lines, part);
+  if (threadIdx.x == 0) atomicAdd(out, static_cast<unsigned long long>(lines));
 }
 
 __global__ __launch_bounds__(kT) void pbb_fill_i32(int *__restrict__ a, long n, int v) {
@@ -512,12 +514,10 @@ std::unique_ptr<PbMatrix> pb_build_gpu(const DeviceMatrix &d, int n) {
     hipLaunchKernelGGL(pbb_local_place, dim3(blocks_for(nloc)), dim3(kT), 0, s, rel.as<int>(), lrow.as<int>(),
                        lcol.as<int>(), le.as<int>(), pb->lp.as<int>(), nloc, rows, pb->lkey.as<unsigned short>(),
                        pb->lbase.as<unsigned short>(), pb->loc_src.as<int>());
-    DevBuf lines;
-    lines.alloc(sizeof(unsigned long long));
-    hipLaunchKernelGGL(pbb_local_lines, dim3(blocks_for(nl / kPbLocalGroup)), dim3(kT), 0, s,
-                       pb->lkey.as<unsigned short>(), nl / kPbLocalGroup, lines.as<unsigned long long>());
-    unsigned long long v = 0;
-    TBSLA_HIP_CHECK(hipMemcpy(&v, lines.get(), sizeof(v), hipMemcpyDeviceToHost));
+    unsigned long long *const lines = err.as<unsigned long long>() + 1, v = 0;  // (ints 2 and 3)
+    hipLaunchKernelGGL(pbb_local_lines, dim3(std::min(1024u, blocks_for(nl / kPbLocalGroup))), dim3(kT), 0, s,
+                       pb->lkey.as<unsigned short>(), nl / kPbLocalGroup, lines);
+    TBSLA_HIP_CHECK(hipMemcpy(&v, lines, sizeof(v), hipMemcpyDeviceToHost));
     pb->loc_lines = static_cast<long>(v);
   }
   TBSLA_HIP_CHECK(hipGetLastError());
