@@ -511,9 +511,10 @@ def main():
         tg["pagerank_mixed_speedup_vs_fp64"] = mixed
         l1key = "l1_vs_oracle_pstar" if "l1_vs_oracle_pstar" in var[best] else "l1_vs_gpu_fp64_limit"
         tg["pagerank_mixed_best"] = {"variant": best, "speedup_vs_fp64": mixed[best], l1key: var[best][l1key]}
-        stored = {k: v for k, v in mixed.items() if k in ("f32", "bf16")}
-        bs = max(stored, key=stored.get)
-        tg["pagerank_stored_values_best"] = {"variant": bs, "speedup_vs_fp64": stored[bs], l1key: var[bs][l1key]}
+        # (the graph's columns hold one value each, so these read no stored values either)
+        plain = {k: v for k, v in mixed.items() if k in ("f32", "bf16")}
+        bs = max(plain, key=plain.get)
+        tg["pagerank_f32_bf16_best"] = {"variant": bs, "speedup_vs_fp64": plain[bs], l1key: var[bs][l1key]}
     out["targets"] = tg
 
     print(json.dumps(out), flush=True)

@@ -9,12 +9,14 @@
 // Device layout:
 //   single-RHS graphs  one block-diagonal CSR (graphs concatenated, columns
 //                      offset), entry tiles as in the single-graph product
-//                      but of 2048 entries; iterate vectors concatenated.
+//                      but of the tuned size, with 32-bit columns; iterate
+//                      vectors concatenated.
 //   multi-RHS graphs   one CSR per graph with up to 64 RHS; iterates stored
 //                      row-major n x 64 so a gathered row of X is 64
 //                      consecutive values (one coalesced load per wavefront).
 //
-// One iteration is three launches, captured in a hipGraph and replayed:
+// One iteration is three launches (four where many small graphs stand beside
+// multi-RHS ones), captured in a hipGraph and replayed:
 //   batch_step          persistent work-queue kernel over every tile of the
 //                       block-diagonal matrix and every 64-row block of the
 //                       multi-RHS graphs (SpMM: lane = RHS), fused with

@@ -1,15 +1,18 @@
 // Device mirror of one host matrix: the HBM layout the kernels read.
 //
 //   CSR   rowptr/colidx as stored, values in the requested type, plus the
-//         entry-tile table: tile t = entries [t*kCsrTileNnz, (t+1)*kCsrTileNnz)
-//         owns rows [tile_row[t], tile_row[t+1]) (the rows whose first entry
-//         lies in the tile), and the list of rows longer than kCsrLongRow.
+//         entry-tile table: tile t = entries [t*T, (t+1)*T), T = tile_nnz
+//         (1024, 2048 or 3072 by the entries), owns rows [tile_row[t],
+//         tile_row[t+1]) (the rows whose first entry lies in the tile), the
+//         list of rows longer than kCsrLongRow, and the columns a second time
+//         packed in three bytes where they fit and the memory is there.
 //   ELL   sliced column-major: slice b = rows [b*kEllSlice, (b+1)*kEllSlice)
 //         holds its K slots contiguously, slot j of row i at
 //         ((i / kEllSlice) * K + j) * kEllSlice + i % kEllSlice, so one
 //         workgroup streams one contiguous block.  Columns are stored local
 //         and clamped, max(col - f_col, 0) (MatrixELL.cpp:110); the slice's
-//         rows past the last hold column 0, value 0.
+//         rows past the last hold column 0, value 0.  Columns are packed in
+//         three bytes where that is less.
 //   COO / SCOO
 //         entries in a row-sorted view (a stable counting sort by row when the
 //         input is not already sorted), compressed to row segments: segment s
@@ -80,8 +83,6 @@ struct DeviceMatrix {
   // DENSE
   int dcols = 0;
   DevBuf dvals;
-  // count-stochastic CSR: 1/count of each local column
-  DevBuf colscale;
   // transposed CSR structure: CSR entry index of each transposed entry
   DevBuf perm;
   std::size_t algorithmic_bytes(std::size_t x_elem, std::size_t y_elem) const;

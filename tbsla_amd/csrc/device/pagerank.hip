@@ -1,6 +1,7 @@
 // PageRank iteration kernels and their host driver (see pagerank.hpp).
 //
-// One iteration of the CSR engine is two launches (three with long rows):
+// One iteration of the CSR engine on the entry tiles is two launches on
+// matrices of up to 2^20 entries (three with long rows):
 //   pr_update_csr     first the step decision of the iteration before (every
 //                     block merges that normalise pass's partials, at most
 //                     256, and takes the same decision; block 0 stores it),
@@ -13,7 +14,7 @@
 // The step decision updates the state: iteration count, convergence, the next
 // teleport term, and (mixed precision) whether to move the anchor.  A launch
 // of its own (pr_finalize_norm) takes it at the end of a launch batch, before
-// the host reads the state.
+// the host reads the state, and in every iteration on larger matrices.
 // Partial results cross workgroups only at kernel boundaries, so no kernel
 // needs a device-wide fence.
 // Every kernel returns at once when the state says the run has converged, so
@@ -937,12 +938,13 @@ bool column_values(const cpp::Matrix &m, const DeviceMatrix &d64, long n, hipStr
 
 // ---------------------------------------------------------------------------
 // Propagation-blocked product (layout in mirror.hpp, PbMatrix).
-//   pb_scatter  one workgroup per column superblock (8192 columns): the
+//   pb_scatter  one workgroup per column superblock (at most 8192 columns, in
+//               the wide order 16384; fewer on small graphs, pb_width): the
 //               superblock's slice of x is staged in LDS, then every far
 //               product v * x[c] is written to its slot in the bin-grouped
 //               product array; entries come in (bin, column) order, so
 //               consecutive threads write runs of consecutive slots.
-//   pb_gather   one 1024-thread workgroup per bin of 8192 rows: the bin's
+//   pb_gather   one 1024-thread workgroup per bin (at most 8192 rows): the bin's
 //               far products and local products (x from the bin's own slice)
 //               are added into LDS, then the row epilogue runs on the sums.
 // The LDS additions are atomic, so the summation order within a row is not

@@ -1,13 +1,14 @@
 // SpMV kernels for gfx950 (MI355X, CDNA4, 64-wide wavefronts).
 //
-// csr_tile_kernel   one workgroup per fixed 3072-entry tile.  Entries are
-//                   read with 16-byte loads (12 entries per thread),
-//                   multiplied by the gathered x, and staged in LDS; each row
-//                   that starts in the tile is then summed by one thread in
-//                   entry order.  With FP64 this reproduces the reference loop
-//                   MatrixCSR.cpp:133-139 bit for bit (product rounded, then a
-//                   left-to-right sum starting from 0).  Columns are read
-//                   packed in three bytes where they fit (pack_columns).
+// csr_tile_kernel   one workgroup per tile of 1024, 2048 or 3072 entries.
+//                   Entries are read with 16-byte loads (4, 8 or 12 entries
+//                   per thread), multiplied by the gathered x, and staged in
+//                   LDS; each row that starts in the tile is then summed by
+//                   one thread in entry order.  With FP64 this reproduces the
+//                   reference loop MatrixCSR.cpp:133-139 bit for bit (product
+//                   rounded, then a left-to-right sum starting from 0).
+//                   Columns are read packed in three bytes where they fit
+//                   (pack_columns).
 // csr_long_kernel   rows longer than 1536 entries, one workgroup each.
 // ell_kernel        one row per thread over the sliced column-major slots (one
 //                   contiguous block per workgroup), eight slots per step;

@@ -2,16 +2,15 @@
 // include only from .hip translation units).
 //
 // CSR products use fixed entry tiles: tile t holds entries [t*T, (t+1)*T)
-// (T = kCsrTileNnz, 3072, or the caller's TN) and owns the rows whose first
-// entry lies in it
-// (tile_row[t] .. tile_row[t+1]).  A tile's entries are read with 16-byte
-// loads (packed columns: 12 bytes) at an aligned offset that needs no
-// descriptor load, the products
-// v * x[c] are rounded and staged in LDS, and each owned row is summed by one
-// thread from 0, left to right; of a row that runs past the tile the rest is
-// staged too (kTileTail).  That reproduces the sequential FP64 row
-// sum of MatrixCSR.cpp:133-139 exactly.  Rows longer than T / 2 entries are
-// left to csr_long_row (one workgroup per row, fixed-order tree).
+// (T = the caller's TN, 1024 to kCsrTileNnz) and owns the rows whose first
+// entry lies in it (tile_row[t] .. tile_row[t+1]).  A tile's entries are read
+// with 16-byte loads (packed columns: 12 bytes) at an aligned offset that needs
+// no descriptor load, the products v * x[c] are rounded and staged in LDS, and
+// each owned row is summed by one thread from 0, left to right; of a row that
+// runs past the tile the rest is staged too (kTileTail).  That reproduces the
+// sequential FP64 row sum of MatrixCSR.cpp:133-139 exactly.  Rows longer than
+// kCsrLongRow entries (the batch: kBatchLongRow) are left to csr_long_row (one
+// workgroup per row, fixed-order tree).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -206,8 +205,7 @@ constexpr int kLongSum = 64;
 // 18.0, 300,007 of 12 13.0 -> 11.8, 62 million entries 146.2 -> 144.8).
 constexpr int kTileTail = kTileThreads;
 
-// TN: entries per tile (kCsrTileNnz unless a caller builds its own tile
-// table with another size); rows longer than TN / 2 go to csr_long_row.
+// TN: entries per tile of the caller's table.
 // Product i of the tile is at slot(i): a free slot after every 16, so that the
 // threads of a wavefront, each reading its own row, meet in few LDS banks (rows
 // of 16 doubles start in two of the 64 without it): 500,009 rows of 16 FP64
