@@ -14,7 +14,7 @@ def window_graph(tb, n, c, w, per_column=True):
     base = np.repeat(np.arange(n, dtype=np.int64), c)
     off = np.tile(np.arange(c), n) if w == 0 else rng.integers(-w, w + 1, base.size)
     col = np.sort(((base + off) % n).reshape(n, c), axis=1).ravel().astype(np.int32)
-    v = (1.0 / np.bincount(col, minlength=n))[col]
+    v = (1.0 / np.maximum(np.bincount(col, minlength=n), 1))[col]
     if not per_column:
         v = v * (0.5 + 0.5 * rng.random(v.size))
     return tb.MatrixCSR(n, n, v, (np.arange(n + 1) * c).astype(np.int32), col)
